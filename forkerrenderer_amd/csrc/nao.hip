@@ -1098,85 +1098,149 @@ static inline void fused34_tiles(int lW, int lH, int &tx, int &ty)
 
 // Weight gradient: dW[co][tap*CIN+ci] = sum_p dout[p][co] * in[p+off(tap)][ci]
 // and db[co] = sum_p dout[p][co], per workgroup over a 64 x WG_ROWS pixel
-// tile, written as partials [block][...] for a fixed-order reduction.  Tap
-// offsets are (dy, dx) * dil.  Two rows of pixels per stage: their output
+// tile, written as partials [block][dW, db] for a fixed-order reduction.  Tap
+// offsets are (dy, dx) * DIL.  Two rows of pixels per stage: their output
 // gradients, and the six input rows the three tap rows reach, each with a
-// dil-pixel halo left and right.
-template <int CIN>
+// DIL-pixel halo left and right; the next stage's loads are in flight while
+// a stage is multiplied.
+//
+// A GEMM with pixels as its K dimension, while memory and LDS hold a pixel's
+// channels together: both operands come out of LDS through the transposing
+// read (ds_read_b64_tr_b16: 16 lanes x 8 bytes, four pixels' 16 channels,
+// returned as one channel's four pixels per lane), two per 16x16x32 operand;
+// gathered two bytes at a time the kernel took 107 us a 32-channel layer (16
+// crops of 192 x 192), so 38 to 41 us.  Both operands take the same pixel order
+// (lane group q: pixels 4q..4q+3 and 16+4q..16+4q+3 of a 32-pixel step), so
+// the sums are over the same products.  The two 32-byte halves of a
+// 32-channel pixel swap places every four pixels: 16 consecutive pixels'
+// halves then cover all 64 banks evenly (two passes, the least 512 bytes
+// take).  db is the same product with a B operand of ones, on the wavefront
+// that has a column block less.
+template <int CIN, int DIL>
+struct WgradStage {
+    static constexpr int SR = 2;                        // pixel rows per stage
+    static constexpr int SW = 64 + 2 * DIL;             // staged row width
+    static constexpr int CPO = CH / 8, CPI = CIN / 8;   // 16-byte chunks per pixel
+    static constexpr int NO = SR * 64 * CPO / 256;
+    static constexpr int NI = (3 * SR * SW * CPI + 255) / 256;
+    uint4 o[NO], i[NI];
+};
+
+// Chunk c (16 bytes) of pixel p in a staged array of CC-channel pixels.
+template <int CC>
+__device__ __forceinline__ int wgrad_chunk(int p, int c)
+{
+    return CC == 32 ? p * 4 + (c ^ (((p >> 2) & 1) << 1)) : p * (CC / 8) + c;
+}
+
+template <int CIN, int DIL>
+__device__ __forceinline__ void wgrad_load(WgradStage<CIN, DIL> &st, const uint16_t *__restrict__ in,
+                                           const uint16_t *__restrict__ dout, size_t img, int xb, int y0, int W, int H)
+{
+    using S = WgradStage<CIN, DIL>;
+#pragma unroll
+    for (int k = 0; k < S::NO; ++k) {
+        const int e = threadIdx.x + 256 * k, pix = e / S::CPO, c = e % S::CPO;
+        const int yy = y0 + pix / 64, xx = xb + pix % 64;
+        st.o[k] = make_uint4(0, 0, 0, 0);
+        if (yy < H && xx < W) st.o[k] = *(const uint4 *)(dout + (img + (size_t)yy * W + xx) * CH + c * 8);
+    }
+    // stage row (dyi * SR + r) is image row y0 + r + (dyi - 1) * DIL, column
+    // c is image column xb - DIL + c
+#pragma unroll
+    for (int k = 0; k < S::NI; ++k) {
+        const int e = threadIdx.x + 256 * k, pix = e / S::CPI, c = e % S::CPI;
+        const int srow = pix / S::SW, col = pix % S::SW;
+        const int yy = y0 + srow % S::SR + (srow / S::SR - 1) * DIL, xx = xb - DIL + col;
+        st.i[k] = make_uint4(0, 0, 0, 0);
+        if (srow < 3 * S::SR && yy >= 0 && yy < H && xx >= 0 && xx < W)
+            st.i[k] = *(const uint4 *)(in + (img + (size_t)yy * W + xx) * CIN + c * 8);
+    }
+}
+
+// Operand of one 32-pixel step: channel block cb (16 channels) of pixels
+// p .. p + 31 of a staged array.
+template <int CC>
+__device__ __forceinline__ v8bf wgrad_operand(const uint4 *arr, int p, int cb)
+{
+    typedef __attribute__((address_space(3))) v4s lds_v4s;
+    const int lane = threadIdx.x & 63, lq = lane >> 4, li = lane & 15;
+    const int p0 = p + lq * 4 + (li >> 2), p1 = p0 + 16;
+    const int c = cb * 2 + ((li >> 1) & 1), half = li & 1;
+    const char *base = (const char *)arr;
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(base + wgrad_chunk<CC>(p0, c) * 16 + half * 8));
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(base + wgrad_chunk<CC>(p1, c) * 16 + half * 8));
+    typedef short v8s __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(v8bf, (v8s)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int CIN, int DIL>
 __global__ __launch_bounds__(256) void k_conv_wgrad(const uint16_t *__restrict__ in,
                                                     const uint16_t *__restrict__ dout,
-                                                    float *__restrict__ part_dw,
-                                                    float *__restrict__ part_db, int W, int H, int dil)
+                                                    float *__restrict__ part, int W, int H)
 {
+    using S = WgradStage<CIN, DIL>;
     constexpr int K = 9 * CIN, NB = K / 16;
-    constexpr int NBW = (NB + 3) / 4;  // n-blocks per wavefront
-    constexpr int SR = 2;              // pixel rows per stage
-    __shared__ uint16_t s_out[SR * 64 * CH];
-    __shared__ uint16_t s_in[3 * SR * (64 + 2 * kMaxDil) * CIN];
-    const int SW = 64 + 2 * dil;
+    constexpr int NBW = (NB + 3) / 4;  // column blocks per wavefront
+    constexpr int SR = S::SR, SW = S::SW;
+    __shared__ uint4 s_out[SR * 64 * S::CPO];
+    __shared__ uint4 s_in[3 * SR * SW * S::CPI];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, lq = lane >> 4;
     const int xb = blockIdx.x * 64, yb = blockIdx.y * WG_ROWS, n = blockIdx.z;
     const size_t img = (size_t)n * H * W;
-    v4f acc[2][NBW];
+    v4f acc[2][NBW], db[2];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < 2; ++mb) {
+        db[mb] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < NBW; ++j) acc[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    float dbacc = 0.f;
+    }
+    v8bf ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = (__bf16)1.f;
+    S st;
+    wgrad_load<CIN, DIL>(st, in, dout, img, xb, yb, W, H);
     for (int r0 = 0; r0 < WG_ROWS; r0 += SR) {
-        const int y0 = yb + r0;
-        // output gradients: SR rows x 64 px x 32 ch
-        for (int e = tid; e < SR * 64 * CH / 4; e += 256) {
-            const int pix = e / (CH / 4), c4 = e % (CH / 4);
-            const int yy = y0 + pix / 64, xx = xb + pix % 64;
-            uint64_t v = 0;
-            if (yy < H && xx < W) v = *(const uint64_t *)(dout + (img + (size_t)yy * W + xx) * CH + c4 * 4);
-            *(uint64_t *)(s_out + pix * CH + c4 * 4) = v;
+#pragma unroll
+        for (int k = 0; k < S::NO; ++k) {
+            const int e = tid + 256 * k;
+            s_out[wgrad_chunk<CH>(e / S::CPO, e % S::CPO)] = st.o[k];
         }
-        // inputs: stage row (dyi * SR + r) is image row y0 + r + (dyi - 1) * dil,
-        // column c is image column xb - dil + c
-        for (int e = tid; e < 3 * SR * SW * CIN / 4; e += 256) {
-            const int pix = e / (CIN / 4), c4 = e % (CIN / 4);
-            const int srow = pix / SW, col = pix % SW;
-            const int yy = y0 + srow % SR + (srow / SR - 1) * dil, xx = xb - dil + col;
-            uint64_t v = 0;
-            if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = *(const uint64_t *)(in + (img + (size_t)yy * W + xx) * CIN + c4 * 4);
-            *(uint64_t *)(s_in + pix * CIN + c4 * 4) = v;
+#pragma unroll
+        for (int k = 0; k < S::NI; ++k) {
+            const int e = tid + 256 * k;
+            if (e < 3 * SR * SW * S::CPI) s_in[wgrad_chunk<CIN>(e / S::CPI, e % S::CPI)] = st.i[k];
         }
         __syncthreads();
-        if (tid < CH)
-            for (int p = 0; p < SR * 64; ++p) dbacc += bf2f(s_out[p * CH + tid]);
-        // K dimension of this GEMM = SR * 64 pixels in steps of 16
-        for (int ps = 0; ps < SR * 4; ++ps) {
-            v4s a[2];
+        if (r0 + SR < WG_ROWS) wgrad_load<CIN, DIL>(st, in, dout, img, xb, yb + r0 + SR, W, H);
+        // K dimension of this GEMM = SR * 64 pixels in steps of 32
 #pragma unroll
-            for (int mb = 0; mb < 2; ++mb)
+        for (int ps = 0; ps < SR * 2; ++ps) {
+            const int pr = ps / 2, pc = (ps % 2) * 32;
+            v8bf a[2];
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    a[mb][j] = (short)s_out[(ps * 16 + lq * 4 + j) * CH + mb * 16 + lr];
+            for (int mb = 0; mb < 2; ++mb) a[mb] = wgrad_operand<CH>(s_out, ps * 32, mb);
 #pragma unroll
             for (int jb = 0; jb < NBW; ++jb) {
                 const int nb = wave + 4 * jb;
                 if (nb >= NB) break;
-                const int k = nb * 16 + lr, tap = k / CIN, ci = k % CIN;
+                const int tap = nb / (CIN / 16), cb = nb % (CIN / 16);
                 const int dyi = tap / 3, dxi = tap % 3;
-                v4s b;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int pix = ps * 16 + lq * 4 + j;
-                    const int pr = pix / 64, pc = pix % 64;
-                    b[j] = (short)s_in[((dyi * SR + pr) * SW + pc + dxi * dil) * CIN + ci];
-                }
+                const v8bf b = wgrad_operand<CIN>(s_in, (dyi * SR + pr) * SW + pc + dxi * DIL, cb);
 #pragma unroll
                 for (int mb = 0; mb < 2; ++mb)
-                    acc[mb][jb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mb], b, acc[mb][jb], 0, 0, 0);
+                    acc[mb][jb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mb], b, acc[mb][jb], 0, 0, 0);
+            }
+            if (wave == 3) {
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+                    db[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mb], ones, db[mb], 0, 0, 0);
             }
         }
         __syncthreads();
     }
     const size_t blk = ((size_t)n * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    float *pd = part_dw + blk * CH * K;
+    float *pd = part + blk * (CH * K + CH);
 #pragma unroll
     for (int jb = 0; jb < NBW; ++jb) {
         const int nb = wave + 4 * jb;
@@ -1186,25 +1250,73 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const uint16_t *__restrict__
 #pragma unroll
             for (int i = 0; i < 4; ++i) pd[(size_t)(mb * 16 + lq * 4 + i) * K + nb * 16 + lr] = acc[mb][jb][i];
     }
-    if (tid < CH) part_db[blk * CH + tid] = dbacc;
+    if (wave == 3 && lr == 0) {
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pd[CH * K + mb * 16 + lq * 4 + i] = db[mb][i];
+    }
 }
 
-// out[i] = sum over b of part[b*len + i], b ascending (fixed order).
-__global__ __launch_bounds__(256) void k_reduce_cols(const float *__restrict__ part, int nb, int len,
-                                                     float *__restrict__ out)
+template <int DIL>
+static void launch_wgrad(hipStream_t s, const uint16_t *in, const uint16_t *dout, float *part, int S, int N)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= len) return;
+    constexpr int CIN = DIL == layer_dil(0) ? C0 : CH;
+    hipLaunchKernelGGL((k_conv_wgrad<CIN, DIL>), dim3(S / 64, S / WG_ROWS, N), dim3(256), 0, s, in, dout, part, S, S);
+}
+
+// Sum over b of part[b*len + i], in a fixed order (bitwise reproducible): 64
+// columns to a workgroup, row b in group b mod kReduceGroups -- each group
+// one wavefront, whose loads run 8 rows ahead of its sum -- and the groups'
+// sums combined in ascending order.  Columns below split go to out, the
+// others to out2 from its start.  Bound by the read of the partials (21 MB a
+// layer at 16 crops of 192 x 192): one thread per column walked its 576 rows
+// one load at a time, 169 us a call on average; so split, 5.2 us.
+constexpr int kReduceGroups = 16;
+__global__ __launch_bounds__(64 * kReduceGroups) void k_reduce_cols(const float *__restrict__ part, int nb, int len,
+                                                                    float *__restrict__ out, int split,
+                                                                    float *__restrict__ out2)
+{
+    __shared__ float sum[kReduceGroups][64];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int i = blockIdx.x * 64 + lane;
     float s = 0.f;
-    for (int b = 0; b < nb; ++b) s += part[(size_t)b * len + i];
-    out[i] = s;
+    if (i < len) {
+        int b = grp;
+        for (; b + 7 * kReduceGroups < nb; b += 8 * kReduceGroups) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = part[(size_t)(b + e * kReduceGroups) * len + i];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s += v[e];
+        }
+        for (; b < nb; b += kReduceGroups) s += part[(size_t)b * len + i];
+    }
+    sum[grp][lane] = s;
+    __syncthreads();
+    if (grp == 0 && i < len) {
+        for (int g = 1; g < kReduceGroups; ++g) s += sum[g][lane];
+        if (i < split) out[i] = s;
+        else out2[i - split] = s;
+    }
 }
 
 // ---------------- head backward (training) ----------------
 
 // Loss = sum over covered pixels of (y - t)^2 / n_total.  Writes the data
-// gradient of a4 and per-block partials of [dW5 (32), db5, loss, |err|, count].
+// gradient of a4 and per-workgroup partials of [dW5 (32), db5, loss, |err|,
+// count].  Bound by HBM (64 B read and 64 B written per pixel): a thread
+// takes every kHeadWgs*256-th pixel and keeps the 36 sums in registers, so
+// they are reduced once per workgroup instead of once per 256 pixels through
+// 38 KB of LDS (118 us for 590 k pixels then, 28 us now).
 constexpr int HEAD_PART = CH + 4;
+constexpr int kHeadWgs = 512;
+static inline int head_workgroups(size_t px)
+{
+    const size_t b = (px + 255) / 256;
+    return (int)(b < (size_t)kHeadWgs ? b : (size_t)kHeadWgs);
+}
+
 __global__ __launch_bounds__(256) void k_head_bwd(const float *__restrict__ params,
                                                   const uint16_t *__restrict__ a4,
                                                   const float *__restrict__ target,
@@ -1212,37 +1324,60 @@ __global__ __launch_bounds__(256) void k_head_bwd(const float *__restrict__ para
                                                   uint16_t *__restrict__ da4,
                                                   float *__restrict__ part)
 {
-    __shared__ float red[256][HEAD_PART + 1];
-    const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
+    __shared__ float red[4][HEAD_PART];
     float loc[HEAD_PART];
+#pragma unroll
     for (int k = 0; k < HEAD_PART; ++k) loc[k] = 0.f;
-    if (p < n) {
-        const uint16_t *a = a4 + p * CH;
-        const float *w5 = params + OFF_W5;
+    const float *w5 = params + OFF_W5;
+    for (size_t p = (size_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (size_t)gridDim.x * 256) {
+        uint16_t a[CH], o[CH];
+        const uint4 *src = (const uint4 *)(a4 + p * CH);
+#pragma unroll
+        for (int q = 0; q < CH / 8; ++q) {
+            const uint4 v = src[q];
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                a[8 * q + 2 * e] = (uint16_t)(w[e] & 0xffffu);
+                a[8 * q + 2 * e + 1] = (uint16_t)(w[e] >> 16);
+            }
+        }
         const float z = head_z(w5, params[OFF_B5], a);
         const float y = 1.f / (1.f + expf(-z));
         const bool m = mask[p] != 0;
         const float diff = y - target[p];
         const float g = m ? 2.f * diff / (float)n : 0.f;
         const float dz = g * y * (1.f - y);
+#pragma unroll
         for (int c = 0; c < CH; ++c) {
             const float av = bf2f(a[c]);
-            da4[p * CH + c] = f2bf(av > 0.f ? dz * w5[c] : 0.f);
-            loc[c] = dz * av;
+            o[c] = f2bf(av > 0.f ? dz * w5[c] : 0.f);
+            loc[c] += dz * av;
         }
-        loc[CH] = dz;
-        loc[CH + 1] = m ? diff * diff : 0.f;
-        loc[CH + 2] = m ? fabsf(diff) : 0.f;
-        loc[CH + 3] = m ? 1.f : 0.f;
+        uint4 *dst = (uint4 *)(da4 + p * CH);
+#pragma unroll
+        for (int q = 0; q < CH / 8; ++q) {
+            uint32_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = (uint32_t)o[8 * q + 2 * e] | ((uint32_t)o[8 * q + 2 * e + 1] << 16);
+            dst[q] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        loc[CH] += dz;
+        loc[CH + 1] += m ? diff * diff : 0.f;
+        loc[CH + 2] += m ? fabsf(diff) : 0.f;
+        loc[CH + 3] += m ? 1.f : 0.f;
     }
-    for (int k = 0; k < HEAD_PART; ++k) red[threadIdx.x][k] = loc[k];
+#pragma unroll
+    for (int k = 0; k < HEAD_PART; ++k) {
+        float v = loc[k];
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = v;
+    }
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s)
-            for (int k = 0; k < HEAD_PART; ++k) red[threadIdx.x][k] += red[threadIdx.x + s][k];
-        __syncthreads();
-    }
-    if (threadIdx.x < HEAD_PART) part[(size_t)blockIdx.x * HEAD_PART + threadIdx.x] = red[0][threadIdx.x];
+    if (threadIdx.x < HEAD_PART)
+        part[(size_t)blockIdx.x * HEAD_PART + threadIdx.x] =
+            (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 // ---------------- weights, Adam ----------------
@@ -1308,7 +1443,7 @@ struct fgl_nao {
     uint16_t *d[4] = {nullptr, nullptr, nullptr, nullptr};
     float *target = nullptr, *y = nullptr;
     uint8_t *mask = nullptr;
-    float *part = nullptr, *part_db = nullptr, *head_part = nullptr, *head_red = nullptr;
+    float *part = nullptr, *head_part = nullptr, *head_red = nullptr;
     size_t part_cap = 0;
     // inference buffers (grow-only): network-grid inputs, activations,
     // coverage and AO; frame-pixel coverage
@@ -1464,11 +1599,9 @@ int fgl_nao_create(fgl_ctx *ctx, int batch, int crop, int scale, fgl_nao **out)
     rc |= nao_alloc((void **)&n->mask, px);
     const size_t nblk = (size_t)(crop / 64) * (crop / WG_ROWS) * batch;
     n->part_cap = nblk;
-    rc |= nao_alloc((void **)&n->part, nblk * CH * K2 * 4);
-    rc |= nao_alloc((void **)&n->part_db, nblk * CH * 4);
-    const size_t hb = (px + 255) / 256;
-    rc |= nao_alloc((void **)&n->head_part, hb * HEAD_PART * 4);
-    rc |= nao_alloc((void **)&n->head_red, HEAD_PART * 4);
+    rc |= nao_alloc((void **)&n->part, nblk * (CH * K2 + CH) * 4);
+    rc |= nao_alloc((void **)&n->head_part, (size_t)head_workgroups(px) * HEAD_PART * 4);
+    rc |= nao_alloc((void **)&n->head_red, 3 * 4);
     if (hipHostMalloc((void **)&n->h_stats, 64 * 4, hipHostMallocDefault) != hipSuccess) rc = FGL_ERR_NOMEM;
     if (rc != FGL_OK) {
         fgl_nao_destroy(n);   // frees what was allocated, leaves the context
@@ -1494,7 +1627,7 @@ void fgl_nao_destroy(fgl_nao *n)
     }
     (void)hipDeviceSynchronize();
     void *ps[] = {n->params, n->grads, n->m, n->v, n->w1, n->w234, n->wt234, n->feat, n->target, n->y,
-                  n->mask, n->part, n->part_db, n->head_part, n->head_red, n->ifeat, n->ia, n->ib,
+                  n->mask, n->part, n->head_part, n->head_red, n->ifeat, n->ia, n->ib,
                   n->imask, n->fmask, n->lao};
     for (void *p : ps)
         if (p) (void)hipFree(p);
@@ -1589,30 +1722,30 @@ static int run_batch(fgl_nao *n, bool update, float lr, float *stats)
     const size_t px = (size_t)N * S * S;
     forward_convs(n, s, n->feat, n->a, S, S, N);
     // head forward + loss + data gradient of a4
-    const int hb = (int)((px + 255) / 256);
+    const int hb = head_workgroups(px);
     hipLaunchKernelGGL(k_head_bwd, dim3(hb), dim3(256), 0, s, n->params, n->a[3], n->target, n->mask, px,
                        n->d[3], n->head_part);
-    hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, s, n->head_part, hb, HEAD_PART, n->head_red);
-    if (hipMemcpyAsync(n->grads + OFF_W5, n->head_red, CH * 4, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(n->grads + OFF_B5, n->head_red + CH, 4, hipMemcpyDeviceToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(n->h_stats, n->head_red + CH + 1, 3 * 4, hipMemcpyDeviceToHost, s) != hipSuccess)
-        return FGL_ERR_DEVICE;
+    // dW5 and db5 (adjacent in the parameters), then the statistics
+    static_assert(OFF_B5 == OFF_W5 + CH, "head layout");
+    hipLaunchKernelGGL(k_reduce_cols, dim3((HEAD_PART + 63) / 64), dim3(64 * kReduceGroups), 0, s, n->head_part, hb,
+                       HEAD_PART, n->grads + OFF_W5, CH + 1, n->head_red);
+    if (hipMemcpyAsync(n->h_stats, n->head_red, 3 * 4, hipMemcpyDeviceToHost, s) != hipSuccess) return FGL_ERR_DEVICE;
     // layers 4..1: weight gradient from (input, output gradient), then the
     // data gradient of the layer input (not needed for layer 1)
-    const dim3 wg(S / 64, S / WG_ROWS, N);
-    const int nblk = (int)(wg.x * wg.y * wg.z);
-    const int woffs[4] = {OFF_W1, OFF_W2, OFF_W3, OFF_W4}, boffs[4] = {OFF_B1, OFF_B2, OFF_B3, OFF_B4};
+    const int nblk = (S / 64) * (S / WG_ROWS) * N;
+    const int woffs[4] = {OFF_W1, OFF_W2, OFF_W3, OFF_W4};
+    static_assert(OFF_B1 == OFF_W1 + CH * K1 && OFF_B2 == OFF_W2 + CH * K2 && OFF_B3 == OFF_W3 + CH * K2 &&
+                  OFF_B4 == OFF_W4 + CH * K2, "a layer's biases follow its weights");
     for (int l = 3; l >= 0; --l) {
-        const int K = l == 0 ? K1 : K2;
-        if (l == 0)
-            hipLaunchKernelGGL((k_conv_wgrad<C0>), wg, dim3(256), 0, s, n->feat, n->d[0], n->part, n->part_db, S, S,
-                               layer_dil(0));
-        else
-            hipLaunchKernelGGL((k_conv_wgrad<CH>), wg, dim3(256), 0, s, n->a[l - 1], n->d[l], n->part, n->part_db, S, S,
-                               layer_dil(l));
-        hipLaunchKernelGGL(k_reduce_cols, dim3((CH * K + 255) / 256), dim3(256), 0, s, n->part, nblk, CH * K,
-                           n->grads + woffs[l]);
-        hipLaunchKernelGGL(k_reduce_cols, dim3(1), dim3(256), 0, s, n->part_db, nblk, CH, n->grads + boffs[l]);
+        const int len = CH * (l == 0 ? K1 : K2) + CH;
+        switch (l) {
+        case 0: launch_wgrad<layer_dil(0)>(s, n->feat, n->d[0], n->part, S, N); break;
+        case 1: launch_wgrad<layer_dil(1)>(s, n->a[0], n->d[1], n->part, S, N); break;
+        case 2: launch_wgrad<layer_dil(2)>(s, n->a[1], n->d[2], n->part, S, N); break;
+        default: launch_wgrad<layer_dil(3)>(s, n->a[2], n->d[3], n->part, S, N); break;
+        }
+        hipLaunchKernelGGL(k_reduce_cols, dim3((len + 63) / 64), dim3(64 * kReduceGroups), 0, s, n->part, nblk, len,
+                           n->grads + woffs[l], len, (float *)nullptr);
         if (l > 0)
             launch_conv<CH, 1>(s, n->d[l], n->wt234 + (size_t)(l - 1) * CH * K2, nullptr, n->a[l - 1], n->d[l - 1], S,
                                S, N, layer_dil(l));
