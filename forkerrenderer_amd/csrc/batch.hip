@@ -158,9 +158,13 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     const DevView &v = b.views[vi];
     ResolveArgs a;
     a.draws = b.draws;
+    a.n_draws = 0;
     a.screen = b.screen;
     a.tri_v = b.tri_v;
     a.vis = b.vis + v.px_off;
+    a.key = nullptr;
+    a.fix = nullptr;
+    a.depth = nullptr;
     a.W = v.W;
     a.H = v.H;
     a.fresh = 1;
@@ -171,7 +175,7 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     a.textures = b.textures;
     a.shadow_map = nullptr;
     a.ss = ShadowSamples{nullptr, nullptr, 0u};
-    gbuffer_px(a, v.u, x, y);
+    gbuffer_px<false>(a, v.u, x, y);
 }
 
 __global__ __launch_bounds__(256) void k_bv_lighting(BvPixelArgs b)

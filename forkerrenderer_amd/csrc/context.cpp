@@ -28,12 +28,20 @@ struct DevBuf {
     size_t cap = 0;
 };
 
+constexpr int kFewVertices = 256;
+
 struct ModelRes {
     float *pos = nullptr, *uv = nullptr, *nrm = nullptr, *tan = nullptr;
     int *vi = nullptr, *ti = nullptr, *ni = nullptr, *fmat = nullptr;
+    int4 *tri = nullptr;       // the faces in spatial order
     float *corner = nullptr;   // per face corner: pos, uv, nrm, tan (12 floats)
     int n_pos = 0, n_faces = 0;
     bool has_tan = false, pbr = false;
+    // extent of the faces' corners and the longest face edge; bounded: they
+    // are finite
+    double lo[3], hi[3], edge = 0.0;
+    bool bounded = false;
+    std::vector<float> few;    // the positions, of a model with at most kFewVertices
 };
 
 struct TimedKernel {
@@ -88,6 +96,10 @@ struct fgl_ctx {
     // pass scratch
     DevBuf d_draws, screen, rect, counts, offs, scan_tmp, keys, vals, keys_alt, vals_alt, sort_tmp,
         tile_start, tile_end, tri_v, big_list, counters, ndc_z;
+    // the direct rasteriser: pixel keys, NaN plane (all ones between passes),
+    // large-triangle items and two passes' counters used in turn
+    DevBuf key, key_nan, items;
+    int direct_turn = 0;
     // forward pass with a stochastic shadow filter: per-pixel passing counts
     // (+ scan scratch), the passing fragments (triangle ids then pixels) and
     // the sort's other copy, its scratch, their shadow inputs, and each
@@ -339,7 +351,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     for (auto &m : c->models) {
         (void)hipFree(m.pos); (void)hipFree(m.uv); (void)hipFree(m.nrm);
         if (m.tan) (void)hipFree(m.tan);
-        (void)hipFree(m.vi); (void)hipFree(m.ti); (void)hipFree(m.ni); (void)hipFree(m.fmat); (void)hipFree(m.corner);
+        (void)hipFree(m.vi); (void)hipFree(m.ti); (void)hipFree(m.ni); (void)hipFree(m.fmat); (void)hipFree(m.corner); (void)hipFree(m.tri);
     }
     DevBuf *bufs[] = {&c->d_textures, &c->d_materials, &c->depth, &c->fb, &c->gbuf, &c->ao,
                       &c->blur_tmp, &c->shadow, &c->shadow_depth, &c->img, &c->vis, &c->d_draws,
@@ -348,6 +360,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
                       &c->screen, &c->rect, &c->counts, &c->offs, &c->scan_tmp, &c->keys,
                       &c->vals, &c->keys_alt, &c->vals_alt, &c->sort_tmp, &c->tile_start,
                       &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z,
+                      &c->key, &c->key_nan, &c->items,
                       &c->frag_cnt, &c->frag_tri, &c->frag_alt, &c->frag_tmp, &c->frag_planes,
                       &c->frag_offs_px};
     for (DevBuf *b : bufs) free_buf(*b);
@@ -444,6 +457,65 @@ int fgl_upload_material(fgl_ctx *c, const fgl_material *m, int *out_id)
     return FGL_OK;
 }
 
+// The faces in the order of a Morton curve through their first corners (10
+// bits an axis of the model's extent; face order breaks ties), and each
+// position's place in the order of first use (unused positions last).
+static void spatial_order(const fgl_model_desc *d, std::vector<int32_t> &order, std::vector<int32_t> &rank)
+{
+    const size_t nf = (size_t)d->n_faces;
+    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    for (size_t f = 0; f < nf; ++f)
+        for (int j = 0; j < 3; ++j) {
+            const float x = d->pos[3 * (size_t)d->vi[3 * f] + j];
+            if (x < lo[j]) lo[j] = x;
+            if (x > hi[j]) hi[j] = x;
+        }
+    float scale[3];
+    for (int j = 0; j < 3; ++j) {
+        scale[j] = 1023.f / (hi[j] - lo[j]);
+        if (!std::isfinite(scale[j])) scale[j] = 0.f;
+    }
+    auto spread = [](uint32_t x) {
+        x = (x | x << 16) & 0x030000ffu;
+        x = (x | x << 8) & 0x0300f00fu;
+        x = (x | x << 4) & 0x030c30c3u;
+        return (x | x << 2) & 0x09249249u;
+    };
+    std::vector<uint32_t> key(nf), key2(nf);
+    std::vector<int32_t> tmp(nf);
+    order.resize(nf);
+    for (size_t f = 0; f < nf; ++f) {
+        uint32_t q[3];
+        for (int j = 0; j < 3; ++j) {
+            const float x = (d->pos[3 * (size_t)d->vi[3 * f] + j] - lo[j]) * scale[j];
+            q[j] = x >= 0.f && x <= 1023.f ? (uint32_t)x : 0u;   // also a NaN
+        }
+        key[f] = spread(q[0]) | spread(q[1]) << 1 | spread(q[2]) << 2;
+        order[f] = (int32_t)f;
+    }
+    for (int shift = 0; shift < 30; shift += 10) {   // stable counting sort, ten bits a pass
+        uint32_t at[1025] = {0};
+        for (size_t f = 0; f < nf; ++f) ++at[(key[f] >> shift & 1023u) + 1];
+        for (int k = 0; k < 1024; ++k) at[k + 1] += at[k];
+        for (size_t f = 0; f < nf; ++f) {
+            const uint32_t o = at[key[f] >> shift & 1023u]++;
+            key2[o] = key[f];
+            tmp[o] = order[f];
+        }
+        key.swap(key2);
+        order.swap(tmp);
+    }
+    rank.assign((size_t)d->n_pos, -1);
+    int32_t next = 0;
+    for (size_t k = 0; k < nf; ++k)
+        for (int j = 0; j < 3; ++j) {
+            int32_t &r = rank[d->vi[3 * (size_t)order[k] + j]];
+            if (r < 0) r = next++;
+        }
+    for (int32_t &r : rank)
+        if (r < 0) r = next++;
+}
+
 int fgl_upload_model(fgl_ctx *c, const fgl_model_desc *d, int *out_id)
 {
     if (!c || !d || !out_id) return FGL_ERR_INVALID;
@@ -460,26 +532,61 @@ int fgl_upload_model(fgl_ctx *c, const fgl_model_desc *d, int *out_id)
             return fail(c, FGL_ERR_INVALID, "face material out of range");
     ModelRes m;
     int rc;
-    if ((rc = upload_array(c, &m.pos, d->pos, 3 * (size_t)d->n_pos))) return rc;
+    // The positions are kept in the order the faces, taken in spatial order,
+    // first use them, so that neighbouring triangles' vertex records are
+    // neighbours; vi indexes that order.
+    std::vector<int32_t> order, rank, vi;
+    std::vector<float> pos;
+    spatial_order(d, order, rank);
+    pos.resize(3 * (size_t)d->n_pos);
+    for (int k = 0; k < d->n_pos; ++k) std::memcpy(&pos[3 * (size_t)rank[k]], d->pos + 3 * (size_t)k, 3 * sizeof(float));
+    vi.resize(3 * nf);
+    for (size_t k = 0; k < 3 * nf; ++k) vi[k] = rank[d->vi[k]];
+    std::vector<int4> tri(nf);
+    for (size_t k = 0; k < nf; ++k) {
+        const int f = order[k];
+        tri[k] = make_int4(vi[3 * (size_t)f], vi[3 * (size_t)f + 1], vi[3 * (size_t)f + 2], f);
+    }
+    if ((rc = upload_array(c, &m.pos, pos.data(), pos.size()))) return rc;
+    if ((rc = upload_array(c, &m.tri, tri.data(), nf))) return rc;
     if ((rc = upload_array(c, &m.uv, d->uv, 2 * (size_t)d->n_uv))) return rc;
     if ((rc = upload_array(c, &m.nrm, d->nrm, 3 * (size_t)d->n_nrm))) return rc;
-    if (d->tan && (rc = upload_array(c, &m.tan, d->tan, 3 * (size_t)d->n_pos))) return rc;
-    if ((rc = upload_array(c, &m.vi, (const int *)d->vi, 3 * nf))) return rc;
+    if (d->tan) {   // in the positions' order
+        for (int k = 0; k < d->n_pos; ++k)
+            std::memcpy(&pos[3 * (size_t)rank[k]], d->tan + 3 * (size_t)k, 3 * sizeof(float));
+        if ((rc = upload_array(c, &m.tan, pos.data(), pos.size()))) return rc;
+    }
+    if ((rc = upload_array(c, &m.vi, (const int *)vi.data(), 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.ti, (const int *)d->ti, 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.ni, (const int *)d->ni, 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.fmat, (const int *)d->face_material, nf))) return rc;
-    {
-        std::vector<float> corner(3 * nf * 12, 0.f);
-        for (size_t k = 0; k < 3 * nf; ++k) {
-            float *o = &corner[12 * k];
-            const int vi = d->vi[k], ti = d->ti[k], ni = d->ni[k];
-            o[0] = d->pos[3 * vi]; o[1] = d->pos[3 * vi + 1]; o[2] = d->pos[3 * vi + 2];
-            o[3] = d->uv[2 * ti]; o[4] = d->uv[2 * ti + 1];
-            o[5] = d->nrm[3 * ni]; o[6] = d->nrm[3 * ni + 1]; o[7] = d->nrm[3 * ni + 2];
-            if (d->tan) { o[8] = d->tan[3 * vi]; o[9] = d->tan[3 * vi + 1]; o[10] = d->tan[3 * vi + 2]; }
-        }
-        if ((rc = upload_array(c, &m.corner, corner.data(), corner.size()))) return rc;
+    HIPCHK(c, hipMalloc((void **)&m.corner, (nf ? 3 * nf * 12 : 1) * sizeof(float)));
+    launch_corners(m.pos, m.uv, m.nrm, m.tan, m.vi, m.ti, m.ni, 3 * nf, (float4 *)m.corner, c->stream);
+    HIPCHK(c, hipGetLastError());
+    for (int k = 0; k < 3; ++k) {
+        m.lo[k] = HUGE_VAL;
+        m.hi[k] = -HUGE_VAL;
     }
+    bool finite = nf > 0;
+    double edge2 = 0.0;
+    for (size_t f = 0; f < nf; ++f) {
+        const float *p[3];
+        for (int k = 0; k < 3; ++k) p[k] = d->pos + 3 * (size_t)d->vi[3 * f + k];
+        for (int k = 0; k < 3; ++k) {
+            double e2 = 0.0;
+            for (int j = 0; j < 3; ++j) {
+                const double x = p[k][j], e = x - p[(k + 1) % 3][j];
+                finite = finite && std::isfinite(x);
+                m.lo[j] = x < m.lo[j] ? x : m.lo[j];
+                m.hi[j] = x > m.hi[j] ? x : m.hi[j];
+                e2 += e * e;
+            }
+            edge2 = e2 > edge2 ? e2 : edge2;
+        }
+    }
+    m.edge = std::sqrt(edge2);
+    m.bounded = finite;
+    if (d->n_pos <= kFewVertices) m.few.assign(d->pos, d->pos + 3 * (size_t)d->n_pos);
     m.n_pos = d->n_pos;
     m.n_faces = d->n_faces;
     m.has_tan = d->tan != nullptr;
@@ -530,7 +637,7 @@ int fgl_init_targets(fgl_ctx *c, int w, int h)
     size_t P = (size_t)w * h;
     if ((rc = ensure(c, c->depth, P * 4)) || (rc = ensure(c, c->fb, 3 * P * 4)) ||
         (rc = ensure(c, c->gbuf, kGbufPlanes * P * 4)) || (rc = ensure(c, c->ao, P * 4)) ||
-        (rc = ensure(c, c->blur_tmp, P * 4)) || (rc = ensure(c, c->vis, P * 4)))
+        (rc = ensure(c, c->blur_tmp, P * 4)))
         return rc;
     c->W = w;
     c->H = h;
@@ -785,6 +892,7 @@ static void fill_draw(fgl_ctx *c, const ModelRes &m, const float M[16], DevDraw 
     d.pos = m.pos; d.uv = m.uv; d.nrm = m.nrm; d.tan = m.tan;
     d.vi = m.vi; d.ti = m.ti; d.ni = m.ni; d.face_mat = m.fmat;
     d.corner = (const float4 *)m.corner;
+    d.tri = m.tri;
     d.n_pos = m.n_pos;
     d.n_faces = m.n_faces;
     d.has_tangents = m.has_tan;
@@ -964,89 +1072,197 @@ static int stochastic_shadow_samples(fgl_ctx *c, const FrameUniforms &u, const f
     return FGL_OK;
 }
 
-static int flush_pass(fgl_ctx *c)
+// Model to clip space of one draw in double precision, and the same product
+// of absolute values, which bounds what the vertex stage's roundings can move.
+struct ClipBound {
+    double m[16], a[16];
+};
+
+static void mat_mul_d(const double *x, const float *y, double *o, bool absolute)
 {
-    if (c->draws.empty()) return FGL_OK;
-    const int pass = c->pass == FGL_PASS_SHADOW ? kPassShadow
-                   : c->pass == FGL_PASS_GEOMETRY ? kPassGeometry : kPassForward;
-    const bool shadow = pass == kPassShadow;
-    const int W = shadow ? c->SW : c->W, H = shadow ? c->SH : c->H;
-    if (W <= 0 || H <= 0 || (shadow && !c->shadow.p) || (!shadow && !c->depth.p)) {
-        c->draws.clear();
-        return fail(c, FGL_ERR_INVALID, "render targets not initialised for this pass");
-    }
-    if (pass == kPassForward && c->shadow_on && !c->shadow.p) {
-        c->draws.clear();
-        return fail(c, FGL_ERR_INVALID, "forward pass with shadows needs a shadow buffer");
-    }
-    // The forward shaders with a stochastic shadow filter draw samples for
-    // every fragment that passes the depth test, in raster order: the pass
-    // replays that sequence (k_frag_walk) to find each winner's samples.
-    const bool stoch = pass == kPassForward && c->shadow_on && !c->lights.empty() &&
-                       (c->shadow_cfg.mode == FGL_SHADOW_REF_PCF || c->shadow_cfg.mode == FGL_SHADOW_REF_PCSS);
-    if (stoch && (size_t)c->W * c->H > 0xffffffffull) {
-        c->draws.clear();
-        return fail(c, FGL_ERR_CAPACITY, "stochastic shadows in the forward pass: too many pixels");
-    }
-    int rc = upload_tables(c);
-    if (rc) return rc;
+    for (int r = 0; r < 4; ++r)
+        for (int j = 0; j < 4; ++j) {
+            double v = 0.0;
+            for (int k = 0; k < 4; ++k) {
+                const double e = x[4 * r + k] * (double)y[4 * k + j];
+                v += absolute ? std::fabs(e) : e;
+            }
+            o[4 * r + j] = v;
+        }
+}
 
-    // draw table in submission order
-    std::vector<DevDraw> dd(c->draws.size());
-    long long nt = 0, nv = 0;
-    int max_pos = 0, max_faces = 0;
-    for (size_t i = 0; i < c->draws.size(); ++i) {
-        const ModelRes &m = c->models[c->draws[i].model];
-        DevDraw &d = dd[i];
-        fill_draw(c, m, c->draws[i].m, d);
-        if (c->draws[i].has_normal) std::memcpy(d.normal, c->draws[i].n, sizeof(d.normal));
-        d.vert_base = (int)nv;
-        d.tri_base = (int)nt;
-        nt += m.n_faces;
-        nv += m.n_pos;
-        max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
-        max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
-    }
-    const int n_draws = (int)c->draws.size();
-    c->draws.clear();
-    if (nt > 0x7fffffffLL || nv > 0x7fffffffLL) return fail(c, FGL_ERR_CAPACITY, "pass too large");
-    // Whether this pass starts from the cleared targets: then it writes
-    // every pixel (winner or clear value) and no separate clear runs.
-    bool fresh;
-    if (shadow) {
-        fresh = c->pend_shadow;
-    } else if (pass == kPassGeometry) {
-        if (c->pend_depth != c->pend_gbuf && (rc = materialize(c, true, true, false, false, false))) return rc;
-        fresh = c->pend_depth;
-    } else {
-        if (c->pend_depth != c->pend_fb && (rc = materialize(c, true, false, true, false, false))) return rc;
-        if (c->shadow_on && (rc = materialize(c, false, false, false, false, true))) return rc;
-        fresh = c->pend_depth;
-    }
-    if (nt == 0) return FGL_OK;
+// The pass's camera (model matrix still to come).
+static ClipBound camera_bound(const fgl_ctx *c, bool shadow)
+{
+    const double I[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
+    ClipBound b, p;
+    mat_mul_d(I, shadow ? c->light_space : c->proj, b.m, false);
+    mat_mul_d(I, shadow ? c->light_space : c->proj, b.a, true);
+    if (shadow) return b;
+    mat_mul_d(b.m, c->view, p.m, false);
+    mat_mul_d(b.a, c->view, p.a, true);
+    return p;
+}
 
-    if (dd.size() != c->last_draws.size() ||
-        std::memcmp(dd.data(), c->last_draws.data(), dd.size() * sizeof(DevDraw)) != 0) {
-        if ((rc = ensure(c, c->d_draws, dd.size() * sizeof(DevDraw)))) return rc;
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        HIPCHK(c, hipMemcpy(c->d_draws.p, dd.data(), dd.size() * sizeof(DevDraw), hipMemcpyHostToDevice));
-        c->last_draws = dd;
-    }
+// Share of the vertex stage's largest intermediate that its roundings cannot
+// reach (they are about a millionth of it).
+constexpr double kClipMargin = 1e-4;
 
-    FrameUniforms u;
-    build_uniforms(c, u);
+// Whether every vertex of m has a finite window depth below 1e30: then no
+// fragment's depth is NaN.  Each vertex is tried for models of few vertices,
+// else the model's extent, which has to lie on one side of the camera plane.
+static bool depths_finite(const ModelRes &m, const ClipBound &b)
+{
+    if (!m.bounded) return false;
+    auto far_from_camera = [&](const double lo[3], const double hi[3]) {
+        double w = b.m[15], ext = 0.0, mag = b.a[15], z = b.a[11], top = 0.0;
+        for (int j = 0; j < 3; ++j) {
+            const double most = std::fmax(std::fabs(lo[j]), std::fabs(hi[j]));
+            w += b.m[12 + j] * 0.5 * (lo[j] + hi[j]);
+            ext += std::fabs(b.m[12 + j]) * 0.5 * (hi[j] - lo[j]);
+            mag += b.a[12 + j] * most;
+            z += b.a[8 + j] * most;
+            top += most;
+        }
+        const double least = std::fabs(w) - ext;
+        return least > kClipMargin * mag && z < 1e30 * least && least > 1e-30 && mag < 1e30 && top < 1e30;
+    };
+    if (m.few.empty()) return far_from_camera(m.lo, m.hi);
+    for (size_t k = 0; k < m.few.size(); k += 3) {
+        const double p[3] = {m.few[k], m.few[k + 1], m.few[k + 2]};
+        if (!far_from_camera(p, p)) return false;
+    }
+    return true;
+}
+
+// The tile lists refuse a pass with 2^32 - 1 or more (tile, triangle) pairs,
+// whatever rasterises it: a pass that could have as many goes to the lists,
+// which count them.  pairs_bound bounds the pairs of m's faces: each face by
+// the tiles its window rectangle can meet, from the model's extent and its
+// longest edge, when all of the extent is in front of the camera; by the
+// whole screen otherwise.
+static double pairs_bound(const ModelRes &m, const ClipBound &b, const float vp[16], int W, int H, int TS)
+{
+    const double tx = (W + TS - 1) / TS, ty = (H + TS - 1) / TS;
+    double all = tx * ty;
+    if (!m.bounded) return all * m.n_faces;
+    double wmin = HUGE_VAL, nx = 0.0, ny = 0.0;
+    for (int k = 0; k < 8; ++k) {
+        const double p[4] = {k & 1 ? m.hi[0] : m.lo[0], k & 2 ? m.hi[1] : m.lo[1], k & 4 ? m.hi[2] : m.lo[2], 1.0};
+        double q[4], mag = 0.0;
+        for (int r = 0; r < 4; ++r) {
+            q[r] = 0.0;
+            for (int j = 0; j < 4; ++j) q[r] += b.m[4 * r + j] * p[j];
+        }
+        for (int j = 0; j < 4; ++j) mag += b.a[12 + j] * std::fabs(p[j]);
+        if (!(q[3] > kClipMargin * mag) || !std::isfinite(q[0]) || !std::isfinite(q[1])) return all * m.n_faces;
+        wmin = std::fmin(wmin, q[3]);
+        nx = std::fmax(nx, std::fabs(q[0] / q[3]));
+        ny = std::fmax(ny, std::fabs(q[1] / q[3]));
+    }
+    // |x/w - x'/w'| <= (|x - x'| + |x'/w'| |w - w'|) / w over an edge
+    double row[4];
+    for (int r = 0; r < 4; ++r)
+        row[r] = std::sqrt(b.m[4 * r] * b.m[4 * r] + b.m[4 * r + 1] * b.m[4 * r + 1] + b.m[4 * r + 2] * b.m[4 * r + 2]);
+    const double ex = std::fabs((double)vp[0]) * (row[0] + nx * row[3]) * m.edge / wmin;
+    const double ey = std::fabs((double)vp[5]) * (row[1] + ny * row[3]) * m.edge / wmin;
+    const double face = std::fmin(tx, (1.01 * ex + 4.0) / TS + 2.0) * std::fmin(ty, (1.01 * ey + 4.0) / TS + 2.0);
+    if (face < all) all = face;   // also when face is NaN
+    return all * m.n_faces;
+}
+
+// What a pass's draws allow: its pairs are sure to be fewer than the lists
+// can hold; no fragment can have a NaN depth.
+static void bound_pass(const fgl_ctx *c, bool shadow, long long nt, int W, int H, int TS, bool &pairs_fit, bool &no_nan)
+{
+    const double most = 4294967295.0;
+    const bool count = (double)nt * ((W + TS - 1) / TS) * ((H + TS - 1) / TS) >= most;
+    const ClipBound cam = camera_bound(c, shadow);
+    double sum = 0.0;
+    no_nan = true;
+    for (const fgl_ctx::Rec &r : c->draws) {
+        const ModelRes &m = c->models[r.model];
+        ClipBound b;
+        mat_mul_d(cam.m, r.m, b.m, false);
+        mat_mul_d(cam.a, r.m, b.a, true);
+        no_nan = no_nan && depths_finite(m, b);
+        if (count) sum += pairs_bound(m, b, shadow ? c->shadow_viewport : c->viewport, W, H, TS);
+    }
+    pairs_fit = !count || sum < most;
+}
+
+// The pass's fragments through the direct rasteriser: its keys are left for
+// the resolve, the shadow pass's targets are written.  n_draws and the
+// largest draw bound the launches' grids (direct_fits).
+static bool direct_fits(int n_draws, int max_faces, int max_pos, size_t px)
+{
+    const long long most = 0x7fffffffLL;
+    return (long long)n_draws * ((max_faces + 15) / 16) <= most &&
+           (long long)n_draws * ((max_pos + 255) / 256) + (long long)(px / 256) + 1 <= most;
+}
+
+static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, int max_pos, int max_faces, long long nt,
+                       bool shadow, bool no_nan, int W, int H)
+{
+    // large triangles' items: room for every 64 x 16 block of the screen many
+    // times over; a pass that needs more rasterises the rest in place
+    constexpr uint32_t kItems = 1u << 18;
+    const size_t px = (size_t)W * H;
+    int rc;
+    if ((rc = ensure(c, c->key, px * 8))) return rc;
+    if (!c->items.p) {
+        // the items, then two passes' counters (one allocation)
+        if ((rc = ensure(c, c->items, (size_t)kItems * sizeof(uint2) + 2 * sizeof(DirectCtr)))) return rc;
+        launch_fill_u32((uint32_t *)((uint2 *)c->items.p + kItems), 0u, 2 * sizeof(DirectCtr) / 4, c->stream);
+    }
+    if (!no_nan) {
+        const size_t cap = c->key_nan.cap;
+        if ((rc = ensure(c, c->key_nan, px * 8))) return rc;
+        if (c->key_nan.cap != cap)
+            launch_fill_u32((uint32_t *)c->key_nan.p, 0xffffffffu, c->key_nan.cap / 4, c->stream);
+    }
+    DirectCtr *ctr = (DirectCtr *)((uint2 *)c->items.p + kItems);
+    DirectArgs a;
+    a.draws = (const DevDraw *)c->d_draws.p;
+    a.n_draws = n_draws;
+    a.screen = (const int4 *)c->screen.p;
+    a.key = (unsigned long long *)c->key.p;
+    a.fix = no_nan ? nullptr : (unsigned long long *)c->key_nan.p;
+    a.items = (uint2 *)c->items.p;
+    a.n_items = kItems;
+    a.ctr = ctr + c->direct_turn;
+    a.W = W;
+    a.H = H;
+    c->direct_turn ^= 1;
+    {
+        KernelTimer t(c, "vertex");
+        launch_direct_vertex(shadow, a.draws, n_draws, max_pos, u, (int4 *)c->screen.p,
+                             shadow ? (float *)c->ndc_z.p : nullptr, a, ctr + c->direct_turn, c->stream);
+    }
+    KernelTimer t(c, shadow ? "raster_shadow" : "raster");
+    launch_direct(a, max_faces, nt, c->stream);
+    if (shadow)
+        launch_direct_shadow(a, (const float *)c->ndc_z.p, (float *)c->shadow_depth.p, (float *)c->shadow.p, c->stream);
+    return FGL_OK;
+}
+
+// The pass through the tile lists; with stoch also the sequence of passing
+// fragments (n_frag of them).
+static int list_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, int max_pos, int max_faces, long long nt, bool shadow,
+                     int W, int H, bool fresh, bool stoch, uint32_t &n_frag)
+{
     const int TS = shadow ? c->TS_shadow : c->TS;
     const int tiles_x = (W + TS - 1) / TS, tiles_y = (H + TS - 1) / TS;
     const uint32_t ntiles = (uint32_t)(tiles_x * tiles_y);
-    if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) ||
-        (rc = ensure(c, c->rect, (size_t)nt * sizeof(uint2))) ||
+    int rc;
+    if ((rc = ensure(c, c->rect, (size_t)nt * sizeof(uint2))) ||
         (rc = ensure(c, c->counts, (size_t)nt * 4)) || (rc = ensure(c, c->offs, ((size_t)nt + 1) * 4)) ||
         (rc = ensure(c, c->scan_tmp, scan_tmp_words((size_t)nt) * 4)) ||
         (rc = ensure(c, c->tile_start, (size_t)ntiles * 4)) ||
         (rc = ensure(c, c->tile_end, (size_t)ntiles * 4)) ||
         (rc = ensure(c, c->tri_v, (size_t)nt * sizeof(int4))) ||
         (rc = ensure(c, c->big_list, (size_t)nt * 4)) || (rc = ensure(c, c->counters, 64)) ||
-        (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))))
+        (!shadow && (rc = ensure(c, c->vis, (size_t)W * H * 4))))
         return rc;
     const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
     uint32_t *big_count = (uint32_t *)c->counters.p;
@@ -1093,7 +1309,6 @@ static int flush_pass(fgl_ctx *c)
         launch_tile_ranges((const uint32_t *)c->keys.p, npairs, nullptr, (uint32_t *)c->tile_start.p,
                            (uint32_t *)c->tile_end.p, c->stream);
     }
-    uint32_t n_frag = 0;
     if (stoch) {
         // the passing fragments in raster order: count, scan, emit, sort
         KernelTimer t(c, "frag_walk");
@@ -1155,15 +1370,111 @@ static int flush_pass(fgl_ctx *c)
         KernelTimer t(c, shadow ? "raster_shadow" : "raster");
         launch_raster(shadow, TS, a, c->stream);
     }
+    return FGL_OK;
+}
+
+static int flush_pass(fgl_ctx *c)
+{
+    if (c->draws.empty()) return FGL_OK;
+    const int pass = c->pass == FGL_PASS_SHADOW ? kPassShadow
+                   : c->pass == FGL_PASS_GEOMETRY ? kPassGeometry : kPassForward;
+    const bool shadow = pass == kPassShadow;
+    const int W = shadow ? c->SW : c->W, H = shadow ? c->SH : c->H;
+    if (W <= 0 || H <= 0 || (shadow && !c->shadow.p) || (!shadow && !c->depth.p)) {
+        c->draws.clear();
+        return fail(c, FGL_ERR_INVALID, "render targets not initialised for this pass");
+    }
+    if (pass == kPassForward && c->shadow_on && !c->shadow.p) {
+        c->draws.clear();
+        return fail(c, FGL_ERR_INVALID, "forward pass with shadows needs a shadow buffer");
+    }
+    // The forward shaders with a stochastic shadow filter draw samples for
+    // every fragment that passes the depth test, in raster order: the pass
+    // replays that sequence (k_frag_walk) to find each winner's samples.
+    const bool stoch = pass == kPassForward && c->shadow_on && !c->lights.empty() &&
+                       (c->shadow_cfg.mode == FGL_SHADOW_REF_PCF || c->shadow_cfg.mode == FGL_SHADOW_REF_PCSS);
+    if (stoch && (size_t)c->W * c->H > 0xffffffffull) {
+        c->draws.clear();
+        return fail(c, FGL_ERR_CAPACITY, "stochastic shadows in the forward pass: too many pixels");
+    }
+    int rc = upload_tables(c);
+    if (rc) return rc;
+
+    // draw table in submission order
+    std::vector<DevDraw> dd(c->draws.size());
+    long long nt = 0, nv = 0;
+    int max_pos = 0, max_faces = 0;
+    for (size_t i = 0; i < c->draws.size(); ++i) {
+        const ModelRes &m = c->models[c->draws[i].model];
+        DevDraw &d = dd[i];
+        fill_draw(c, m, c->draws[i].m, d);
+        if (c->draws[i].has_normal) std::memcpy(d.normal, c->draws[i].n, sizeof(d.normal));
+        d.vert_base = (int)nv;
+        d.tri_base = (int)nt;
+        nt += m.n_faces;
+        nv += m.n_pos;
+        max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
+        max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
+    }
+    const int n_draws = (int)c->draws.size();
+    bool fits, no_nan;
+    bound_pass(c, shadow, nt, W, H, shadow ? c->TS_shadow : c->TS, fits, no_nan);
+    c->draws.clear();
+    if (nt > 0x7fffffffLL || nv > 0x7fffffffLL) return fail(c, FGL_ERR_CAPACITY, "pass too large");
+    // Whether this pass starts from the cleared targets: then it writes
+    // every pixel (winner or clear value) and no separate clear runs.
+    bool fresh;
+    if (shadow) {
+        fresh = c->pend_shadow;
+    } else if (pass == kPassGeometry) {
+        if (c->pend_depth != c->pend_gbuf && (rc = materialize(c, true, true, false, false, false))) return rc;
+        fresh = c->pend_depth;
+    } else {
+        if (c->pend_depth != c->pend_fb && (rc = materialize(c, true, false, true, false, false))) return rc;
+        if (c->shadow_on && (rc = materialize(c, false, false, false, false, true))) return rc;
+        fresh = c->pend_depth;
+    }
+    if (nt == 0) return FGL_OK;
+
+    if (dd.size() != c->last_draws.size() ||
+        std::memcmp(dd.data(), c->last_draws.data(), dd.size() * sizeof(DevDraw)) != 0) {
+        if ((rc = ensure(c, c->d_draws, dd.size() * sizeof(DevDraw)))) return rc;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        HIPCHK(c, hipMemcpy(c->d_draws.p, dd.data(), dd.size() * sizeof(DevDraw), hipMemcpyHostToDevice));
+        c->last_draws = dd;
+    }
+
+    FrameUniforms u;
+    build_uniforms(c, u);
+    // A pass from cleared targets folds its fragments into a key plane; one
+    // that goes on from earlier depths, or replays the fragment sequence, takes
+    // the tile lists.
+    const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
+    const size_t px = (size_t)W * H;
+    const bool direct = fresh && !stoch && fits && direct_fits(n_draws, max_faces, max_pos, px);
+    if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))))
+        return rc;
+    uint32_t n_frag = 0;
+    if (direct) {
+        if ((rc = direct_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, no_nan, W, H))) return rc;
+    } else if ((rc = list_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, W, H, fresh, stoch, n_frag))) {
+        return rc;
+    }
     if (shadow) {
         c->pend_shadow = false;
     } else {
         ResolveArgs r;
         std::memset(&r, 0, sizeof(r));
         r.draws = ddraws;
-        r.screen = a.screen;
-        r.tri_v = a.tri_v;
-        r.vis = a.vis;
+        r.n_draws = n_draws;
+        r.screen = (const int4 *)c->screen.p;
+        r.tri_v = (const int4 *)c->tri_v.p;
+        r.vis = (const int *)c->vis.p;
+        if (direct) {
+            r.key = (unsigned long long *)c->key.p;
+            r.fix = no_nan ? nullptr : (unsigned long long *)c->key_nan.p;
+            r.depth = (float *)c->depth.p;
+        }
         r.W = W;
         r.H = H;
         r.fresh = fresh;

@@ -35,6 +35,8 @@ struct DevDraw {
     // (tan.xyz, 0) -- one 48-byte record instead of four arrays behind three
     // index streams
     const float4 *corner;
+    // the faces in spatial order: position indices (as vi) and the face
+    const int4 *tri;
     int n_pos, n_faces, vert_base, tri_base;
     int has_tangents, support_pbr;
     int view;      // batched views: index of the draw's view (0 otherwise)

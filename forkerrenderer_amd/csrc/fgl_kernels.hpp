@@ -38,11 +38,35 @@ struct ShadowSamples {
     uint32_t stride;
 };
 
+// Its counters: items claimed (64 bits: claims past the list's end still
+// count), and whether a NaN mark was made.
+struct DirectCtr {
+    unsigned long long items;
+    uint32_t nan, pad;
+};
+
+// A pass of the direct rasteriser (raster_core.hpp): its key plane and the
+// second plane of pixels with NaN marks (null when none can be made), the item list of large triangles,
+// the counters.
+struct DirectArgs {
+    const DevDraw *draws;
+    int n_draws;
+    const int4 *screen;
+    unsigned long long *key, *fix;
+    uint2 *items;
+    uint32_t n_items;          // the list's capacity
+    DirectCtr *ctr;
+    int W, H;
+};
+
 struct ResolveArgs {
     const DevDraw *draws;
+    int n_draws;
     const int4 *screen;
     const int4 *tri_v;
-    const int *vis;
+    const int *vis;            // the tile rasteriser's winners, or
+    unsigned long long *key, *fix;   // the direct rasteriser's keys (key != nullptr) and
+    float *depth;              // the depth target its resolve writes
     int W, H, fresh;
     float clear[3];            // forward pass background colour
     float *gbuf;               // 19 planes (geometry pass)
@@ -103,6 +127,9 @@ struct SsaoArgs {
 };
 
 // raster.hip
+// The corner records of a model from its attribute arrays (tan may be null).
+void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti,
+                    const int *ni, size_t n, float4 *out, hipStream_t s);
 // Window records of every (draw, position); shadow pass: also the NDC z of
 // each vertex into ndc_z; zero (may be null): a word set to 0 on the way.
 void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos,
@@ -123,6 +150,15 @@ void launch_fill_f32(float *p, float v, size_t n, hipStream_t s);
 void launch_tile_ranges(const uint32_t *keys, uint32_t n, const uint32_t *n_dev, uint32_t *start,
                         uint32_t *end, hipStream_t s);
 void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s);
+// The direct rasteriser.  launch_direct_vertex: launch_vertex, the key plane
+// cleared and the next pass's counters zeroed on the way; launch_direct: the
+// pass's fragments into the keys (max_faces: the largest draw's; n_tri: all
+// draws'); launch_direct_shadow: the shadow pass's depth and ShadowBuffer
+// value of every texel from the keys.
+void launch_direct_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
+                          float *ndc_z, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s);
+void launch_direct(const DirectArgs &a, int max_faces, long long n_tri, hipStream_t s);
+void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth, float *shadow_out, hipStream_t s);
 void launch_gbuffer_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);
 void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);
 // emit = false: the count walk; true: the emit walk.

@@ -15,9 +15,30 @@
 //   resolve       one thread per pixel: the pass's fragment program for the
 //                 winning triangle (G-buffer or forward colour), coalesced
 //                 SoA writes; the shadow pass resolves inside k_raster.
+//
+// A pass that starts from cleared targets and replays no fragment sequence
+// (every pass of a frame but the stochastic forward one) takes the direct
+// rasteriser instead of the lists: k_direct_vertex, k_direct, k_direct_big,
+// k_direct_nan, then the resolve (k_direct_shadow for the shadow pass).
 #include "raster_core.hpp"
 
 namespace fgl {
+
+// A model's corner records (DevDraw::corner), a thread per corner: gathered
+// here, not built on the host and copied (144 bytes a face).
+__global__ __launch_bounds__(256) void k_corners(const float *__restrict__ pos, const float *__restrict__ uv,
+                                                 const float *__restrict__ nrm, const float *__restrict__ tan,
+                                                 const int *__restrict__ vi, const int *__restrict__ ti,
+                                                 const int *__restrict__ ni, size_t n, float4 *__restrict__ out)
+{
+    const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= n) return;
+    const float *p = pos + 3 * (size_t)vi[k], *t = uv + 2 * (size_t)ti[k], *m = nrm + 3 * (size_t)ni[k];
+    out[3 * k] = make_float4(p[0], p[1], p[2], t[0]);
+    out[3 * k + 1] = make_float4(t[1], m[0], m[1], m[2]);
+    const float *g = tan ? tan + 3 * (size_t)vi[k] : nullptr;
+    out[3 * k + 2] = g ? make_float4(g[0], g[1], g[2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+}
 
 // One thread per (draw, position); the first thread also zeroes *zero (the
 // pass's big-triangle counter, which setup counts up next).
@@ -148,12 +169,99 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TS == 32 
     raster_tile<TS, BLOCK, SHADOW>(a, tile, lds);
 }
 
+// Direct rasteriser, first launch of a pass: the vertex records, the key
+// plane cleared (8 keys a thread) by the workgroups past the vertices', and
+// the counters of the next pass zeroed (this pass's were by the one before).
+constexpr int kClearKeys = 8;
+template <bool SHADOW>
+__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, int n_vert_blocks, int bx,
+                                                       FrameUniforms u, int4 *__restrict__ out,
+                                                       float *__restrict__ ndc_z, unsigned long long *__restrict__ key,
+                                                       size_t n_keys, DirectCtr *__restrict__ next_ctr)
+{
+    const int b = blockIdx.x;
+    if (b >= n_vert_blocks) {
+        const size_t k0 = (size_t)(b - n_vert_blocks) * (256 * kClearKeys);
+        if (b == n_vert_blocks && threadIdx.x == 0) *next_ctr = DirectCtr{0ull, 0u, 0u};
+        ulonglong2 c;
+        c.x = c.y = kDirectClear;
+#pragma unroll
+        for (int e = 0; e < kClearKeys / 2; ++e) {
+            const size_t k = k0 + 2 * ((size_t)e * 256 + threadIdx.x);
+            if (k + 1 < n_keys) *(ulonglong2 *)(key + k) = c;
+            else if (k < n_keys) key[k] = kDirectClear;
+        }
+        return;
+    }
+    const DevDraw &dr = draws[b / bx];
+    const int vi = (b % bx) * 256 + threadIdx.x;
+    if (vi >= dr.n_pos) return;
+    if (SHADOW) {
+        const Vec4 n = depth_ndc(dr, vi);
+        out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
+        ndc_z[dr.vert_base + vi] = n.z;
+    } else {
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_ndc(dr, u, vi));
+    }
+}
+
+// G lanes per triangle: as many as fill the chip (a triangle's pixels are
+// its lanes' serial work).  Workgroups are dealt to the XCDs in runs:
+// neighbouring triangles share vertices and pixels.
+constexpr long long kDirectTris16 = 32768, kDirectTris4 = 262144;
+template <int G>
+__global__ __launch_bounds__(256) void k_direct(DirectArgs a, int bx)
+{
+    __shared__ DirectLds lds;
+    const int b = xcd_remap(blockIdx.x, gridDim.x);
+    direct_group<G>(a, a.draws[b / bx], (b % bx) * (256 / G), lds);
+}
+
+// The large triangles' items, a wavefront each.
+__global__ __launch_bounds__(256) void k_direct_big(DirectArgs a)
+{
+    const unsigned long long claimed = a.ctr->items;
+    const uint32_t n = claimed < a.n_items ? (uint32_t)claimed : a.n_items;
+    for (uint32_t k = blockIdx.x * 4 + (threadIdx.x >> 6); k < n; k += gridDim.x * 4) direct_item(a, a.items[k]);
+}
+
+// The second walk of a pass with NaN marks.
+__global__ __launch_bounds__(256) void k_direct_nan(DirectArgs a, int bx, int blocks)
+{
+    if (a.ctr->nan == 0u) return;
+    for (int b = blockIdx.x; b < blocks; b += gridDim.x) {
+        const DevDraw &dr = a.draws[b / bx];
+        const int n = (b % bx) * 256 + threadIdx.x;
+        TriL t;
+        const bool keep = n < dr.n_faces && direct_stage(a, dr, n, t);
+        direct_walk<1>(t, keep, keep ? direct_area(t) : 0, FoldAfterNan{a});
+    }
+}
+
+// DepthShader::ProcessFragment (depthshader.h:30-36) for the winners, with
+// the vertices' NDC z as the vertex pass computed them.
+__global__ __launch_bounds__(256) void k_direct_shadow(DirectArgs a, const float *__restrict__ ndc_z,
+                                                       float *__restrict__ depth, float *__restrict__ shadow_out)
+{
+    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (x >= a.W || y >= a.H) return;
+    const size_t i = (size_t)x + (size_t)y * a.W;
+    const Winner w = direct_winner(a.draws, a.n_draws, a.key, a.fix, a.screen, a.W, a.H, i, x, y);
+    float z = 0.f;
+    if (w.g >= 0) z = dot3(vec3(ndc_z[w.tv.x], ndc_z[w.tv.y], ndc_z[w.tv.z]), w.b) * 0.5f + 0.5f;
+    depth[i] = w.depth;
+    shadow_out[i] = z;
+    if (w.mark) a.fix[i] = ~0ull;
+}
+
+template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_gbuffer_resolve(ResolveArgs a, FrameUniforms u)
 {
     const int x = blockIdx.x * 64 + (threadIdx.x & 63);
     const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
     if (x >= a.W || y >= a.H) return;
-    gbuffer_px(a, u, x, y);
+    gbuffer_px<DIRECT>(a, u, x, y);
 }
 
 // Forward pass resolve: BlinnPhongShader / PBRShader::ProcessFragment
@@ -199,7 +307,7 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
 
 // Forward resolve, one thread per pixel; draw and material records through
 // readfirstlane when the wavefront shares them (as in gbuffer_px).
-template <bool STREAM>
+template <bool STREAM, bool DIRECT>
 __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUniforms u)
 {
     const int x = blockIdx.x * 64 + (threadIdx.x & 63);
@@ -207,31 +315,32 @@ __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUni
     if (x >= a.W || y >= a.H) return;
     const size_t i = (size_t)x + (size_t)y * a.W;
     const size_t P = (size_t)a.W * a.H;
-    const int g = a.vis[i];
-    if (g < 0) {
+    const Winner w = resolve_winner<DIRECT>(a, i, x, y);
+    if (w.g < 0) {
         if (a.fresh) {
             a.fb[i] = a.clear[0];
             a.fb[P + i] = a.clear[1];
             a.fb[2 * P + i] = a.clear[2];
         }
+        resolve_end<DIRECT>(a, i, w);
         return;
     }
-    int4 tv;
-    const Vec3 b = winner_bary(a.screen, a.tri_v, g, a.W, a.H, x, y, tv);
-    const int d0 = __builtin_amdgcn_readfirstlane(tv.w);
-    if (__ballot(tv.w != d0) == 0ull) {
+    const int d0 = __builtin_amdgcn_readfirstlane(w.tv.w);
+    if (__ballot(w.tv.w != d0) == 0ull) {
         const DevDraw &dr = a.draws[d0];
-        const int f = g - dr.tri_base;
+        const int f = w.g - dr.tri_base;
         const int mi = dr.face_mat[f];
         const int m0 = __builtin_amdgcn_readfirstlane(mi);
         if (__ballot(mi != m0) == 0ull) {
-            forward_shade<STREAM>(a, u, dr, a.materials[m0], f, b, i, P);
+            forward_shade<STREAM>(a, u, dr, a.materials[m0], f, w.b, i, P);
+            resolve_end<DIRECT>(a, i, w);
             return;
         }
     }
-    const DevDraw &dr = a.draws[tv.w];
-    const int f = g - dr.tri_base;
-    forward_shade<STREAM>(a, u, dr, a.materials[dr.face_mat[f]], f, b, i, P);
+    const DevDraw &dr = a.draws[w.tv.w];
+    const int f = w.g - dr.tri_base;
+    forward_shade<STREAM>(a, u, dr, a.materials[dr.face_mat[f]], f, w.b, i, P);
+    resolve_end<DIRECT>(a, i, w);
 }
 
 // ---------------- the forward pass's fragment sequence ----------------
@@ -373,6 +482,7 @@ __global__ __launch_bounds__(256) void k_frag_pixel_offsets(const uint32_t *__re
 // ---------------- launch wrappers ----------------
 
 static inline unsigned blocks_for(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
+static inline dim3 grid2(int W, int H) { return dim3((W + 63) / 64, (H + 3) / 4); }
 
 void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos,
                    const FrameUniforms &u, int4 *out, float *ndc_z, uint32_t *zero, hipStream_t s)
@@ -384,6 +494,13 @@ void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos,
     dim3 grid(blocks_for(max_pos, 256), n_draws);
     if (shadow) hipLaunchKernelGGL(k_vertex<true>, grid, dim3(256), 0, s, draws, u, out, ndc_z, zero);
     else hipLaunchKernelGGL(k_vertex<false>, grid, dim3(256), 0, s, draws, u, out, ndc_z, zero);
+}
+
+void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti,
+                    const int *ni, size_t n, float4 *out, hipStream_t s)
+{
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_corners, dim3(blocks_for(n, 256)), dim3(256), 0, s, pos, uv, nrm, tan, vi, ti, ni, n, out);
 }
 
 void launch_setup(const DevDraw *draws, int n_draws, int max_faces, const int4 *screen, int W,
@@ -449,19 +566,58 @@ void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s)
     else launch_raster_t<false>(TS, a, s);
 }
 
-static inline dim3 grid2(int W, int H) { return dim3((W + 63) / 64, (H + 3) / 4); }
+void launch_direct_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
+                          float *ndc_z, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s)
+{
+    const size_t P = (size_t)a.W * a.H;
+    const unsigned bx = blocks_for(max_pos, 256), nv = bx * (unsigned)n_draws;
+    const unsigned grid = nv + blocks_for(P, 256 * kClearKeys);
+    if (shadow)
+        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z, a.key,
+                           P, next_ctr);
+    else
+        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z,
+                           a.key, P, next_ctr);
+}
+
+void launch_direct(const DirectArgs &a, int max_faces, long long n_tri, hipStream_t s)
+{
+    const unsigned nd = (unsigned)a.n_draws;
+    if (n_tri <= kDirectTris16) {
+        const unsigned bx = blocks_for(max_faces, 256 / 16);
+        hipLaunchKernelGGL(k_direct<16>, dim3(bx * nd), dim3(256), 0, s, a, (int)bx);
+    } else if (n_tri <= kDirectTris4) {
+        const unsigned bx = blocks_for(max_faces, 256 / 4);
+        hipLaunchKernelGGL(k_direct<4>, dim3(bx * nd), dim3(256), 0, s, a, (int)bx);
+    } else {
+        const unsigned bx = blocks_for(max_faces, 256);
+        hipLaunchKernelGGL(k_direct<1>, dim3(bx * nd), dim3(256), 0, s, a, (int)bx);
+    }
+    hipLaunchKernelGGL(k_direct_big, dim3(1024), dim3(256), 0, s, a);
+    if (!a.fix) return;
+    const unsigned bx = blocks_for(max_faces, 256), nb = bx * nd;
+    hipLaunchKernelGGL(k_direct_nan, dim3(nb < 256u ? nb : 256u), dim3(256), 0, s, a, (int)bx, (int)nb);
+}
+
+void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth, float *shadow_out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_direct_shadow, grid2(a.W, a.H), dim3(256), 0, s, a, ndc_z, depth, shadow_out);
+}
 
 void launch_gbuffer_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s)
 {
     if (a.W <= 0 || a.H <= 0) return;
-    hipLaunchKernelGGL(k_gbuffer_resolve, grid2(a.W, a.H), dim3(256), 0, s, a, u);
+    if (a.key) hipLaunchKernelGGL(k_gbuffer_resolve<true>, grid2(a.W, a.H), dim3(256), 0, s, a, u);
+    else hipLaunchKernelGGL(k_gbuffer_resolve<false>, grid2(a.W, a.H), dim3(256), 0, s, a, u);
 }
 
 void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s)
 {
     if (a.W <= 0 || a.H <= 0) return;
-    if (a.ss.pairs) hipLaunchKernelGGL(k_forward_resolve<true>, grid2(a.W, a.H), dim3(256), 0, s, a, u);
-    else hipLaunchKernelGGL(k_forward_resolve<false>, grid2(a.W, a.H), dim3(256), 0, s, a, u);
+    const dim3 g = grid2(a.W, a.H);
+    if (a.ss.pairs) hipLaunchKernelGGL((k_forward_resolve<true, false>), g, dim3(256), 0, s, a, u);
+    else if (a.key) hipLaunchKernelGGL((k_forward_resolve<false, true>), g, dim3(256), 0, s, a, u);
+    else hipLaunchKernelGGL((k_forward_resolve<false, false>), g, dim3(256), 0, s, a, u);
 }
 
 template <bool EMIT>

@@ -48,6 +48,22 @@ __device__ __forceinline__ bool nondegenerate_general(int4 a, int4 b, int4 c)
     return fabs(uz) > 1e-2;
 }
 
+// Whether a triangle can cover a pixel of the W x H screen: not degenerate
+// and, in the exact regime, not off the screen.
+__device__ __forceinline__ bool keep_tri(int4 a, int4 b, int4 c, int W, int H)
+{
+    if (a.w && b.w && c.w && W <= 8192 && H <= 8192) {
+        int cz = (b.x - a.x) * (c.y - a.y) - (c.x - a.x) * (b.y - a.y);
+        int ux0 = imin(a.x, imin(b.x, c.x)), ux1 = imax(a.x, imax(b.x, c.x));
+        int uy0 = imin(a.y, imin(b.y, c.y)), uy1 = imax(a.y, imax(b.y, c.y));
+        // Every clamped-bbox pixel of an off-screen triangle lies strictly
+        // outside it, and in the exact regime one computed weight is then
+        // strictly negative: nothing can be covered.
+        return cz != 0 && !(ux1 < 0 || ux0 > W - 1 || uy1 < 0 || uy0 > H - 1);
+    }
+    return nondegenerate_general(a, b, c);
+}
+
 // Triangle setup of face f of draw d (pass-wide triangle id g): clamped
 // bbox, degenerate / off-screen cull, screen-tile rectangle and count.
 __device__ __forceinline__ void setup_tri(const DevDraw &dr, int d, int f,
@@ -63,19 +79,7 @@ __device__ __forceinline__ void setup_tri(const DevDraw &dr, int d, int f,
     const int4 a = screen[v0], b = screen[v1], c = screen[v2];
     int minx, miny, maxx, maxy;
     clamped_bbox(a, b, c, W, H, minx, miny, maxx, maxy);
-    const bool exact = a.w && b.w && c.w && W <= 8192 && H <= 8192;
-    bool keep;
-    if (exact) {
-        int cz = (b.x - a.x) * (c.y - a.y) - (c.x - a.x) * (b.y - a.y);
-        int ux0 = imin(a.x, imin(b.x, c.x)), ux1 = imax(a.x, imax(b.x, c.x));
-        int uy0 = imin(a.y, imin(b.y, c.y)), uy1 = imax(a.y, imax(b.y, c.y));
-        // Every clamped-bbox pixel of an off-screen triangle lies strictly
-        // outside it, and in the exact regime one computed weight is then
-        // strictly negative: nothing can be covered.
-        keep = cz != 0 && !(ux1 < 0 || ux0 > W - 1 || uy1 < 0 || uy0 > H - 1);
-    } else {
-        keep = nondegenerate_general(a, b, c);
-    }
+    const bool keep = keep_tri(a, b, c, W, H);
     const uint32_t tx0 = minx / TS, tx1 = maxx / TS, ty0 = miny / TS, ty1 = maxy / TS;
     const uint32_t n = keep ? (tx1 - tx0 + 1) * (ty1 - ty0 + 1) : 0u;
     rect[g] = make_uint2(tx0 | (tx1 << 16), ty0 | (ty1 << 16));
@@ -401,6 +405,358 @@ __device__ __forceinline__ void raster_tile(const RasterArgs &a, int tile, Raste
     }
 }
 
+// ---------------- direct rasteriser ----------------
+//
+// A pass that starts from cleared targets needs no tile lists: the depth
+// fold is a minimum over keys, so workgroups fold their triangles' fragments
+// into a plane of 64-bit keys in HBM with device-scope atomic minima, and the
+// resolve reads each pixel's key.
+//
+// A workgroup takes 256 / G neighbouring triangles (the model's faces in
+// spatial order, fgl_upload_model) and folds them in LDS over the box of
+// pixels they share, then folds the box's pixels into the plane, neighbouring
+// lanes neighbouring pixels.  What bounds the fold is the atomics' memory
+// traffic -- one by one, in the faces' own order, each fetched and wrote back
+// a cache line (5.2 M triangles at 3840 x 2160: 668 us for the main pass, 137
+// without the atomics) -- and a box touches each of its lines once (205 us,
+// of which the items below take a quarter; the tile lists' own setup, scan,
+// emit, sort, ranges and rasteriser took 515).  A box of more than kDirectBox pixels folds straight into the plane: its
+// triangles are large, their own rows of pixels neighbours.
+//
+// kDirectBig bounds what one triangle costs the lanes that own it: a larger
+// one goes to the item list, 64 x 16 pixels an item, and any wavefront of
+// k_direct_big takes it (a list that is full leaves the triangle to its own
+// wavefront).
+//
+// NaN depths (a vertex on the camera plane) follow the rule above in two
+// more steps: the first walk marks the pixel with the NaN fragment's id --
+// high word 0, below every real depth's -- and the mark with the highest id
+// is the minimum; k_direct_nan, which returns at once unless a mark was made,
+// walks the triangles again and folds the fragments after the mark into a
+// second plane (all ones between passes: the resolve puts back what it
+// read).  A pass whose vertices the host has shown to have finite depths
+// (context.cpp, bound_pass) has neither that plane nor that walk.
+constexpr unsigned long long kDirectClear = 0xff7fffffull << 32;   // depth_order(FLT_MAX), no fragment
+constexpr int kDirectItemW = 64, kDirectItemH = 16;
+constexpr int kDirectBig = 4096;      // pixels of the bounding box
+constexpr int kDirectBox = 2048;      // pixels of a workgroup's LDS box: 16 KiB, nine workgroups a CU
+
+struct DirectLds {
+    unsigned long long key[kDirectBox];
+    uint32_t lo[4], hi[4];            // per wavefront: (min x | min y << 16), the complement of the maxima
+};
+
+// A fragment's key; a NaN depth's is its mark.
+__device__ __forceinline__ unsigned long long direct_key(const DirectArgs &a, const TriL &t, float dd)
+{
+    if (dd != dd) {
+        a.ctr->nan = 1u;
+        return (unsigned long long)(uint32_t)~(uint32_t)t.g;
+    }
+    return ((unsigned long long)depth_order(dd) << 32) | (unsigned long long)(uint32_t)(t.g + 1);
+}
+
+__device__ __forceinline__ void direct_min(unsigned long long *key, unsigned long long k)
+{
+    (void)__hip_atomic_fetch_min(key, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Where a walk's fragments go: the key plane,
+struct FoldPlane {
+    const DirectArgs &a;
+    __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd) const
+    {
+        direct_min(a.key + (size_t)px + (size_t)py * a.W, direct_key(a, t, dd));
+    }
+};
+
+// the workgroup's box in LDS (w pixels wide, its corner at (x0, y0)),
+struct FoldBox {
+    const DirectArgs &a;
+    DirectLds &L;
+    int x0, y0, w;
+    __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd) const
+    {
+        atomicMin(&L.key[(px - x0) + (py - y0) * w], direct_key(a, t, dd));
+    }
+};
+
+// or, in the second walk of a pass with NaN marks, the second plane: the
+// fragments after the pixel's mark.
+struct FoldAfterNan {
+    const DirectArgs &a;
+    __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd) const
+    {
+        const size_t i = (size_t)px + (size_t)py * a.W;
+        const unsigned long long m = a.key[i];
+        if ((m >> 32) != 0ull || dd != dd || t.g <= (int)~(uint32_t)m) return;
+        direct_min(a.fix + i, ((unsigned long long)depth_order(dd) << 32) | (unsigned long long)(uint32_t)(t.g + 1));
+    }
+};
+
+// Pixels first, first + step, ... of t's box, row by row: its fragments
+// among them to fold.  first < step <= 64.
+template <typename Fold>
+__device__ __forceinline__ void direct_box(const TriL &t, int first, int step, const Fold &fold)
+{
+    const int x0 = t.bb0 & 0xffff, y0 = t.bb0 >> 16;
+    const int w = (t.bb1 & 0xffff) - x0 + 1, h = (t.bb1 >> 16) - y0 + 1;
+    int y = 0, x = 0, sy = 0, sx = 1;
+    if (step > 1) {
+        // first / w and step / w: at most 64 and off an integer by 0.5 / w or
+        // more after the half is added, so the product truncates exactly
+        const float inv = __builtin_amdgcn_rcpf((float)w);
+        y = (int)(((float)first + 0.5f) * inv);
+        x = first - y * w;
+        sy = (int)(((float)step + 0.5f) * inv);
+        sx = step - sy * w;
+    }
+    while (y < h) {
+        float b0, b1, b2;
+        if (cover(t, x0 + x, y0 + y, b0, b1, b2)) fold(t, x0 + x, y0 + y, tri_depth(t, b0, b1, b2));
+        x += sx;
+        y += sy;
+        if (x >= w) {
+            x -= w;
+            ++y;
+        }
+    }
+}
+
+__device__ __forceinline__ int direct_area(const TriL &t)
+{
+    return ((t.bb1 & 0xffff) - (t.bb0 & 0xffff) + 1) * ((t.bb1 >> 16) - (t.bb0 >> 16) + 1);
+}
+
+// Face number n of draw dr in the model's spatial order, staged; false when
+// it covers nothing (degenerate, or off the screen in the exact regime).
+__device__ __forceinline__ bool direct_stage(const DirectArgs &a, const DevDraw &dr, int n, TriL &t)
+{
+    const int4 v = dr.tri[n];
+    const int4 p = a.screen[dr.vert_base + v.x], q = a.screen[dr.vert_base + v.y], r = a.screen[dr.vert_base + v.z];
+    if (!keep_tri(p, q, r, a.W, a.H)) return false;
+    stage_tri(t, dr.tri_base + v.w, p, q, r, a.W, a.H);
+    return true;
+}
+
+__device__ __forceinline__ TriL direct_lane(const TriL &t, int l)
+{
+    TriL o;
+    o.X0 = __builtin_amdgcn_readlane(t.X0, l);
+    o.Y0 = __builtin_amdgcn_readlane(t.Y0, l);
+    o.q0 = __builtin_amdgcn_readlane(t.q0, l);
+    o.q1 = __builtin_amdgcn_readlane(t.q1, l);
+    o.q2 = __builtin_amdgcn_readlane(t.q2, l);
+    o.q3 = __builtin_amdgcn_readlane(t.q3, l);
+    o.z0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.z0), l));
+    o.z1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.z1), l));
+    o.z2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t.z2), l));
+    o.bb0 = __builtin_amdgcn_readlane(t.bb0, l);
+    o.bb1 = __builtin_amdgcn_readlane(t.bb1, l);
+    o.cz = __builtin_amdgcn_readlane(t.cz, l);
+    o.exact = __builtin_amdgcn_readlane(t.exact, l);
+    o.g = __builtin_amdgcn_readlane(t.g, l);
+    const long long iv = __double_as_longlong(t.inv);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)iv, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(iv >> 32), l);
+    o.inv = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    return o;
+}
+
+// The wavefront's triangles, G lanes each: a box of up to kSmallTriArea
+// pixels a lane stays with its group, the whole wavefront takes a larger one.
+template <int G, typename Fold>
+__device__ __forceinline__ void direct_walk(const TriL &t, bool keep, int area, const Fold &fold)
+{
+    const int lane = threadIdx.x & 63, sub = lane % G;
+    const bool small = area <= kSmallTriArea * G;
+    if (keep && small) direct_box(t, sub, G, fold);
+    unsigned long long m = __ballot(keep && !small && sub == 0);
+    while (m) {
+        const int l = __builtin_ctzll(m);
+        m &= m - 1;
+        direct_box(direct_lane(t, l), lane, 64, fold);
+    }
+}
+
+// Triangles of more than kDirectBig pixels to the item list, one claim a
+// wavefront, the items written by all its lanes; true when this lane's
+// triangle (n items of it, 0 if it is no such triangle) went there.
+__device__ __forceinline__ bool direct_items(const DirectArgs &a, int g, uint32_t n)
+{
+    unsigned long long m = __ballot(n != 0u);
+    if (!m) return false;
+    const int lane = threadIdx.x & 63;
+    uint32_t inc = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    unsigned long long at = 0;
+    if (lane == 63) at = atomicAdd(&a.ctr->items, (unsigned long long)total);
+    at = __shfl(at, 63, 64);
+    if (at + total > a.n_items) {
+        // no room: what was claimed inside the list holds no item
+        for (unsigned long long k = at + lane; k < a.n_items; k += 64) a.items[k] = make_uint2(0xffffffffu, 0u);
+        return false;
+    }
+    const uint32_t off = (uint32_t)at + inc - n;
+    while (m) {
+        const int l = __builtin_ctzll(m);
+        m &= m - 1;
+        const uint32_t ln = (uint32_t)__builtin_amdgcn_readlane((int)n, l);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)off, l);
+        const uint32_t lg = (uint32_t)__builtin_amdgcn_readlane(g, l);
+        for (uint32_t k = lane; k < ln; k += 64) a.items[lo + k] = make_uint2(lg, k);
+    }
+    return n != 0u;
+}
+
+// A workgroup's 256 / G triangles of draw dr, from number first of its
+// spatial order on.
+template <int G>
+__device__ __forceinline__ void direct_group(const DirectArgs &a, const DevDraw &dr, int first, DirectLds &L)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = first + tid / G;
+    TriL t;
+    bool keep = n < dr.n_faces && direct_stage(a, dr, n, t);
+    int area = keep ? direct_area(t) : 0;
+    {
+        const int w = keep ? (t.bb1 & 0xffff) - (t.bb0 & 0xffff) + 1 : 0, h = keep ? (t.bb1 >> 16) - (t.bb0 >> 16) + 1 : 0;
+        const bool big = area > kDirectBig;
+        const uint32_t k = big && lane % G == 0 ? (uint32_t)((w + kDirectItemW - 1) / kDirectItemW) *
+                                                      (uint32_t)((h + kDirectItemH - 1) / kDirectItemH) : 0u;
+        // a group's first lane decides for the group
+        const int listed = __shfl((int)direct_items(a, keep ? t.g : 0, k), lane - lane % G, 64);
+        keep = keep && !listed;
+    }
+    // the box of what is left
+    typedef unsigned short v2u __attribute__((ext_vector_type(2)));
+    v2u lo = {0xffff, 0xffff}, hi = {0xffff, 0xffff};
+    if (keep) {
+        lo = __builtin_bit_cast(v2u, t.bb0);
+        hi = __builtin_bit_cast(v2u, ~t.bb1);
+    }
+#pragma unroll
+    for (int o = G; o < 64; o <<= 1) {
+        lo = __builtin_elementwise_min(lo, __builtin_bit_cast(v2u, __shfl_xor(__builtin_bit_cast(int, lo), o, 64)));
+        hi = __builtin_elementwise_min(hi, __builtin_bit_cast(v2u, __shfl_xor(__builtin_bit_cast(int, hi), o, 64)));
+    }
+    if (lane == 0) {
+        L.lo[wave] = __builtin_bit_cast(uint32_t, lo);
+        L.hi[wave] = __builtin_bit_cast(uint32_t, hi);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        lo = __builtin_elementwise_min(lo, __builtin_bit_cast(v2u, L.lo[v]));
+        hi = __builtin_elementwise_min(hi, __builtin_bit_cast(v2u, L.hi[v]));
+    }
+    const int x0 = lo.x, y0 = lo.y, w = (int)(uint16_t)~hi.x - x0 + 1, h = (int)(uint16_t)~hi.y - y0 + 1;
+    if (lo.x == 0xffff) return;   // nothing kept (a screen is at most 16384 wide)
+    if (w * h > kDirectBox) {
+        direct_walk<G>(t, keep, area, FoldPlane{a});
+        return;
+    }
+    for (int p = tid; p < w * h; p += 256) L.key[p] = ~0ull;
+    __syncthreads();
+    direct_walk<G>(t, keep, area, FoldBox{a, L, x0, y0, w});
+    __syncthreads();
+    for (int p = tid; p < w * h; p += 256) {
+        const unsigned long long k = L.key[p];
+        const int y = p / w, x = p - y * w;
+        if (k != ~0ull) direct_min(a.key + (size_t)(x0 + x) + (size_t)(y0 + y) * a.W, k);
+    }
+}
+
+// The draw of pass-wide triangle g (their tri_base ascend).
+__device__ __forceinline__ int draw_of(const DevDraw *draws, int n_draws, int g)
+{
+    int lo = 0, hi = n_draws - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (draws[mid].tri_base <= g) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Triangle g staged from its face, and its vertex ids and draw.
+__device__ __forceinline__ int4 direct_face(const DevDraw *draws, int d, const int4 *screen, int g, int W, int H, TriL &t)
+{
+    const DevDraw &dr = draws[d];
+    const int f = g - dr.tri_base;
+    const int4 tv = make_int4(dr.vert_base + dr.vi[3 * f], dr.vert_base + dr.vi[3 * f + 1],
+                              dr.vert_base + dr.vi[3 * f + 2], d);
+    stage_tri(t, g, screen[tv.x], screen[tv.y], screen[tv.z], W, H);
+    return tv;
+}
+
+// Item it of the list by one wavefront.
+__device__ __forceinline__ void direct_item(const DirectArgs &a, uint2 it)
+{
+    if (it.x == 0xffffffffu) return;
+    TriL t;
+    direct_face(a.draws, draw_of(a.draws, a.n_draws, (int)it.x), a.screen, (int)it.x, a.W, a.H, t);
+    const int bx = t.bb0 & 0xffff, by = t.bb0 >> 16, w = (t.bb1 & 0xffff) - bx + 1, h = (t.bb1 >> 16) - by + 1;
+    const int nx = (w + kDirectItemW - 1) / kDirectItemW;
+    const int ox = ((int)it.y % nx) * kDirectItemW, oy = ((int)it.y / nx) * kDirectItemH;
+    const int x = ox + (int)(threadIdx.x & 63);
+    if (x >= w) return;
+    const int y1 = imin(oy + kDirectItemH, h);
+    const FoldPlane fold{a};
+    for (int y = oy; y < y1; ++y) {
+        float b0, b1, b2;
+        if (cover(t, bx + x, by + y, b0, b1, b2)) fold(t, bx + x, by + y, tri_depth(t, b0, b1, b2));
+    }
+}
+
+// A pixel's winner: its triangle (-1: none), vertex ids and draw, weights;
+// with the direct rasteriser also its depth as the fold leaves it, and
+// whether the pixel has a NaN mark.
+struct Winner {
+    int g;
+    int4 tv;
+    Vec3 b;
+    float depth;
+    bool mark;
+};
+
+// The winner of pixel i = (px, py) from its key.  Wavefronts whose winners
+// belong to one draw find it once.
+__device__ __forceinline__ Winner direct_winner(const DevDraw *draws, int n_draws, const unsigned long long *key,
+                                                const unsigned long long *fix, const int4 *screen, int W, int H, size_t i,
+                                                int px, int py)
+{
+    Winner w;
+    unsigned long long k = key[i];
+    bool nan = false;
+    w.mark = (k >> 32) == 0ull && fix;
+    if ((k >> 32) == 0ull) {
+        const unsigned long long after = fix ? fix[i] : ~0ull;
+        nan = after == ~0ull;
+        w.g = nan ? (int)~(uint32_t)k : (int)(uint32_t)after - 1;
+        k = after;
+    } else {
+        w.g = (int)(uint32_t)k - 1;
+    }
+    w.depth = 3.40282347e+38f;
+    if (w.g < 0) return w;
+    const int d0 = draw_of(draws, n_draws, __builtin_amdgcn_readfirstlane(w.g));
+    const int f0 = w.g - draws[d0].tri_base;
+    const int d = f0 >= 0 && f0 < draws[d0].n_faces ? d0 : draw_of(draws, n_draws, w.g);
+    TriL t;
+    w.tv = direct_face(draws, d, screen, w.g, W, H, t);
+    w.b = vec3(0.f, 0.f, 0.f);
+    cover(t, px, py, w.b.x, w.b.y, w.b.z);
+    w.depth = depth_from_order((uint32_t)(k >> 32));
+    if (nan || w.depth == 0.f) w.depth = tri_depth(t, w.b.x, w.b.y, w.b.z);   // NaN, or a zero with its sign
+    return w;
+}
+
 // Barycentric weights of the winning triangle at (px,py), recomputed with the
 // same staged arithmetic as the coverage loop.
 __device__ __forceinline__ Vec3 winner_bary(const int4 *__restrict__ screen,
@@ -413,6 +769,27 @@ __device__ __forceinline__ Vec3 winner_bary(const int4 *__restrict__ screen,
     float b0 = 0.f, b1 = 0.f, b2 = 0.f;
     cover(t, px, py, b0, b1, b2);
     return vec3(b0, b1, b2);
+}
+
+// The winner of pixel i = (x, y), and the end of its resolve: the depth
+// target, and the second plane all ones again (last, so that the loads
+// between keep their scalar form).
+template <bool DIRECT>
+__device__ __forceinline__ Winner resolve_winner(const ResolveArgs &a, size_t i, int x, int y)
+{
+    if (DIRECT) return direct_winner(a.draws, a.n_draws, a.key, a.fix, a.screen, a.W, a.H, i, x, y);
+    Winner w;
+    w.g = a.vis[i];
+    if (w.g >= 0) w.b = winner_bary(a.screen, a.tri_v, w.g, a.W, a.H, x, y, w.tv);
+    return w;
+}
+
+template <bool DIRECT>
+__device__ __forceinline__ void resolve_end(const ResolveArgs &a, size_t i, const Winner &w)
+{
+    if (!DIRECT) return;
+    a.depth[i] = w.depth;
+    if (w.mark) a.fix[i] = ~0ull;
 }
 
 // GShader::ProcessFragment + the seven buffer writes (gshader.h:95-202,
@@ -466,33 +843,37 @@ __device__ __forceinline__ void gbuffer_shade(const ResolveArgs &a, const FrameU
 // neighbouring pixels show the same mesh), the draw and material records are
 // addressed through readfirstlane, so their fields (matrices, flags, texture
 // descriptors) come in as scalar loads instead of one vector load per field.
+// DIRECT: winners come from the direct rasteriser's keys, and the depth
+// target is written here.
+template <bool DIRECT>
 __device__ __forceinline__ void gbuffer_px(const ResolveArgs &a, const FrameUniforms &u, int x, int y)
 {
     const size_t i = (size_t)x + (size_t)y * a.W;
     const size_t P = (size_t)a.W * a.H;
     float *gb = a.gbuf;
-    const int g = a.vis[i];
-    if (g < 0) {
+    const Winner w = resolve_winner<DIRECT>(a, i, x, y);
+    if (w.g < 0) {
         if (a.fresh)
             for (int c = 0; c < kGbufPlanes; ++c) gb[c * P + i] = 0.f;
+        resolve_end<DIRECT>(a, i, w);
         return;
     }
-    int4 tv;
-    const Vec3 b = winner_bary(a.screen, a.tri_v, g, a.W, a.H, x, y, tv);
-    const int d0 = __builtin_amdgcn_readfirstlane(tv.w);
-    if (__ballot(tv.w != d0) == 0ull) {
+    const int d0 = __builtin_amdgcn_readfirstlane(w.tv.w);
+    if (__ballot(w.tv.w != d0) == 0ull) {
         const DevDraw &dr = a.draws[d0];
-        const int f = g - dr.tri_base;
+        const int f = w.g - dr.tri_base;
         const int mi = dr.face_mat[f];
         const int m0 = __builtin_amdgcn_readfirstlane(mi);
         if (__ballot(mi != m0) == 0ull) {
-            gbuffer_shade(a, u, dr, a.materials[m0], f, b, i, P);
+            gbuffer_shade(a, u, dr, a.materials[m0], f, w.b, i, P);
+            resolve_end<DIRECT>(a, i, w);
             return;
         }
     }
-    const DevDraw &dr = a.draws[tv.w];
-    const int f = g - dr.tri_base;
-    gbuffer_shade(a, u, dr, a.materials[dr.face_mat[f]], f, b, i, P);
+    const DevDraw &dr = a.draws[w.tv.w];
+    const int f = w.g - dr.tri_base;
+    gbuffer_shade(a, u, dr, a.materials[dr.face_mat[f]], f, w.b, i, P);
+    resolve_end<DIRECT>(a, i, w);
 }
 
 }  // namespace fgl

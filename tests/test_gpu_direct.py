@@ -1,0 +1,106 @@
+"""The direct rasteriser (passes from cleared targets) against the tile lists
+(passes that go on from earlier depths), bit for bit, over what their rules
+divide: lanes per triangle, the workgroup's LDS box, the item list of large
+triangles and its overflow, NaN depths, screens of one pixel and wider than
+the exact regime, several draws with equal depths.
+
+The second rendering starts with a draw that covers nothing and a change of
+state, which flushes it: the rest of the pass then continues from existing
+depths and takes the tile lists."""
+import numpy as np
+import pytest
+
+import forkerrenderer_amd as F
+
+pytestmark = pytest.mark.gpu
+
+EYE4 = np.eye(4, dtype=np.float32)
+
+
+def _model(ctx, mat, pos):
+    """Separate triangles, pos (n, 3, 3) in clip space."""
+    n = len(pos)
+    f = np.arange(3 * n, dtype=np.int32).reshape(n, 3)
+    return ctx.upload_model({"pos": pos.reshape(-1, 3).astype(np.float32), "uv": np.zeros((3 * n, 2), np.float32),
+                             "nrm": np.tile(np.array([[0, 0, 1]], np.float32), (3 * n, 1)), "tan": None, "vi": f, "ti": f,
+                             "ni": f, "face_material": np.full(n, mat, np.int32), "support_pbr": False})
+
+
+def _triangles(rng, n, size, spread=1.1):
+    """n triangles of about `size` of the screen's half width, anywhere on it."""
+    c = rng.uniform(-spread, spread, (n, 1, 3)) * np.array([1, 1, 0.45])
+    return c + rng.uniform(-size, size, (n, 3, 3)) * np.array([1, 1, 0.05])
+
+
+def _scene(name, rng):
+    """(models, W, H): each model's triangles."""
+    if name == "few_mixed":        # 16 lanes a triangle, boxes below and above the LDS box, items
+        return [np.concatenate([_triangles(rng, 300, s) for s in (0.01, 0.05, 0.2, 0.9)])], 333, 201
+    if name == "four_lanes":
+        return [_triangles(rng, 40000, 0.02)], 640, 400
+    if name == "one_lane":
+        return [_triangles(rng, 270000, 0.004), _triangles(rng, 5, 1.5)], 512, 300
+    if name == "items_overflow":   # 1,200 full screens of 300 items each: more than the list holds
+        full = np.array([[-3, -3, 0], [3, -3, 0], [0, 3, 0]]) + 0.0
+        return [full[None] + rng.uniform(-0.4, 0.4, (1200, 3, 1)) * np.array([0, 0, 1]), _triangles(rng, 100, 0.1)], 640, 480
+    if name == "ties":             # the same triangles drawn three times: the first draw's win
+        t = _triangles(rng, 200, 0.3)
+        return [t, _triangles(rng, 50, 0.3), t, t[::-1]], 160, 90
+    if name == "one_pixel":
+        return [_triangles(rng, 50, 2.0)], 1, 1
+    if name == "thin":
+        return [_triangles(rng, 2000, 0.3)], 5, 300
+    if name == "inexact":          # wider than 8192: the general coverage sequence
+        return [_triangles(rng, 400, 0.1)], 8300, 6
+    if name == "nan":              # NaN and infinite depths among ordinary ones
+        t = _triangles(rng, 400, 0.4)
+        t[::7, 1, 2] = np.nan
+        t[3::11, 2, 2] = np.inf
+        return [t, _triangles(rng, 100, 0.4)], 120, 80
+    raise AssertionError(name)
+
+
+@pytest.mark.parametrize("name", ["few_mixed", "four_lanes", "one_lane", "items_overflow", "ties", "one_pixel", "thin",
+                                  "inexact", "nan"])
+@pytest.mark.parametrize("shadow", [False, True])
+def test_direct_equals_lists(ctx, name, shadow):
+    rng = np.random.default_rng(len(name))
+    tris, W, H = _scene(name, rng)
+    m = F.Material()
+    for f in ("map_kd", "map_ks", "map_ke", "map_bump", "map_base", "map_rough", "map_metal", "map_ao", "map_pbr_ke"):
+        setattr(m, f, -1)
+    mat = ctx.upload_material(m)
+    models = [_model(ctx, mat, t) for t in tris]
+    off = _model(ctx, mat, np.full((1, 3, 3), 9.0) + np.eye(3)[None])
+    ctx.set_tile_size(16)
+    ctx.set_shadow(False)
+    eye = np.ascontiguousarray(EYE4)
+    ctx.set_matrix(F.MAT_PROJ, eye)
+    ctx.set_matrix(F.MAT_VIEW, eye)
+    ctx.set_matrix(F.MAT_LIGHT_SPACE, eye)
+    ctx.set_viewport(0, 0, W, H, shadow=shadow)
+    out = []
+    for lists in (False, True):
+        print(f"direct test {name} {W}x{H} shadow {shadow} lists {lists}", flush=True)
+        if shadow:
+            ctx.init_shadow_buffer(W, H)
+        else:
+            ctx.init_targets(W, H)
+        ctx.set_eye((0.0, 0.0, 1.0))
+        ctx.begin_pass(F.PASS_SHADOW if shadow else F.PASS_GEOMETRY)
+        if lists:
+            ctx.draw_model(off, eye)
+            ctx.set_eye((0.0, 0.0, 2.0))   # flushes the pass so far
+        for k in models:
+            ctx.draw_model(k, eye)
+        ctx.end_pass()
+        which = (F.TARGET_SHADOW_DEPTH, F.TARGET_SHADOW) if shadow else (F.TARGET_DEPTH, F.TARGET_GBUFFER)
+        out.append([ctx.read(t).view(np.uint32) for t in which])
+    for a, b, what in zip(out[0], out[1], ("depth", "shadow value" if shadow else "G-buffer")):
+        if name == "nan":   # a NaN's payload is not the fold's
+            na, nb = np.isnan(a.view(np.float32)), np.isnan(b.view(np.float32))
+            assert np.array_equal(na, nb), what
+            a, b = np.where(na, 0, a), np.where(nb, 0, b)
+        assert np.array_equal(a, b), f"{what}: {(a != b).sum()} of {a.size} differ"
+    depth = out[0][0].view(np.float32)
+    assert (depth < 3e38).any()
