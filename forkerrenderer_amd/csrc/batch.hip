@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     a.materials = b.materials;
     a.textures = b.textures;
     a.shadow_map = nullptr;
-    a.ss = ShadowSamples{nullptr, nullptr, 0u};
+    a.ss = ShadowSamples{};
     gbuffer_px<false>(a, v.u, x, y);
 }
 
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void k_bv_lighting(BvPixelArgs b)
     int vi, x, y;
     if (!bv_pixel(b, vi, x, y)) return;
     const DevView &v = b.views[vi];
-    const ShadowSamples none = {nullptr, nullptr, 0};
+    const ShadowSamples none = {};
     lighting_px(v.u, b.gbuf + kGbufPlanes * v.px_off, b.ao + v.px_off, b.ao_is_one, b.shadow + v.spx_off, none,
                 b.fb + 3 * v.px_off, x, y);
 }

@@ -116,15 +116,14 @@ struct fgl_ctx {
     // the PCSS sample offsets, the DoSSAO powf table
     DevBuf rng, rng_samples, rng_offs, ssao_pow3;
     uint32_t rng_seed = 5489u;
-    // the parallel generator: base sequence, jumped chunk arrays, raw draws,
-    // the per-workgroup counts of kept tries and their scan, the jump
-    // polynomials uploaded so far; the last fill's tries (T of D draws) for
-    // its commit
-    DevBuf mt_base, mt_states, mt_raw, mt_pos;
+    // the parallel generator: base sequence, jumped chunk arrays, the chunks'
+    // kept vectors, their counts and checkpoints, the jump polynomials uploaded
+    // so far; the last fill and the vectors asked of it, for its commit
+    DevBuf mt_base, mt_states, mt_vec, mt_ck;
     DevBuf mt_polys[2];          // jump polynomials for the two chunk lengths
     int mt_polys_n[2] = {0, 0};
-    uint32_t fill_T = 0, fill_n = 0;
-    int fill_D = 0;
+    MtFill fill{};
+    uint32_t fill_n = 0;
 
     // device address of the allocation-free entry point's scratch array
     float *noalloc_scratch = nullptr;
@@ -356,7 +355,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     DevBuf *bufs[] = {&c->d_textures, &c->d_materials, &c->depth, &c->fb, &c->gbuf, &c->ao,
                       &c->blur_tmp, &c->shadow, &c->shadow_depth, &c->img, &c->vis, &c->d_draws,
                       &c->rng, &c->rng_samples, &c->rng_offs, &c->ssao_pow3,
-                      &c->mt_base, &c->mt_states, &c->mt_raw, &c->mt_pos, &c->mt_polys[0], &c->mt_polys[1],
+                      &c->mt_base, &c->mt_states, &c->mt_vec, &c->mt_ck, &c->mt_polys[0], &c->mt_polys[1],
                       &c->screen, &c->rect, &c->counts, &c->offs, &c->scan_tmp, &c->keys,
                       &c->vals, &c->keys_alt, &c->vals_alt, &c->sort_tmp, &c->tile_start,
                       &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z,
@@ -903,43 +902,55 @@ static void fill_draw(fgl_ctx *c, const ModelRes &m, const float M[16], DevDraw 
 }
 
 // The stream's next n vectors (RandomVectorInUnitDisk for D = 2,
-// RandomVectorInUnitSphere for D = 3) into out, in stream order, without
+// RandomVectorInUnitSphere for D = 3) in stream order (c->fill), without
 // consuming them: rng_take then moves the stream past the first m <= n.  The
-// draws are generated in parallel chunks of K blocks, each chunk's array
-// reached by a jump from the context's (rng.hip, mt_jump.hpp); the draws
-// needed are estimated from the acceptance rate (pi/4 for the disk, pi/6 for
-// the sphere) with a margin, and doubled in the rare case that too few tries
-// are kept.  A chunk's generation takes time in proportion to K, and the
-// jumps (a workgroup each, one per CU) take a fixed time per 256 chunks:
-// K = 256 while 256 chunks of it cover the request, else 512.
+// draws are generated in parallel chunks of K blocks, each chunk's first
+// window reached by a jump from the context's next draw (rng.hip,
+// mt_jump.hpp); the draws needed are estimated from the acceptance rate (pi/4
+// for the disk, pi/6 for the sphere) with a margin, and doubled in the rare
+// case that too few tries are kept.  A chunk's generation takes time in
+// proportion to K, and the jumps (a workgroup each, one per CU) take a fixed
+// time per 256 chunks: K = 256 while 256 chunks of it cover the request, else
+// 512.
 static constexpr int kMtChunkShort = 256, kMtChunkLong = 512;
 
-static int rng_fill(fgl_ctx *c, int D, float *out, uint32_t n)
+static int rng_fill(fgl_ctx *c, int D, uint32_t n)
 {
     int rc;
-    c->fill_T = 0;
+    c->fill = MtFill{};
+    c->fill.D = D;
     c->fill_n = 0;
-    c->fill_D = D;
     if (n == 0) return FGL_OK;
     const double keep = D == 2 ? 0.78539816339744831 : 0.52359877559829887;
     uint64_t R = (uint64_t)((double)n * D / keep * 1.01) + 4096;
     for (;;) {
         const int kind = R <= 256ull * 624 * kMtChunkShort ? 0 : 1;
         const uint64_t C = 624ull * (kind ? kMtChunkLong : kMtChunkShort);
-        uint64_t Nc = (R + C - 1) / C;
+        const uint64_t Nc = (R + C - 1) / C;
         int K = kind ? kMtChunkLong : kMtChunkShort;
         if (Nc == 1) K = (int)((R + 623) / 624);   // one chunk: only the blocks needed
         const uint64_t len = Nc * (uint64_t)K * 624;
         if (len + 624 >= 0xffffffffull || Nc > 0x7fffffffull)
             return fail(c, FGL_ERR_CAPACITY, "random stream: too many draws in one request");
-        const uint32_t T = (uint32_t)(len / (uint64_t)D);
-        const uint32_t nb = mt_try_blocks(T);
-        if ((rc = ensure(c, c->mt_raw, (len + 624) * 4)) ||
-            (rc = ensure(c, c->mt_pos, ((size_t)nb + 1 + scan_tmp_words(nb)) * 4)))
+        MtFill f;
+        f.D = D;
+        f.chunks = (uint32_t)Nc;
+        f.T = (uint32_t)K * 624u / (uint32_t)D;
+        f.stride = (f.T + kStreamRun + 3u) & ~3u;
+        f.n_ck = mt_checkpoints(f.T);
+        const size_t cks = (size_t)Nc * f.n_ck;
+        if ((rc = ensure(c, c->mt_vec, (size_t)Nc * f.stride * D * sizeof(float))) ||
+            (rc = ensure(c, c->mt_ck, (cks * 625 + 2 * (size_t)Nc + 1) * 4)) ||
+            (rc = ensure(c, c->mt_base, (size_t)kMtBaseWords * 4)))
             return rc;
-        MtState *st = (MtState *)c->rng.p;
-        uint32_t *raw = (uint32_t *)c->mt_raw.p, *pos = (uint32_t *)c->mt_pos.p;
+        f.out = (float *)c->mt_vec.p;
+        f.ck_words = (uint32_t *)c->mt_ck.p;
+        f.ck_kept = f.ck_words + cks * 624;
+        f.kept = f.ck_kept + cks;
+        f.prefix = f.kept + Nc;
+        uint32_t *base = (uint32_t *)c->mt_base.p;
         const uint32_t *states = nullptr;
+        launch_mt_base((const MtState *)c->rng.p, Nc > 1 ? (uint32_t)kMtBaseWords : 624u, base, c->stream);
         if (Nc > 1) {
             const int nj = (int)Nc - 1;
             if (nj > c->mt_polys_n[kind]) {
@@ -952,22 +963,15 @@ static int rng_fill(fgl_ctx *c, int D, float *out, uint32_t n)
                 HIPCHK(c, hipStreamSynchronize(c->stream));
                 c->mt_polys_n[kind] = nj;
             }
-            if ((rc = ensure(c, c->mt_base, (size_t)kMtBaseWords * 4)) ||
-                (rc = ensure(c, c->mt_states, (size_t)Nc * 624 * 4)))
-                return rc;
-            launch_mt_base(st, (uint32_t *)c->mt_base.p, c->stream);
-            launch_mt_jump((const uint32_t *)c->mt_base.p, (const uint64_t *)c->mt_polys[kind].p, nj,
-                           (uint32_t *)c->mt_states.p, c->stream);
+            if ((rc = ensure(c, c->mt_states, (size_t)Nc * 624 * 4))) return rc;
+            launch_mt_jump(base, (const uint64_t *)c->mt_polys[kind].p, nj, (uint32_t *)c->mt_states.p, c->stream);
             states = (const uint32_t *)c->mt_states.p;
         }
-        launch_mt_gen(st, states, (int)Nc, K, raw, c->stream);
-        launch_mt_count(D, raw, T, pos, c->stream);
-        launch_exclusive_scan(pos, pos, nb, pos + nb + 1, c->stream);
-        HIPCHK(c, hipMemcpyAsync(c->h_total, pos + nb, 4, hipMemcpyDeviceToHost, c->stream));
+        launch_mt_fill(base, states, f, c->stream);
+        HIPCHK(c, hipMemcpyAsync(c->h_total, f.prefix + Nc, 4, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         if (c->h_total[0] >= n) {
-            launch_mt_take(D, raw, T, pos, n, out, c->stream);
-            c->fill_T = T;
+            c->fill = f;
             c->fill_n = n;
             HIPCHK(c, hipGetLastError());
             return FGL_OK;
@@ -980,8 +984,7 @@ static int rng_take(fgl_ctx *c, uint32_t m)
 {
     if (m == 0) return FGL_OK;
     if (m > c->fill_n) return fail(c, FGL_ERR_INVALID, "random stream: taking more vectors than were drawn");
-    launch_mt_commit(c->fill_D, (MtState *)c->rng.p, (const uint32_t *)c->mt_raw.p, (const uint32_t *)c->mt_pos.p,
-                     c->fill_T, m, c->stream);
+    launch_mt_commit((MtState *)c->rng.p, c->fill, m, c->stream);
     HIPCHK(c, hipGetLastError());
     return FGL_OK;
 }
@@ -1003,10 +1006,8 @@ static int stochastic_shadow_samples(fgl_ctx *c, const FrameUniforms &u, const f
     if (mode == FGL_SHADOW_REF_PCF) {
         const size_t total = n * np;
         if (total > 0xffffffffull) return fail(c, FGL_ERR_CAPACITY, "stochastic shadows: too many samples");
-        if ((rc = ensure(c, c->rng_samples, (total > np ? total : np) * 2 * sizeof(float)))) return rc;
-        float *pairs = (float *)c->rng_samples.p;
-        if ((rc = rng_fill(c, 2, pairs, (uint32_t)total)) || (rc = rng_take(c, (uint32_t)total))) return rc;
-        ss = {pairs, nullptr, np};
+        if ((rc = rng_fill(c, 2, (uint32_t)total)) || (rc = rng_take(c, (uint32_t)total))) return rc;
+        ss = {c->fill.vectors(), nullptr, np};
         return FGL_OK;
     }
     // PCSS takes n_pcf more samples only where its blocker search finds a
@@ -1039,9 +1040,8 @@ static int stochastic_shadow_samples(fgl_ctx *c, const FrameUniforms &u, const f
     // n_pcf per undecided point: every offset the walk evaluates reads
     // inside it (point k of the undecided ones at most n_pcf k past its base)
     const size_t most = (size_t)c->h_total[0] + (size_t)np * n_unc;
-    if ((rc = ensure(c, c->rng_samples, (most > nb + np ? most : nb + np) * 2 * sizeof(float)))) return rc;
-    float *pairs = (float *)c->rng_samples.p;
-    if ((rc = rng_fill(c, 2, pairs, (uint32_t)most))) return rc;
+    if ((rc = rng_fill(c, 2, (uint32_t)most))) return rc;
+    const StreamVectors pairs = c->fill.vectors();
     // the undecided points in order, a segment at a time (shade.hip): the
     // band of miss counts each point is evaluated at follows the miss rate
     // seen so far
@@ -1503,11 +1503,11 @@ static int flush_pass(fgl_ctx *c)
                     launch_frag_shadow_inputs(r, u, ftri, fq, n_frag, (float *)c->frag_planes.p, c->stream);
                     planes = (const float *)c->frag_planes.p;
                 }
-                ShadowSamples ss = {nullptr, nullptr, 0};
+                ShadowSamples ss = {};
                 if ((rc = stochastic_shadow_samples(c, u, planes, n_frag, ss))) return rc;
                 launch_frag_pixel_offsets(ftri, fq, n_frag, W, H, (const int *)c->vis.p, ss.offs, ss.stride, offs_px,
                                           c->stream);
-                r.ss = {ss.pairs, offs_px, 0};
+                r.ss = {ss.sv, offs_px, 0};
             }
             KernelTimer t(c, "forward_resolve");
             launch_forward_resolve(r, u, c->stream);
@@ -1535,7 +1535,7 @@ int fgl_draw_screen_space_pixels(fgl_ctx *c)
     if ((rc = materialize(c, false, true, false, false, c->shadow_on != 0))) return rc;
     FrameUniforms u;
     build_uniforms(c, u);
-    ShadowSamples ss = {nullptr, nullptr, 0};
+    ShadowSamples ss = {};
     const int mode = c->shadow_cfg.mode;
     if (c->shadow_on && !c->lights.empty() && (mode == FGL_SHADOW_REF_PCF || mode == FGL_SHADOW_REF_PCSS)) {
         // the filters' unit-disk samples from the stream, pixels in row order
@@ -1587,11 +1587,9 @@ int fgl_ssao(fgl_ctx *c, const fgl_ssao_cfg *cfg)
         // 32 hemisphere samples per pixel, pixels in row order, from the stream
         const size_t n = (size_t)c->W * c->H * 32;
         if (n > 0xffffffffull) return fail(c, FGL_ERR_CAPACITY, "stochastic SSAO: too many samples");
-        if ((rc = ensure(c, c->rng_samples, n * 3 * sizeof(float)))) return rc;
         KernelTimer t(c, "ssao_reference");
-        if ((rc = rng_fill(c, 3, (float *)c->rng_samples.p, (uint32_t)n)) || (rc = rng_take(c, (uint32_t)n)))
-            return rc;
-        launch_ssao_reference(u, (const float *)c->rng_samples.p, (const float *)c->ssao_pow3.p,
+        if ((rc = rng_fill(c, 3, (uint32_t)n)) || (rc = rng_take(c, (uint32_t)n))) return rc;
+        launch_ssao_reference(u, c->fill.vectors(), (const float *)c->ssao_pow3.p,
                               (const float *)c->depth.p, (const float *)c->gbuf.p, (float *)c->ao.p, c->stream);
     } else {
         KernelTimer t(c, "ssao");
@@ -1778,7 +1776,8 @@ int fgl_rng_vectors(fgl_ctx *c, int kind, uint32_t n, float *out)
     if (n == 0) return FGL_OK;
     const size_t bytes = (size_t)n * kind * sizeof(float);
     if ((rc = ensure(c, c->rng_samples, bytes))) return rc;
-    if ((rc = rng_fill(c, kind, (float *)c->rng_samples.p, n)) || (rc = rng_take(c, n))) return rc;
+    if ((rc = rng_fill(c, kind, n)) || (rc = rng_take(c, n))) return rc;
+    launch_mt_gather(c->fill, n, (float *)c->rng_samples.p, c->stream);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(out, c->rng_samples.p, bytes, hipMemcpyDeviceToHost));

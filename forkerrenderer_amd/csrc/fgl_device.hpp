@@ -328,6 +328,33 @@ __device__ __forceinline__ float pcss_blocker_depth(const FrameUniforms &u, cons
     return (nb < 1.f) ? 0.f : blocker / nb;
 }
 
+// Accepted vectors of the random stream, in stream order, in chunks: chunk
+// c's lie at v + c * stride * D (D floats each), prefix[c] of them before it;
+// at least kStreamRun more follow each chunk's own (the next chunk's first),
+// so a run of that many starting in a chunk is contiguous.  Chunks keep their
+// tries' expected share within a fraction of a percent, so the chunk of a
+// vector is guessed from it (inv: chunks per vector) and settled by the
+// prefixes.
+constexpr int kStreamRun = 128;
+static_assert(kStreamRun >= 2 * kMaxDisk, "a point's blocker and PCF samples in one run");
+
+struct StreamVectors {
+    const float *v;
+    const uint32_t *prefix;
+    uint32_t chunks, stride;
+    float inv;
+};
+
+template <int D>
+__device__ __forceinline__ const float *stream_at(const StreamVectors &s, uint32_t j)
+{
+    uint32_t c = (uint32_t)((float)j * s.inv);
+    c = c < s.chunks ? c : s.chunks - 1;
+    while (c > 0 && j < s.prefix[c]) --c;
+    while (c + 1 < s.chunks && j >= s.prefix[c + 1]) ++c;
+    return s.v + ((size_t)c * s.stride + (j - s.prefix[c])) * D;
+}
+
 // The random stream's samples (modes 4 and 5) are each pixel's own, 512
 // bytes or more apart between neighbouring lanes: read one sample per load,
 // every load would fetch a cache line per lane.  So they are taken

@@ -30,12 +30,16 @@ struct RasterArgs {
 };
 
 // Per-pixel unit-disk samples of the stochastic shadow filters: pixel i's
-// samples start at pair offs[i] of `pairs`, or at i * stride when offs is
-// null (fixed count per pixel).
+// samples start at vector offs[i] of sv, or at i * stride when offs is null
+// (fixed count per pixel).  sv.v == nullptr: not in use.
 struct ShadowSamples {
-    const float *pairs;
+    StreamVectors sv;
     const uint32_t *offs;
     uint32_t stride;
+    __device__ __forceinline__ const float *at(size_t i) const
+    {
+        return stream_at<2>(sv, offs ? offs[i] : (uint32_t)i * stride);
+    }
 };
 
 // Its counters: items claimed (64 bits: claims past the list's end still
@@ -197,36 +201,42 @@ struct MtState {
     unsigned long long draws;
 };
 void mt_seed_state(uint32_t seed, MtState &st);
-// The stream's next draws in parallel chunks of K blocks (624 K draws each):
-// base = the context's array and the 32 blocks after it (kMtBaseWords
-// words); states[c] (c = 1..n_jumps, 624 words each) = chunk c's starting
-// array from jump polynomial c (mt_jump.hpp; kMtPolyWords words each);
-// raw = the tempered draws from the context's next one on,
-// (624 - idx) + n_chunks 624 K of them.
+// The stream's next draws in parallel chunks of 624 K draws: base = the words
+// from the context's next draw on, n of them (kMtBaseWords for jumps, one
+// window otherwise); states[c] (c = 1..n_jumps, 624 words each) = chunk c's
+// first window from jump polynomial c (mt_jump.hpp; kMtPolyWords words each).
 constexpr int kMtBaseWords = 33 * 624;
-void launch_mt_base(const MtState *st, uint32_t *base, hipStream_t s);
+void launch_mt_base(const MtState *st, uint32_t n, uint32_t *base, hipStream_t s);
 void launch_mt_jump(const uint32_t *base, const uint64_t *polys, int n_jumps, uint32_t *states, hipStream_t s);
-void launch_mt_gen(const MtState *st, const uint32_t *states, int n_chunks, int K, uint32_t *raw, hipStream_t s);
-// Rejection-sampled unit vectors from raw's T tries of D draws (D = 3:
-// RandomVectorInUnitSphere (x, y, z); 2: RandomVectorInUnitDisk (x, y)),
-// kMtTryTile tries to a workgroup: part[b] = workgroup b's count of kept
-// tries (mt_try_blocks(T) of them); after an exclusive scan of part (the
-// total at part[nb]) the first n kept vectors go to out in stream order, and
-// a commit moves the stream past the try that kept the m-th.
-constexpr uint32_t kMtTryTile = 2048;
-uint32_t mt_try_blocks(uint32_t T);
-void launch_mt_count(int D, const uint32_t *raw, uint32_t T, uint32_t *part, hipStream_t s);
-void launch_mt_take(int D, const uint32_t *raw, uint32_t T, const uint32_t *part, uint32_t n, float *out,
-                    hipStream_t s);
-void launch_mt_commit(int D, MtState *st, const uint32_t *raw, const uint32_t *part, uint32_t T, uint32_t m,
-                      hipStream_t s);
+// A fill of rejection-sampled unit vectors (D = 3: RandomVectorInUnitSphere
+// (x, y, z); 2: RandomVectorInUnitDisk (x, y)): T tries of D draws a chunk,
+// the kept vectors of chunk c at out + c stride D (stride >= T + kStreamRun),
+// prefix[c] = vectors kept before it (chunks + 1 entries), n_ck checkpoints a
+// chunk (mt_checkpoints(T); 624 words and a count each).  A commit moves the
+// stream past the try that kept the m-th vector.
+struct MtFill {
+    int D;
+    uint32_t chunks, T, stride, n_ck;
+    float *out;
+    uint32_t *kept, *prefix, *ck_words, *ck_kept;
+    StreamVectors vectors() const
+    {
+        const float per = (float)T * (D == 2 ? 0.785398163f : 0.523598776f);
+        return StreamVectors{out, prefix, chunks, stride, 1.f / per};
+    }
+};
+uint32_t mt_checkpoints(uint32_t T);
+void launch_mt_fill(const uint32_t *base, const uint32_t *states, const MtFill &f, hipStream_t s);
+void launch_mt_commit(MtState *st, const MtFill &f, uint32_t m, hipStream_t s);
+// The fill's first n vectors as one array.
+void launch_mt_gather(const MtFill &f, uint32_t n, float *out, hipStream_t s);
 
 // shade.hip
 void launch_lighting(const FrameUniforms &u, const float *gbuf, const float *ao, int ao_is_one, const NetAo &net,
                      const float *shadow_map, const ShadowSamples &ss, float *fb, hipStream_t s);
 // Render::DoSSAO with the stream's hemisphere samples (32 (x, y, z) per
 // pixel in row order); pow3[c] = powf(1 - c / 32, 3) from the host libm.
-void launch_ssao_reference(const FrameUniforms &u, const float *samples, const float *pow3,
+void launch_ssao_reference(const FrameUniforms &u, const StreamVectors &samples, const float *pow3,
                            const float *depth, const float *gbuf, float *ao, hipStream_t s);
 // Offsets of the PCSS filter's samples for P shading points in the order
 // they shade (a point takes n_blocker pairs, plus n_pcf when its blocker
@@ -255,7 +265,7 @@ constexpr size_t kPcssChainFbits = (size_t)(kPcssSegmentMax / kPcssChainBlock) *
 constexpr size_t kPcssChainRes = 2 * (size_t)(kPcssSegmentMax / kPcssChainBlock) * kPcssBandWidth;
 void launch_pcss_points(const FrameUniforms &u, const float *g, size_t P, const uint32_t *base, const uint32_t *list,
                         uint32_t n, float4 *pt, uint32_t *pbase, hipStream_t s);
-void launch_pcss_segment(const FrameUniforms &u, const float *shadow_map, const float *pairs, const float4 *pt,
+void launch_pcss_segment(const FrameUniforms &u, const float *shadow_map, const StreamVectors &pairs, const float4 *pt,
                          const uint32_t *pbase, uint32_t s0, uint32_t L, uint32_t M0, float rate, uint32_t *pred,
                          uint32_t *scan_tmp, unsigned long long *masks, unsigned long long *fbits, uint32_t *res,
                          uint32_t *found, uint32_t *out, hipStream_t s);

@@ -278,7 +278,7 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
     FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump);
     // the stochastic shadow filters: this fragment's samples in the stream
     const float *rdisk = nullptr;
-    if (STREAM && a.ss.pairs) rdisk = a.ss.pairs + 2 * (a.ss.offs ? (size_t)a.ss.offs[i] : i * (size_t)a.ss.stride);
+    if (STREAM && a.ss.sv.v) rdisk = a.ss.at(i);
     Vec3 c;
     if (!dr.support_pbr) {
         Vec3 dc = m.map_kd >= 0 ? tex_sample(a.textures, m.map_kd, fg.uv)
@@ -615,7 +615,7 @@ void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStr
 {
     if (a.W <= 0 || a.H <= 0) return;
     const dim3 g = grid2(a.W, a.H);
-    if (a.ss.pairs) hipLaunchKernelGGL((k_forward_resolve<true, false>), g, dim3(256), 0, s, a, u);
+    if (a.ss.sv.v) hipLaunchKernelGGL((k_forward_resolve<true, false>), g, dim3(256), 0, s, a, u);
     else if (a.key) hipLaunchKernelGGL((k_forward_resolve<false, true>), g, dim3(256), 0, s, a, u);
     else hipLaunchKernelGGL((k_forward_resolve<false, false>), g, dim3(256), 0, s, a, u);
 }

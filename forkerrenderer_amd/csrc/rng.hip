@@ -5,10 +5,10 @@
 // (src/utility.h:90-103), and builds its random vectors by rejection
 // (src/geometry.h:947-990).  Its consumers (Render::DoSSAO, the PCF / PCSS
 // shadow filters) take the stream strictly in pixel (or fragment) order, so
-// the device replays it in two steps: the generator's draws are produced in
-// parallel chunks reached by jumping ahead, and the accepted vectors written
-// in stream order; the per-pixel kernels then read the vectors of their
-// pixel at a known offset.
+// the device replays it in parallel chunks reached by jumping ahead, each
+// chunk writing its accepted vectors in stream order into its own region;
+// the per-pixel kernels then read the vectors of their pixel at a known
+// offset (StreamVectors, fgl_device.hpp).
 //
 // Arithmetic, fixed by the C++ library the reference is built with:
 //  * MT19937: the standard twist and tempering on 624 words;
@@ -63,97 +63,101 @@ __device__ __forceinline__ float random_pm1(uint32_t u)
 // The generator as one sequence: x_{n+624} = twist(x_n, x_{n+1}, x_{n+397})
 // (a block's twist is this recurrence, new words used as they appear).  The
 // 227 words x_n .. x_{n+226} read only words at least 227 back, so a
-// workgroup makes them together, one barrier per step, keeping the last 1024
-// words in an LDS ring (word n in slot n % 1024).  In step s thread t makes
+// workgroup makes them together, one barrier per step, keeping the last 2048
+// words in an LDS ring (word n in slot n % 2048).  In step s thread t makes
 // x_{624+j}, j = 227 s + t, from x_j and x_{j+1} (made two steps back or
 // earlier, so read during the step before, while it computes) and x_{j+397}
-// (the word the thread made in the step before).  A step writes the slots of
-// words 1024 back, none of which it or the next step's reads touch, so the
-// next step's reads are issued first and their latency overlaps the twist.
-constexpr uint32_t kMtRing = 1024, kMtLag = kMtN - kMtM;
+// (the word the thread made in the step before).
+//
+// The barrier orders LDS alone: a __syncthreads() also waits for the step's
+// global stores, which made a step 860 cycles.
+constexpr uint32_t kMtRing = 2048, kMtLag = kMtN - kMtM;
 
-// ring holds x_0 .. x_623 (slots 0..623); the next `total` words x_624 ..
-// go through emit(j, x_{624+j}) once each, in steps of 227.  Needs at least
-// 227 threads; every thread of the workgroup calls it.  Past the end the
-// last step computes and stores words nobody reads, and emits only j < total.
-template <typename Emit>
-__device__ __forceinline__ void mt_run(uint32_t *ring, uint32_t total, Emit emit)
+__device__ __forceinline__ void mt_barrier()
 {
-    constexpr uint32_t R = kMtRing - 1;
-    const uint32_t tid = threadIdx.x;
-    const bool lane_on = tid < kMtLag;
-    uint32_t cur = 0, nxt = 0, far = 0;
-    if (lane_on) {
-        cur = ring[tid];
-        nxt = ring[tid + 1];
-        far = ring[tid + kMtM];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// A running generator: the ring holds x_0 .. x_{623 + made}.  Needs at least
+// 227 threads; every thread of the workgroup calls it.
+struct MtRun {
+    uint32_t *ring;
+    uint32_t made, cur, nxt, far;
+    __device__ __forceinline__ explicit MtRun(uint32_t *r) : ring(r), made(0), cur(0), nxt(0), far(0)
+    {
+        if (threadIdx.x < kMtLag) {
+            cur = ring[threadIdx.x];
+            nxt = ring[threadIdx.x + 1];
+            far = ring[threadIdx.x + kMtM];
+        }
     }
-    for (uint32_t j0 = 0; j0 < total; j0 += kMtLag) {
-        if (lane_on) {
-            const uint32_t j = j0 + tid;
+    // 227 more words; this thread's (the first 227 threads) is returned.
+    __device__ __forceinline__ uint32_t step()
+    {
+        constexpr uint32_t R = kMtRing - 1;
+        uint32_t v = 0;
+        if (threadIdx.x < kMtLag) {
+            const uint32_t j = made + threadIdx.x;
             const uint32_t ncur = ring[(j + kMtLag) & R], nnxt = ring[(j + kMtLag + 1) & R];
-            const uint32_t v = mt_twist_word(cur, nxt, far);
+            v = mt_twist_word(cur, nxt, far);
             ring[(j + kMtN) & R] = v;
-            if (j < total) emit(j, v);
             cur = ncur;
             nxt = nnxt;
             far = v;
         }
-        __syncthreads();
+        made += kMtLag;
+        mt_barrier();
+        return v;
     }
-}
+};
 
-__device__ __forceinline__ uint32_t mt_untemper(uint32_t y)
-{
-    y ^= y >> 18;
-    y ^= (y << 15) & 0xefc60000u;
-    uint32_t x = y;
-#pragma unroll
-    for (int i = 0; i < 5; ++i) x = y ^ ((x << 7) & 0x9d2c5680u);
-    return x ^ (x >> 11) ^ (x >> 22);
-}
-
-// One try of D draws at p: the vector (x, y, z) and whether it is kept.
+// The try of D draws at word p of the sequence in the ring: the vector (x, y,
+// z) and whether it is kept.
 template <int D>
-__device__ __forceinline__ bool mt_try(const uint32_t *__restrict__ p, float &x, float &y, float &z)
+__device__ __forceinline__ bool mt_try(const uint32_t *ring, uint32_t p, float &x, float &y, float &z)
 {
-    z = 0.f;
-    if (D == 3) {
-        z = random_pm1(p[0]);
-        y = random_pm1(p[1]);
-        x = random_pm1(p[2]);
-    } else {
-        y = random_pm1(p[0]);
-        x = random_pm1(p[1]);
-    }
+    constexpr uint32_t R = kMtRing - 1;
+    float r[D];
+#pragma unroll
+    for (int e = 0; e < D; ++e) r[e] = random_pm1(mt_temper(ring[(p + e) & R]));
+    z = D == 3 ? r[0] : 0.f;
+    y = r[D - 2];
+    x = r[D - 1];
     return (x * x + y * y) + z * z < 1.f;
 }
 
 // ---- the stream in parallel: jump ahead, generate, keep ----
 //
-// A fill takes the stream's next draws in chunks of K blocks (624 K draws).
-// Chunk 0 continues from the context's array; chunk c > 0 starts from the
-// array c 624 K words further on, which the jump gives (mt_jump.hpp): the XOR
-// of the windows x_{B+i} .. x_{B+i+623} of the base sequence over the set
-// bits i of t^(c 624 K) mod phi, x_B .. being the context's array and the 32
-// blocks after it.  The tries are then counted, scanned and kept in
-// parallel, and a commit moves the context's stream past the tries a caller
-// used.  Every window of a jump, x_{B + 19967 + 623} at most, lies in the
-// base sequence.
+// A fill takes the stream's next draws in chunks of L = 624 K draws, L a
+// multiple of D, so that no try crosses chunks.  The base sequence x_0, x_1 ..
+// starts at the context's next draw; chunk c starts from the 624 words c L
+// words into it, which the jump gives (mt_jump.hpp): the XOR of the windows
+// x_i .. x_{i+623} over the set bits i of t^(c L) mod phi.  A chunk makes its
+// words in an LDS ring, tests its tries there and writes the kept vectors
+// only; its draws never reach memory.  Checkpoints -- the generator's words
+// and the vectors kept so far, every kMtCkRounds rounds -- let a commit find
+// the try that kept the m-th vector without the draws.  Every window of a
+// jump, x_{19967 + 623} at most, lies in the base sequence.
 static_assert(kMtBaseWords >= 64 * kMtPolyWords + 623, "the jump's windows stay in the base sequence");
 
-// One workgroup: the context's array and the 32 blocks after it, untempered.
-__global__ __launch_bounds__(256) void k_mt_base(const MtState *__restrict__ st, uint32_t *__restrict__ base)
+// One workgroup: the base sequence's first n words, untempered.
+__global__ __launch_bounds__(256) void k_mt_base(const MtState *__restrict__ st, uint32_t n, uint32_t *__restrict__ base)
 {
     __shared__ uint32_t ring[kMtRing];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < (int)kMtN; i += 256) {
+    const uint32_t tid = threadIdx.x, idx = st->idx;
+    for (uint32_t i = tid; i < kMtN; i += 256) {
         const uint32_t v = st->mt[i];
         ring[i] = v;
-        base[i] = v;
+        if (i >= idx && i - idx < n) base[i - idx] = v;
     }
     __syncthreads();
-    mt_run(ring, (uint32_t)(kMtBaseWords - (int)kMtN), [&](uint32_t j, uint32_t v) { base[kMtN + j] = v; });
+    MtRun run(ring);
+    for (uint32_t at = kMtN - idx; at < n; at += kMtLag) {
+        const uint32_t v = run.step();
+        if (tid < kMtLag && at + tid < n) base[at + tid] = v;
+    }
 }
 
 // Workgroup c - 1 jumps to chunk c's array: states[c][k] = XOR of base[i + k]
@@ -276,195 +280,174 @@ __global__ __launch_bounds__(kJumpThreads) void k_mt_jump(const uint32_t *__rest
         states[(size_t)c * kMtN + k] = part[0][k] ^ part[1][k + 1] ^ part[2][k + 2] ^ part[3][k + 3];
 }
 
-// Workgroup c generates chunk c: K blocks of tempered draws at
-// raw[(624 - idx) + c 624 K ..]; chunk 0 first writes the rest of the
-// context's current block at raw[0 .. 624 - idx).
-__global__ __launch_bounds__(256) void k_mt_gen(const MtState *__restrict__ st, const uint32_t *__restrict__ states,
-                                                int K, uint32_t *__restrict__ raw)
+// Workgroup c runs chunk c: rounds of D steps, 227 tries a round (a thread
+// each), T tries in all.  A round's tries are read, tempered and tested in
+// the interval before its last steps' barrier and written after it, when
+// every wavefront's count is known.  The step is bound by its LDS latency and
+// barrier; written as tempered draws, counted, scanned and read back by two
+// more kernels, the same fill took 1,390 us for 187 M draws (D = 3).
+constexpr uint32_t kMtCkRounds = 32;
+
+template <int D>
+__global__ __launch_bounds__(256) void k_mt_fill(const uint32_t *__restrict__ base, const uint32_t *__restrict__ states,
+                                                 uint32_t T, uint32_t stride, uint32_t n_ck, float *__restrict__ out,
+                                                 uint32_t *__restrict__ kept, uint32_t *__restrict__ ck_words,
+                                                 uint32_t *__restrict__ ck_kept)
 {
+    constexpr uint32_t R = kMtRing - 1;
     __shared__ uint32_t ring[kMtRing];
-    const int tid = threadIdx.x, c = blockIdx.x;
-    const uint32_t idx = st->idx;
-    const uint32_t *src = c == 0 ? st->mt : states + (size_t)c * kMtN;
-    for (int i = tid; i < (int)kMtN; i += 256) ring[i] = src[i];
+    __shared__ uint32_t cnt[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = blockIdx.x;
+    const uint32_t *src = c == 0 ? base : states + (size_t)c * kMtN;
+    for (uint32_t i = tid; i < kMtN; i += 256) ring[i] = src[i];
     __syncthreads();
-    const size_t a = kMtN - idx;
-    if (c == 0)
-        for (uint32_t i = tid; i < a; i += 256) raw[i] = mt_temper(ring[idx + i]);
-    uint32_t *out = raw + a + (size_t)c * K * kMtN;
-    mt_run(ring, (uint32_t)K * kMtN, [&](uint32_t j, uint32_t v) { out[j] = mt_temper(v); });
-}
-
-// Tries are taken 2048 to a workgroup, 8 consecutive ones to a thread (its
-// 8 D draws read as 16-byte loads): k_mt_count writes each workgroup's count
-// of kept tries, a scan of the counts gives each workgroup its first
-// vector's index, and k_mt_take recounts its own tries and writes the kept
-// vectors in order.  No per-try array is written.
-constexpr uint32_t kTryItems = 8, kTryTile = kTryItems * 256;
-static_assert(kTryTile == kMtTryTile, "tries per workgroup");
-
-// The kept flags (bit k) of tries t0 .. t0 + 7 (those below T), their
-// vectors in xyz[3 k ..].
-template <int D>
-__device__ __forceinline__ uint32_t mt_tries8(const uint32_t *__restrict__ raw, uint32_t T, uint32_t t0, float *xyz)
-{
-    uint32_t w[kTryItems * D];
-    if (t0 + kTryItems <= T) {
-        // D t0 words from a 16-byte aligned array: t0 is a multiple of 8
-        const uint4 *p = (const uint4 *)(raw + (size_t)D * t0);
-#pragma unroll
-        for (int e = 0; e < 2 * D; ++e) {
-            const uint4 q = p[e];
-            w[4 * e] = q.x;
-            w[4 * e + 1] = q.y;
-            w[4 * e + 2] = q.z;
-            w[4 * e + 3] = q.w;
+    MtRun run(ring);
+    float *o = out + (size_t)c * stride * D;
+    uint32_t total = 0;
+    for (uint32_t t0 = 0, r = 0; t0 < T; t0 += kMtLag, ++r) {
+        if (r % kMtCkRounds == 0) {
+            const size_t k = (size_t)c * n_ck + r / kMtCkRounds;
+            for (uint32_t i = tid; i < kMtN; i += 256) ck_words[k * kMtN + i] = ring[(D * t0 + i) & R];
+            if (tid == 0) ck_kept[k] = total;
         }
-    } else {
-#pragma unroll
-        for (int e = 0; e < (int)kTryItems * D; ++e) w[e] = t0 + (uint32_t)(e / D) < T ? raw[(size_t)D * t0 + e] : 0u;
-    }
-    uint32_t kept = 0;
-#pragma unroll
-    for (int k = 0; k < (int)kTryItems; ++k) {
+        run.step();
         float x, y, z;
-        const bool ok = mt_try<D>(w + D * k, x, y, z);
-        xyz[3 * k] = x;
-        xyz[3 * k + 1] = y;
-        xyz[3 * k + 2] = z;
-        if (ok && t0 + (uint32_t)k < T) kept |= 1u << k;
-    }
-    return kept;
-}
-
-// Exclusive scan of one value per thread over a 256-thread workgroup.
-__device__ __forceinline__ uint32_t try_block_scan(uint32_t v, uint32_t *lds4, uint32_t &total)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint32_t inc = v;
+        const bool ok = mt_try<D>(ring, D * (t0 + tid), x, y, z) && tid < kMtLag && t0 + tid < T;
+        const unsigned long long m = __ballot(ok);
+        if (lane == 0) cnt[wave] = (uint32_t)__popcll(m);
+        run.step();
+        uint32_t at = total + (uint32_t)__popcll(m & ((1ull << lane) - 1));
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(inc, o, 64);
-        if (lane >= o) inc += y;
-    }
-    if (lane == 63) lds4[wave] = inc;
-    __syncthreads();
-    uint32_t prefix = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        const uint32_t c = lds4[w];
-        if (w < wave) prefix += c;
-        tot += c;
-    }
-    __syncthreads();
-    total = tot;
-    return prefix + inc - v;
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void k_mt_count(const uint32_t *__restrict__ raw, uint32_t T,
-                                                  uint32_t *__restrict__ part)
-{
-    __shared__ uint32_t lds4[4];
-    float xyz[3 * kTryItems];
-    const uint32_t t0 = blockIdx.x * kTryTile + threadIdx.x * kTryItems;
-    const uint32_t c = (uint32_t)__popc(mt_tries8<D>(raw, T, t0, xyz));
-    uint32_t total;
-    try_block_scan(c, lds4, total);
-    if (threadIdx.x == 0) part[blockIdx.x] = total;
-}
-
-// part: exclusive scan of the workgroups' counts (part[nb] = every kept
-// try); the first n kept vectors to out in stream order.
-template <int D>
-__global__ __launch_bounds__(256) void k_mt_take(const uint32_t *__restrict__ raw, uint32_t T,
-                                                 const uint32_t *__restrict__ part, uint32_t n, float *__restrict__ out)
-{
-    __shared__ uint32_t lds4[4];
-    const uint32_t first = part[blockIdx.x];
-    if (first >= n) return;   // the whole workgroup: its vectors are not asked for
-    float xyz[3 * kTryItems];
-    const uint32_t t0 = blockIdx.x * kTryTile + threadIdx.x * kTryItems;
-    const uint32_t kept = mt_tries8<D>(raw, T, t0, xyz);
-    uint32_t total;
-    uint32_t p = first + try_block_scan((uint32_t)__popc(kept), lds4, total);
-#pragma unroll
-    for (int k = 0; k < (int)kTryItems; ++k)
-        if ((kept >> k) & 1u) {
-            if (p < n) {
-                float *o = out + (size_t)p * D;
-                o[0] = xyz[3 * k];
-                o[1] = xyz[3 * k + 1];
-                if (D == 3) o[2] = xyz[3 * k + 2];
-            }
-            ++p;
+        for (uint32_t w = 0; w < 4; ++w) {
+            const uint32_t k = cnt[w];
+            if (w < wave) at += k;
+            total += k;
         }
+        if (ok) {
+            float *v = o + (size_t)at * D;
+            if (D == 2) {
+                *(float2 *)v = make_float2(x, y);
+            } else {
+                v[0] = x;
+                v[1] = y;
+                v[2] = z;
+            }
+        }
+        if (D == 3) run.step();
+    }
+    if (tid == 0) kept[c] = total;
+}
+
+// One workgroup: prefix[c] = vectors kept before chunk c, prefix[n] the total.
+__global__ __launch_bounds__(256) void k_mt_prefix(const uint32_t *__restrict__ kept, uint32_t n,
+                                                   uint32_t *__restrict__ prefix)
+{
+    __shared__ uint32_t part[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint32_t carry = 0;
+    for (uint32_t c0 = 0; c0 < n; c0 += 256) {
+        const uint32_t v = c0 + tid < n ? kept[c0 + tid] : 0u;
+        uint32_t inc = v;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(inc, d, 64);
+            if (lane >= (uint32_t)d) inc += o;
+        }
+        if (lane == 63) part[wave] = inc;
+        __syncthreads();
+        uint32_t at = carry + inc - v;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+            const uint32_t k = part[w];
+            if (w < wave) at += k;
+            carry += k;
+        }
+        if (c0 + tid < n) prefix[c0 + tid] = at;
+        __syncthreads();
+    }
+    if (tid == 0) prefix[n] = carry;
+}
+
+// The first kStreamRun vectors of chunk c + 1 behind chunk c's own, so that
+// a reader's run of that many never leaves the region it starts in.
+template <int D>
+__global__ __launch_bounds__(128) void k_mt_join(const uint32_t *__restrict__ kept, uint32_t stride, float *__restrict__ out)
+{
+    const size_t c = blockIdx.x;
+    float *dst = out + (c * stride + kept[c]) * D;
+    const float *src = out + (c + 1) * stride * D;
+    for (int i = threadIdx.x; i < kStreamRun * D; i += 128) dst[i] = src[i];
+}
+
+// The fill's first n vectors as one array.
+template <int D>
+__global__ __launch_bounds__(256) void k_mt_gather(StreamVectors sv, uint32_t n, float *__restrict__ out)
+{
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    if (j >= n) return;
+    const float *v = stream_at<D>(sv, j);
+#pragma unroll
+    for (int e = 0; e < D; ++e) out[(size_t)j * D + e] = v[e];
 }
 
 // The stream moves past the try that kept the m-th vector (m >= 1, at most
-// part[nb]): the draws up to it are consumed, and the array becomes the
-// block holding the next draw (its words untempered from raw), idx its
-// position there -- 624 when the next draw starts a new block, as the
-// generator itself leaves it.  The workgroup holding the m-th kept try is
-// found by a binary search over part, the try by recounting its tries.
+// the total): the chunk and the checkpoint before it are found by every
+// thread at once, its rounds run again to the try, and the context's array
+// becomes the 624 words from the next draw on (idx 0).
 template <int D>
-__global__ __launch_bounds__(256) void k_mt_commit(MtState *__restrict__ st, const uint32_t *__restrict__ raw,
-                                                   const uint32_t *__restrict__ part, uint32_t nb, uint32_t T,
-                                                   uint32_t m)
+__global__ __launch_bounds__(256) void k_mt_commit(MtState *__restrict__ st, const uint32_t *__restrict__ prefix, uint32_t n,
+                                                   uint32_t T, uint32_t n_ck, const uint32_t *__restrict__ ck_words,
+                                                   const uint32_t *__restrict__ ck_kept, uint32_t m)
 {
-    __shared__ uint32_t s_b, s_t;
-    __shared__ uint32_t lds4[4];
-    const int tid = threadIdx.x;
-    const uint32_t idx0 = st->idx;
-    if (tid == 0) {
-        uint32_t lo = 0, hi = nb - 1;   // the smallest b with part[b + 1] >= m
-        while (lo < hi) {
-            const uint32_t mid = lo + (hi - lo) / 2;
-            if (part[mid + 1] >= m) hi = mid;
-            else lo = mid + 1;
+    constexpr uint32_t R = kMtRing - 1;
+    __shared__ uint32_t ring[kMtRing];
+    __shared__ uint32_t cnt[4];
+    __shared__ uint32_t s_c, s_k, s_t;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (uint32_t c = tid; c < n; c += 256)
+        if (prefix[c] < m && m <= prefix[c + 1]) s_c = c;
+    __syncthreads();
+    const uint32_t c = s_c, want = m - prefix[c];   // the want-th kept of chunk c
+    const uint32_t *ck = ck_kept + (size_t)c * n_ck;
+    for (uint32_t k = tid; k < n_ck; k += 256)
+        if (ck[k] < want && (k + 1 == n_ck || want <= ck[k + 1])) s_k = k;
+    __syncthreads();
+    const uint32_t k = s_k;
+    for (uint32_t i = tid; i < kMtN; i += 256) ring[i] = ck_words[((size_t)c * n_ck + k) * kMtN + i];
+    __syncthreads();
+    MtRun run(ring);
+    uint32_t total = ck[k], t0 = 0;
+    const uint32_t first = k * kMtCkRounds * kMtLag;   // the checkpoint's try
+    for (; first + t0 < T; t0 += kMtLag) {
+        run.step();
+        float x, y, z;
+        const bool ok = mt_try<D>(ring, D * (t0 + tid), x, y, z) && tid < kMtLag && first + t0 + tid < T;
+        const unsigned long long b = __ballot(ok);
+        if (lane == 0) cnt[wave] = (uint32_t)__popcll(b);
+        run.step();
+        uint32_t at = total + (uint32_t)__popcll(b & ((1ull << lane) - 1));
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+            const uint32_t q = cnt[w];
+            if (w < wave) at += q;
+            total += q;
         }
-        s_b = lo;
+        if (ok && at + 1 == want) s_t = t0 + tid;
+        if (D == 3) run.step();
+        if (total >= want) break;
     }
     __syncthreads();
-    {
-        float xyz[3 * kTryItems];
-        const uint32_t t0 = s_b * kTryTile + (uint32_t)tid * kTryItems;
-        const uint32_t kept = mt_tries8<D>(raw, T, t0, xyz);
-        const uint32_t cnt = (uint32_t)__popc(kept);
-        uint32_t total;
-        const uint32_t ex = part[s_b] + try_block_scan(cnt, lds4, total);
-        if (ex < m && m <= ex + cnt) {
-            // the (m - ex)-th kept try of this thread's eight
-            uint32_t j = m - ex, k = 0;
-            for (; k < kTryItems; ++k)
-                if (((kept >> k) & 1u) && --j == 0) break;
-            s_t = t0 + k;
-        }
-    }
-    __syncthreads();
-    const unsigned long long e = (unsigned long long)D * (s_t + 1ull);
-    unsigned long long blk = (idx0 + e) / kMtN;
-    uint32_t idx1 = (uint32_t)((idx0 + e) % kMtN);
-    if (idx1 == 0) {
-        blk -= 1;
-        idx1 = kMtN;
-    }
-    if (blk > 0) {
-        const uint32_t *src = raw + (kMtN - idx0) + (size_t)(blk - 1) * kMtN;
-        for (int i = tid; i < (int)kMtN; i += 256) st->mt[i] = mt_untemper(src[i]);
-    }
-    __syncthreads();   // every thread has read idx before it changes
+    const uint32_t w = D * (s_t + 1);   // the next draw, in words past the checkpoint
+    for (uint32_t i = tid; i < kMtN; i += 256) st->mt[i] = ring[(w + i) & R];
     if (tid == 0) {
-        st->idx = idx1;
-        st->draws += e;
+        st->idx = 0;
+        st->draws += (unsigned long long)D * ((unsigned long long)c * T + first + s_t + 1ull);
     }
 }
 
-static inline unsigned blocks256(size_t n) { return (unsigned)((n + 255) / 256); }
-
-void launch_mt_base(const MtState *st, uint32_t *base, hipStream_t s)
+void launch_mt_base(const MtState *st, uint32_t n, uint32_t *base, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mt_base, dim3(1), dim3(256), 0, s, st, base);
+    hipLaunchKernelGGL(k_mt_base, dim3(1), dim3(256), 0, s, st, n, base);
 }
 
 void launch_mt_jump(const uint32_t *base, const uint64_t *polys, int n_jumps, uint32_t *states, hipStream_t s)
@@ -473,35 +456,40 @@ void launch_mt_jump(const uint32_t *base, const uint64_t *polys, int n_jumps, ui
     hipLaunchKernelGGL(k_mt_jump, dim3(n_jumps), dim3(kJumpThreads), 0, s, base, polys, states);
 }
 
-void launch_mt_gen(const MtState *st, const uint32_t *states, int n_chunks, int K, uint32_t *raw, hipStream_t s)
+uint32_t mt_checkpoints(uint32_t T) { return (T + kMtLag * kMtCkRounds - 1) / (kMtLag * kMtCkRounds); }
+
+template <int D>
+static void launch_mt_fill_t(const uint32_t *base, const uint32_t *states, const MtFill &f, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mt_gen, dim3(n_chunks), dim3(256), 0, s, st, states, K, raw);
+    hipLaunchKernelGGL(k_mt_fill<D>, dim3(f.chunks), dim3(256), 0, s, base, states, f.T, f.stride, f.n_ck, f.out, f.kept,
+                       f.ck_words, f.ck_kept);
+    hipLaunchKernelGGL(k_mt_prefix, dim3(1), dim3(256), 0, s, f.kept, f.chunks, f.prefix);
+    if (f.chunks > 1) hipLaunchKernelGGL(k_mt_join<D>, dim3(f.chunks - 1), dim3(128), 0, s, f.kept, f.stride, f.out);
 }
 
-uint32_t mt_try_blocks(uint32_t T) { return (T + kTryTile - 1) / kTryTile; }
-
-void launch_mt_count(int D, const uint32_t *raw, uint32_t T, uint32_t *part, hipStream_t s)
+void launch_mt_fill(const uint32_t *base, const uint32_t *states, const MtFill &f, hipStream_t s)
 {
-    if (T == 0) return;
-    if (D == 3) hipLaunchKernelGGL(k_mt_count<3>, dim3(mt_try_blocks(T)), dim3(256), 0, s, raw, T, part);
-    else hipLaunchKernelGGL(k_mt_count<2>, dim3(mt_try_blocks(T)), dim3(256), 0, s, raw, T, part);
+    if (f.D == 3) launch_mt_fill_t<3>(base, states, f, s);
+    else launch_mt_fill_t<2>(base, states, f, s);
 }
 
-void launch_mt_take(int D, const uint32_t *raw, uint32_t T, const uint32_t *part, uint32_t n, float *out,
-                    hipStream_t s)
+void launch_mt_commit(MtState *st, const MtFill &f, uint32_t m, hipStream_t s)
 {
-    if (T == 0 || n == 0) return;
-    if (D == 3) hipLaunchKernelGGL(k_mt_take<3>, dim3(mt_try_blocks(T)), dim3(256), 0, s, raw, T, part, n, out);
-    else hipLaunchKernelGGL(k_mt_take<2>, dim3(mt_try_blocks(T)), dim3(256), 0, s, raw, T, part, n, out);
+    if (m == 0) return;
+    if (f.D == 3)
+        hipLaunchKernelGGL(k_mt_commit<3>, dim3(1), dim3(256), 0, s, st, f.prefix, f.chunks, f.T, f.n_ck, f.ck_words,
+                           f.ck_kept, m);
+    else
+        hipLaunchKernelGGL(k_mt_commit<2>, dim3(1), dim3(256), 0, s, st, f.prefix, f.chunks, f.T, f.n_ck, f.ck_words,
+                           f.ck_kept, m);
 }
 
-void launch_mt_commit(int D, MtState *st, const uint32_t *raw, const uint32_t *part, uint32_t T, uint32_t m,
-                      hipStream_t s)
+void launch_mt_gather(const MtFill &f, uint32_t n, float *out, hipStream_t s)
 {
-    if (T == 0 || m == 0) return;
-    const uint32_t nb = mt_try_blocks(T);
-    if (D == 3) hipLaunchKernelGGL(k_mt_commit<3>, dim3(1), dim3(256), 0, s, st, raw, part, nb, T, m);
-    else hipLaunchKernelGGL(k_mt_commit<2>, dim3(1), dim3(256), 0, s, st, raw, part, nb, T, m);
+    if (n == 0) return;
+    const unsigned b = (unsigned)(((size_t)n + 255) / 256);
+    if (f.D == 3) hipLaunchKernelGGL(k_mt_gather<3>, dim3(b), dim3(256), 0, s, f.vectors(), n, out);
+    else hipLaunchKernelGGL(k_mt_gather<2>, dim3(b), dim3(256), 0, s, f.vectors(), n, out);
 }
 
 }  // namespace fgl

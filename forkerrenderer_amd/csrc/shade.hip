@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void k_lighting(FrameUniforms u, const float *
     lighting_px<STREAM>(u, g, ao, ao_is_one, smap, ss, fb, x, y, net);
 }
 
-__global__ __launch_bounds__(256) void k_ssao_ref(FrameUniforms u, const float *__restrict__ samples,
+__global__ __launch_bounds__(256) void k_ssao_ref(FrameUniforms u, StreamVectors samples,
                                                   const float *__restrict__ pow3,
                                                   const float *__restrict__ depth,
                                                   const float *__restrict__ g, float *__restrict__ ao)
@@ -155,9 +155,9 @@ constexpr int kGuesses = 2;     // prediction rounds per segment (more do not pa
 // The blocker search of an undecided point at sample offset o (the stream
 // samples' loads grouped as in the shading, fgl_device.hpp).
 __device__ __forceinline__ bool pcss_search(const FrameUniforms &u, const float *__restrict__ smap,
-                                            const float *__restrict__ pairs, float4 q, uint32_t o)
+                                            const StreamVectors &pairs, float4 q, uint32_t o)
 {
-    const float dB = pcss_blocker_stream(u, smap, vec3(q.x, q.y, q.z), q.w, pairs + 2 * (size_t)o, u.shadow.n_blocker);
+    const float dB = pcss_blocker_stream(u, smap, vec3(q.x, q.y, q.z), q.w, stream_at<2>(pairs, o), u.shadow.n_blocker);
     return !((double)dB < 0.001);
 }
 
@@ -172,7 +172,7 @@ __device__ __forceinline__ uint32_t pcss_predict(const uint32_t *__restrict__ pr
 }
 
 __global__ __launch_bounds__(256) void k_pcss_guess(FrameUniforms u, const float *__restrict__ smap,
-                                                    const float *__restrict__ pairs, const float4 *__restrict__ pt,
+                                                    StreamVectors pairs, const float4 *__restrict__ pt,
                                                     const uint32_t *__restrict__ pbase, uint32_t s0, uint32_t L,
                                                     uint32_t M0, float rate, const uint32_t *__restrict__ pred,
                                                     uint32_t *__restrict__ miss)
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void k_pcss_guess(FrameUniforms u, const float
 }
 
 __global__ __launch_bounds__(256) void k_pcss_band(FrameUniforms u, const float *__restrict__ smap,
-                                                   const float *__restrict__ pairs, const float4 *__restrict__ pt,
+                                                   StreamVectors pairs, const float4 *__restrict__ pt,
                                                    const uint32_t *__restrict__ pbase, uint32_t s0, uint32_t L,
                                                    uint32_t M0, const uint32_t *__restrict__ pred,
                                                    unsigned long long *__restrict__ masks)
@@ -564,7 +564,7 @@ void launch_lighting(const FrameUniforms &u, const float *gbuf, const float *ao,
                      const float *shadow_map, const ShadowSamples &ss, float *fb, hipStream_t s)
 {
     if (u.W <= 0 || u.H <= 0) return;
-    if (ss.pairs)
+    if (ss.sv.v)
         hipLaunchKernelGGL(k_lighting<true>, grid2(u.W, u.H), dim3(256), 0, s, u, gbuf, ao, ao_is_one, net,
                            shadow_map, ss, fb);
     else
@@ -572,7 +572,7 @@ void launch_lighting(const FrameUniforms &u, const float *gbuf, const float *ao,
                            shadow_map, ss, fb);
 }
 
-void launch_ssao_reference(const FrameUniforms &u, const float *samples, const float *pow3,
+void launch_ssao_reference(const FrameUniforms &u, const StreamVectors &samples, const float *pow3,
                            const float *depth, const float *gbuf, float *ao, hipStream_t s)
 {
     if (u.W <= 0 || u.H <= 0) return;
@@ -600,7 +600,7 @@ void launch_pcss_points(const FrameUniforms &u, const float *g, size_t P, const 
     hipLaunchKernelGGL(k_pcss_points, dim3((n + 255) / 256), dim3(256), 0, s, u, g, P, base, list, n, pt, pbase);
 }
 
-void launch_pcss_segment(const FrameUniforms &u, const float *shadow_map, const float *pairs, const float4 *pt,
+void launch_pcss_segment(const FrameUniforms &u, const float *shadow_map, const StreamVectors &pairs, const float4 *pt,
                          const uint32_t *pbase, uint32_t s0, uint32_t L, uint32_t M0, float rate, uint32_t *pred,
                          uint32_t *scan_tmp, unsigned long long *masks, unsigned long long *fbits, uint32_t *res,
                          uint32_t *found, uint32_t *out, hipStream_t s)

@@ -32,7 +32,7 @@ __device__ __forceinline__ void lighting_px(const FrameUniforms &u, const float 
     if (net.lao) pa.x *= net.fmask[i] ? net_ao_interp(net.lao, net.lW, net.lH, net.f, x, y) : 1.f;
     else if (!ao_is_one) pa.x *= ao[i];
     const float *rdisk = nullptr;
-    if (STREAM && ss.pairs) rdisk = ss.pairs + 2 * (ss.offs ? (size_t)ss.offs[i] : i * (size_t)ss.stride);
+    if (STREAM && ss.sv.v) rdisk = ss.at(i);
     Vec3 c = shade_point<STREAM>(u, smap, !(type < 0.5f), true, Pw, N, L, al, em, pa, rdisk);
     fb[i] = c.x;
     fb[P + i] = c.y;
@@ -143,8 +143,11 @@ __device__ __forceinline__ void ssao_px_with(const FrameUniforms &u, const SsaoA
 // (undefined in the reference; here no occlusion).  Each occluding sample
 // adds 1/32 (exact); ao = powf(1 - occlusion, 3) by table.  The samples are
 // the pixel's own (384 bytes a pixel), so they are read 8 at a time (16-byte
-// loads), and the 8 depths they project to are loaded together.
-__device__ __forceinline__ void ssao_ref_px(const FrameUniforms &u, const float *__restrict__ samples,
+// loads, 4-byte aligned: a vector is 12 bytes), and the 8 depths they project
+// to are loaded together.
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ void ssao_ref_px(const FrameUniforms &u, const StreamVectors &samples,
                                             const float *__restrict__ pow3, const float *__restrict__ depth,
                                             const float *__restrict__ g, float *__restrict__ ao, int x, int y)
 {
@@ -153,13 +156,13 @@ __device__ __forceinline__ void ssao_ref_px(const FrameUniforms &u, const float 
     const Vec3 N = vec3(g[i], g[P + i], g[2 * P + i]);
     const Vec3 Pw = vec3(g[3 * P + i], g[4 * P + i], g[5 * P + i]);
     const float fd = depth[i];
-    const float4 *smp = (const float4 *)(samples + i * 96);   // 16-byte aligned: 384 bytes a pixel
+    const v4f_any *smp = (const v4f_any *)stream_at<3>(samples, (uint32_t)i * 32u);
     int count = 0;
     for (int s0 = 0; s0 < 32; s0 += 8) {
         float v[24];
 #pragma unroll
         for (int e = 0; e < 6; ++e) {
-            const float4 q = smp[(s0 * 3) / 4 + e];
+            const v4f_any q = smp[(s0 * 3) / 4 + e];
             v[4 * e] = q.x;
             v[4 * e + 1] = q.y;
             v[4 * e + 2] = q.z;
