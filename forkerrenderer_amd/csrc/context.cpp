@@ -937,7 +937,7 @@ static int rng_fill(fgl_ctx *c, int D, uint32_t n)
         f.chunks = (uint32_t)Nc;
         f.T = (uint32_t)K * 624u / (uint32_t)D;
         f.stride = (f.T + kStreamRun + 3u) & ~3u;
-        f.n_ck = mt_checkpoints(f.T);
+        f.n_ck = mt_checkpoints(f.T * (uint32_t)D);
         const size_t cks = (size_t)Nc * f.n_ck;
         if ((rc = ensure(c, c->mt_vec, (size_t)Nc * f.stride * D * sizeof(float))) ||
             (rc = ensure(c, c->mt_ck, (cks * 625 + 2 * (size_t)Nc + 1) * 4)) ||

@@ -212,7 +212,7 @@ void launch_mt_jump(const uint32_t *base, const uint64_t *polys, int n_jumps, ui
 // (x, y, z); 2: RandomVectorInUnitDisk (x, y)): T tries of D draws a chunk,
 // the kept vectors of chunk c at out + c stride D (stride >= T + kStreamRun),
 // prefix[c] = vectors kept before it (chunks + 1 entries), n_ck checkpoints a
-// chunk (mt_checkpoints(T); 624 words and a count each).  A commit moves the
+// chunk (mt_checkpoints(T D); 624 words and a count each).  A commit moves the
 // stream past the try that kept the m-th vector.
 struct MtFill {
     int D;
@@ -225,7 +225,7 @@ struct MtFill {
         return StreamVectors{out, prefix, chunks, stride, 1.f / per};
     }
 };
-uint32_t mt_checkpoints(uint32_t T);
+uint32_t mt_checkpoints(uint32_t words);
 void launch_mt_fill(const uint32_t *base, const uint32_t *states, const MtFill &f, hipStream_t s);
 void launch_mt_commit(MtState *st, const MtFill &f, uint32_t m, hipStream_t s);
 // The fill's first n vectors as one array.

@@ -61,17 +61,17 @@ __device__ __forceinline__ float random_pm1(uint32_t u)
 }
 
 // The generator as one sequence: x_{n+624} = twist(x_n, x_{n+1}, x_{n+397})
-// (a block's twist is this recurrence, new words used as they appear).  The
-// 227 words x_n .. x_{n+226} read only words at least 227 back, so a
-// workgroup makes them together, one barrier per step, keeping the last 2048
-// words in an LDS ring (word n in slot n % 2048).  In step s thread t makes
-// x_{624+j}, j = 227 s + t, from x_j and x_{j+1} (made two steps back or
-// earlier, so read during the step before, while it computes) and x_{j+397}
-// (the word the thread made in the step before).
+// (a block's twist is this recurrence, new words used as they appear).  227
+// consecutive words read only words at least 227 back, so a workgroup makes
+// them together, a thread each -- and the next 227 as well before anyone has
+// to wait: thread t's second word reads x_{j+227} and x_{j+228}, at least 396
+// back, and its own first word.  So a pair of steps, 454 words, takes one
+// barrier.  The last 2048 words are kept in an LDS ring (word n in slot n %
+// 2048).
 //
-// The barrier orders LDS alone: a __syncthreads() also waits for the step's
-// global stores, which made a step 860 cycles.
-constexpr uint32_t kMtRing = 2048, kMtLag = kMtN - kMtM;
+// The barrier orders LDS alone: a __syncthreads() also waits for the
+// interval's global stores, which made a step of 227 words 860 cycles.
+constexpr uint32_t kMtRing = 2048, kMtLag = kMtN - kMtM, kMtPair = 2 * kMtLag;
 
 __device__ __forceinline__ void mt_barrier()
 {
@@ -80,36 +80,30 @@ __device__ __forceinline__ void mt_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// A running generator: the ring holds x_0 .. x_{623 + made}.  Needs at least
-// 227 threads; every thread of the workgroup calls it.
+// A running generator: the ring holds x_0 .. x_{623 + made}.  The first 227
+// threads make words; `far` is x_{made + 397 + t}, the thread's own last one.
 struct MtRun {
     uint32_t *ring;
-    uint32_t made, cur, nxt, far;
-    __device__ __forceinline__ explicit MtRun(uint32_t *r) : ring(r), made(0), cur(0), nxt(0), far(0)
+    uint32_t made, far;
+    __device__ __forceinline__ explicit MtRun(uint32_t *r) : ring(r), made(0), far(0)
     {
-        if (threadIdx.x < kMtLag) {
-            cur = ring[threadIdx.x];
-            nxt = ring[threadIdx.x + 1];
-            far = ring[threadIdx.x + kMtM];
-        }
+        if (threadIdx.x < kMtLag) far = ring[threadIdx.x + kMtM];
     }
-    // 227 more words; this thread's (the first 227 threads) is returned.
-    __device__ __forceinline__ uint32_t step()
+    // 454 more words (w0, w1: this thread's), ready after the next barrier.
+    __device__ __forceinline__ void pair(uint32_t &w0, uint32_t &w1)
     {
         constexpr uint32_t R = kMtRing - 1;
-        uint32_t v = 0;
         if (threadIdx.x < kMtLag) {
             const uint32_t j = made + threadIdx.x;
-            const uint32_t ncur = ring[(j + kMtLag) & R], nnxt = ring[(j + kMtLag + 1) & R];
-            v = mt_twist_word(cur, nxt, far);
-            ring[(j + kMtN) & R] = v;
-            cur = ncur;
-            nxt = nnxt;
-            far = v;
+            const uint32_t c0 = ring[j & R], n0 = ring[(j + 1) & R];
+            const uint32_t c1 = ring[(j + kMtLag) & R], n1 = ring[(j + kMtLag + 1) & R];
+            w0 = mt_twist_word(c0, n0, far);
+            w1 = mt_twist_word(c1, n1, w0);
+            ring[(j + kMtN) & R] = w0;
+            ring[(j + kMtN + kMtLag) & R] = w1;
+            far = w1;
         }
-        made += kMtLag;
-        mt_barrier();
-        return v;
+        made += kMtPair;
     }
 };
 
@@ -137,7 +131,7 @@ __device__ __forceinline__ bool mt_try(const uint32_t *ring, uint32_t p, float &
 // x_i .. x_{i+623} over the set bits i of t^(c L) mod phi.  A chunk makes its
 // words in an LDS ring, tests its tries there and writes the kept vectors
 // only; its draws never reach memory.  Checkpoints -- the generator's words
-// and the vectors kept so far, every kMtCkRounds rounds -- let a commit find
+// and the vectors kept so far, every kMtCkEvery intervals -- let a commit find
 // the try that kept the m-th vector without the draws.  Every window of a
 // jump, x_{19967 + 623} at most, lies in the base sequence.
 static_assert(kMtBaseWords >= 64 * kMtPolyWords + 623, "the jump's windows stay in the base sequence");
@@ -154,9 +148,14 @@ __global__ __launch_bounds__(256) void k_mt_base(const MtState *__restrict__ st,
     }
     __syncthreads();
     MtRun run(ring);
-    for (uint32_t at = kMtN - idx; at < n; at += kMtLag) {
-        const uint32_t v = run.step();
-        if (tid < kMtLag && at + tid < n) base[at + tid] = v;
+    for (uint32_t at = kMtN - idx; at < n; at += kMtPair) {
+        uint32_t w0, w1;
+        run.pair(w0, w1);
+        if (tid < kMtLag) {
+            if (at + tid < n) base[at + tid] = w0;
+            if (at + kMtLag + tid < n) base[at + kMtLag + tid] = w1;
+        }
+        mt_barrier();
     }
 }
 
@@ -280,62 +279,103 @@ __global__ __launch_bounds__(kJumpThreads) void k_mt_jump(const uint32_t *__rest
         states[(size_t)c * kMtN + k] = part[0][k] ^ part[1][k + 1] ^ part[2][k + 2] ^ part[3][k + 3];
 }
 
-// Workgroup c runs chunk c: rounds of D steps, 227 tries a round (a thread
-// each), T tries in all.  A round's tries are read, tempered and tested in
-// the interval before its last steps' barrier and written after it, when
-// every wavefront's count is known.  The step is bound by its LDS latency and
-// barrier; written as tempered draws, counted, scanned and read back by two
-// more kernels, the same fill took 1,390 us for 187 M draws (D = 3).
-constexpr uint32_t kMtCkRounds = 32;
-
+// The tries of interval q (the words of one pair): [mt_first(q), mt_first(q +
+// 1)), at most 227, all of whose words the ring holds when the interval
+// starts.
 template <int D>
-__global__ __launch_bounds__(256) void k_mt_fill(const uint32_t *__restrict__ base, const uint32_t *__restrict__ states,
-                                                 uint32_t T, uint32_t stride, uint32_t n_ck, float *__restrict__ out,
-                                                 uint32_t *__restrict__ kept, uint32_t *__restrict__ ck_words,
-                                                 uint32_t *__restrict__ ck_kept)
-{
-    constexpr uint32_t R = kMtRing - 1;
-    __shared__ uint32_t ring[kMtRing];
-    __shared__ uint32_t cnt[4];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = blockIdx.x;
-    const uint32_t *src = c == 0 ? base : states + (size_t)c * kMtN;
-    for (uint32_t i = tid; i < kMtN; i += 256) ring[i] = src[i];
-    __syncthreads();
-    MtRun run(ring);
-    float *o = out + (size_t)c * stride * D;
-    uint32_t total = 0;
-    for (uint32_t t0 = 0, r = 0; t0 < T; t0 += kMtLag, ++r) {
-        if (r % kMtCkRounds == 0) {
-            const size_t k = (size_t)c * n_ck + r / kMtCkRounds;
-            for (uint32_t i = tid; i < kMtN; i += 256) ck_words[k * kMtN + i] = ring[(D * t0 + i) & R];
-            if (tid == 0) ck_kept[k] = total;
-        }
-        run.step();
-        float x, y, z;
-        const bool ok = mt_try<D>(ring, D * (t0 + tid), x, y, z) && tid < kMtLag && t0 + tid < T;
-        const unsigned long long m = __ballot(ok);
-        if (lane == 0) cnt[wave] = (uint32_t)__popcll(m);
-        run.step();
-        uint32_t at = total + (uint32_t)__popcll(m & ((1ull << lane) - 1));
+__device__ __forceinline__ uint32_t mt_first(uint32_t q) { return q * kMtPair / (uint32_t)D; }
+
+// Half a workgroup's tries over the generator's intervals: in an interval a
+// thread tests one try of it and writes the vector it kept in the one
+// before, whose wavefronts' counts the barrier between has published.
+template <int D>
+struct MtTries {
+    uint32_t total;       // kept before the interval being tested
+    uint32_t rank;        // this thread's vector among its wavefront's
+    bool ok;
+    float x, y, z;
+    __device__ __forceinline__ MtTries() : total(0), rank(0), ok(false), x(0.f), y(0.f), z(0.f) {}
+    // The interval before, counted: where this thread's vector goes (valid
+    // when ok).
+    __device__ __forceinline__ uint32_t settle(const uint32_t *cnt, uint32_t wave)
+    {
+        uint32_t at = total + rank;
 #pragma unroll
         for (uint32_t w = 0; w < 4; ++w) {
             const uint32_t k = cnt[w];
             if (w < wave) at += k;
             total += k;
         }
-        if (ok) {
+        return at;
+    }
+    __device__ __forceinline__ void test(const uint32_t *ring, uint32_t *cnt, uint32_t q, uint32_t T, uint32_t i)
+    {
+        const uint32_t t = mt_first<D>(q) + i, end = mt_first<D>(q + 1);
+        ok = mt_try<D>(ring, D * t, x, y, z) && t < end && t < T;
+        const unsigned long long m = __ballot(ok);
+        rank = (uint32_t)__popcll(m & ((1ull << (i & 63)) - 1));
+        if ((i & 63) == 0) cnt[i >> 6] = (uint32_t)__popcll(m);
+    }
+};
+
+// Workgroup c runs chunk c, T tries: four wavefronts make words, four test
+// tries and write the kept vectors.  An interval is bound by either half's
+// chain (LDS reads, some 60 operations, barrier); written as tempered draws,
+// counted, scanned and read back by two more kernels, 187 M draws (D = 3) took
+// 890 us.
+constexpr uint32_t kMtCkEvery = 33;   // intervals between checkpoints, a multiple of 3: whole tries
+
+template <int D>
+__global__ __launch_bounds__(512) void k_mt_fill(const uint32_t *__restrict__ base, const uint32_t *__restrict__ states,
+                                                 uint32_t T, uint32_t stride, uint32_t n_ck, float *__restrict__ out,
+                                                 uint32_t *__restrict__ kept, uint32_t *__restrict__ ck_words,
+                                                 uint32_t *__restrict__ ck_kept)
+{
+    constexpr uint32_t R = kMtRing - 1;
+    __shared__ uint32_t ring[kMtRing];
+    __shared__ uint32_t cnt[2][4];
+    const uint32_t tid = threadIdx.x, c = blockIdx.x;
+    const uint32_t *src = c == 0 ? base : states + (size_t)c * kMtN;
+    for (uint32_t i = tid; i < kMtN; i += 512) ring[i] = src[i];
+    if (tid < 8) cnt[tid >> 2][tid & 3] = 0u;
+    __syncthreads();
+    const uint32_t Q = (T * D + kMtPair - 1) / kMtPair;
+    if (tid < 256) {
+        MtRun run(ring);
+        for (uint32_t q = 0; q < Q; ++q) {
+            uint32_t w0, w1;
+            if (q % kMtCkEvery == 0) {
+                const size_t k = (size_t)c * n_ck + q / kMtCkEvery;
+                for (uint32_t i = tid; i < kMtN; i += 256) ck_words[k * kMtN + i] = ring[(kMtPair * q + i) & R];
+            }
+            run.pair(w0, w1);
+            mt_barrier();
+        }
+    } else {
+        const uint32_t i = tid - 256, wave = i >> 6;
+        float *o = out + (size_t)c * stride * D;
+        MtTries<D> tries;
+        auto write = [&](uint32_t q) {
+            const uint32_t at = tries.settle(cnt[(q + 1) & 1], wave);
+            if (!tries.ok) return;
             float *v = o + (size_t)at * D;
             if (D == 2) {
-                *(float2 *)v = make_float2(x, y);
+                *(float2 *)v = make_float2(tries.x, tries.y);
             } else {
-                v[0] = x;
-                v[1] = y;
-                v[2] = z;
+                v[0] = tries.x;
+                v[1] = tries.y;
+                v[2] = tries.z;
             }
+        };
+        for (uint32_t q = 0; q < Q; ++q) {
+            write(q);
+            if (q % kMtCkEvery == 0 && i == 0) ck_kept[(size_t)c * n_ck + q / kMtCkEvery] = tries.total;
+            tries.test(ring, cnt[q & 1], q, T, i);
+            mt_barrier();
         }
-        if (D == 3) run.step();
+        write(Q);
+        if (i == 0) kept[c] = tries.total;
     }
-    if (tid == 0) kept[c] = total;
 }
 
 // One workgroup: prefix[c] = vectors kept before chunk c, prefix[n] the total.
@@ -392,53 +432,52 @@ __global__ __launch_bounds__(256) void k_mt_gather(StreamVectors sv, uint32_t n,
 
 // The stream moves past the try that kept the m-th vector (m >= 1, at most
 // the total): the chunk and the checkpoint before it are found by every
-// thread at once, its rounds run again to the try, and the context's array
+// thread at once, its intervals run again to the try, and the context's array
 // becomes the 624 words from the next draw on (idx 0).
 template <int D>
-__global__ __launch_bounds__(256) void k_mt_commit(MtState *__restrict__ st, const uint32_t *__restrict__ prefix, uint32_t n,
+__global__ __launch_bounds__(512) void k_mt_commit(MtState *__restrict__ st, const uint32_t *__restrict__ prefix, uint32_t n,
                                                    uint32_t T, uint32_t n_ck, const uint32_t *__restrict__ ck_words,
                                                    const uint32_t *__restrict__ ck_kept, uint32_t m)
 {
     constexpr uint32_t R = kMtRing - 1;
     __shared__ uint32_t ring[kMtRing];
-    __shared__ uint32_t cnt[4];
+    __shared__ uint32_t cnt[2][4];
     __shared__ uint32_t s_c, s_k, s_t;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (uint32_t c = tid; c < n; c += 256)
+    const uint32_t tid = threadIdx.x;
+    if (tid < 8) cnt[tid >> 2][tid & 3] = 0u;
+    for (uint32_t c = tid; c < n; c += 512)
         if (prefix[c] < m && m <= prefix[c + 1]) s_c = c;
     __syncthreads();
     const uint32_t c = s_c, want = m - prefix[c];   // the want-th kept of chunk c
     const uint32_t *ck = ck_kept + (size_t)c * n_ck;
-    for (uint32_t k = tid; k < n_ck; k += 256)
+    for (uint32_t k = tid; k < n_ck; k += 512)
         if (ck[k] < want && (k + 1 == n_ck || want <= ck[k + 1])) s_k = k;
     __syncthreads();
     const uint32_t k = s_k;
-    for (uint32_t i = tid; i < kMtN; i += 256) ring[i] = ck_words[((size_t)c * n_ck + k) * kMtN + i];
+    for (uint32_t i = tid; i < kMtN; i += 512) ring[i] = ck_words[((size_t)c * n_ck + k) * kMtN + i];
     __syncthreads();
+    const uint32_t first = mt_first<D>(k * kMtCkEvery);   // the checkpoint's try
+    const bool maker = tid < 256;
+    const uint32_t i = tid & 255, wave = i >> 6;
     MtRun run(ring);
-    uint32_t total = ck[k], t0 = 0;
-    const uint32_t first = k * kMtCkRounds * kMtLag;   // the checkpoint's try
-    for (; first + t0 < T; t0 += kMtLag) {
-        run.step();
-        float x, y, z;
-        const bool ok = mt_try<D>(ring, D * (t0 + tid), x, y, z) && tid < kMtLag && first + t0 + tid < T;
-        const unsigned long long b = __ballot(ok);
-        if (lane == 0) cnt[wave] = (uint32_t)__popcll(b);
-        run.step();
-        uint32_t at = total + (uint32_t)__popcll(b & ((1ull << lane) - 1));
-#pragma unroll
-        for (uint32_t w = 0; w < 4; ++w) {
-            const uint32_t q = cnt[w];
-            if (w < wave) at += q;
-            total += q;
-        }
-        if (ok && at + 1 == want) s_t = t0 + tid;
-        if (D == 3) run.step();
-        if (total >= want) break;
+    MtTries<D> tries;
+    uint32_t w0, w1;
+    // The vector lies in the checkpoint's kMtCkEvery intervals; every thread
+    // follows the counts and stops at the same one.
+    for (uint32_t q = 0; q <= kMtCkEvery; ++q) {
+        const uint32_t at = tries.settle(cnt[(q + 1) & 1], wave);
+        if (!maker && tries.ok && at + 1 + ck[k] == want) s_t = mt_first<D>(q - 1) + i;
+        if (tries.total + ck[k] >= want) break;
+        if (maker) run.pair(w0, w1);
+        else tries.test(ring, cnt[q & 1], q, T - first, i);
+        mt_barrier();
     }
+    // the window after a try at the end of its interval reaches into the
+    // next pair's words
+    if (maker) run.pair(w0, w1);
     __syncthreads();
     const uint32_t w = D * (s_t + 1);   // the next draw, in words past the checkpoint
-    for (uint32_t i = tid; i < kMtN; i += 256) st->mt[i] = ring[(w + i) & R];
+    for (uint32_t j = tid; j < kMtN; j += 512) st->mt[j] = ring[(w + j) & R];
     if (tid == 0) {
         st->idx = 0;
         st->draws += (unsigned long long)D * ((unsigned long long)c * T + first + s_t + 1ull);
@@ -456,12 +495,12 @@ void launch_mt_jump(const uint32_t *base, const uint64_t *polys, int n_jumps, ui
     hipLaunchKernelGGL(k_mt_jump, dim3(n_jumps), dim3(kJumpThreads), 0, s, base, polys, states);
 }
 
-uint32_t mt_checkpoints(uint32_t T) { return (T + kMtLag * kMtCkRounds - 1) / (kMtLag * kMtCkRounds); }
+uint32_t mt_checkpoints(uint32_t words) { return (words + kMtPair * kMtCkEvery - 1) / (kMtPair * kMtCkEvery); }
 
 template <int D>
 static void launch_mt_fill_t(const uint32_t *base, const uint32_t *states, const MtFill &f, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mt_fill<D>, dim3(f.chunks), dim3(256), 0, s, base, states, f.T, f.stride, f.n_ck, f.out, f.kept,
+    hipLaunchKernelGGL(k_mt_fill<D>, dim3(f.chunks), dim3(512), 0, s, base, states, f.T, f.stride, f.n_ck, f.out, f.kept,
                        f.ck_words, f.ck_kept);
     hipLaunchKernelGGL(k_mt_prefix, dim3(1), dim3(256), 0, s, f.kept, f.chunks, f.prefix);
     if (f.chunks > 1) hipLaunchKernelGGL(k_mt_join<D>, dim3(f.chunks - 1), dim3(128), 0, s, f.kept, f.stride, f.out);
@@ -477,10 +516,10 @@ void launch_mt_commit(MtState *st, const MtFill &f, uint32_t m, hipStream_t s)
 {
     if (m == 0) return;
     if (f.D == 3)
-        hipLaunchKernelGGL(k_mt_commit<3>, dim3(1), dim3(256), 0, s, st, f.prefix, f.chunks, f.T, f.n_ck, f.ck_words,
+        hipLaunchKernelGGL(k_mt_commit<3>, dim3(1), dim3(512), 0, s, st, f.prefix, f.chunks, f.T, f.n_ck, f.ck_words,
                            f.ck_kept, m);
     else
-        hipLaunchKernelGGL(k_mt_commit<2>, dim3(1), dim3(256), 0, s, st, f.prefix, f.chunks, f.T, f.n_ck, f.ck_words,
+        hipLaunchKernelGGL(k_mt_commit<2>, dim3(1), dim3(512), 0, s, st, f.prefix, f.chunks, f.T, f.n_ck, f.ck_words,
                            f.ck_kept, m);
 }
 
