@@ -338,7 +338,9 @@ __global__ __launch_bounds__(256) void k_pcss_offsets(const uint32_t *__restrict
 // the workgroup first copies the depth plane around its tile, 32 pixels
 // each side, into LDS (coalesced 16-byte loads), and taps that land there
 // read LDS; the others read the plane.  Per tap it issues about 42 vector
-// ALU operations (projection, reciprocal, bounds, address, compare).
+// ALU operations (projection, reciprocal, bounds, address, compare).  A
+// workgroup none of whose pixels can be occluded (nothing drawn there) is
+// done before the copy, a wavefront of a mixed one before its taps.
 constexpr int kSsaoTW = 64, kSsaoTH = 16, kSsaoHalo = 32;
 static_assert(kSsaoTW * kSsaoTH == 1024 && kSsaoHalo % 4 == 0, "one thread per pixel; 16-byte staging");
 constexpr int kSsaoLW = kSsaoTW + 2 * kSsaoHalo, kSsaoLH = kSsaoTH + 2 * kSsaoHalo;
@@ -351,6 +353,16 @@ __global__ __launch_bounds__(1024) void k_ssao_tiled(FrameUniforms u, SsaoArgs s
     __shared__ float tile[kSsaoLH * kSsaoLW];
     const int x0 = blockIdx.x * kSsaoTW, y0 = blockIdx.y * kSsaoTH;
     const int lx0 = x0 - kSsaoHalo, ly0 = y0 - kSsaoHalo;
+    const int x = x0 + (int)(threadIdx.x % kSsaoTW), y = y0 + (int)(threadIdx.x / kSsaoTW);
+    const bool on = x < u.W && y < u.H;
+    SsaoPx px;
+    px.none = true;
+    if (on) px = ssao_setup(u, sa, depth, g, x, y);
+    float *out = ao + (size_t)x + (size_t)y * u.W;
+    if (__syncthreads_and(px.none)) {
+        if (on) *out = 1.f;
+        return;
+    }
     const bool vec = (u.W & 3) == 0;   // rows start 16-byte aligned
     for (int k = threadIdx.x; k < kSsaoLH * kSsaoLW / 4; k += 1024) {
         const int row = k / (kSsaoLW / 4), c4 = k - row * (kSsaoLW / 4);
@@ -371,15 +383,18 @@ __global__ __launch_bounds__(1024) void k_ssao_tiled(FrameUniforms u, SsaoArgs s
         for (int e = 0; e < 4; ++e) tile[row * kSsaoLW + 4 * c4 + e] = v[e];
     }
     __syncthreads();
-    const int x = x0 + (int)(threadIdx.x % kSsaoTW), y = y0 + (int)(threadIdx.x / kSsaoTW);
-    if (x >= u.W || y >= u.H) return;
+    if (!on) return;
+    if (__all(px.none)) {
+        *out = 1.f;
+        return;
+    }
     const uint32_t W = (uint32_t)u.W;
     // The plane is read through a global-address-space pointer: with two
     // generic pointers the compiler merges both reads into one flat load,
     // which sends the LDS taps down the vector-memory path as well.
     const __attribute__((address_space(1))) float *gdepth =
         (const __attribute__((address_space(1))) float *)depth;
-    ssao_px_with(u, sa, depth, g, ao, x, y, [&](int sx, int sy) {
+    *out = ssao_taps(u, sa, px, [&](int sx, int sy) {
         const uint32_t tx = (uint32_t)(sx - lx0), ty = (uint32_t)(sy - ly0);
         const bool near = tx < (uint32_t)kSsaoLW && ty < (uint32_t)kSsaoLH;
         // Every lane reads LDS (a far lane at the tile's first word) and far
