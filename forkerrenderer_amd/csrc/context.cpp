@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <cstddef>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -65,6 +66,12 @@ struct fgl_ctx {
     DevBuf d_materials;
     bool materials_dirty = true;
     std::vector<ModelRes> models;
+    // map bundles made so far, by their texture ids (A, Z, N, Y; -1: not held)
+    struct Bundle {
+        int ids[4];
+        DevBundle b;
+    };
+    std::vector<Bundle> bundles;
 
     // ForkerGL state
     int W = 0, H = 0, SW = 0, SH = 0;
@@ -447,12 +454,60 @@ int fgl_upload_material(fgl_ctx *c, const fgl_material *m, int *out_id)
     for (int id : ids)
         if (id < -1 || id >= (int)c->textures.size())
             return fail(c, FGL_ERR_INVALID, "material references an unknown texture id");
-    DevMaterial d;
-    static_assert(sizeof(DevMaterial) == sizeof(fgl_material), "material layout");
-    std::memcpy(&d, m, sizeof(d));
+    DevMaterial d{};
+    static_assert(offsetof(DevMaterial, bundle) >= sizeof(fgl_material) &&
+                      offsetof(DevMaterial, map_pbr_ke) == offsetof(fgl_material, map_pbr_ke), "material layout");
+    std::memcpy((void *)&d, m, sizeof(fgl_material));
     c->materials.push_back(d);
     c->materials_dirty = true;
     *out_id = (int)c->materials.size() - 1;
+    return FGL_OK;
+}
+
+// The bundle (DevBundle) of material k's maps for the Blinn-Phong (0) or PBR
+// (1) shaders, made on first use from the maps that share the first one's
+// size, wrap and filter; a single map has none.
+static int ensure_bundle(fgl_ctx *c, int k, int pbr)
+{
+    DevMaterial &m = c->materials[k];
+    if (m.bundle[pbr].t) return FGL_OK;
+    fgl_ctx::Bundle n{{pbr ? m.map_base : m.map_kd, pbr ? m.map_rough : m.map_ks, m.map_bump, pbr ? m.map_metal : -1}, {}};
+    const DevTexture *first = nullptr, *t[4];
+    int maps = 0;
+    for (int j = 0; j < 4; ++j) {
+        t[j] = n.ids[j] >= 0 ? &c->textures[n.ids[j]] : nullptr;
+        if (t[j] && !first) first = t[j];
+        if (t[j] && (t[j]->w != first->w || t[j]->h != first->h || t[j]->wrap != first->wrap || t[j]->filter != first->filter)) {
+            t[j] = nullptr;
+            n.ids[j] = -1;
+        }
+        if (t[j]) {
+            n.b.has |= 1 << j;
+            ++maps;
+        }
+    }
+    if (maps < 2) return FGL_OK;
+    for (const fgl_ctx::Bundle &o : c->bundles)
+        if (std::memcmp(o.ids, n.ids, sizeof(n.ids)) == 0) {
+            m.bundle[pbr] = o.b;
+            c->materials_dirty = true;
+            return FGL_OK;
+        }
+    const int w = first->w, h = first->h;
+    void *mem = nullptr;
+    HIPCHK(c, hipMalloc(&mem, (size_t)((w + 3) / 4) * ((h + 3) / 4) * 16 * sizeof(uint2)));
+    c->texture_mem.push_back(mem);
+    launch_bundle(w, h, t[0] ? t[0]->texels : nullptr, t[1] ? t[1]->zb : nullptr, t[2] ? t[2]->texels : nullptr,
+                  t[3] ? t[3]->zb : nullptr, (uint2 *)mem, c->stream);
+    HIPCHK(c, hipGetLastError());
+    n.b.t = (const uint2 *)mem;
+    n.b.w = w;
+    n.b.h = h;
+    n.b.wrap = first->wrap;
+    n.b.filter = first->filter;
+    c->bundles.push_back(n);
+    m.bundle[pbr] = n.b;
+    c->materials_dirty = true;
     return FGL_OK;
 }
 
@@ -531,6 +586,10 @@ int fgl_upload_model(fgl_ctx *c, const fgl_model_desc *d, int *out_id)
             return fail(c, FGL_ERR_INVALID, "face material out of range");
     ModelRes m;
     int rc;
+    for (size_t f = 0; f < nf; ++f)
+        if ((f == 0 || d->face_material[f] != d->face_material[f - 1]) &&
+            (rc = ensure_bundle(c, d->face_material[f], d->support_pbr != 0)))
+            return rc;
     // The positions are kept in the order the faces, taken in spatial order,
     // first use them, so that neighbouring triangles' vertex records are
     // neighbours; vi indexes that order.

@@ -131,6 +131,9 @@ struct SsaoArgs {
 };
 
 // raster.hip
+// The texels of a bundle of w x h maps (null: not held), in its block order.
+void launch_bundle(int w, int h, const uint32_t *a, const uint8_t *z, const uint32_t *n, const uint8_t *y, uint2 *out,
+                   hipStream_t s);
 // The corner records of a model from its attribute arrays (tan may be null).
 void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti,
                     const int *ni, size_t n, float4 *out, hipStream_t s);

@@ -40,6 +40,23 @@ __global__ __launch_bounds__(256) void k_corners(const float *__restrict__ pos, 
     out[3 * k + 2] = g ? make_float4(g[0], g[1], g[2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
+// A bundle's texels (DevBundle) from its maps' own, a thread per texel in the
+// bundle's order; maps it does not hold are null.
+__global__ __launch_bounds__(256) void k_bundle(int w, int h, const uint32_t *__restrict__ a, const uint8_t *__restrict__ z,
+                                                const uint32_t *__restrict__ n, const uint8_t *__restrict__ y,
+                                                uint2 *__restrict__ out)
+{
+    const int tx = blockIdx.x * 64 + (threadIdx.x >> 4) * 4 + (threadIdx.x & 3), ty = blockIdx.y * 4 + ((threadIdx.x >> 2) & 3);
+    if (tx >= w || ty >= h) return;
+    const size_t i = (size_t)tx + (size_t)ty * w;
+    uint2 o = make_uint2(0u, 0u);
+    if (a) o.x = a[i] & 0xffffffu;
+    if (z) o.x |= (uint32_t)z[i] << 24;
+    if (n) o.y = n[i] & 0xffffffu;
+    if (y) o.y |= (uint32_t)y[i] << 24;
+    out[bundle_index(w, tx, ty)] = o;
+}
+
 // One thread per (draw, position); the first thread also zeroes *zero (the
 // pass's big-triangle counter, which setup counts up next).
 template <bool SHADOW>
@@ -275,27 +292,33 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
     Varying v0 = main_vertex(dr, u, f, 0);
     Varying v1 = main_vertex(dr, u, f, 1);
     Varying v2 = main_vertex(dr, u, f, 2);
-    FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump);
+    const DevBundle &bn = m.bundle[dr.support_pbr ? 1 : 0];
+    FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, bn);
     // the stochastic shadow filters: this fragment's samples in the stream
     const float *rdisk = nullptr;
     if (STREAM && a.ss.sv.v) rdisk = a.ss.at(i);
     Vec3 c;
     if (!dr.support_pbr) {
-        Vec3 dc = m.map_kd >= 0 ? tex_sample(a.textures, m.map_kd, fg.uv)
-                                : vec3(m.kd[0], m.kd[1], m.kd[2]);
+        Vec3 dc = (bn.has & kBundleA) ? fg.maps.a
+                : m.map_kd >= 0       ? tex_sample(a.textures, m.map_kd, fg.uv)
+                                      : vec3(m.kd[0], m.kd[1], m.kd[2]);
         Vec3 em = m.map_ke >= 0 ? tex_sample(a.textures, m.map_ke, fg.uv)
                                 : vec3(m.ke[0], m.ke[1], m.ke[2]);
         float shin = 1.f;
-        if (m.map_ks >= 0) shin = tex_samplef(a.textures, m.map_ks, fg.uv) + 5;
+        if (bn.has & kBundleZ) shin = fg.maps.z + 5;
+        else if (m.map_ks >= 0) shin = tex_samplef(a.textures, m.map_ks, fg.uv) + 5;
         c = shade_point<STREAM>(u, a.shadow_map, false, false, fg.pos, fg.normal, fg.lndc, dc, em,
                         vec3(m.ka[0], m.ks[0], shin), rdisk);
     } else {
-        Vec3 al = m.map_base >= 0 ? tex_sample(a.textures, m.map_base, fg.uv)
-                                  : vec3(m.albedo[0], m.albedo[1], m.albedo[2]);
+        Vec3 al = (bn.has & kBundleA) ? fg.maps.a
+                : m.map_base >= 0     ? tex_sample(a.textures, m.map_base, fg.uv)
+                                      : vec3(m.albedo[0], m.albedo[1], m.albedo[2]);
         Vec3 em = m.map_pbr_ke >= 0 ? tex_sample(a.textures, m.map_pbr_ke, fg.uv)
                                     : vec3(m.pbr_ke[0], m.pbr_ke[1], m.pbr_ke[2]);
-        float rough = m.map_rough >= 0 ? tex_samplef(a.textures, m.map_rough, fg.uv) : m.roughness;
-        float metal = m.map_metal >= 0 ? tex_samplef(a.textures, m.map_metal, fg.uv) : m.metalness;
+        float rough = (bn.has & kBundleZ) ? fg.maps.z
+                    : m.map_rough >= 0    ? tex_samplef(a.textures, m.map_rough, fg.uv) : m.roughness;
+        float metal = (bn.has & kBundleY) ? fg.maps.y
+                    : m.map_metal >= 0    ? tex_samplef(a.textures, m.map_metal, fg.uv) : m.metalness;
         float ao = m.map_ao >= 0 ? tex_samplef(a.textures, m.map_ao, fg.uv) : 1.f;
         c = shade_point<STREAM>(u, a.shadow_map, true, false, fg.pos, fg.normal, fg.lndc, al, em,
                         vec3(ao, metal, rough), rdisk);
@@ -450,7 +473,7 @@ __global__ __launch_bounds__(256) void k_frag_shadow_inputs(ResolveArgs a, Frame
     Varying v0 = main_vertex(dr, u, f, 0);
     Varying v1 = main_vertex(dr, u, f, 1);
     Varying v2 = main_vertex(dr, u, f, 2);
-    const FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump);
+    const FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, m.bundle[dr.support_pbr ? 1 : 0]);
     const size_t N = n;
     out[k] = fg.normal.x;
     out[N + k] = fg.normal.y;
@@ -501,6 +524,12 @@ void launch_corners(const float *pos, const float *uv, const float *nrm, const f
 {
     if (n == 0) return;
     hipLaunchKernelGGL(k_corners, dim3(blocks_for(n, 256)), dim3(256), 0, s, pos, uv, nrm, tan, vi, ti, ni, n, out);
+}
+
+void launch_bundle(int w, int h, const uint32_t *a, const uint8_t *z, const uint32_t *n, const uint8_t *y, uint2 *out,
+                   hipStream_t s)
+{
+    hipLaunchKernelGGL(k_bundle, dim3((w + 63) / 64, (h + 3) / 4), dim3(256), 0, s, w, h, a, z, n, y, out);
 }
 
 void launch_setup(const DevDraw *draws, int n_draws, int max_faces, const int4 *screen, int W,

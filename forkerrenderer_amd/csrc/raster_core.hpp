@@ -802,25 +802,31 @@ __device__ __forceinline__ void gbuffer_shade(const ResolveArgs &a, const FrameU
     Varying v0 = main_vertex(dr, u, f, 0);
     Varying v1 = main_vertex(dr, u, f, 1);
     Varying v2 = main_vertex(dr, u, f, 2);
-    FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump);
+    const DevBundle &bn = m.bundle[dr.support_pbr ? 1 : 0];
+    FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, bn);
     Vec3 albedo, emissive, param;
     float type;
     if (dr.support_pbr) {
-        albedo = m.map_base >= 0 ? tex_sample(a.textures, m.map_base, fg.uv)
-                                 : vec3(m.albedo[0], m.albedo[1], m.albedo[2]);
+        albedo = (bn.has & kBundleA) ? fg.maps.a
+               : m.map_base >= 0     ? tex_sample(a.textures, m.map_base, fg.uv)
+                                     : vec3(m.albedo[0], m.albedo[1], m.albedo[2]);
         emissive = m.map_pbr_ke >= 0 ? tex_sample(a.textures, m.map_pbr_ke, fg.uv)
                                      : vec3(m.ke[0], m.ke[1], m.ke[2]);
-        float rough = m.map_rough >= 0 ? tex_samplef(a.textures, m.map_rough, fg.uv) : m.roughness;
-        float metal = m.map_metal >= 0 ? tex_samplef(a.textures, m.map_metal, fg.uv) : m.metalness;
+        float rough = (bn.has & kBundleZ) ? fg.maps.z
+                    : m.map_rough >= 0    ? tex_samplef(a.textures, m.map_rough, fg.uv) : m.roughness;
+        float metal = (bn.has & kBundleY) ? fg.maps.y
+                    : m.map_metal >= 0    ? tex_samplef(a.textures, m.map_metal, fg.uv) : m.metalness;
         float ao = m.map_ao >= 0 ? tex_samplef(a.textures, m.map_ao, fg.uv) : 1.f;
         param = vec3(ao, metal, rough);
         type = 1.f;
     } else {
         emissive = m.map_ke >= 0 ? tex_sample(a.textures, m.map_ke, fg.uv)
                                  : vec3(m.ke[0], m.ke[1], m.ke[2]);
-        albedo = m.map_kd >= 0 ? tex_sample(a.textures, m.map_kd, fg.uv)
-                               : vec3(m.kd[0], m.kd[1], m.kd[2]);
-        float shin = m.map_ks >= 0 ? tex_samplef(a.textures, m.map_ks, fg.uv) + 5 : 1.f;
+        albedo = (bn.has & kBundleA) ? fg.maps.a
+               : m.map_kd >= 0       ? tex_sample(a.textures, m.map_kd, fg.uv)
+                                     : vec3(m.kd[0], m.kd[1], m.kd[2]);
+        float shin = (bn.has & kBundleZ) ? fg.maps.z + 5
+                   : m.map_ks >= 0       ? tex_samplef(a.textures, m.map_ks, fg.uv) + 5 : 1.f;
         param = vec3(1.f, m.ks[0], shin);
         type = 0.f;
     }
