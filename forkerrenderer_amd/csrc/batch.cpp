@@ -116,6 +116,9 @@ struct fgl_batch {
     uint32_t cap[2] = {0, 0};       // allocated capacities
     uint64_t last_pairs[2] = {0, 0};
     bool measured = false;
+    // the direct rasteriser: its passes' pairs are known (last_pairs) for this
+    // plan; every draw's depths are finite
+    bool pairs_known = false, direct_ok = false;
     bool use_graph = true;
     hipGraphExec_t exec = nullptr;
 
@@ -139,6 +142,11 @@ struct fgl_batch {
     Buf depth, vis, gbuf, ao, fb, img, shadow, shadow_depth;
     Buf screen, ndc_z, rect, counts, offs, scan_tmp, tri_v, big_list, tile_start, tile_end;
     Buf keys[2], vals[2], keys_alt[2], vals_alt[2], sort_tmp[2];
+    Buf key, items, direct_ctr;   // pixel keys, large-triangle items, a counter record per pass
+    uint32_t n_direct_items = 0;
+    Buf d_dblocks[2], d_sblk_view;   // triangle groups of each pass; view of each 64 x 4 shadow-map block
+    int n_dblocks[2] = {0, 0};
+    uint32_t n_sblocks = 0;
     Buf counters;   // [0] big count, [1] queue, [2], [3] overflow flags (shadow, main)
     uint32_t *h_flags = nullptr;
     uint32_t *h_tot = nullptr;
@@ -164,7 +172,8 @@ static int plan(fgl_batch *b)
     b->hv.assign(b->n, DevView());
     std::vector<DevDraw> dd[2];
     std::vector<uint32_t> items[2];
-    std::vector<uint8_t> blk_view, lblk_view;
+    std::vector<uint8_t> blk_view, lblk_view, sblk_view;
+    b->direct_ok = true;
     std::vector<BatchPixView> pix(b->n);
     const int nscale = b->ao_mode == FGL_AO_NEURAL ? nao_scale(b->nao) : 1;
     size_t lpx = 0;
@@ -203,6 +212,10 @@ static int plan(fgl_batch *b)
             for (uint32_t t = 0; t < nt; ++t) items[p].push_back(((uint32_t)i << 24) | t);
             tiles[p] += nt;
         }
+        dv.sblk_base = (uint32_t)sblk_view.size();
+        sblk_view.insert(sblk_view.end(), (size_t)((S + 63) / 64) * ((S + 3) / 4), (uint8_t)i);
+        for (int p = 0; p < 2; ++p) dv.draw_base[p] = (int)dd[p].size();
+        dv.n_draws = v.n_draws;
         dv.blk_base = blocks;
         const uint32_t nb = (uint32_t)(((v.width + 63) / 64) * ((v.height + 3) / 4));
         blk_view.insert(blk_view.end(), nb, (uint8_t)i);
@@ -230,6 +243,9 @@ static int plan(fgl_batch *b)
             d.view = i;
             for (int p = 0; p < 2; ++p) {
                 if (p == kBvShadow && !v.shadow_on) continue;
+                if (d.n_faces > 0x3fffffff || !ctx_depths_finite(c, b->views[i].models[k], &b->views[i].mats[16 * k],
+                                                                 p == kBvShadow))
+                    b->direct_ok = false;
                 DevDraw e = d;
                 e.vert_base = (int)b->nv[p];
                 e.tri_base = (int)b->nt[p];
@@ -270,12 +286,41 @@ static int plan(fgl_batch *b)
         grow(b->big_list, (size_t)mt * 4) || grow(b->tile_start, (size_t)mtiles * 4) ||
         grow(b->tile_end, (size_t)mtiles * 4) || grow(b->counters, 256))
         return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
+    if (b->direct_ok) {
+        // items: every view's 64 x 16 blocks several times over
+        const size_t kp = std::max(px, spx);
+        b->n_direct_items = (uint32_t)std::min<size_t>((size_t)1 << 28, std::max<size_t>((size_t)1 << 18, kp / 128 + 256 * b->n));
+        if (grow(b->key, kp * 8) || grow(b->items, (size_t)b->n_direct_items * sizeof(uint2)) ||
+            grow(b->direct_ctr, 2 * sizeof(DirectCtr)) || grow(b->d_sblk_view, sblk_view.size() + 1))
+            return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
+        launch_fill_u32((uint32_t *)b->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, ctx_stream(c));
+        if (!sblk_view.empty() &&
+            hipMemcpy(b->d_sblk_view.p, sblk_view.data(), sblk_view.size(), hipMemcpyHostToDevice))
+            return bfail(b, FGL_ERR_DEVICE, "upload failed");
+        b->n_sblocks = (uint32_t)sblk_view.size();
+    }
     for (int p = 0; p < 2; ++p) {
         std::vector<uint2> vb, fb;
         for (size_t k = 0; k < dd[p].size(); ++k) {
             for (int v0 = 0; v0 < dd[p][k].n_pos; v0 += 256) vb.push_back(make_uint2((uint32_t)k, (uint32_t)v0));
             for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256) fb.push_back(make_uint2((uint32_t)k, (uint32_t)f0));
         }
+        // triangle groups of the direct rasteriser: lanes per triangle by the
+        // pixels its view has for it
+        std::vector<uint2> db;
+        for (size_t k = 0; b->direct_ok && k < dd[p].size(); ++k) {
+            const DevView &v = b->hv[dd[p][k].view];
+            const double area = p == kBvShadow ? (double)v.S * v.S : (double)v.W * v.H;
+            const double per = area / (dd[p][k].n_faces > 0 ? dd[p][k].n_faces : 1);
+            const uint32_t code = per >= 48.0 ? 2u : per >= 6.0 ? 1u : 0u;
+            for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256 / bv_lanes(code))
+                db.push_back(make_uint2((uint32_t)k, (uint32_t)f0 | code << 30));
+        }
+        b->n_dblocks[p] = (int)db.size();
+        if (grow(b->d_dblocks[p], (db.size() + 1) * sizeof(uint2)))
+            return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
+        if (!db.empty() && hipMemcpy(b->d_dblocks[p].p, db.data(), db.size() * sizeof(uint2), hipMemcpyHostToDevice))
+            return bfail(b, FGL_ERR_DEVICE, "upload failed");
         b->n_vblocks[p] = (int)vb.size();
         b->n_fblocks[p] = (int)fb.size();
         if (grow(b->d_vblocks[p], (vb.size() + 1) * sizeof(uint2)) || grow(b->d_fblocks[p], (fb.size() + 1) * sizeof(uint2)))
@@ -311,6 +356,7 @@ static int plan(fgl_batch *b)
         }
     }
     b->measured = false;
+    b->pairs_known = false;
     return FGL_OK;
 }
 
@@ -328,6 +374,50 @@ static int ensure_capacity(fgl_batch *b, int p, uint32_t need)
     return FGL_OK;
 }
 
+// Whether the passes can take the direct rasteriser: the views do not change,
+// so once a plan's pairs are counted they are known to fit their capacities
+// (where they would not, the lists find out and report it as before).
+static bool use_direct(const fgl_batch *b)
+{
+    return b->direct_ok && b->pairs_known && (!b->have_shadow || b->last_pairs[kBvShadow] <= b->cap[kBvShadow]) &&
+           b->last_pairs[kBvMain] <= b->cap[kBvMain];
+}
+
+static BvDirectArgs direct_args(fgl_batch *b, int p)
+{
+    BvDirectArgs a;
+    a.draws = (const DevDraw *)b->d_draws[p].p;
+    a.n_draws = b->n_draws[p];
+    a.views = (const DevView *)b->d_views.p;
+    a.screen = (const int4 *)b->screen.p;
+    a.key = (unsigned long long *)b->key.p;
+    a.items = (uint2 *)b->items.p;
+    a.n_items = b->n_direct_items;
+    a.ctr = (DirectCtr *)b->direct_ctr.p + p;
+    return a;
+}
+
+// The raster passes of one render through the direct rasteriser, up to the
+// G-buffer resolve.
+static void enqueue_direct(fgl_batch *b, bool timed, hipStream_t s)
+{
+    uint32_t *flags = (uint32_t *)b->counters.p + 2;
+    for (int p = 0; p < 2; ++p) {
+        if (p == kBvShadow && !b->have_shadow) continue;
+        const BvDirectArgs a = direct_args(b, p);
+        {
+            CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_binning" : "batch_main_binning") : nullptr);
+            launch_bv_direct_vertex(p, a, (const uint2 *)b->d_vblocks[p].p, b->n_vblocks[p], (int4 *)b->screen.p,
+                                    (float *)b->ndc_z.p, p == kBvShadow ? b->total_spx : b->total_px, flags, s);
+        }
+        CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_raster" : "batch_main_raster") : nullptr);
+        launch_bv_direct(p, a, (const uint2 *)b->d_dblocks[p].p, b->n_dblocks[p], s);
+        if (p == kBvShadow)
+            launch_bv_direct_shadow(a, (const uint8_t *)b->d_sblk_view.p, b->n_sblocks, (const float *)b->ndc_z.p,
+                                    (float *)b->shadow_depth.p, (float *)b->shadow.p, s);
+    }
+}
+
 // Enqueues one render of every view.  measure: read each pass's pair count
 // back (host sync) and size the pair buffers before emitting -- not
 // capturable; otherwise the pass runs with the allocated capacity and raises
@@ -338,7 +428,9 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
     uint32_t *ctr = (uint32_t *)b->counters.p;
     const DevView *views = (const DevView *)b->d_views.p;
     int rc;
-    for (int p = 0; p < 2; ++p) {
+    const bool direct = !measure && use_direct(b);
+    if (direct) enqueue_direct(b, timed, s);
+    for (int p = 0; p < 2 && !direct; ++p) {
         if (p == kBvShadow && !b->have_shadow) {
             launch_fill_u32(ctr + 2, 0, 1, s);
             continue;
@@ -436,6 +528,9 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
     pa.screen = (const int4 *)b->screen.p;
     pa.tri_v = (const int4 *)b->tri_v.p;
     pa.vis = (const int *)b->vis.p;
+    pa.key = direct ? (const unsigned long long *)b->key.p : nullptr;
+    pa.depth = (float *)b->depth.p;
+    pa.ctr = (DirectCtr *)b->direct_ctr.p + kBvMain;
     pa.materials = b->materials;
     pa.textures = b->textures;
     pa.gbuf = (float *)b->gbuf.p;
@@ -444,6 +539,7 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
     pa.shadow = (const float *)b->shadow.p;
     pa.ao_is_one = b->ao_mode == FGL_AO_NEURAL ? 0 : 1;
     pa.img = (uint8_t *)b->img.p;
+    if (measure) b->pairs_known = true;
     {
         CtxTimer t(b->ctx, timed ? "batch_gbuffer" : nullptr);
         launch_bv_gbuffer(pa, s);
@@ -588,7 +684,8 @@ void fgl_batch_destroy(fgl_batch *b)
                    &b->d_lblk_view,
                    &b->d_pix_views, &b->depth, &b->vis, &b->gbuf, &b->ao, &b->fb, &b->img, &b->shadow,
                    &b->shadow_depth, &b->screen, &b->ndc_z, &b->rect, &b->counts, &b->offs, &b->scan_tmp, &b->tri_v,
-                   &b->big_list, &b->tile_start, &b->tile_end, &b->counters};
+                   &b->big_list, &b->tile_start, &b->tile_end, &b->counters, &b->key, &b->items, &b->direct_ctr,
+                   &b->d_dblocks[0], &b->d_dblocks[1], &b->d_sblk_view};
     for (Buf *x : bufs) release(*x);
     for (int p = 0; p < 2; ++p) {
         release(b->keys[p]); release(b->vals[p]); release(b->keys_alt[p]); release(b->vals_alt[p]);

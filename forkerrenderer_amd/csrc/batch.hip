@@ -5,6 +5,13 @@
 // per-pixel bodies are the single-view ones (raster_core.hpp,
 // shade_core.hpp), so a view's results are those of its single-view render.
 //
+// A batch is rendered through the tile lists while its (tile, triangle) pairs
+// are being counted or may not fit their capacity, and through the direct
+// rasteriser (raster_core.hpp) once they are known to fit.  24 views of 24,600
+// to 384,400 pixels, 6.1 M shadow-map pixels: the tile rasteriser's
+// two launches alone 760 us, all direct kernels 670 us; a render 3,715 -> 3,311
+// us, of which copying the images out takes 820.
+//
 // The pair count of a pass is known only on the device: the emit kernels
 // drop pairs beyond the capacity, the sort and tile-range kernels read the
 // count from device memory, and an overflow flag tells the host to re-render
@@ -139,11 +146,113 @@ __global__ __launch_bounds__(BLOCK) void k_bv_raster(BvRasterArgs b)
     }
 }
 
+// ---- the direct rasteriser over all views ----
+
+// The vertex records, the key plane cleared (8 keys a thread) by the
+// workgroups past the vertices', the overflow flags zeroed (views do not
+// change, so a batch whose pairs were counted has none).
+constexpr int kBvClearKeys = 8;
+template <int PASS>
+__global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const uint2 *__restrict__ blocks, int n_blocks,
+                                                          int4 *__restrict__ out, float *__restrict__ ndc_z, size_t n_keys,
+                                                          uint32_t *__restrict__ flags)
+{
+    const int b = blockIdx.x;
+    if (b >= n_blocks) {
+        if (b == n_blocks && threadIdx.x < 2) flags[threadIdx.x] = 0u;
+        const size_t k0 = (size_t)(b - n_blocks) * (256 * kBvClearKeys);
+        ulonglong2 c;
+        c.x = c.y = kDirectClear;
+#pragma unroll
+        for (int e = 0; e < kBvClearKeys / 2; ++e) {
+            const size_t k = k0 + 2 * ((size_t)e * 256 + threadIdx.x);
+            if (k + 1 < n_keys) *(ulonglong2 *)(a.key + k) = c;
+            else if (k < n_keys) a.key[k] = kDirectClear;
+        }
+        return;
+    }
+    const uint2 bk = blocks[b];
+    const DevDraw &dr = a.draws[bk.x];
+    const int vi = (int)bk.y + threadIdx.x;
+    if (vi >= dr.n_pos) return;
+    const FrameUniforms &u = a.views[dr.view].u;
+    if (PASS == kBvShadow) {
+        const Vec4 n = depth_ndc(dr, vi);
+        out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
+        ndc_z[dr.vert_base + vi] = n.z;
+    } else {
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_ndc(dr, u, vi));
+    }
+}
+
+template <int PASS>
+__device__ __forceinline__ DirectArgs bv_direct_args(const BvDirectArgs &b, const DevView &v)
+{
+    DirectArgs a;
+    a.draws = b.draws;
+    a.n_draws = b.n_draws;
+    a.screen = b.screen;
+    a.key = b.key + (PASS == kBvShadow ? v.spx_off : v.px_off);
+    a.fix = nullptr;
+    a.items = b.items;
+    a.n_items = b.n_items;
+    a.ctr = b.ctr;
+    a.W = PASS == kBvShadow ? v.S : v.W;
+    a.H = PASS == kBvShadow ? v.S : v.H;
+    return a;
+}
+
+template <int PASS>
+__global__ __launch_bounds__(256) void k_bv_direct(BvDirectArgs b, const uint2 *__restrict__ blocks)
+{
+    __shared__ DirectLds lds;
+    const uint2 bk = blocks[xcd_remap(blockIdx.x, gridDim.x)];
+    const DevDraw &dr = b.draws[bk.x];
+    const DirectArgs a = bv_direct_args<PASS>(b, b.views[dr.view]);
+    const int first = (int)(bk.y & 0x3fffffffu);
+    const uint32_t code = bk.y >> 30;
+    if (code == 0) direct_group<1>(a, dr, first, lds);
+    else if (code == 1) direct_group<4>(a, dr, first, lds);
+    else direct_group<16>(a, dr, first, lds);
+}
+
+template <int PASS>
+__global__ __launch_bounds__(256) void k_bv_direct_big(BvDirectArgs b)
+{
+    const unsigned long long claimed = b.ctr->items;
+    const uint32_t n = claimed < b.n_items ? (uint32_t)claimed : b.n_items;
+    for (uint32_t k = blockIdx.x * 4 + (threadIdx.x >> 6); k < n; k += gridDim.x * 4) {
+        const uint2 it = b.items[k];
+        if (it.x == 0xffffffffu) continue;
+        const int d = draw_of(b.draws, b.n_draws, (int)it.x);
+        direct_item(bv_direct_args<PASS>(b, b.views[b.draws[d].view]), it, d);
+    }
+}
+
+// The shadow targets of every view, and the pass's counters zeroed.
+__global__ __launch_bounds__(256) void k_bv_direct_shadow(BvDirectArgs b, const uint8_t *__restrict__ sblk_view,
+                                                          const float *__restrict__ ndc_z, float *__restrict__ depth,
+                                                          float *__restrict__ shadow)
+{
+    const DevView &v = b.views[__builtin_amdgcn_readfirstlane(sblk_view[blockIdx.x])];
+    const int lb = (int)(blockIdx.x - v.sblk_base), nbx = (v.S + 63) / 64;
+    const int x = (lb % nbx) * 64 + (threadIdx.x & 63), y = (lb / nbx) * 4 + (threadIdx.x >> 6);
+    if (x >= v.S || y >= v.S) return;
+    const size_t i = (size_t)x + (size_t)y * v.S;
+    const Winner w = direct_winner(b.draws + v.draw_base[kBvShadow], v.n_draws, b.key + v.spx_off, nullptr, b.screen, v.S, v.S,
+                                   i, x, y);
+    float z = 0.f;
+    if (w.g >= 0) z = dot3(vec3(ndc_z[w.tv.x], ndc_z[w.tv.y], ndc_z[w.tv.z]), w.b) * 0.5f + 0.5f;
+    depth[v.spx_off + i] = w.depth;
+    shadow[v.spx_off + i] = z;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *b.ctr = DirectCtr{0ull, 0u, 0u};
+}
+
 // Pixel (x, y) of the view owning 64 x 4 block blockIdx.x; false when it is
 // outside the view.
 __device__ __forceinline__ bool bv_pixel(const BvPixelArgs &a, int &vi, int &x, int &y)
 {
-    vi = a.blk_view[blockIdx.x];
+    vi = __builtin_amdgcn_readfirstlane(a.blk_view[blockIdx.x]);
     const DevView &v = a.views[vi];
     const int lb = (int)(blockIdx.x - v.blk_base), nbx = (v.W + 63) / 64;
     x = (lb % nbx) * 64 + (threadIdx.x & 63);
@@ -151,20 +260,21 @@ __device__ __forceinline__ bool bv_pixel(const BvPixelArgs &a, int &vi, int &x, 
     return x < v.W && y < v.H;
 }
 
+template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
 {
     int vi, x, y;
     if (!bv_pixel(b, vi, x, y)) return;
     const DevView &v = b.views[vi];
     ResolveArgs a;
-    a.draws = b.draws;
-    a.n_draws = 0;
+    a.draws = DIRECT ? b.draws + v.draw_base[kBvMain] : b.draws;
+    a.n_draws = v.n_draws;
     a.screen = b.screen;
     a.tri_v = b.tri_v;
     a.vis = b.vis + v.px_off;
-    a.key = nullptr;
+    a.key = DIRECT ? const_cast<unsigned long long *>(b.key) + v.px_off : nullptr;
     a.fix = nullptr;
-    a.depth = nullptr;
+    a.depth = DIRECT ? b.depth + v.px_off : nullptr;
     a.W = v.W;
     a.H = v.H;
     a.fresh = 1;
@@ -175,7 +285,9 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     a.textures = b.textures;
     a.shadow_map = nullptr;
     a.ss = ShadowSamples{};
-    gbuffer_px<false>(a, v.u, x, y);
+    gbuffer_px<DIRECT>(a, v.u, x, y);
+    // last: a store before them would keep the loads above from their scalar form
+    if (DIRECT && blockIdx.x == 0 && threadIdx.x == 0) *b.ctr = DirectCtr{0ull, 0u, 0u};
 }
 
 __global__ __launch_bounds__(256) void k_bv_lighting(BvPixelArgs b)
@@ -259,9 +371,43 @@ void launch_bv_raster(int pass, int TS, unsigned n_wg, const BvRasterArgs &a, hi
     else bv_raster_t<false>(TS, n_wg, a, s);
 }
 
+void launch_bv_direct_vertex(int pass, const BvDirectArgs &a, const uint2 *vblocks, int n_vblocks, int4 *screen,
+                             float *ndc_z, size_t n_keys, uint32_t *flags, hipStream_t s)
+{
+    const unsigned grid = (unsigned)n_vblocks + nblk(n_keys, 256 * kBvClearKeys);
+    if (grid == 0) return;
+    if (pass == kBvShadow)
+        hipLaunchKernelGGL(k_bv_direct_vertex<kBvShadow>, dim3(grid), dim3(256), 0, s, a, vblocks, n_vblocks, screen, ndc_z,
+                           n_keys, flags);
+    else
+        hipLaunchKernelGGL(k_bv_direct_vertex<kBvMain>, dim3(grid), dim3(256), 0, s, a, vblocks, n_vblocks, screen, ndc_z,
+                           n_keys, flags);
+}
+
+void launch_bv_direct(int pass, const BvDirectArgs &a, const uint2 *fblocks, int n_fblocks, hipStream_t s)
+{
+    if (n_fblocks <= 0) return;
+    const unsigned big_grid = 1024;
+    if (pass == kBvShadow) {
+        hipLaunchKernelGGL(k_bv_direct<kBvShadow>, dim3(n_fblocks), dim3(256), 0, s, a, fblocks);
+        hipLaunchKernelGGL(k_bv_direct_big<kBvShadow>, dim3(big_grid), dim3(256), 0, s, a);
+    } else {
+        hipLaunchKernelGGL(k_bv_direct<kBvMain>, dim3(n_fblocks), dim3(256), 0, s, a, fblocks);
+        hipLaunchKernelGGL(k_bv_direct_big<kBvMain>, dim3(big_grid), dim3(256), 0, s, a);
+    }
+}
+
+void launch_bv_direct_shadow(const BvDirectArgs &a, const uint8_t *sblk_view, uint32_t n_sblocks, const float *ndc_z,
+                             float *depth, float *shadow, hipStream_t s)
+{
+    if (n_sblocks) hipLaunchKernelGGL(k_bv_direct_shadow, dim3(n_sblocks), dim3(256), 0, s, a, sblk_view, ndc_z, depth, shadow);
+}
+
 void launch_bv_gbuffer(const BvPixelArgs &a, hipStream_t s)
 {
-    if (a.n_blocks) hipLaunchKernelGGL(k_bv_gbuffer, dim3(a.n_blocks), dim3(256), 0, s, a);
+    if (!a.n_blocks) return;
+    if (a.key) hipLaunchKernelGGL(k_bv_gbuffer<true>, dim3(a.n_blocks), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_bv_gbuffer<false>, dim3(a.n_blocks), dim3(256), 0, s, a);
 }
 
 void launch_bv_lighting(const BvPixelArgs &a, hipStream_t s)

@@ -16,13 +16,16 @@ constexpr int kBvMain = 1;
 // px_off, G-buffer planes at 19 * px_off, frame planes at 3 * px_off, image
 // bytes at 3 * px_off), shadow targets at spx_off.  Its tiles of pass p are
 // global tiles tile_base[p] .. tile_base[p] + tiles_x[p] * tiles_y[p] - 1;
-// its 64 x 4 pixel blocks are batch blocks blk_base ...
+// its 64 x 4 pixel blocks are batch blocks blk_base .., those of its shadow
+// map sblk_base .., its draws of pass p draw_base[p] ...
 struct DevView {
     FrameUniforms u;   // ForkerGL state of the view (both passes)
     int W, H, S, shadow_on;
     int tiles_x[2], tiles_y[2];
     uint32_t tile_base[2];
-    uint32_t blk_base, pad;
+    uint32_t blk_base, sblk_base;
+    int draw_base[2], n_draws;
+    int pad;
     size_t px_off, spx_off;
 };
 
@@ -54,6 +57,19 @@ struct BvRasterArgs {
     const float *ndc_z;       // shadow pass: per vertex NDC z
 };
 
+// A pass through the direct rasteriser: the key plane of every view's
+// targets (indexed as they are), the item list of all views' large triangles.
+struct BvDirectArgs {
+    const DevDraw *draws;
+    int n_draws;
+    const DevView *views;
+    const int4 *screen;
+    unsigned long long *key;
+    uint2 *items;
+    uint32_t n_items;
+    DirectCtr *ctr;
+};
+
 struct BvPixelArgs {
     const DevDraw *draws;
     const DevView *views;
@@ -62,6 +78,9 @@ struct BvPixelArgs {
     const int4 *screen;
     const int4 *tri_v;
     const int *vis;
+    const unsigned long long *key;   // the direct rasteriser's keys instead of vis (null: vis)
+    float *depth;                    // with key: written by the resolve
+    DirectCtr *ctr;                  // with key: zeroed by the resolve for the next render
     const DevMaterial *materials;
     const DevTexture *textures;
     float *gbuf, *ao, *fb;
@@ -80,6 +99,16 @@ void launch_bv_emit(int pass, const BvBinArgs &a, hipStream_t s);
 // flag = (*total > cap): the pass's pairs did not fit
 void launch_bv_overflow(const uint32_t *total, uint32_t cap, uint32_t *flag, hipStream_t s);
 void launch_bv_raster(int pass, int TS, unsigned n_wg, const BvRasterArgs &a, hipStream_t s);
+// The direct rasteriser (raster_core.hpp) over all views.  vblocks as above,
+// fblocks: (draw, first triangle | lanes code << 30) of each workgroup
+// (bv_lanes); n_keys pixels of the pass's targets; flags: the two overflow
+// words, zeroed.  launch_bv_direct_shadow also zeroes the pass's counters.
+__host__ __device__ inline int bv_lanes(uint32_t code) { return code == 0 ? 1 : code == 1 ? 4 : 16; }
+void launch_bv_direct_vertex(int pass, const BvDirectArgs &a, const uint2 *vblocks, int n_vblocks, int4 *screen,
+                             float *ndc_z, size_t n_keys, uint32_t *flags, hipStream_t s);
+void launch_bv_direct(int pass, const BvDirectArgs &a, const uint2 *fblocks, int n_fblocks, hipStream_t s);
+void launch_bv_direct_shadow(const BvDirectArgs &a, const uint8_t *sblk_view, uint32_t n_sblocks, const float *ndc_z,
+                             float *depth, float *shadow, hipStream_t s);
 void launch_bv_gbuffer(const BvPixelArgs &a, hipStream_t s);
 void launch_bv_lighting(const BvPixelArgs &a, hipStream_t s);
 void launch_bv_resolve(const BvPixelArgs &a, hipStream_t s);

@@ -2028,6 +2028,15 @@ int ctx_draw_record(fgl_ctx *c, int model, const float M[16], DevDraw *out)
     return FGL_OK;
 }
 
+bool ctx_depths_finite(fgl_ctx *c, int model, const float M[16], bool shadow)
+{
+    const ClipBound cam = camera_bound(c, shadow);
+    ClipBound b;
+    mat_mul_d(cam.m, M, b.m, false);
+    mat_mul_d(cam.a, M, b.a, true);
+    return depths_finite(c->models[model], b);
+}
+
 int ctx_tables(fgl_ctx *c, const DevMaterial **materials, const DevTexture **textures)
 {
     int rc = upload_tables(c);

@@ -37,6 +37,10 @@ void ctx_uniforms(fgl_ctx *c, FrameUniforms *u);
 // light-space matrix: geometry pointers, normal matrix, light * model.  The
 // pass-wide bases (vert_base, tri_base) and the view index are left zero.
 int ctx_draw_record(fgl_ctx *c, int model, const float M[16], DevDraw *out);
+// Whether every window depth of `model` under M is finite, in the shadow or
+// the main pass of the context's current matrices (then no fragment's depth
+// is NaN).
+bool ctx_depths_finite(fgl_ctx *c, int model, const float M[16], bool shadow);
 // Uploads pending texture / material tables; returns their device copies.
 int ctx_tables(fgl_ctx *c, const DevMaterial **materials, const DevTexture **textures);
 hipStream_t ctx_stream(fgl_ctx *c);

@@ -239,7 +239,10 @@ __global__ __launch_bounds__(256) void k_direct_big(DirectArgs a)
 {
     const unsigned long long claimed = a.ctr->items;
     const uint32_t n = claimed < a.n_items ? (uint32_t)claimed : a.n_items;
-    for (uint32_t k = blockIdx.x * 4 + (threadIdx.x >> 6); k < n; k += gridDim.x * 4) direct_item(a, a.items[k]);
+    for (uint32_t k = blockIdx.x * 4 + (threadIdx.x >> 6); k < n; k += gridDim.x * 4) {
+        const uint2 it = a.items[k];
+        if (it.x != 0xffffffffu) direct_item(a, it, draw_of(a.draws, a.n_draws, (int)it.x));
+    }
 }
 
 // The second walk of a pass with NaN marks.

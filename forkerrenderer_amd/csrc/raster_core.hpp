@@ -695,12 +695,11 @@ __device__ __forceinline__ int4 direct_face(const DevDraw *draws, int d, const i
     return tv;
 }
 
-// Item it of the list by one wavefront.
-__device__ __forceinline__ void direct_item(const DirectArgs &a, uint2 it)
+// Item it of the list, a triangle of draw d, by one wavefront.
+__device__ __forceinline__ void direct_item(const DirectArgs &a, uint2 it, int d)
 {
-    if (it.x == 0xffffffffu) return;
     TriL t;
-    direct_face(a.draws, draw_of(a.draws, a.n_draws, (int)it.x), a.screen, (int)it.x, a.W, a.H, t);
+    direct_face(a.draws, d, a.screen, (int)it.x, a.W, a.H, t);
     const int bx = t.bb0 & 0xffff, by = t.bb0 >> 16, w = (t.bb1 & 0xffff) - bx + 1, h = (t.bb1 >> 16) - by + 1;
     const int nx = (w + kDirectItemW - 1) / kDirectItemW;
     const int ox = ((int)it.y % nx) * kDirectItemW, oy = ((int)it.y / nx) * kDirectItemH;
