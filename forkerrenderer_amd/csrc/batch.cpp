@@ -140,7 +140,7 @@ struct fgl_batch {
     int n_vblocks[2] = {0, 0}, n_fblocks[2] = {0, 0};
     uint32_t n_conv_items[2] = {0, 0};
     Buf depth, vis, gbuf, ao, fb, img, shadow, shadow_depth;
-    Buf screen, ndc_z, rect, counts, offs, scan_tmp, tri_v, big_list, tile_start, tile_end;
+    Buf screen, ndc_z, vary, rect, counts, offs, scan_tmp, tri_v, big_list, tile_start, tile_end;
     Buf keys[2], vals[2], keys_alt[2], vals_alt[2], sort_tmp[2];
     Buf key, items, direct_ctr;   // pixel keys, large-triangle items, a counter record per pass
     uint32_t n_direct_items = 0;
@@ -280,6 +280,7 @@ static int plan(fgl_batch *b)
         grow(b->gbuf, (size_t)kGbufPlanes * px * 4) || grow(b->ao, px * 4) || grow(b->fb, 3 * px * 4) ||
         grow(b->img, 3 * px) || grow(b->shadow, spx * 4) || grow(b->shadow_depth, spx * 4) ||
         grow(b->screen, (size_t)mv * sizeof(int4)) || grow(b->ndc_z, (size_t)mv * 4) ||
+        grow(b->vary, (size_t)b->nv[kBvMain] * 2 * sizeof(float4)) ||
         grow(b->rect, (size_t)mt * sizeof(uint2)) ||
         grow(b->counts, (size_t)mt * 4) || grow(b->offs, ((size_t)mt + 1) * 4) ||
         grow(b->scan_tmp, scan_tmp_words((size_t)mt) * 4) || grow(b->tri_v, (size_t)mt * sizeof(int4)) ||
@@ -408,7 +409,8 @@ static void enqueue_direct(fgl_batch *b, bool timed, hipStream_t s)
         {
             CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_binning" : "batch_main_binning") : nullptr);
             launch_bv_direct_vertex(p, a, (const uint2 *)b->d_vblocks[p].p, b->n_vblocks[p], (int4 *)b->screen.p,
-                                    (float *)b->ndc_z.p, p == kBvShadow ? b->total_spx : b->total_px, flags, s);
+                                    (float *)b->ndc_z.p, (float4 *)b->vary.p,
+                                    p == kBvShadow ? b->total_spx : b->total_px, flags, s);
         }
         CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_raster" : "batch_main_raster") : nullptr);
         launch_bv_direct(p, a, (const uint2 *)b->d_dblocks[p].p, b->n_dblocks[p], s);
@@ -442,7 +444,7 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
             CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_binning" : "batch_main_binning") : nullptr);
             if (nt > 0) {
                 launch_bv_vertex(p, draws, views, (const uint2 *)b->d_vblocks[p].p, b->n_vblocks[p], (int4 *)b->screen.p,
-                                 (float *)b->ndc_z.p, s);
+                                 (float *)b->ndc_z.p, (float4 *)b->vary.p, s);
                 launch_fill_u32(ctr, 0, 1, s);
                 launch_bv_setup(p, draws, views, (const uint2 *)b->d_fblocks[p].p, b->n_fblocks[p],
                                 (const int4 *)b->screen.p,
@@ -527,6 +529,7 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
     pa.n_blocks = b->n_blocks;
     pa.screen = (const int4 *)b->screen.p;
     pa.tri_v = (const int4 *)b->tri_v.p;
+    pa.vary = (const float4 *)b->vary.p;
     pa.vis = (const int *)b->vis.p;
     pa.key = direct ? (const unsigned long long *)b->key.p : nullptr;
     pa.depth = (float *)b->depth.p;
@@ -683,7 +686,7 @@ void fgl_batch_destroy(fgl_batch *b)
     Buf *bufs[] = {&b->d_views, &b->d_draws[0], &b->d_draws[1], &b->d_items[0], &b->d_items[1], &b->d_blk_view,
                    &b->d_lblk_view,
                    &b->d_pix_views, &b->depth, &b->vis, &b->gbuf, &b->ao, &b->fb, &b->img, &b->shadow,
-                   &b->shadow_depth, &b->screen, &b->ndc_z, &b->rect, &b->counts, &b->offs, &b->scan_tmp, &b->tri_v,
+                   &b->shadow_depth, &b->screen, &b->ndc_z, &b->vary, &b->rect, &b->counts, &b->offs, &b->scan_tmp, &b->tri_v,
                    &b->big_list, &b->tile_start, &b->tile_end, &b->counters, &b->key, &b->items, &b->direct_ctr,
                    &b->d_dblocks[0], &b->d_dblocks[1], &b->d_sblk_view};
     for (Buf *x : bufs) release(*x);

@@ -31,7 +31,8 @@ template <int PASS>
 __global__ __launch_bounds__(256) void k_bv_vertex(const DevDraw *__restrict__ draws,
                                                    const DevView *__restrict__ views,
                                                    const uint2 *__restrict__ blocks,
-                                                   int4 *__restrict__ out, float *__restrict__ ndc_z)
+                                                   int4 *__restrict__ out, float *__restrict__ ndc_z,
+                                                   float4 *__restrict__ vary)
 {
     const uint2 bk = blocks[blockIdx.x];
     const DevDraw &dr = draws[bk.x];
@@ -43,7 +44,8 @@ __global__ __launch_bounds__(256) void k_bv_vertex(const DevDraw *__restrict__ d
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        out[dr.vert_base + vi] = to_screen(u.viewport, main_ndc(dr, u, vi));
+        const size_t v = (size_t)dr.vert_base + vi;
+        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
     }
 }
 
@@ -154,7 +156,8 @@ __global__ __launch_bounds__(BLOCK) void k_bv_raster(BvRasterArgs b)
 constexpr int kBvClearKeys = 8;
 template <int PASS>
 __global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const uint2 *__restrict__ blocks, int n_blocks,
-                                                          int4 *__restrict__ out, float *__restrict__ ndc_z, size_t n_keys,
+                                                          int4 *__restrict__ out, float *__restrict__ ndc_z,
+                                                          float4 *__restrict__ vary, size_t n_keys,
                                                           uint32_t *__restrict__ flags)
 {
     const int b = blockIdx.x;
@@ -181,7 +184,8 @@ __global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const 
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        out[dr.vert_base + vi] = to_screen(u.viewport, main_ndc(dr, u, vi));
+        const size_t v = (size_t)dr.vert_base + vi;
+        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
     }
 }
 
@@ -271,6 +275,7 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     a.n_draws = v.n_draws;
     a.screen = b.screen;
     a.tri_v = b.tri_v;
+    a.vary = b.vary;
     a.vis = b.vis + v.px_off;
     a.key = DIRECT ? const_cast<unsigned long long *>(b.key) + v.px_off : nullptr;
     a.fix = nullptr;
@@ -313,15 +318,15 @@ __global__ __launch_bounds__(256) void k_bv_resolve(BvPixelArgs b)
 static inline unsigned nblk(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
 void launch_bv_vertex(int pass, const DevDraw *draws, const DevView *views, const uint2 *blocks, int n_blocks,
-                      int4 *screen, float *ndc_z, hipStream_t s)
+                      int4 *screen, float *ndc_z, float4 *vary, hipStream_t s)
 {
     if (n_blocks <= 0) return;
     if (pass == kBvShadow)
         hipLaunchKernelGGL(k_bv_vertex<kBvShadow>, dim3(n_blocks), dim3(256), 0, s, draws, views, blocks, screen,
-                           ndc_z);
+                           ndc_z, vary);
     else
         hipLaunchKernelGGL(k_bv_vertex<kBvMain>, dim3(n_blocks), dim3(256), 0, s, draws, views, blocks, screen,
-                           ndc_z);
+                           ndc_z, vary);
 }
 
 void launch_bv_setup(int pass, const DevDraw *draws, const DevView *views, const uint2 *blocks, int n_blocks,
@@ -372,16 +377,16 @@ void launch_bv_raster(int pass, int TS, unsigned n_wg, const BvRasterArgs &a, hi
 }
 
 void launch_bv_direct_vertex(int pass, const BvDirectArgs &a, const uint2 *vblocks, int n_vblocks, int4 *screen,
-                             float *ndc_z, size_t n_keys, uint32_t *flags, hipStream_t s)
+                             float *ndc_z, float4 *vary, size_t n_keys, uint32_t *flags, hipStream_t s)
 {
     const unsigned grid = (unsigned)n_vblocks + nblk(n_keys, 256 * kBvClearKeys);
     if (grid == 0) return;
     if (pass == kBvShadow)
         hipLaunchKernelGGL(k_bv_direct_vertex<kBvShadow>, dim3(grid), dim3(256), 0, s, a, vblocks, n_vblocks, screen, ndc_z,
-                           n_keys, flags);
+                           vary, n_keys, flags);
     else
         hipLaunchKernelGGL(k_bv_direct_vertex<kBvMain>, dim3(grid), dim3(256), 0, s, a, vblocks, n_vblocks, screen, ndc_z,
-                           n_keys, flags);
+                           vary, n_keys, flags);
 }
 
 void launch_bv_direct(int pass, const BvDirectArgs &a, const uint2 *fblocks, int n_fblocks, hipStream_t s)

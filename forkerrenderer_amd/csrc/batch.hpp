@@ -77,6 +77,7 @@ struct BvPixelArgs {
     uint32_t n_blocks;
     const int4 *screen;
     const int4 *tri_v;
+    const float4 *vary;       // the main vertex pass's varyings
     const int *vis;
     const unsigned long long *key;   // the direct rasteriser's keys instead of vis (null: vis)
     float *depth;                    // with key: written by the resolve
@@ -91,7 +92,7 @@ struct BvPixelArgs {
 
 // blocks: (draw, first vertex / face) of each 256-item block
 void launch_bv_vertex(int pass, const DevDraw *draws, const DevView *views, const uint2 *blocks, int n_blocks,
-                      int4 *screen, float *ndc_z, hipStream_t s);
+                      int4 *screen, float *ndc_z, float4 *vary, hipStream_t s);
 void launch_bv_setup(int pass, const DevDraw *draws, const DevView *views, const uint2 *blocks, int n_blocks,
                      const int4 *screen, int TS, uint2 *rect, uint32_t *count, int4 *tri_v,
                      uint32_t *big_list, uint32_t *big_count, hipStream_t s);
@@ -105,7 +106,7 @@ void launch_bv_raster(int pass, int TS, unsigned n_wg, const BvRasterArgs &a, hi
 // words, zeroed.  launch_bv_direct_shadow also zeroes the pass's counters.
 __host__ __device__ inline int bv_lanes(uint32_t code) { return code == 0 ? 1 : code == 1 ? 4 : 16; }
 void launch_bv_direct_vertex(int pass, const BvDirectArgs &a, const uint2 *vblocks, int n_vblocks, int4 *screen,
-                             float *ndc_z, size_t n_keys, uint32_t *flags, hipStream_t s);
+                             float *ndc_z, float4 *vary, size_t n_keys, uint32_t *flags, hipStream_t s);
 void launch_bv_direct(int pass, const BvDirectArgs &a, const uint2 *fblocks, int n_fblocks, hipStream_t s);
 void launch_bv_direct_shadow(const BvDirectArgs &a, const uint8_t *sblk_view, uint32_t n_sblocks, const float *ndc_z,
                              float *depth, float *shadow, hipStream_t s);

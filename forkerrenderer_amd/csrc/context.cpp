@@ -35,7 +35,7 @@ struct ModelRes {
     float *pos = nullptr, *uv = nullptr, *nrm = nullptr, *tan = nullptr;
     int *vi = nullptr, *ti = nullptr, *ni = nullptr, *fmat = nullptr;
     int4 *tri = nullptr;       // the faces in spatial order
-    float *corner = nullptr;   // per face corner: pos, uv, nrm, tan (12 floats)
+    float *corner = nullptr;   // per face corner: uv, normal, tangent (8 floats)
     int n_pos = 0, n_faces = 0;
     bool has_tan = false, pbr = false;
     // extent of the faces' corners and the longest face edge; bounded: they
@@ -102,7 +102,7 @@ struct fgl_ctx {
 
     // pass scratch
     DevBuf d_draws, screen, rect, counts, offs, scan_tmp, keys, vals, keys_alt, vals_alt, sort_tmp,
-        tile_start, tile_end, tri_v, big_list, counters, ndc_z;
+        tile_start, tile_end, tri_v, big_list, counters, ndc_z, vary;
     // the direct rasteriser: pixel keys, NaN plane (all ones between passes),
     // large-triangle items and two passes' counters used in turn
     DevBuf key, key_nan, items;
@@ -365,7 +365,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
                       &c->mt_base, &c->mt_states, &c->mt_vec, &c->mt_ck, &c->mt_polys[0], &c->mt_polys[1],
                       &c->screen, &c->rect, &c->counts, &c->offs, &c->scan_tmp, &c->keys,
                       &c->vals, &c->keys_alt, &c->vals_alt, &c->sort_tmp, &c->tile_start,
-                      &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z,
+                      &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z, &c->vary,
                       &c->key, &c->key_nan, &c->items,
                       &c->frag_cnt, &c->frag_tri, &c->frag_alt, &c->frag_tmp, &c->frag_planes,
                       &c->frag_offs_px};
@@ -618,8 +618,8 @@ int fgl_upload_model(fgl_ctx *c, const fgl_model_desc *d, int *out_id)
     if ((rc = upload_array(c, &m.ti, (const int *)d->ti, 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.ni, (const int *)d->ni, 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.fmat, (const int *)d->face_material, nf))) return rc;
-    HIPCHK(c, hipMalloc((void **)&m.corner, (nf ? 3 * nf * 12 : 1) * sizeof(float)));
-    launch_corners(m.pos, m.uv, m.nrm, m.tan, m.vi, m.ti, m.ni, 3 * nf, (float4 *)m.corner, c->stream);
+    HIPCHK(c, hipMalloc((void **)&m.corner, (nf ? 3 * nf * 8 : 1) * sizeof(float)));
+    launch_corners(m.uv, m.nrm, m.tan, m.vi, m.ti, m.ni, 3 * nf, (float4 *)m.corner, c->stream);
     HIPCHK(c, hipGetLastError());
     for (int k = 0; k < 3; ++k) {
         m.lo[k] = HUGE_VAL;
@@ -1296,7 +1296,8 @@ static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, int max_
     {
         KernelTimer t(c, "vertex");
         launch_direct_vertex(shadow, a.draws, n_draws, max_pos, u, (int4 *)c->screen.p,
-                             shadow ? (float *)c->ndc_z.p : nullptr, a, ctr + c->direct_turn, c->stream);
+                             shadow ? (float *)c->ndc_z.p : nullptr, shadow ? nullptr : (float4 *)c->vary.p, a,
+                             ctr + c->direct_turn, c->stream);
     }
     KernelTimer t(c, shadow ? "raster_shadow" : "raster");
     launch_direct(a, max_faces, nt, c->stream);
@@ -1328,7 +1329,8 @@ static int list_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, int max_po
     {
         KernelTimer t(c, "vertex");
         launch_vertex(shadow, ddraws, n_draws, max_pos, u, (int4 *)c->screen.p,
-                      shadow ? (float *)c->ndc_z.p : nullptr, big_count, c->stream);
+                      shadow ? (float *)c->ndc_z.p : nullptr, shadow ? nullptr : (float4 *)c->vary.p, big_count,
+                      c->stream);
     }
     {
         KernelTimer t(c, "setup");
@@ -1511,7 +1513,8 @@ static int flush_pass(fgl_ctx *c)
     const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
     const size_t px = (size_t)W * H;
     const bool direct = fresh && !stoch && fits && direct_fits(n_draws, max_faces, max_pos, px);
-    if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))))
+    if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))) ||
+        (!shadow && (rc = ensure(c, c->vary, (size_t)nv * 2 * sizeof(float4)))))
         return rc;
     uint32_t n_frag = 0;
     if (direct) {
@@ -1528,6 +1531,7 @@ static int flush_pass(fgl_ctx *c)
         r.n_draws = n_draws;
         r.screen = (const int4 *)c->screen.p;
         r.tri_v = (const int4 *)c->tri_v.p;
+        r.vary = (const float4 *)c->vary.p;
         r.vis = (const int *)c->vis.p;
         if (direct) {
             r.key = (unsigned long long *)c->key.p;

@@ -48,9 +48,9 @@ struct DevDraw {
     const float *pos, *uv, *nrm, *tan;
     const int *vi, *ti, *ni, *face_mat;
     // per face corner (3 per face), the attributes the main vertex programs
-    // read, interleaved as 3 float4: (pos.xyz, uv.x), (uv.y, nrm.xyz),
-    // (tan.xyz, 0) -- one 48-byte record instead of four arrays behind three
-    // index streams
+    // read beside the position, interleaved as 2 float4: (uv, n.xy), (n.z,
+    // t.xyz), the normal and tangent normalised as ProcessVertex does -- one
+    // 32-byte record instead of three arrays behind three index streams
     const float4 *corner;
     // the faces in spatial order: position indices (as vi) and the face
     const int4 *tri;
@@ -250,52 +250,47 @@ struct Varying {
 };
 
 // BlinnPhong/PBR/G ProcessVertex (phongshader.h:35-85, pbrshader.h:35-85,
-// gshader.h:41-92) of corner k of face f, with the corner's attributes as
-// Mesh::Vert / TexCoord / Normal / Tangent fetch them (mesh.cpp:34-56).
-__device__ __forceinline__ Varying main_vertex(const DevDraw &d, const FrameUniforms &u, int f, int k)
+// gshader.h:41-92), the part that depends on the position alone: made once a
+// vertex by the vertex pass (its NDC, and the varyings as two float4:
+// position / w and 1 / w, light NDC / w), where the resolves used to make it
+// for every corner of every pixel (some 120 operations each; 24-view batch
+// G-buffer 671 -> 628 us, 957 x 603 2x forward resolve 159 -> 154, 1920 x 1080
+// G-buffer 73 -> 65; where faces are a few pixels large the resolve is bound by
+// its gathers and stays as it was).
+__device__ __forceinline__ Vec4 main_position(const DevDraw &d, const FrameUniforms &u, int vi, float4 &v0, float4 &v1)
 {
-    Varying o;
-    const float4 *r = d.corner + (size_t)(3 * f + k) * 3;
-    const float4 r0 = r[0], r1 = r[1], r2 = r[2];
-    Vec4 p = vec4(r0.x, r0.y, r0.z, 1.f);
+    Vec4 p = vec4(d.pos[3 * vi], d.pos[3 * vi + 1], d.pos[3 * vi + 2], 1.f);
     Vec4 ws = mv4(d.model, p);
-    Vec4 vs = mv4(u.view, ws);
-    Vec4 cs = mv4(u.proj, vs);
-    Vec2 uv = vec2(r0.w, r1.x);
-    Vec3 n = norm3(vec3(r1.y, r1.z, r1.w));
-    Vec3 nws = mv3(d.normal, n);
-    Vec3 tws = vec3(0.f, 0.f, 0.f);
-    if (d.has_tangents) {
-        Vec3 t = norm3(vec3(r2.x, r2.y, r2.z));
-        tws = mv3(d.normal, t);
-    }
+    Vec4 cs = mv4(u.proj, mv4(u.view, ws));
     Vec4 l = vec4(0.f, 0.f, 0.f, 0.f);
     if (u.shadow_on) {
         l = mv4(u.light_space, ws);
         l = divs4(l, l.w);
     }
-    float oow = recip(cs.w);
+    const float oow = recip(cs.w);
     ws = scale4(ws, oow);
-    uv.x *= oow;
-    uv.y *= oow;
-    nws = scale3(nws, oow);
-    if (d.has_tangents) tws = scale3(tws, oow);
     if (u.shadow_on) l = scale4(l, oow);
-    o.ws = vec3(ws.x, ws.y, ws.z);
-    o.uv = uv;
-    o.nws = nws;
-    o.tws = tws;
-    o.lndc = vec3(l.x, l.y, l.z);
-    o.oow = oow;
-    return o;
+    v0 = make_float4(ws.x, ws.y, ws.z, oow);
+    v1 = make_float4(l.x, l.y, l.z, 0.f);
+    return divs4(cs, cs.w);
 }
 
-// Clip-space -> NDC of the main shaders: positionCS / positionCS.w.
-__device__ __forceinline__ Vec4 main_ndc(const DevDraw &d, const FrameUniforms &u, int vi)
+// Corner k of face f, a corner at vertex v of the pass's varyings, with its
+// attributes as Mesh::TexCoord / Normal / Tangent fetch them (mesh.cpp:34-56).
+__device__ __forceinline__ Varying main_vertex(const DevDraw &d, const float4 *vary, int v, int f, int k)
 {
-    Vec4 p = vec4(d.pos[3 * vi], d.pos[3 * vi + 1], d.pos[3 * vi + 2], 1.f);
-    Vec4 cs = mv4(u.proj, mv4(u.view, mv4(d.model, p)));
-    return divs4(cs, cs.w);
+    Varying o;
+    const float4 *r = d.corner + (size_t)(3 * f + k) * 2;
+    const float4 r0 = r[0], r1 = r[1], p0 = vary[2 * (size_t)v], p1 = vary[2 * (size_t)v + 1];
+    const float oow = p0.w;
+    o.ws = vec3(p0.x, p0.y, p0.z);
+    o.lndc = vec3(p1.x, p1.y, p1.z);
+    o.oow = oow;
+    o.uv = vec2(r0.x * oow, r0.y * oow);
+    o.nws = scale3(mv3(d.normal, vec3(r0.z, r0.w, r1.x)), oow);
+    o.tws = vec3(0.f, 0.f, 0.f);
+    if (d.has_tangents) o.tws = scale3(mv3(d.normal, vec3(r1.y, r1.z, r1.w)), oow);
+    return o;
 }
 
 // DepthShader::ProcessVertex (src/shaders/depthshader.h:21-28)

@@ -75,6 +75,7 @@ struct ResolveArgs {
     float clear[3];            // forward pass background colour
     float *gbuf;               // 19 planes (geometry pass)
     float *fb;                 // 3 planes (forward pass)
+    const float4 *vary;        // the vertex pass's varyings (main_position)
     const DevMaterial *materials;
     const DevTexture *textures;
     const float *shadow_map;
@@ -135,12 +136,13 @@ struct SsaoArgs {
 void launch_bundle(int w, int h, const uint32_t *a, const uint8_t *z, const uint32_t *n, const uint8_t *y, uint2 *out,
                    hipStream_t s);
 // The corner records of a model from its attribute arrays (tan may be null).
-void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti,
-                    const int *ni, size_t n, float4 *out, hipStream_t s);
+void launch_corners(const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti, const int *ni,
+                    size_t n, float4 *out, hipStream_t s);
 // Window records of every (draw, position); shadow pass: also the NDC z of
-// each vertex into ndc_z; zero (may be null): a word set to 0 on the way.
-void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos,
-                   const FrameUniforms &u, int4 *out, float *ndc_z, uint32_t *zero, hipStream_t s);
+// each vertex into ndc_z, main passes: its varyings into vary; zero (may be
+// null): a word set to 0 on the way.
+void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
+                   float *ndc_z, float4 *vary, uint32_t *zero, hipStream_t s);
 void launch_setup(const DevDraw *draws, int n_draws, int max_faces, const int4 *screen, int W,
                   int H, int TS, uint2 *rect, uint32_t *count, int4 *tri_v, uint32_t *big_list,
                   uint32_t *big_count, hipStream_t s);
@@ -163,7 +165,7 @@ void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s);
 // draws'); launch_direct_shadow: the shadow pass's depth and ShadowBuffer
 // value of every texel from the keys.
 void launch_direct_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
-                          float *ndc_z, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s);
+                          float *ndc_z, float4 *vary, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s);
 void launch_direct(const DirectArgs &a, int max_faces, long long n_tri, hipStream_t s);
 void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth, float *shadow_out, hipStream_t s);
 void launch_gbuffer_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);

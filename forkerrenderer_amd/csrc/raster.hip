@@ -25,19 +25,23 @@
 namespace fgl {
 
 // A model's corner records (DevDraw::corner), a thread per corner: gathered
-// here, not built on the host and copied (144 bytes a face).
-__global__ __launch_bounds__(256) void k_corners(const float *__restrict__ pos, const float *__restrict__ uv,
-                                                 const float *__restrict__ nrm, const float *__restrict__ tan,
-                                                 const int *__restrict__ vi, const int *__restrict__ ti,
-                                                 const int *__restrict__ ni, size_t n, float4 *__restrict__ out)
+// here, not built on the host and copied (96 bytes a face).
+__global__ __launch_bounds__(256) void k_corners(const float *__restrict__ uv, const float *__restrict__ nrm,
+                                                 const float *__restrict__ tan, const int *__restrict__ vi,
+                                                 const int *__restrict__ ti, const int *__restrict__ ni, size_t n,
+                                                 float4 *__restrict__ out)
 {
     const size_t k = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= n) return;
-    const float *p = pos + 3 * (size_t)vi[k], *t = uv + 2 * (size_t)ti[k], *m = nrm + 3 * (size_t)ni[k];
-    out[3 * k] = make_float4(p[0], p[1], p[2], t[0]);
-    out[3 * k + 1] = make_float4(t[1], m[0], m[1], m[2]);
-    const float *g = tan ? tan + 3 * (size_t)vi[k] : nullptr;
-    out[3 * k + 2] = g ? make_float4(g[0], g[1], g[2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float *t = uv + 2 * (size_t)ti[k], *m = nrm + 3 * (size_t)ni[k];
+    const Vec3 nn = norm3(vec3(m[0], m[1], m[2]));
+    Vec3 tt = vec3(0.f, 0.f, 0.f);
+    if (tan) {
+        const float *g = tan + 3 * (size_t)vi[k];
+        tt = norm3(vec3(g[0], g[1], g[2]));
+    }
+    out[2 * k] = make_float4(t[0], t[1], nn.x, nn.y);
+    out[2 * k + 1] = make_float4(nn.z, tt.x, tt.y, tt.z);
 }
 
 // A bundle's texels (DevBundle) from its maps' own, a thread per texel in the
@@ -62,7 +66,7 @@ __global__ __launch_bounds__(256) void k_bundle(int w, int h, const uint32_t *__
 template <bool SHADOW>
 __global__ __launch_bounds__(256) void k_vertex(const DevDraw *__restrict__ draws, FrameUniforms u,
                                                 int4 *__restrict__ out, float *__restrict__ ndc_z,
-                                                uint32_t *__restrict__ zero)
+                                                float4 *__restrict__ vary, uint32_t *__restrict__ zero)
 {
     const DevDraw &dr = draws[blockIdx.y];
     const int vi = blockIdx.x * blockDim.x + threadIdx.x;
@@ -73,7 +77,8 @@ __global__ __launch_bounds__(256) void k_vertex(const DevDraw *__restrict__ draw
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        out[dr.vert_base + vi] = to_screen(u.viewport, main_ndc(dr, u, vi));
+        const size_t v = (size_t)dr.vert_base + vi;
+        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
     }
 }
 
@@ -193,7 +198,8 @@ constexpr int kClearKeys = 8;
 template <bool SHADOW>
 __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, int n_vert_blocks, int bx,
                                                        FrameUniforms u, int4 *__restrict__ out,
-                                                       float *__restrict__ ndc_z, unsigned long long *__restrict__ key,
+                                                       float *__restrict__ ndc_z, float4 *__restrict__ vary,
+                                                       unsigned long long *__restrict__ key,
                                                        size_t n_keys, DirectCtr *__restrict__ next_ctr)
 {
     const int b = blockIdx.x;
@@ -218,7 +224,8 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        out[dr.vert_base + vi] = to_screen(u.viewport, main_ndc(dr, u, vi));
+        const size_t v = (size_t)dr.vert_base + vi;
+        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
     }
 }
 
@@ -290,11 +297,12 @@ __global__ __launch_bounds__(256) void k_gbuffer_resolve(ResolveArgs a, FrameUni
 // m, barycentrics b) at pixel i.
 template <bool STREAM>
 __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameUniforms &u, const DevDraw &dr,
-                                              const DevMaterial &m, int f, const Vec3 &b, size_t i, size_t P)
+                                              const DevMaterial &m, int f, const int4 &tv, const Vec3 &b, size_t i,
+                                              size_t P)
 {
-    Varying v0 = main_vertex(dr, u, f, 0);
-    Varying v1 = main_vertex(dr, u, f, 1);
-    Varying v2 = main_vertex(dr, u, f, 2);
+    Varying v0 = main_vertex(dr, a.vary, tv.x, f, 0);
+    Varying v1 = main_vertex(dr, a.vary, tv.y, f, 1);
+    Varying v2 = main_vertex(dr, a.vary, tv.z, f, 2);
     const DevBundle &bn = m.bundle[dr.support_pbr ? 1 : 0];
     FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, bn);
     // the stochastic shadow filters: this fragment's samples in the stream
@@ -358,14 +366,14 @@ __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUni
         const int mi = dr.face_mat[f];
         const int m0 = __builtin_amdgcn_readfirstlane(mi);
         if (__ballot(mi != m0) == 0ull) {
-            forward_shade<STREAM>(a, u, dr, a.materials[m0], f, w.b, i, P);
+            forward_shade<STREAM>(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
             resolve_end<DIRECT>(a, i, w);
             return;
         }
     }
     const DevDraw &dr = a.draws[w.tv.w];
     const int f = w.g - dr.tri_base;
-    forward_shade<STREAM>(a, u, dr, a.materials[dr.face_mat[f]], f, w.b, i, P);
+    forward_shade<STREAM>(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
     resolve_end<DIRECT>(a, i, w);
 }
 
@@ -473,9 +481,9 @@ __global__ __launch_bounds__(256) void k_frag_shadow_inputs(ResolveArgs a, Frame
     const DevDraw &dr = a.draws[tv.w];
     const int f = g - dr.tri_base;
     const DevMaterial &m = a.materials[dr.face_mat[f]];
-    Varying v0 = main_vertex(dr, u, f, 0);
-    Varying v1 = main_vertex(dr, u, f, 1);
-    Varying v2 = main_vertex(dr, u, f, 2);
+    Varying v0 = main_vertex(dr, a.vary, tv.x, f, 0);
+    Varying v1 = main_vertex(dr, a.vary, tv.y, f, 1);
+    Varying v2 = main_vertex(dr, a.vary, tv.z, f, 2);
     const FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, m.bundle[dr.support_pbr ? 1 : 0]);
     const size_t N = n;
     out[k] = fg.normal.x;
@@ -510,23 +518,23 @@ __global__ __launch_bounds__(256) void k_frag_pixel_offsets(const uint32_t *__re
 static inline unsigned blocks_for(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 static inline dim3 grid2(int W, int H) { return dim3((W + 63) / 64, (H + 3) / 4); }
 
-void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos,
-                   const FrameUniforms &u, int4 *out, float *ndc_z, uint32_t *zero, hipStream_t s)
+void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
+                   float *ndc_z, float4 *vary, uint32_t *zero, hipStream_t s)
 {
     if (n_draws <= 0 || max_pos <= 0) {
         if (zero) launch_fill_u32(zero, 0u, 1, s);
         return;
     }
     dim3 grid(blocks_for(max_pos, 256), n_draws);
-    if (shadow) hipLaunchKernelGGL(k_vertex<true>, grid, dim3(256), 0, s, draws, u, out, ndc_z, zero);
-    else hipLaunchKernelGGL(k_vertex<false>, grid, dim3(256), 0, s, draws, u, out, ndc_z, zero);
+    if (shadow) hipLaunchKernelGGL(k_vertex<true>, grid, dim3(256), 0, s, draws, u, out, ndc_z, vary, zero);
+    else hipLaunchKernelGGL(k_vertex<false>, grid, dim3(256), 0, s, draws, u, out, ndc_z, vary, zero);
 }
 
-void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti,
-                    const int *ni, size_t n, float4 *out, hipStream_t s)
+void launch_corners(const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti, const int *ni,
+                    size_t n, float4 *out, hipStream_t s)
 {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_corners, dim3(blocks_for(n, 256)), dim3(256), 0, s, pos, uv, nrm, tan, vi, ti, ni, n, out);
+    hipLaunchKernelGGL(k_corners, dim3(blocks_for(n, 256)), dim3(256), 0, s, uv, nrm, tan, vi, ti, ni, n, out);
 }
 
 void launch_bundle(int w, int h, const uint32_t *a, const uint8_t *z, const uint32_t *n, const uint8_t *y, uint2 *out,
@@ -599,16 +607,16 @@ void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s)
 }
 
 void launch_direct_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
-                          float *ndc_z, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s)
+                          float *ndc_z, float4 *vary, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s)
 {
     const size_t P = (size_t)a.W * a.H;
     const unsigned bx = blocks_for(max_pos, 256), nv = bx * (unsigned)n_draws;
     const unsigned grid = nv + blocks_for(P, 256 * kClearKeys);
     if (shadow)
-        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z, a.key,
-                           P, next_ctr);
+        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z, vary,
+                           a.key, P, next_ctr);
     else
-        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z,
+        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z, vary,
                            a.key, P, next_ctr);
 }
 
