@@ -238,9 +238,10 @@ __global__ __launch_bounds__(256) void k_bv_direct_shadow(BvDirectArgs b, const 
                                                           const float *__restrict__ ndc_z, float *__restrict__ depth,
                                                           float *__restrict__ shadow)
 {
-    const DevView &v = b.views[__builtin_amdgcn_readfirstlane(sblk_view[blockIdx.x])];
-    const int lb = (int)(blockIdx.x - v.sblk_base), nbx = (v.S + 63) / 64;
-    const int x = (lb % nbx) * 64 + (threadIdx.x & 63), y = (lb / nbx) * 4 + (threadIdx.x >> 6);
+    const int blk = chunk_remap(blockIdx.x, gridDim.x);
+    const DevView &v = b.views[__builtin_amdgcn_readfirstlane(sblk_view[blk])];
+    int x, y;
+    block_px<32>((int)(blk - v.sblk_base), (v.S + 3) / 4, x, y);
     if (x >= v.S || y >= v.S) return;
     const size_t i = (size_t)x + (size_t)y * v.S;
     const Winner w = direct_winner(b.draws + v.draw_base[kBvShadow], v.n_draws, b.key + v.spx_off, nullptr, b.screen, v.S, v.S,
@@ -252,15 +253,15 @@ __global__ __launch_bounds__(256) void k_bv_direct_shadow(BvDirectArgs b, const 
     if (blockIdx.x == 0 && threadIdx.x == 0) *b.ctr = DirectCtr{0ull, 0u, 0u};
 }
 
-// Pixel (x, y) of the view owning 64 x 4 block blockIdx.x; false when it is
+// Pixel (x, y) of this thread in the view that owns its 64 x 4 block; false when it is
 // outside the view.
+template <int WT>
 __device__ __forceinline__ bool bv_pixel(const BvPixelArgs &a, int &vi, int &x, int &y)
 {
-    vi = __builtin_amdgcn_readfirstlane(a.blk_view[blockIdx.x]);
+    const int blk = chunk_remap(blockIdx.x, gridDim.x);
+    vi = __builtin_amdgcn_readfirstlane(a.blk_view[blk]);
     const DevView &v = a.views[vi];
-    const int lb = (int)(blockIdx.x - v.blk_base), nbx = (v.W + 63) / 64;
-    x = (lb % nbx) * 64 + (threadIdx.x & 63);
-    y = (lb / nbx) * 4 + (threadIdx.x >> 6);
+    block_px<WT>((int)(blk - v.blk_base), (v.H + 3) / 4, x, y);
     return x < v.W && y < v.H;
 }
 
@@ -268,7 +269,7 @@ template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
 {
     int vi, x, y;
-    if (!bv_pixel(b, vi, x, y)) return;
+    if (!bv_pixel<32>(b, vi, x, y)) return;
     const DevView &v = b.views[vi];
     ResolveArgs a;
     a.draws = DIRECT ? b.draws + v.draw_base[kBvMain] : b.draws;
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
 __global__ __launch_bounds__(256) void k_bv_lighting(BvPixelArgs b)
 {
     int vi, x, y;
-    if (!bv_pixel(b, vi, x, y)) return;
+    if (!bv_pixel<16>(b, vi, x, y)) return;
     const DevView &v = b.views[vi];
     const ShadowSamples none = {};
     lighting_px(v.u, b.gbuf + kGbufPlanes * v.px_off, b.ao + v.px_off, b.ao_is_one, b.shadow + v.spx_off, none,
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(256) void k_bv_lighting(BvPixelArgs b)
 __global__ __launch_bounds__(256) void k_bv_resolve(BvPixelArgs b)
 {
     int vi, x, y;
-    if (!bv_pixel(b, vi, x, y)) return;
+    if (!bv_pixel<32>(b, vi, x, y)) return;
     const DevView &v = b.views[vi];
     resolve_px(b.fb + 3 * v.px_off, v.W, v.H, 1, b.img + 3 * v.px_off, x, y);
 }

@@ -270,8 +270,8 @@ __global__ __launch_bounds__(256) void k_direct_nan(DirectArgs a, int bx, int bl
 __global__ __launch_bounds__(256) void k_direct_shadow(DirectArgs a, const float *__restrict__ ndc_z,
                                                        float *__restrict__ depth, float *__restrict__ shadow_out)
 {
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    int x, y;
+    grid_px<32>(x, y);
     if (x >= a.W || y >= a.H) return;
     const size_t i = (size_t)x + (size_t)y * a.W;
     const Winner w = direct_winner(a.draws, a.n_draws, a.key, a.fix, a.screen, a.W, a.H, i, x, y);
@@ -285,8 +285,8 @@ __global__ __launch_bounds__(256) void k_direct_shadow(DirectArgs a, const float
 template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_gbuffer_resolve(ResolveArgs a, FrameUniforms u)
 {
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    int x, y;
+    grid_px<32>(x, y);
     if (x >= a.W || y >= a.H) return;
     gbuffer_px<DIRECT>(a, u, x, y);
 }
@@ -344,8 +344,8 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
 template <bool STREAM, bool DIRECT>
 __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUniforms u)
 {
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    int x, y;
+    grid_px<32>(x, y);
     if (x >= a.W || y >= a.H) return;
     const size_t i = (size_t)x + (size_t)y * a.W;
     const size_t P = (size_t)a.W * a.H;

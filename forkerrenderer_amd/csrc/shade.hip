@@ -11,8 +11,8 @@ __global__ __launch_bounds__(256) void k_lighting(FrameUniforms u, const float *
                                                   const float *__restrict__ smap, ShadowSamples ss,
                                                   float *__restrict__ fb)
 {
-    const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    int x, y;
+    grid_px<16>(x, y);
     if (x >= u.W || y >= u.H) return;
     lighting_px<STREAM>(u, g, ao, ao_is_one, smap, ss, fb, x, y, net);
 }
