@@ -127,8 +127,8 @@ struct fgl_ctx {
     // kept vectors, their counts and checkpoints, the jump polynomials uploaded
     // so far; the last fill and the vectors asked of it, for its commit
     DevBuf mt_base, mt_states, mt_vec, mt_ck;
-    DevBuf mt_polys[2];          // jump polynomials for the two chunk lengths
-    int mt_polys_n[2] = {0, 0};
+    DevBuf mt_lists[2];          // the jumps' read lists for the two chunk lengths
+    int mt_lists_n[2] = {0, 0};
     MtFill fill{};
     uint32_t fill_n = 0;
 
@@ -362,7 +362,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     DevBuf *bufs[] = {&c->d_textures, &c->d_materials, &c->depth, &c->fb, &c->gbuf, &c->ao,
                       &c->blur_tmp, &c->shadow, &c->shadow_depth, &c->img, &c->vis, &c->d_draws,
                       &c->rng, &c->rng_samples, &c->rng_offs, &c->ssao_pow3,
-                      &c->mt_base, &c->mt_states, &c->mt_vec, &c->mt_ck, &c->mt_polys[0], &c->mt_polys[1],
+                      &c->mt_base, &c->mt_states, &c->mt_vec, &c->mt_ck, &c->mt_lists[0], &c->mt_lists[1],
                       &c->screen, &c->rect, &c->counts, &c->offs, &c->scan_tmp, &c->keys,
                       &c->vals, &c->keys_alt, &c->vals_alt, &c->sort_tmp, &c->tile_start,
                       &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z, &c->vary,
@@ -1012,18 +1012,25 @@ static int rng_fill(fgl_ctx *c, int D, uint32_t n)
         launch_mt_base((const MtState *)c->rng.p, Nc > 1 ? (uint32_t)kMtBaseWords : 624u, base, c->stream);
         if (Nc > 1) {
             const int nj = (int)Nc - 1;
-            if (nj > c->mt_polys_n[kind]) {
+            if (nj > c->mt_lists_n[kind]) {
                 std::vector<uint64_t> polys;
                 if (!mt_jump_polys(C, nj, polys))
                     return fail(c, FGL_ERR_DEVICE, "random stream: no characteristic polynomial");
-                if ((rc = ensure(c, c->mt_polys[kind], polys.size() * sizeof(uint64_t)))) return rc;
-                HIPCHK(c, hipMemcpyAsync(c->mt_polys[kind].p, polys.data(), polys.size() * sizeof(uint64_t),
-                                         hipMemcpyHostToDevice, c->stream));
+                c->mt_lists_n[kind] = 0;
+                if ((rc = ensure(c, c->mt_lists[kind], (size_t)nj * (kMtListMax * 2 + kMtListStarts * 4)))) return rc;
+                // the polynomials pass through the vectors' space, which the
+                // fill writes after the lists are made
+                static_assert(624 * kMtChunkShort / 3 * 4 >= kMtPolyWords * 8, "a chunk's vectors hold a polynomial");
+                HIPCHK(c, hipMemcpyAsync(f.out, polys.data(), (size_t)nj * kMtPolyWords * 8, hipMemcpyHostToDevice, c->stream));
+                uint16_t *entries = (uint16_t *)c->mt_lists[kind].p;
+                launch_mt_lists((const uint64_t *)f.out, nj, entries, (uint32_t *)(entries + (size_t)nj * kMtListMax), c->stream);
                 HIPCHK(c, hipStreamSynchronize(c->stream));
-                c->mt_polys_n[kind] = nj;
+                c->mt_lists_n[kind] = nj;
             }
-            if ((rc = ensure(c, c->mt_states, (size_t)Nc * 624 * 4))) return rc;
-            launch_mt_jump(base, (const uint64_t *)c->mt_polys[kind].p, nj, (uint32_t *)c->mt_states.p, c->stream);
+            if ((rc = ensure(c, c->mt_states, (size_t)Nc * kMtStateWords * 4))) return rc;
+            const uint16_t *entries = (const uint16_t *)c->mt_lists[kind].p;
+            launch_mt_jump(base, entries, (const uint32_t *)(entries + (size_t)c->mt_lists_n[kind] * kMtListMax), nj,
+                           (uint32_t *)c->mt_states.p, c->stream);
             states = (const uint32_t *)c->mt_states.p;
         }
         launch_mt_fill(base, states, f, c->stream);

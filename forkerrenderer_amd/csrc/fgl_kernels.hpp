@@ -208,11 +208,18 @@ struct MtState {
 void mt_seed_state(uint32_t seed, MtState &st);
 // The stream's next draws in parallel chunks of 624 K draws: base = the words
 // from the context's next draw on, n of them (kMtBaseWords for jumps, one
-// window otherwise); states[c] (c = 1..n_jumps, 624 words each) = chunk c's
-// first window from jump polynomial c (mt_jump.hpp; kMtPolyWords words each).
+// window otherwise); states[c] (c = 1..n_jumps, kMtStateWords each) = chunk c's
+// first window from jump polynomial c (mt_jump.hpp; kMtPolyWords words each),
+// as lists of what to read (launch_mt_lists: kMtListMax entries and 13 starts
+// a polynomial, made once).
 constexpr int kMtBaseWords = 33 * 624;
+constexpr int kMtListMax = 7056, kMtListStarts = 13;
+// A chunk's window is left in parts of 624 words each, their XOR the window.
+constexpr int kMtStateWords = 3 * 624;
 void launch_mt_base(const MtState *st, uint32_t n, uint32_t *base, hipStream_t s);
-void launch_mt_jump(const uint32_t *base, const uint64_t *polys, int n_jumps, uint32_t *states, hipStream_t s);
+void launch_mt_lists(const uint64_t *polys, int n, uint16_t *entries, uint32_t *start, hipStream_t s);
+void launch_mt_jump(const uint32_t *base, const uint16_t *entries, const uint32_t *start, int n_jumps, uint32_t *states,
+                    hipStream_t s);
 // A fill of rejection-sampled unit vectors (D = 3: RandomVectorInUnitSphere
 // (x, y, z); 2: RandomVectorInUnitDisk (x, y)): T tries of D draws a chunk,
 // the kept vectors of chunk c at out + c stride D (stride >= T + kStreamRun),
