@@ -126,7 +126,7 @@ struct fgl_ctx {
     // the parallel generator: base sequence, jumped chunk arrays, the chunks'
     // kept vectors, their counts and checkpoints, the jump polynomials uploaded
     // so far; the last fill and the vectors asked of it, for its commit
-    DevBuf mt_base, mt_states, mt_vec, mt_ck;
+    DevBuf mt_base, mt_states, mt_vec, mt_ck, pcss_mm;
     DevBuf mt_lists[2];          // the jumps' read lists for the two chunk lengths
     int mt_lists_n[2] = {0, 0};
     MtFill fill{};
@@ -204,6 +204,25 @@ static int ensure(fgl_ctx *c, DevBuf &b, size_t bytes)
     }
     b.cap = want;
     return FGL_OK;
+}
+
+// ensure() for memory that the caller can do without: no error without it.
+static bool room(fgl_ctx *c, DevBuf &b, size_t bytes)
+{
+    if (bytes <= b.cap && b.p) return true;
+    if (b.p) {
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+        (void)hipFree(b.p);
+        b.p = nullptr;
+        b.cap = 0;
+    }
+    if (hipMalloc(&b.p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        b.p = nullptr;
+        return false;
+    }
+    b.cap = bytes;
+    return true;
 }
 
 static void free_buf(DevBuf &b)
@@ -362,7 +381,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     DevBuf *bufs[] = {&c->d_textures, &c->d_materials, &c->depth, &c->fb, &c->gbuf, &c->ao,
                       &c->blur_tmp, &c->shadow, &c->shadow_depth, &c->img, &c->vis, &c->d_draws,
                       &c->rng, &c->rng_samples, &c->rng_offs, &c->ssao_pow3,
-                      &c->mt_base, &c->mt_states, &c->mt_vec, &c->mt_ck, &c->mt_lists[0], &c->mt_lists[1],
+                      &c->mt_base, &c->mt_states, &c->mt_vec, &c->mt_ck, &c->pcss_mm, &c->mt_lists[0], &c->mt_lists[1],
                       &c->screen, &c->rect, &c->counts, &c->offs, &c->scan_tmp, &c->keys,
                       &c->vals, &c->keys_alt, &c->vals_alt, &c->sort_tmp, &c->tile_start,
                       &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z, &c->vary,
@@ -1094,7 +1113,14 @@ static int stochastic_shadow_samples(fgl_ctx *c, const FrameUniforms &u, const f
     uint32_t *pred = res + kPcssChainRes;
     uint32_t *seg_out = pred + 2 * ((size_t)kSegmentMax + 2);
     uint32_t *tmp = seg_out + 4;
-    launch_pcss_classify(u, g, n, (const float *)c->shadow.p, base, upos, c->stream);
+    int bx = 0, by = 0;
+    float2 *mm = nullptr;   // without it (no room) every texel is read
+    if (n > 0 && u.shadow_on && u.n_lights > 0 && pcss_windows(u, n, bx, by) &&
+        room(c, c->pcss_mm, (size_t)u.SW * u.SH * sizeof(float2))) {
+        mm = (float2 *)c->pcss_mm.p;
+        launch_pcss_minmax(u, (const float *)c->shadow.p, bx, by, mm, c->stream);
+    }
+    launch_pcss_classify(u, g, n, (const float *)c->shadow.p, mm, bx, by, base, upos, c->stream);
     launch_exclusive_scan(base, base, n, tmp, c->stream);
     launch_exclusive_scan(upos, upos, n, tmp, c->stream);
     launch_pcss_compact(upos, n, list, c->stream);

@@ -261,8 +261,12 @@ void launch_ssao_reference(const FrameUniforms &u, const StreamVectors &samples,
 // launch_pcss_segment), then
 // offs[i] = base[i] + n_pcf * (blockers found by undecided points before i)
 // for i = 0..P.
-void launch_pcss_classify(const FrameUniforms &u, const float *g, size_t P, const float *shadow_map, uint32_t *cnt,
-                          uint32_t *unc, hipStream_t s);
+// mm (may be null): the depth extremes of bx x by texel windows
+// (launch_pcss_minmax) where pcss_windows finds them worth making.
+bool pcss_windows(const FrameUniforms &u, size_t P, int &bx, int &by);
+void launch_pcss_minmax(const FrameUniforms &u, const float *shadow_map, int bx, int by, float2 *mm, hipStream_t s);
+void launch_pcss_classify(const FrameUniforms &u, const float *g, size_t P, const float *shadow_map, const float2 *mm,
+                          int bx, int by, uint32_t *cnt, uint32_t *unc, hipStream_t s);
 void launch_pcss_compact(const uint32_t *upos, size_t P, uint32_t *list, hipStream_t s);
 // The n undecided points' stream-independent inputs (shadow coordinate and
 // bias, sample base), then segments [s0, s0 + L) of the ordered walk from

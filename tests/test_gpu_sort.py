@@ -55,3 +55,13 @@ def test_rejects_bad_arguments(ctx):
         ctx.sort_pairs(np.zeros(4, np.uint32), np.zeros(4, np.uint32), 0)
     k, v = ctx.sort_pairs(np.zeros(0, np.uint32), np.zeros(0, np.uint32), 8)
     assert k.size == 0 and v.size == 0
+
+
+@pytest.mark.parametrize("n", [262_144, 262_145, 33_554_433])
+def test_scan_sizes(ctx, n):
+    """A pass scans 256 counts per 2,048 items: the most that one workgroup
+    scans (128 blocks), one block more (two launches), and a scan of 2,049
+    blocks (three)."""
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 256, n, dtype=np.uint32)
+    _check(ctx, keys, np.arange(n, dtype=np.uint32), 8)

@@ -251,3 +251,29 @@ def test_batched_views_refuse_the_stochastic_filters(ctx, scene_dir):
     got = gpu_frame(ctx, sc2)
     want = oracle_frame(sc2)
     assert_bitexact("depth after errors", got["depth"], want["depth"])
+
+
+@pytest.mark.parametrize("shadowmap,blocker_filter",
+                         [(96, 0.02), (61, 0.1), (128, 0.3), (128, 1.5), (None, 0.06), (64, 0.0), (2048, 0.05)])
+def test_blocker_search_areas_match_the_oracle(ctx, scene_dir, shadowmap, blocker_filter):
+    """Points are classified by the depth extremes of texel windows: search
+    areas of one window, of several (larger than 16 texels), larger than the
+    map, cut off at its edges (read texel by texel), on odd and non-square
+    maps, and maps too large to make windows of.  The stream moves by what the
+    classification decides, so draw counts and image follow it."""
+    p = G.tiny_scene(os.path.join(scene_dir, f"rb{shadowmap}_{blocker_filter}"), seed=36, width=64, height=48, subdiv=3,
+                     tex=16, shadowmap=shadowmap, extra="shadowfilter refpcss")
+    sc = F.Scene(p)
+    gpu_frame(ctx, sc)
+    sc.info.shadow.blocker_filter = blocker_filter
+    ctx.set_shadow(True, sc.info.shadow)
+    ctx.rng_seed(5489)
+    ctx.begin_pass(F.PASS_LIGHTING)
+    ctx.draw_screen_space_pixels()
+    ctx.end_pass()
+    got = ctx.read(F.TARGET_FRAME)
+    device_draws = ctx.rng_draws()
+    want = oracle_frame(sc)
+    assert device_draws == O.rng_draws(), (device_draws, O.rng_draws())
+    assert np.abs(got.reshape(-1) - np.asarray(want["fb"]).reshape(-1)).max() < 1e-4
+    ctx.rng_seed(5489)
