@@ -743,4 +743,13 @@ __device__ __forceinline__ void grid_px(int &x, int &y)
     block_px<WT>(chunk_remap(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y), gridDim.y, x, y);
 }
 
+// A workgroup's barrier that orders its LDS accesses alone: a __syncthreads()
+// also waits for the global stores before it.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 }  // namespace fgl

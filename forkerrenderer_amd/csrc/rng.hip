@@ -69,16 +69,9 @@ __device__ __forceinline__ float random_pm1(uint32_t u)
 // accesses are one address and constant offsets; a long run copies its last
 // 624 words to the front every kMtLap intervals.
 //
-// The barrier orders LDS alone: a __syncthreads() also waits for the
-// interval's global stores, which made a step of 227 words 860 cycles.
+// The barrier orders LDS alone (a __syncthreads() made a step of 227 words 860
+// cycles).
 constexpr uint32_t kMtLag = kMtN - kMtM, kMtPair = 2 * kMtLag;
-
-__device__ __forceinline__ void mt_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // A running generator: `made` words in, the array holds x_made ..
 // x_{made+623} from at - threadIdx.x on.  The first 227 threads make words;
@@ -156,7 +149,7 @@ __global__ __launch_bounds__(256) void k_mt_base(const MtState *__restrict__ st,
             if (at + tid < n) base[at + tid] = w0;
             if (at + kMtLag + tid < n) base[at + kMtLag + tid] = w1;
         }
-        mt_barrier();
+        lds_barrier();
     }
 }
 
@@ -374,7 +367,7 @@ __global__ __launch_bounds__(kMtFillThreads<D>) void k_mt_fill(const uint32_t *_
                 iq = 0;
                 run.at = words + tid;
                 for (uint32_t i = tid; i < kMtN; i += 256) words[i] = words[kLapWords + i];
-                mt_barrier();
+                lds_barrier();
             }
             if (iq == 0 && q % kMtCkEvery == 0) {
                 uint32_t *ck = ck_words + ((size_t)c * n_ck + q / kMtCkEvery) * kMtN;
@@ -382,7 +375,7 @@ __global__ __launch_bounds__(kMtFillThreads<D>) void k_mt_fill(const uint32_t *_
             }
             uint32_t w0, w1;
             run.pair(w0, w1);
-            mt_barrier();
+            lds_barrier();
         }
     } else {
         const uint32_t i = tid - 256, wave = __builtin_amdgcn_readfirstlane(i >> 6);
@@ -405,7 +398,7 @@ __global__ __launch_bounds__(kMtFillThreads<D>) void k_mt_fill(const uint32_t *_
         for (uint32_t j = 0, ij = 0; j <= J; ++j, ++ij) {
             if (ij == kMtLap / 2 && 2 * j < Q) {
                 ij = 0;
-                mt_barrier();
+                lds_barrier();
             }
             {   // slot 2 j: test the tries of intervals 2 j - 2 and 2 j - 1
                 const uint32_t first = mt_first<D>(2 * j - 2), end = mt_first<D>(2 * j);
@@ -418,7 +411,7 @@ __global__ __launch_bounds__(kMtFillThreads<D>) void k_mt_fill(const uint32_t *_
                 rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(k0 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)k0, 0u));
                 rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(k1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)k1, rank));
                 if ((i & 63) == 0) cnt[j & 1][wave] = (uint16_t)(__popcll(k0) + __popcll(k1));
-                mt_barrier();
+                lds_barrier();
             }
             // slot 2 j + 1: write what was kept of them, read the next ones
             const uint32_t *k = (const uint32_t *)cnt[j & 1];
@@ -444,7 +437,7 @@ __global__ __launch_bounds__(kMtFillThreads<D>) void k_mt_fill(const uint32_t *_
             }
             mt_vector<D>(a, v0[0], v0[1], v0[2]);
             mt_vector<D>(b, v1[0], v1[1], v1[2]);
-            mt_barrier();
+            lds_barrier();
         }
         if (i == 0) kept[c] = total;
     }
@@ -550,7 +543,7 @@ __global__ __launch_bounds__(512) void k_mt_commit(MtState *__restrict__ st, con
             mt_vector<D>(w, tried.x, tried.y, tried.z);
             tried.test<D>(cnt[q & 1], wave, a < e ? (b < e ? b : e) - a : 0u);
         }
-        mt_barrier();
+        lds_barrier();
     }
     // the window after a try at the end of its interval reaches into the
     // next pair's words

@@ -481,83 +481,121 @@ __global__ __launch_bounds__(1024) void k_ssao_tiled(FrameUniforms u, SsaoArgs s
 __constant__ float c_ref_blur_w[5] = {(float)0.227027, (float)0.1945946, (float)0.1216216,
                                       (float)0.054054, (float)0.016216};
 
-// Buffer1f::TwoPassGaussianBlurDenoised (src/buffer.cpp:59-98) along one
-// line of n samples at stride s, in place: each output is the reference's
-// sum in its order -- the centre, then for i = 1..4 the sample i ahead
-// (not yet blurred) and the sample i behind (already blurred), indices
-// clamped to the line.  The last four outputs and the next four inputs stay
-// in registers, and the inputs are loaded kPF steps ahead (samples ahead are
-// never written before they are read), so a step waits on its own
-// arithmetic, not on memory.
-constexpr int kPF = 64;
+// Buffer1f::TwoPassGaussianBlurDenoised (src/buffer.cpp:59-98) along lines of
+// n samples, in place: each output is the reference's sum in its order -- the
+// centre, then for i = 1..4 the sample i ahead (not yet blurred) and the
+// sample i behind (already blurred), indices clamped to the line.
+//
+// A line is a chain: a step needs the output before it, and a frame has fewer
+// lines than the chip has lanes, so the kernel is bound by the instructions of
+// one step.  One wavefront takes the steps of 64 lines and is left only the
+// sums in order and the products of its outputs (8 additions, 4 products); four
+// others make what does not depend on outputs -- centre plus first sample
+// ahead, the other products ahead -- a chunk of samples before it, and carry
+// its results out a chunk after it.  Every step done by its line's thread with
+// its loads and stores: 1280 x 800 rows 128 -> 53 us, columns 64 -> 36.
+constexpr int kRecChunk = 32, kRecWaves = 4, kRecPer = kRecChunk / kRecWaves;
 
-__device__ __forceinline__ void blur_rec_line(float *__restrict__ p, int n, size_t s)
+// ROWS: line l is row l (n = W), else column l (n = H).  vec: rows start
+// 16-byte aligned and hold whole quads.
+template <bool ROWS>
+__global__ __launch_bounds__(64 * (kRecWaves + 1)) void k_blur_rec(float *p, int W, int H, bool vec)
 {
+    __shared__ float4 ahead[2][kRecChunk][64];
+    __shared__ float done[2][kRecChunk][65];
     const float w0 = c_ref_blur_w[0], w1 = c_ref_blur_w[1], w2 = c_ref_blur_w[2], w3 = c_ref_blur_w[3],
                 w4 = c_ref_blur_w[4];
-    auto at = [&](int x) { return p[(size_t)(x < n - 1 ? x : n - 1) * s]; };
-    float a0 = at(0), a1 = at(1), a2 = at(2), a3 = at(3), a4 = at(4);
-    // x = 0: every sample behind clamps to sample 0, not yet blurred
-    float r = a0 * w0;
-    r += a1 * w1;
-    r += a0 * w1;
-    r += a2 * w2;
-    r += a0 * w2;
-    r += a3 * w3;
-    r += a0 * w3;
-    r += a4 * w4;
-    r += a0 * w4;
-    p[0] = r;
-    float o1 = r, o2 = r, o3 = r, o4 = r;   // from here on they clamp to the blurred sample 0
-    a0 = a1;
-    a1 = a2;
-    a2 = a3;
-    a3 = a4;
-    float ring[kPF];
+    const int lines = ROWS ? H : W, n = ROWS ? W : H, l0 = blockIdx.x * 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int line = imin(l0 + lane, lines - 1);   // past the last: computed, not written
+    const size_t step = ROWS ? 1 : W;
+    float *mine = p + (ROWS ? (size_t)line * W : (size_t)line);
+    const int chunks = (n + kRecChunk - 1) / kRecChunk;
+    // slot t: chunk t is prepared, chunk t - 1 stepped through, chunk t - 2 written
+    if (wave == 0) {
+        const float first = mine[0];   // x = 0: every sample behind clamps to sample 0, not yet blurred
+        float p1 = first * w1, p2[2] = {first * w2, 0.f}, p3[3] = {first * w3, 0.f, 0.f}, p4[4] = {first * w4, 0.f, 0.f, 0.f};
+        lds_barrier();
+        for (int c = 0; c < chunks; ++c) {
+            const int buf = c & 1;
+#pragma unroll 1
+            for (int e0 = 0; e0 < kRecChunk; e0 += 8) {
+                float4 v[8];
 #pragma unroll
-    for (int j = 0; j < kPF; ++j) ring[j] = at(5 + j);
-    for (int x0 = 1; x0 < n; x0 += kPF) {
+                for (int e = 0; e < 8; ++e) v[e] = ahead[buf][e0 + e][lane];
 #pragma unroll
-        for (int j = 0; j < kPF; ++j) {
-            const int x = x0 + j;
-            if (x < n) {
-                a4 = ring[j];                   // sample x + 4
-                ring[j] = at(x + 4 + kPF);      // for step x + kPF
-                float q = a0 * w0;
-                q += a1 * w1;
-                q += o1 * w1;
-                q += a2 * w2;
-                q += o2 * w2;
-                q += a3 * w3;
-                q += o3 * w3;
-                q += a4 * w4;
-                q += o4 * w4;
-                p[(size_t)x * s] = q;
-                o4 = o3;
-                o3 = o2;
-                o2 = o1;
-                o1 = q;
-                a0 = a1;
-                a1 = a2;
-                a2 = a3;
-                a3 = a4;
+                for (int e = 0; e < 8; ++e) {
+                    float q = v[e].x + p1;
+                    q += v[e].y;
+                    q += p2[0];
+                    q += v[e].z;
+                    q += p3[0];
+                    q += v[e].w;
+                    q += p4[0];
+                    done[buf][e0 + e][lane] = q;
+                    const float r2 = q * w2, r3 = q * w3, r4 = q * w4;
+                    p1 = q * w1;
+                    p2[0] = p2[1]; p2[1] = r2;
+                    p3[0] = p3[1]; p3[1] = p3[2]; p3[2] = r3;
+                    p4[0] = p4[1]; p4[1] = p4[2]; p4[2] = p4[3]; p4[3] = r4;
+                    if (e == 0 && e0 == 0 && c == 0) {   // from here on they clamp to the blurred sample 0
+                        p2[0] = r2;
+                        p3[0] = p3[1] = r3;
+                        p4[0] = p4[1] = p4[2] = r4;
+                    }
+                }
+            }
+            lds_barrier();
+        }
+        return;
+    }
+    const int w = wave - 1, tid = threadIdx.x - 64;
+    float a[kRecPer + 4];   // the samples of this thread's part of the next chunk, and four ahead
+    auto load = [&](int c) {
+        const int x0 = c * kRecChunk + w * kRecPer;
+        if (ROWS && vec) {
+#pragma unroll
+            for (int e = 0; e < kRecPer + 4; e += 4) {
+                if (x0 + e < n) {
+                    const float4 v = *(const float4 *)(mine + x0 + e);
+                    a[e] = v.x; a[e + 1] = v.y; a[e + 2] = v.z; a[e + 3] = v.w;
+                } else {
+                    a[e] = a[e + 1] = a[e + 2] = a[e + 3] = mine[n - 1];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < kRecPer + 4; ++e) a[e] = mine[(size_t)imin(x0 + e, n - 1) * step];
+        }
+    };
+    load(0);
+    for (int t = 0; t < chunks + 2; ++t) {
+        if (t < chunks) {
+#pragma unroll
+            for (int e = 0; e < kRecPer; ++e)
+                ahead[t & 1][w * kRecPer + e][lane] = make_float4(a[e] * w0 + a[e + 1] * w1, a[e + 2] * w2, a[e + 3] * w3,
+                                                                  a[e + 4] * w4);
+            if (t + 1 < chunks) load(t + 1);
+        }
+        if (t >= 2) {
+            const int c = t - 2;
+            if (ROWS) {
+                const int x = tid & 31, at = c * kRecChunk + x;
+#pragma unroll
+                for (int r = 0; r < 64; r += 2 * kRecWaves) {
+                    const int row = r + (tid >> 5);
+                    if (at < n && l0 + row < lines) p[(size_t)(l0 + row) * W + at] = done[c & 1][x][row];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < kRecPer; ++e) {
+                    const int x = c * kRecChunk + w * kRecPer + e;
+                    if (x < n && l0 + lane < lines) p[(size_t)x * W + l0 + lane] = done[c & 1][w * kRecPer + e][lane];
+                }
             }
         }
+        lds_barrier();
     }
-}
-
-__global__ __launch_bounds__(64) void k_blur_rec_rows(float *__restrict__ a, int W, int H)
-{
-    const int h = blockIdx.x * 64 + threadIdx.x;
-    if (h >= H) return;
-    blur_rec_line(a + (size_t)h * W, W, 1);
-}
-
-__global__ __launch_bounds__(64) void k_blur_rec_cols(float *__restrict__ a, int W, int H)
-{
-    const int x = blockIdx.x * 64 + threadIdx.x;
-    if (x >= W) return;
-    blur_rec_line(a + x, H, (size_t)W);
 }
 
 struct BlurWeights {
@@ -745,8 +783,10 @@ void launch_ssao(const FrameUniforms &u, const SsaoArgs &sa, const float *depth,
 void launch_blur_recursive(float *ao, int W, int H, hipStream_t s)
 {
     if (W <= 0 || H <= 0) return;
-    hipLaunchKernelGGL(k_blur_rec_rows, dim3((H + 63) / 64), dim3(64), 0, s, ao, W, H);
-    hipLaunchKernelGGL(k_blur_rec_cols, dim3((W + 63) / 64), dim3(64), 0, s, ao, W, H);
+    const bool vec = (W & 3) == 0 && ((uintptr_t)ao & 15) == 0;
+    const dim3 block(64 * (kRecWaves + 1));
+    hipLaunchKernelGGL(k_blur_rec<true>, dim3((H + 63) / 64), block, 0, s, ao, W, H, vec);
+    hipLaunchKernelGGL(k_blur_rec<false>, dim3((W + 63) / 64), block, 0, s, ao, W, H, vec);
 }
 
 void launch_blur_separable(const float *src, float *dst, int W, int H, const float *w, int R, hipStream_t s)
