@@ -424,6 +424,21 @@ __device__ __forceinline__ const float *stream_at(const StreamVectors &s, uint32
     return s.v + ((size_t)c * s.stride + (j - s.prefix[c])) * D;
 }
 
+// The pairs from j on that lie in one run: their address and how many.
+struct StreamRun {
+    const float *v;
+    uint32_t left;
+};
+
+__device__ __forceinline__ StreamRun stream_run(const StreamVectors &s, uint32_t j)
+{
+    uint32_t c = (uint32_t)((float)j * s.inv);
+    c = c < s.chunks ? c : s.chunks - 1;
+    while (c > 0 && j < s.prefix[c]) --c;
+    while (c + 1 < s.chunks && j >= s.prefix[c + 1]) ++c;
+    return StreamRun{s.v + ((size_t)c * s.stride + (j - s.prefix[c])) * 2, s.prefix[c + 1] - j};
+}
+
 // The random stream's samples (modes 4 and 5) are each pixel's own, 512
 // bytes or more apart between neighbouring lanes: read one sample per load,
 // every load would fetch a cache line per lane.  So they are taken

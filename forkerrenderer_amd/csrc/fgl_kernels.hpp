@@ -275,7 +275,7 @@ void launch_pcss_compact(const uint32_t *upos, size_t P, uint32_t *list, hipStre
 // 64-bit words), fbits (kPcssChainFbits 64-bit words) and res
 // (kPcssChainRes words) for the walks of the segment's blocks; out = (first
 // unsettled point, misses before it).
-constexpr uint32_t kPcssSegmentMax = 32768, kPcssChainBlock = 1024;
+constexpr uint32_t kPcssSegmentMax = 32768, kPcssChainBlock = 512;
 constexpr int kPcssBandWidth = 63;
 constexpr size_t kPcssChainFbits = (size_t)(kPcssSegmentMax / kPcssChainBlock) * kPcssBandWidth * (kPcssChainBlock / 64);
 constexpr size_t kPcssChainRes = 2 * (size_t)(kPcssSegmentMax / kPcssChainBlock) * kPcssBandWidth;

@@ -207,7 +207,8 @@ __global__ __launch_bounds__(256) void k_pcss_points(FrameUniforms u, const floa
 //    straight line at the miss rate so far) -- exact wherever the outcomes
 //    do not depend on the samples' offset, which is most points;
 //  * k_pcss_band evaluates every point at the 63 values of M_k around its
-//    prediction, a wavefront per point, the outcomes as a bit mask;
+//    prediction, a wavefront per point, eight of them at a time, the outcomes
+//    as a bit mask;
 //  * k_pcss_walk_blocks and k_pcss_chain follow the actual M_k through the
 //    masks in order, write found[k] (1: a blocker) and stop where M_k
 //    leaves the band or the segment ends; the host starts the next segment
@@ -219,13 +220,65 @@ __global__ __launch_bounds__(256) void k_pcss_points(FrameUniforms u, const floa
 constexpr int kBandHalf = 31;   // M_k in [prediction - 31, prediction + 31]: a wavefront per point
 constexpr int kGuesses = 2;     // prediction rounds per segment (more do not pay)
 
-// The blocker search of an undecided point at sample offset o (the stream
-// samples' loads grouped as in the shading, fgl_device.hpp).
-__device__ __forceinline__ bool pcss_search(const FrameUniforms &u, const float *__restrict__ smap,
-                                            const StreamVectors &pairs, float4 q, uint32_t o)
+// The blocker search of an undecided point by the kSearchLanes lanes whose
+// lowest is a multiple of that, with its samples from offset o of the stream:
+// lane j takes the samples j, j + kSearchLanes ..., so a load of the group's is
+// one run of the stream and a guess's chain of loads a quarter as long (all 32
+// of a point in one lane, a line per lane and load: segments of 8,192 to 32,768
+// points 10.3 -> 4.9 us a guess, 48.5 -> 44.8 a band).  Found is whether a
+// blocker's depth lies beyond 0.0011: no depth is below 0.001f, and the average
+// of up to 64 of them with that one does not round below 0.001; where the only
+// blockers are within reach of 0.001 the search is run as it is.
+constexpr int kSearchLanes = 8;   // also the rounds of a band's 64 candidates
+template <bool INSIDE>
+__device__ __forceinline__ void pcss_samples(const FrameUniforms &u, const float *__restrict__ smap, const float2 *d, float4 q,
+                                             int n, int sub, bool &any, bool &sure)
 {
-    const float dB = pcss_blocker_stream(u, smap, vec3(q.x, q.y, q.z), q.w, stream_at<2>(pairs, o), u.shadow.n_blocker);
-    return !((double)dB < 0.001);
+    const double filter = u.shadow.blocker_filter;
+    const int w = (int)((float)u.SW - 0.001f), h = (int)((float)u.SH - 0.001f);
+    constexpr int G = 4;   // 32 samples: one group
+    for (int s0 = sub; s0 < n; s0 += G * kSearchLanes) {
+        float2 ds[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) ds[e] = d[imin(s0 + e * kSearchLanes, n - 1)];   // (the last again: nothing new)
+        float dd[G];
+        bool in[G];
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            const float su = q.x + (float)((double)ds[e].x * filter);
+            const float sv = q.y + (float)((double)ds[e].y * filter);
+            in[e] = true;
+            if (INSIDE) dd[e] = smap[(uint32_t)((int)((float)w * su) + (int)((float)h * sv) * u.SW)];
+            else dd[e] = smap[shadow_texel(u.SW, w, h, su, sv, in[e])];
+        }
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            const float v = shadow_value(in[e], dd[e]);
+            const bool blk = q.z > v + q.w;
+            any = any || blk;
+            sure = sure || (blk && v > 0.0011f);
+        }
+    }
+}
+
+// Every sample of the point q on the map (true of its whole search area).
+__device__ __forceinline__ bool pcss_inside(const FrameUniforms &u, float4 q)
+{
+    const float F = fabsf((float)u.shadow.blocker_filter);
+    return q.x - F >= 0.f && q.x + F <= 1.f && q.y - F >= 0.f && q.y + F <= 1.f && (size_t)u.SW * u.SH < 0x80000000ull;
+}
+
+// OR over a group's lanes.
+__device__ __forceinline__ uint32_t search_or(uint32_t v)
+{
+#pragma unroll
+    for (int d = 1; d < kSearchLanes; d <<= 1) v |= __shfl_xor(v, d, 64);
+    return v;
+}
+
+__device__ __forceinline__ bool pcss_search_exact(const FrameUniforms &u, const float *__restrict__ smap, const float *d, float4 q)
+{
+    return !((double)pcss_blocker_stream(u, smap, vec3(q.x, q.y, q.z), q.w, d, u.shadow.n_blocker) < 0.001);
 }
 
 // pred == nullptr: the prediction M0 + round(i * rate); else M0 + pred[i]
@@ -244,10 +297,18 @@ __global__ __launch_bounds__(256) void k_pcss_guess(FrameUniforms u, const float
                                                     uint32_t M0, float rate, const uint32_t *__restrict__ pred,
                                                     uint32_t *__restrict__ miss)
 {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) / kSearchLanes;
     if (i >= L) return;
     const uint32_t k = s0 + i, M = pcss_predict(pred, M0, rate, i);
-    miss[i] = pcss_search(u, smap, pairs, pt[k], pbase[k] + (uint32_t)u.shadow.n_pcf * (k - M)) ? 0u : 1u;
+    const float4 q = pt[k];
+    const float *d = stream_at<2>(pairs, pbase[k] + (uint32_t)u.shadow.n_pcf * (k - M));
+    const int sub = (int)(threadIdx.x & (kSearchLanes - 1)), n = u.shadow.n_blocker;
+    bool any = false, sure = false;
+    if (__all(pcss_inside(u, q))) pcss_samples<true>(u, smap, (const float2 *)d, q, n, sub, any, sure);
+    else pcss_samples<false>(u, smap, (const float2 *)d, q, n, sub, any, sure);
+    const uint32_t got = search_or((any ? 1u : 0u) | (sure ? 2u : 0u));
+    const bool f = got == 1u ? pcss_search_exact(u, smap, d, q) : got != 0u;
+    if ((threadIdx.x & (kSearchLanes - 1)) == 0) miss[i] = f ? 0u : 1u;
 }
 
 __global__ __launch_bounds__(256) void k_pcss_band(FrameUniforms u, const float *__restrict__ smap,
@@ -256,17 +317,50 @@ __global__ __launch_bounds__(256) void k_pcss_band(FrameUniforms u, const float 
                                                    uint32_t M0, const uint32_t *__restrict__ pred,
                                                    unsigned long long *__restrict__ masks)
 {
-    const uint32_t i = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    const uint32_t i = __builtin_amdgcn_readfirstlane((blockIdx.x * 256 + threadIdx.x) >> 6), lane = threadIdx.x & 63;
     if (i >= L) return;   // whole wavefronts
-    const int cand = (int)lane;
-    const long long M = (long long)pcss_predict(pred, M0, 0.f, i) - kBandHalf + cand;
-    bool f = false;
-    if (cand <= 2 * kBandHalf && M >= (long long)M0 && M <= (long long)M0 + i) {
-        const uint32_t k = s0 + i;
-        f = pcss_search(u, smap, pairs, pt[k], pbase[k] + (uint32_t)u.shadow.n_pcf * (k - (uint32_t)M));
+    const uint32_t k = s0 + i, n = (uint32_t)u.shadow.n_blocker, np = (uint32_t)u.shadow.n_pcf;
+    const float4 q = pt[k];
+    const uint32_t base = pbase[k];
+    // candidate c: M = first + c, of those in [M0, M0 + i]; the samples of the
+    // highest come first in the stream
+    const long long first = (long long)pcss_predict(pred, M0, 0.f, i) - kBandHalf;
+    const int lo = first < (long long)M0 ? (int)((long long)M0 - first) : 0;
+    const long long top = (long long)M0 + i - first;
+    const int hi = top < 2 * kBandHalf ? (int)top : 2 * kBandHalf;
+    const uint32_t o_hi = base + np * (k - (uint32_t)(first + hi)), span = np * (uint32_t)(hi - lo);
+    const StreamRun run = stream_run(pairs, o_hi);
+    const bool one = span + n <= run.left, inside = pcss_inside(u, q);
+    const int group = (int)(lane / kSearchLanes), sub = (int)(lane & (kSearchLanes - 1));
+    uint32_t any_bits = 0, sure_bits = 0;   // of candidates group, group + 8, ...
+#pragma unroll 2
+    for (int t = 0; t < kSearchLanes; ++t) {
+        const int c = t * (64 / kSearchLanes) + group;
+        const int at = c < lo ? lo : c > hi ? hi : c;   // outside: masked below
+        const uint32_t o = np * (uint32_t)(hi - at);
+        const float *d = one ? run.v + 2 * (size_t)o : stream_at<2>(pairs, o_hi + o);
+        bool any = false, sure = false;
+        if (inside) pcss_samples<true>(u, smap, (const float2 *)d, q, (int)n, sub, any, sure);
+        else pcss_samples<false>(u, smap, (const float2 *)d, q, (int)n, sub, any, sure);
+        any_bits |= any ? 1u << t : 0u;
+        sure_bits |= sure ? 1u << t : 0u;
     }
-    const unsigned long long b = __ballot(f);
-    if (lane == 0) masks[i] = b;
+    uint32_t got = search_or(any_bits | sure_bits << 16);
+    uint32_t found = got >> 16;
+    for (uint32_t left = got & 0xffffu & ~found; left; left &= left - 1) {   // rare
+        const int t = __builtin_ctz(left), c = t * (64 / kSearchLanes) + group;
+        if (c < lo || c > hi) continue;
+        if (pcss_search_exact(u, smap, stream_at<2>(pairs, o_hi + np * (uint32_t)(hi - c)), q)) found |= 1u << t;
+    }
+    unsigned long long m = 0ull;
+#pragma unroll
+    for (int t = 0; t < kSearchLanes; ++t) {
+        const int c = t * (64 / kSearchLanes) + group;
+        // bit j of the 8 candidates': lane 8 j's
+        const unsigned long long b = __ballot((found >> t & 1u) && c >= lo && c <= hi) & 0x0101010101010101ull;
+        m |= (b * 0x0102040810204080ull >> 56) << 8 * t;
+    }
+    if (lane == 0) masks[i] = m;
 }
 
 // Following the actual M_k through the masks.  With P_i the prediction
@@ -278,7 +372,7 @@ __global__ __launch_bounds__(256) void k_pcss_band(FrameUniforms u, const float 
 // step), the points up to it settle (every one before it with the opposite
 // outcome), and D moves by one from there.
 //
-// The segment is cut into blocks of 1024 points, and every block is walked
+// The segment is cut into blocks of kPcssChainBlock points, and every block is walked
 // from each of the 63 places D can enter it with (k_pcss_walk_blocks: a
 // workgroup per block and 16 places, a wavefront per place; block 0 only
 // from 31), each walk writing its outcomes, the points it settled and the D
@@ -288,7 +382,7 @@ __global__ __launch_bounds__(256) void k_pcss_band(FrameUniforms u, const float 
 // stopped or which D enters from outside the band.
 constexpr int kBandWidth = 2 * kBandHalf + 1;
 constexpr int kChainWaves = 16;   // start places per workgroup
-static_assert(kPcssChainBlock == 1024 && kPcssBandWidth == kBandWidth, "chain layout");
+static_assert(kPcssChainBlock % 64 == 0 && kPcssBandWidth == kBandWidth, "chain layout");
 
 __global__ __launch_bounds__(64 * kChainWaves) void k_pcss_walk_blocks(const unsigned long long *__restrict__ masks,
                                                                       const uint32_t *__restrict__ pred, uint32_t L,
@@ -349,19 +443,20 @@ __global__ __launch_bounds__(64 * kChainWaves) void k_pcss_walk_blocks(const uns
 // One workgroup: the chain through the blocks' walks (their results staged
 // in LDS), then found[] for the settled points.  out = (first unsettled
 // point, M there).
-__global__ __launch_bounds__(256) void k_pcss_chain(const unsigned long long *__restrict__ fbits,
+constexpr uint32_t kChainThreads = 1024;
+__global__ __launch_bounds__(kChainThreads) void k_pcss_chain(const unsigned long long *__restrict__ fbits,
                                                     const uint32_t *__restrict__ res, const uint32_t *__restrict__ pred,
                                                     uint32_t s0, uint32_t L, uint32_t M0, uint32_t *__restrict__ found,
                                                     uint32_t *__restrict__ out)
 {
     constexpr uint32_t kMaxBlocks = kPcssSegmentMax / kPcssChainBlock;
-    __shared__ uint32_t sres[2 * kBandWidth * kMaxBlocks];
+    __shared__ __align__(8) uint32_t sres[2 * kBandWidth * kMaxBlocks];
     __shared__ int pick[kMaxBlocks];
     __shared__ uint32_t s_settled;
     __shared__ int s_D;
     const uint32_t tid = threadIdx.x;
     const uint32_t nblk = (L + kPcssChainBlock - 1) / kPcssChainBlock;
-    for (uint32_t i = tid; i < 2 * kBandWidth * nblk; i += 256) sres[i] = res[i];
+    for (uint32_t i = tid; i < 2 * kBandWidth * nblk; i += kChainThreads) sres[i] = res[i];
     __syncthreads();
     if (tid == 0) {
         int D = kBandHalf;
@@ -369,18 +464,19 @@ __global__ __launch_bounds__(256) void k_pcss_chain(const unsigned long long *__
         for (uint32_t b = 0; b < nblk; ++b) {
             if (D < 0 || D > 2 * kBandHalf) break;
             const uint32_t len = L - b * kPcssChainBlock < kPcssChainBlock ? L - b * kPcssChainBlock : kPcssChainBlock;
-            const uint32_t r = sres[2 * (b * kBandWidth + (uint32_t)D)];
+            const uint2 r = *(const uint2 *)(sres + 2 * (b * kBandWidth + (uint32_t)D));
             pick[b] = D;
-            D = (int)sres[2 * (b * kBandWidth + (uint32_t)D) + 1];
-            settled += r;
-            if (r < len) break;
+            D = (int)r.y;
+            settled += r.x;
+            if (r.x < len) break;
         }
         s_settled = settled;
         s_D = D;
     }
     __syncthreads();
     const uint32_t settled = s_settled;
-    for (uint32_t k = tid; k < settled; k += 256) {
+#pragma unroll 4
+    for (uint32_t k = tid; k < settled; k += kChainThreads) {
         const uint32_t b = k / kPcssChainBlock, kk = k - b * kPcssChainBlock;
         const unsigned long long w = fbits[((size_t)b * kBandWidth + (uint32_t)pick[b]) * (kPcssChainBlock / 64) + kk / 64];
         found[s0 + k] = (uint32_t)(w >> (kk & 63)) & 1u;
@@ -751,7 +847,7 @@ void launch_pcss_segment(const FrameUniforms &u, const float *shadow_map, const 
     const uint32_t *prev = nullptr;
     for (int q = 0; q < kGuesses; ++q) {
         uint32_t *dst = bufs[(kGuesses - 1 - q) & 1];
-        hipLaunchKernelGGL(k_pcss_guess, dim3((L + 255) / 256), dim3(256), 0, s, u, shadow_map, pairs, pt, pbase, s0, L,
+        hipLaunchKernelGGL(k_pcss_guess, dim3((L + 256 / kSearchLanes - 1) / (256 / kSearchLanes)), dim3(256), 0, s, u, shadow_map, pairs, pt, pbase, s0, L,
                            M0, rate, prev, dst);
         launch_exclusive_scan(dst, dst, L, scan_tmp, s);
         prev = dst;
@@ -762,7 +858,7 @@ void launch_pcss_segment(const FrameUniforms &u, const float *shadow_map, const 
     const uint32_t nblk = (L + kPcssChainBlock - 1) / kPcssChainBlock;
     hipLaunchKernelGGL(k_pcss_walk_blocks, dim3(nblk, (kBandWidth + kChainWaves - 1) / kChainWaves),
                        dim3(64 * kChainWaves), 0, s, masks, pred2, L, fbits, res);
-    hipLaunchKernelGGL(k_pcss_chain, dim3(1), dim3(256), 0, s, fbits, res, pred2, s0, L, M0, found, out);
+    hipLaunchKernelGGL(k_pcss_chain, dim3(1), dim3(kChainThreads), 0, s, fbits, res, pred2, s0, L, M0, found, out);
 }
 
 void launch_pcss_offsets(const uint32_t *base, const uint32_t *upos, const uint32_t *fpos, uint32_t n_pcf, size_t P,

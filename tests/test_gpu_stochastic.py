@@ -261,11 +261,25 @@ def test_blocker_search_areas_match_the_oracle(ctx, scene_dir, shadowmap, blocke
     map, cut off at its edges (read texel by texel), on odd and non-square
     maps, and maps too large to make windows of.  The stream moves by what the
     classification decides, so draw counts and image follow it."""
-    p = G.tiny_scene(os.path.join(scene_dir, f"rb{shadowmap}_{blocker_filter}"), seed=36, width=64, height=48, subdiv=3,
-                     tex=16, shadowmap=shadowmap, extra="shadowfilter refpcss")
+    _lighting_matches_the_oracle(ctx, os.path.join(scene_dir, f"rb{shadowmap}_{blocker_filter}"), shadowmap,
+                                 blocker_filter=blocker_filter)
+
+
+@pytest.mark.parametrize("n_blocker,n_pcf", [(1, 1), (5, 3), (33, 64), (64, 64)])
+def test_blocker_search_sample_counts_match_the_oracle(ctx, scene_dir, n_blocker, n_pcf):
+    """The eight lanes of a blocker search: fewer samples than lanes, a
+    remainder, more than one group of loads a lane, the most there are."""
+    _lighting_matches_the_oracle(ctx, os.path.join(scene_dir, f"rn{n_blocker}_{n_pcf}"), 128, blocker_filter=0.05,
+                                 n_blocker=n_blocker, n_pcf=n_pcf)
+
+
+def _lighting_matches_the_oracle(ctx, path, shadowmap, **cfg):
+    p = G.tiny_scene(path, seed=36, width=64, height=48, subdiv=3, tex=16, shadowmap=shadowmap,
+                     extra="shadowfilter refpcss")
     sc = F.Scene(p)
     gpu_frame(ctx, sc)
-    sc.info.shadow.blocker_filter = blocker_filter
+    for k, v in cfg.items():
+        setattr(sc.info.shadow, k, v)
     ctx.set_shadow(True, sc.info.shadow)
     ctx.rng_seed(5489)
     ctx.begin_pass(F.PASS_LIGHTING)
