@@ -566,7 +566,12 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
     }
     {
         CtxTimer t(b->ctx, timed ? "batch_lighting" : nullptr);
-        launch_bv_lighting(pa, s);
+        int mode = -2;
+        for (const DevView &v : b->hv) {
+            const int m = v.u.shadow_on ? v.u.shadow.mode : mode;
+            mode = mode == -2 || m == mode ? m : -1;
+        }
+        launch_bv_lighting(pa, mode == -2 ? 0 : mode, s);
     }
     {
         CtxTimer t(b->ctx, timed ? "batch_resolve" : nullptr);

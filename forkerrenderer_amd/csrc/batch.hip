@@ -296,13 +296,15 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     if (DIRECT && blockIdx.x == 0 && threadIdx.x == 0) *b.ctr = DirectCtr{0ull, 0u, 0u};
 }
 
+// MODE: the shadow filter of every view, or -1.
+template <int MODE>
 __global__ __launch_bounds__(256) void k_bv_lighting(BvPixelArgs b)
 {
     int vi, x, y;
     if (!bv_pixel<16>(b, vi, x, y)) return;
     const DevView &v = b.views[vi];
     const ShadowSamples none = {};
-    lighting_px(v.u, b.gbuf + kGbufPlanes * v.px_off, b.ao + v.px_off, b.ao_is_one, b.shadow + v.spx_off, none,
+    lighting_px<false, MODE>(v.u, b.gbuf + kGbufPlanes * v.px_off, b.ao + v.px_off, b.ao_is_one, b.shadow + v.spx_off, none,
                 b.fb + 3 * v.px_off, x, y);
 }
 
@@ -416,9 +418,17 @@ void launch_bv_gbuffer(const BvPixelArgs &a, hipStream_t s)
     else hipLaunchKernelGGL(k_bv_gbuffer<false>, dim3(a.n_blocks), dim3(256), 0, s, a);
 }
 
-void launch_bv_lighting(const BvPixelArgs &a, hipStream_t s)
+void launch_bv_lighting(const BvPixelArgs &a, int mode, hipStream_t s)
 {
-    if (a.n_blocks) hipLaunchKernelGGL(k_bv_lighting, dim3(a.n_blocks), dim3(256), 0, s, a);
+    if (!a.n_blocks) return;
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(a.n_blocks), dim3(256), 0, s, a); };
+    switch (mode) {
+    case 0: return go(k_bv_lighting<0>);
+    case 1: return go(k_bv_lighting<1>);
+    case 2: return go(k_bv_lighting<2>);
+    case 3: return go(k_bv_lighting<3>);
+    default: return go(k_bv_lighting<-1>);
+    }
 }
 
 void launch_bv_resolve(const BvPixelArgs &a, hipStream_t s)

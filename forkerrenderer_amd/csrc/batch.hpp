@@ -111,7 +111,8 @@ void launch_bv_direct(int pass, const BvDirectArgs &a, const uint2 *fblocks, int
 void launch_bv_direct_shadow(const BvDirectArgs &a, const uint8_t *sblk_view, uint32_t n_sblocks, const float *ndc_z,
                              float *depth, float *shadow, hipStream_t s);
 void launch_bv_gbuffer(const BvPixelArgs &a, hipStream_t s);
-void launch_bv_lighting(const BvPixelArgs &a, hipStream_t s);
+// mode: the shadow filter that every view with shadows uses, -1 if they differ
+void launch_bv_lighting(const BvPixelArgs &a, int mode, hipStream_t s);
 void launch_bv_resolve(const BvPixelArgs &a, hipStream_t s);
 
 }  // namespace fgl

@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) void k_gbuffer_resolve(ResolveArgs a, FrameUni
 // (phongshader.h:90-169, pbrshader.h:90-180) once for the visible fragment.
 // The forward fragment program for the winner (face f of draw dr, material
 // m, barycentrics b) at pixel i.
-template <bool STREAM>
+template <bool STREAM, int MODE>
 __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameUniforms &u, const DevDraw &dr,
                                               const DevMaterial &m, int f, const int4 &tv, const Vec3 &b, size_t i,
                                               size_t P)
@@ -318,7 +318,7 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
         float shin = 1.f;
         if (bn.has & kBundleZ) shin = fg.maps.z + 5;
         else if (m.map_ks >= 0) shin = tex_samplef(a.textures, m.map_ks, fg.uv) + 5;
-        c = shade_point<STREAM>(u, a.shadow_map, false, false, fg.pos, fg.normal, fg.lndc, dc, em,
+        c = shade_point<STREAM, MODE>(u, a.shadow_map, false, false, fg.pos, fg.normal, fg.lndc, dc, em,
                         vec3(m.ka[0], m.ks[0], shin), rdisk);
     } else {
         Vec3 al = (bn.has & kBundleA) ? fg.maps.a
@@ -331,7 +331,7 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
         float metal = (bn.has & kBundleY) ? fg.maps.y
                     : m.map_metal >= 0    ? tex_samplef(a.textures, m.map_metal, fg.uv) : m.metalness;
         float ao = m.map_ao >= 0 ? tex_samplef(a.textures, m.map_ao, fg.uv) : 1.f;
-        c = shade_point<STREAM>(u, a.shadow_map, true, false, fg.pos, fg.normal, fg.lndc, al, em,
+        c = shade_point<STREAM, MODE>(u, a.shadow_map, true, false, fg.pos, fg.normal, fg.lndc, al, em,
                         vec3(ao, metal, rough), rdisk);
     }
     a.fb[i] = c.x;
@@ -341,7 +341,7 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
 
 // Forward resolve, one thread per pixel; draw and material records through
 // readfirstlane when the wavefront shares them (as in gbuffer_px).
-template <bool STREAM, bool DIRECT>
+template <bool STREAM, bool DIRECT, int MODE>
 __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUniforms u)
 {
     int x, y;
@@ -366,14 +366,14 @@ __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUni
         const int mi = dr.face_mat[f];
         const int m0 = __builtin_amdgcn_readfirstlane(mi);
         if (__ballot(mi != m0) == 0ull) {
-            forward_shade<STREAM>(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
+            forward_shade<STREAM, MODE>(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
             resolve_end<DIRECT>(a, i, w);
             return;
         }
     }
     const DevDraw &dr = a.draws[w.tv.w];
     const int f = w.g - dr.tri_base;
-    forward_shade<STREAM>(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
+    forward_shade<STREAM, MODE>(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
     resolve_end<DIRECT>(a, i, w);
 }
 
@@ -655,9 +655,16 @@ void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStr
 {
     if (a.W <= 0 || a.H <= 0) return;
     const dim3 g = grid2(a.W, a.H);
-    if (a.ss.sv.v) hipLaunchKernelGGL((k_forward_resolve<true, false>), g, dim3(256), 0, s, a, u);
-    else if (a.key) hipLaunchKernelGGL((k_forward_resolve<false, true>), g, dim3(256), 0, s, a, u);
-    else hipLaunchKernelGGL((k_forward_resolve<false, false>), g, dim3(256), 0, s, a, u);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, s, a, u); };
+    if (a.ss.sv.v) return go(k_forward_resolve<true, false, -1>);
+    if (!a.key) return go(k_forward_resolve<false, false, -1>);
+    switch (u.shadow_on ? u.shadow.mode : 0) {
+    case 0: return go(k_forward_resolve<false, true, 0>);
+    case 1: return go(k_forward_resolve<false, true, 1>);
+    case 2: return go(k_forward_resolve<false, true, 2>);
+    case 3: return go(k_forward_resolve<false, true, 3>);
+    default: return go(k_forward_resolve<false, true, -1>);
+    }
 }
 
 template <bool EMIT>

@@ -7,7 +7,7 @@
 
 namespace fgl {
 
-template <bool STREAM>
+template <bool STREAM, int MODE>
 __global__ __launch_bounds__(256) void k_lighting(FrameUniforms u, const float *__restrict__ g,
                                                   const float *__restrict__ ao, int ao_is_one, NetAo net,
                                                   const float *__restrict__ smap, ShadowSamples ss,
@@ -16,7 +16,7 @@ __global__ __launch_bounds__(256) void k_lighting(FrameUniforms u, const float *
     int x, y;
     grid_px<16>(x, y);
     if (x >= u.W || y >= u.H) return;
-    lighting_px<STREAM>(u, g, ao, ao_is_one, smap, ss, fb, x, y, net);
+    lighting_px<STREAM, MODE>(u, g, ao, ao_is_one, smap, ss, fb, x, y, net);
 }
 
 __global__ __launch_bounds__(256) void k_ssao_ref(FrameUniforms u, StreamVectors samples,
@@ -780,12 +780,18 @@ void launch_lighting(const FrameUniforms &u, const float *gbuf, const float *ao,
                      const float *shadow_map, const ShadowSamples &ss, float *fb, hipStream_t s)
 {
     if (u.W <= 0 || u.H <= 0) return;
-    if (ss.sv.v)
-        hipLaunchKernelGGL(k_lighting<true>, grid2(u.W, u.H), dim3(256), 0, s, u, gbuf, ao, ao_is_one, net,
-                           shadow_map, ss, fb);
-    else
-        hipLaunchKernelGGL(k_lighting<false>, grid2(u.W, u.H), dim3(256), 0, s, u, gbuf, ao, ao_is_one, net,
-                           shadow_map, ss, fb);
+    const dim3 grid = grid2(u.W, u.H);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, u, gbuf, ao, ao_is_one, net, shadow_map, ss, fb);
+    };
+    if (ss.sv.v) return go(k_lighting<true, -1>);
+    switch (u.shadow_on ? u.shadow.mode : 0) {
+    case 0: return go(k_lighting<false, 0>);
+    case 1: return go(k_lighting<false, 1>);
+    case 2: return go(k_lighting<false, 2>);
+    case 3: return go(k_lighting<false, 3>);
+    default: return go(k_lighting<false, -1>);
+    }
 }
 
 void launch_ssao_reference(const FrameUniforms &u, const StreamVectors &samples, const float *pow3,

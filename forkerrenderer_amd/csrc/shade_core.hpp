@@ -13,7 +13,7 @@ namespace fgl {
 // read the G-buffer (76 B/px) + AO (4 B/px, or the network AO still on its
 // coarse grid: 1 B of coverage and four cached grid values), light, write
 // the frame buffer (12 B/px).
-template <bool STREAM = false>
+template <bool STREAM = false, int MODE = -1>
 __device__ __forceinline__ void lighting_px(const FrameUniforms &u, const float *__restrict__ g,
                                             const float *__restrict__ ao, int ao_is_one,
                                             const float *__restrict__ smap, const ShadowSamples &ss,
@@ -49,7 +49,7 @@ __device__ __forceinline__ void lighting_px(const FrameUniforms &u, const float 
     Vec3 L = vec3(g[6 * P + i], g[7 * P + i], g[8 * P + i]);
     const float *rdisk = nullptr;
     if (STREAM && ss.sv.v) rdisk = ss.at(i);
-    Vec3 c = shade_point<STREAM>(u, smap, !(type < 0.5f), true, Pw, N, L, al, em, pa, rdisk);
+    Vec3 c = shade_point<STREAM, MODE>(u, smap, !(type < 0.5f), true, Pw, N, L, al, em, pa, rdisk);
     fb[i] = c.x;
     fb[P + i] = c.y;
     fb[2 * P + i] = c.z;
