@@ -134,6 +134,7 @@ struct fgl_ctx {
 
     // device address of the allocation-free entry point's scratch array
     float *noalloc_scratch = nullptr;
+    int number = 0;   // of this context among its device's (0: none was free)
     // neural AO still on its network grid (lao != nullptr): the AO target's
     // content until something reads or replaces it; owner = the network
     // whose buffers hold it
@@ -173,6 +174,35 @@ static hipError_t scratch_address(int device, float **out)
     }
     *out = g_scratch_ptr[device];
     return hipSuccess;
+}
+
+// Contexts on a device are numbered (the lowest free number), so that their
+// calls use different parts of `scratch` where it holds a part for each: parts
+// are the frame rounded up to a power of two, by the number.
+static uint64_t g_ctx_numbers[kMaxDevices] = {};
+
+static int take_number(int device)
+{
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    uint64_t &used = g_ctx_numbers[device];
+    if (~used == 0) return 0;
+    const int k = __builtin_ctzll(~used);
+    used |= 1ull << k;
+    return k + 1;
+}
+
+static void give_number(int device, int number)
+{
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    if (number > 0) g_ctx_numbers[device] &= ~(1ull << (number - 1));
+}
+
+static float *scratch_part(float *scratch_base, int number, size_t n)
+{
+    size_t part = 1 << 16;
+    while (part < n) part *= 2;
+    const size_t parts = FGL_SSAO_NOALLOC_MAX_PIXELS / part;   // n is at most that, a power of two
+    return scratch_base + (number > 0 ? (size_t)(number - 1) % parts : 0) * part;
 }
 
 static int fail(fgl_ctx *c, int code, const std::string &msg)
@@ -340,6 +370,7 @@ int fgl_ctx_create(int device, fgl_ctx **out)
         delete c;
         return FGL_ERR_NOMEM;
     }
+    c->number = take_number(device);
     std::memset(c->h_pub, 0, 64);
     float I[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
     std::memcpy(c->viewport, I, sizeof(I));
@@ -393,6 +424,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     if (c->h_total) (void)hipHostFree(c->h_total);
     if (c->h_pub) (void)hipHostFree(c->h_pub);
     (void)hipStreamDestroy(c->stream);
+    give_number(c->device, c->number);
     delete c;
 }
 
@@ -1742,7 +1774,7 @@ int fgl_ssao_noalloc(fgl_ctx *c, int w, int h, const float view[16], const float
     }
     // The separable blur reads the unblurred AO from the scratch array; the
     // SSAO kernel writes every pixel of it first, so nothing is cleared.
-    float *raw = cfg->blur == 2 ? c->noalloc_scratch : ao;
+    float *raw = cfg->blur == 2 ? scratch_part(c->noalloc_scratch, c->number, (size_t)w * h) : ao;
     launch_ssao(u, sa, depth, gbuf, raw, c->stream);
     if (cfg->blur == 1)
         launch_blur_recursive(ao, w, h, c->stream);

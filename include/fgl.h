@@ -216,8 +216,10 @@ int fgl_ssao(fgl_ctx *ctx, const fgl_ssao_cfg *cfg);
  * unblurred AO that the separable blur reads is kept in a static device
  * array of FGL_SSAO_NOALLOC_MAX_PIXELS floats (32 MiB on every device the
  * library runs on, held until the process ends); larger frames fail with
- * FGL_ERR_CAPACITY.  Every call on a device shares that array: calls that
- * overlap on one device (two contexts, two host threads) race.  Work is
+ * FGL_ERR_CAPACITY.  Contexts whose frames round up to the same power of two
+ * use parts of their own while the array holds one for each (64 contexts of
+ * up to 2^17 pixels, one of more than 2^22); other calls that overlap on one
+ * device (larger or mixed frames, two host threads on a context) race.  Work is
  * enqueued on the context's stream; nothing is allocated or freed, and the
  * context's targets and pending draws are left as they are.  Results equal
  * fgl_ssao's on the same frame bit for bit. */
