@@ -11,6 +11,7 @@ depth and shadow map bit-exact; the 8-bit image within +-1 LSB.
 """
 import os
 
+import numpy as np
 import pytest
 
 import forkerrenderer_amd as F
@@ -46,3 +47,62 @@ def test_texture_modes(ctx, scene_dir, wrap, filt, mode):
     mx, frac = lsb_stats(got["image"], want["image"])
     assert frac >= 0.999, (mx, frac)
 
+
+
+@pytest.mark.parametrize("mode", ["deferred", "forward"])
+@pytest.mark.parametrize("tex,other", [(1, None), (3, None), (7, (9, 6)), (33, None), (32, (32, 16))])
+def test_map_sizes(ctx, scene_dir, mode, tex, other):
+    """A material's maps are kept together in 4 x 4 blocks where their sizes
+    agree: sizes that are no multiple of 4, a single texel, and a map of
+    another size, which stays by itself."""
+    d = os.path.join(scene_dir, f"mapsize_{mode}_{tex}")
+    p = G.tiny_scene(d, seed=62, width=97, height=61, subdiv=3, tex=tex, mode=mode, uv_scale=3.0, pbr=(mode == "deferred"))
+    if other:
+        rng = np.random.default_rng(tex)
+        G.write_tga(os.path.join(d, "albedo.tga"), rng.integers(0, 256, (other[1], other[0], 3), dtype=np.uint8))
+    sc = F.Scene(p)
+    print(f"map sizes: {mode} {tex} {other}", flush=True)
+    got = gpu_frame(ctx, sc, 16)
+    want = oracle_frame(sc)
+    assert_bitexact("depth", got["depth"], want["depth"])
+    if mode == "deferred":
+        assert_bitexact("gbuf", got["gbuf"], want["gbuf"])
+    mx, frac = lsb_stats(got["image"], want["image"])
+    assert frac >= 0.999, (mx, frac)
+
+
+@pytest.mark.parametrize("shadow", ["hard", "pcf", "pcss", "grid"])
+@pytest.mark.parametrize("mode,width,height", [("deferred", 333, 201), ("forward", 333, 201), ("deferred", 65, 5),
+                                               ("forward", 1, 1)])
+def test_partly_covered_frames_by_filter(ctx, scene_dir, shadow, mode, width, height):
+    """The kernel of each shadow filter on frames of enough blocks to be dealt
+    out in runs and of fewer, with odd edges, wavefronts nothing was drawn to
+    and wavefronts that are partly covered; SSAO leaves its early ones too."""
+    p = G.tiny_scene(os.path.join(scene_dir, f"part_{shadow}_{mode}_{width}"), seed=63, width=width, height=height,
+                     subdiv=3, tex=16, mode=mode, shadow=shadow, ssao=(mode == "deferred"))
+    sc = F.Scene(p)
+    print(f"partly covered: {shadow} {mode} {width}x{height}", flush=True)
+    got = gpu_frame(ctx, sc, 16)
+    want = oracle_frame(sc)
+    assert_bitexact("depth", got["depth"], want["depth"])
+    assert_bitexact("shadow", got["shadow"], want["shadow"])
+    if mode == "deferred":
+        assert_bitexact("gbuf", got["gbuf"], want["gbuf"])
+    mx, frac = lsb_stats(got["image"], want["image"])
+    assert frac >= 0.998, (mx, frac)   # SSAO taps within rounding of a threshold
+
+
+@pytest.mark.parametrize("mode", ["deferred", "forward"])
+@pytest.mark.parametrize("grid", [1, 3, 4, 5, 7])
+def test_grid_filter_sizes(ctx, scene_dir, mode, grid):
+    """The 3 x 3 and 5 x 5 grids by rows and columns, the others texel by
+    texel, on a map whose edges the grid crosses."""
+    p = G.tiny_scene(os.path.join(scene_dir, f"grid_{mode}_{grid}"), seed=64, width=97, height=61, subdiv=3, tex=16,
+                     mode=mode, shadowmap=23, extra=f"shadowfilter grid {grid}")
+    sc = F.Scene(p)
+    assert sc.info.shadow.grid == grid
+    got = gpu_frame(ctx, sc, 16)
+    want = oracle_frame(sc)
+    assert_bitexact("shadow", got["shadow"], want["shadow"])
+    mx, frac = lsb_stats(got["image"], want["image"])
+    assert frac >= 0.999, (mx, frac)
