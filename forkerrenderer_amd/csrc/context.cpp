@@ -1019,9 +1019,9 @@ static void fill_draw(fgl_ctx *c, const ModelRes &m, const float M[16], DevDraw 
 // mt_jump.hpp); the draws needed are estimated from the acceptance rate (pi/4
 // for the disk, pi/6 for the sphere) with a margin, and doubled in the rare
 // case that too few tries are kept.  A chunk's generation takes time in
-// proportion to K, and the jumps (a workgroup each, one per CU) take a fixed
-// time per 256 chunks: K = 256 while 256 chunks of it cover the request, else
-// 512.
+// proportion to K (0.27 us per 454 words with a workgroup a CU, 0.36 with two),
+// and the jumps (three workgroups each, one per CU) some 0.25 us a chunk: K =
+// 256 while 256 chunks of it cover the request, else 512.
 static constexpr int kMtChunkShort = 256, kMtChunkLong = 512;
 
 static int rng_fill(fgl_ctx *c, int D, uint32_t n)
