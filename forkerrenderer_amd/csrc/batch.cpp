@@ -287,6 +287,24 @@ static int plan(fgl_batch *b)
         grow(b->big_list, (size_t)mt * 4) || grow(b->tile_start, (size_t)mtiles * 4) ||
         grow(b->tile_end, (size_t)mtiles * 4) || grow(b->counters, 256))
         return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
+    // triangle groups of the direct rasteriser: lanes per triangle by the
+    // pixels the draw's view has for it
+    auto lane_code = [&](const DevDraw &d, int p) {
+        const DevView &v = b->hv[d.view];
+        const double area = p == kBvShadow ? (double)v.S * v.S : (double)v.W * v.H;
+        const double per = area / (d.n_faces > 0 ? d.n_faces : 1);
+        return per >= 48.0 ? 2u : per >= 6.0 ? 1u : 0u;
+    };
+    b->direct_ok = b->direct_ok && launch_fits((long long)sblk_view.size());
+    for (int p = 0; p < 2; ++p) {
+        long long groups = 0, vblocks = 0;
+        for (const DevDraw &d : dd[p]) {
+            groups += direct_groups(d.n_faces, bv_lanes(lane_code(d, p)));
+            vblocks += vertex_blocks(d.n_pos);
+        }
+        b->direct_ok = b->direct_ok && launch_fits(groups) &&
+                       launch_fits(vblocks + clear_blocks((long long)(p == kBvShadow ? spx : px)));
+    }
     if (b->direct_ok) {
         // items: every view's 64 x 16 blocks several times over
         const size_t kp = std::max(px, spx);
@@ -306,14 +324,9 @@ static int plan(fgl_batch *b)
             for (int v0 = 0; v0 < dd[p][k].n_pos; v0 += 256) vb.push_back(make_uint2((uint32_t)k, (uint32_t)v0));
             for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256) fb.push_back(make_uint2((uint32_t)k, (uint32_t)f0));
         }
-        // triangle groups of the direct rasteriser: lanes per triangle by the
-        // pixels its view has for it
         std::vector<uint2> db;
         for (size_t k = 0; b->direct_ok && k < dd[p].size(); ++k) {
-            const DevView &v = b->hv[dd[p][k].view];
-            const double area = p == kBvShadow ? (double)v.S * v.S : (double)v.W * v.H;
-            const double per = area / (dd[p][k].n_faces > 0 ? dd[p][k].n_faces : 1);
-            const uint32_t code = per >= 48.0 ? 2u : per >= 6.0 ? 1u : 0u;
+            const uint32_t code = lane_code(dd[p][k], p);
             for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256 / bv_lanes(code))
                 db.push_back(make_uint2((uint32_t)k, (uint32_t)f0 | code << 30));
         }

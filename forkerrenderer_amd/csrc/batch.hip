@@ -153,7 +153,6 @@ __global__ __launch_bounds__(BLOCK) void k_bv_raster(BvRasterArgs b)
 // The vertex records, the key plane cleared (8 keys a thread) by the
 // workgroups past the vertices', the overflow flags zeroed (views do not
 // change, so a batch whose pairs were counted has none).
-constexpr int kBvClearKeys = 8;
 template <int PASS>
 __global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const uint2 *__restrict__ blocks, int n_blocks,
                                                           int4 *__restrict__ out, float *__restrict__ ndc_z,
@@ -163,11 +162,11 @@ __global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const 
     const int b = blockIdx.x;
     if (b >= n_blocks) {
         if (b == n_blocks && threadIdx.x < 2) flags[threadIdx.x] = 0u;
-        const size_t k0 = (size_t)(b - n_blocks) * (256 * kBvClearKeys);
+        const size_t k0 = (size_t)(b - n_blocks) * (256 * kClearKeys);
         ulonglong2 c;
         c.x = c.y = kDirectClear;
 #pragma unroll
-        for (int e = 0; e < kBvClearKeys / 2; ++e) {
+        for (int e = 0; e < kClearKeys / 2; ++e) {
             const size_t k = k0 + 2 * ((size_t)e * 256 + threadIdx.x);
             if (k + 1 < n_keys) *(ulonglong2 *)(a.key + k) = c;
             else if (k < n_keys) a.key[k] = kDirectClear;
@@ -382,7 +381,7 @@ void launch_bv_raster(int pass, int TS, unsigned n_wg, const BvRasterArgs &a, hi
 void launch_bv_direct_vertex(int pass, const BvDirectArgs &a, const uint2 *vblocks, int n_vblocks, int4 *screen,
                              float *ndc_z, float4 *vary, size_t n_keys, uint32_t *flags, hipStream_t s)
 {
-    const unsigned grid = (unsigned)n_vblocks + nblk(n_keys, 256 * kBvClearKeys);
+    const unsigned grid = (unsigned)(n_vblocks + clear_blocks((long long)n_keys));
     if (grid == 0) return;
     if (pass == kBvShadow)
         hipLaunchKernelGGL(k_bv_direct_vertex<kBvShadow>, dim3(grid), dim3(256), 0, s, a, vblocks, n_vblocks, screen, ndc_z,

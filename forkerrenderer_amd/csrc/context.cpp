@@ -1315,18 +1315,17 @@ static void bound_pass(const fgl_ctx *c, bool shadow, long long nt, int W, int H
     pairs_fit = !count || sum < most;
 }
 
-// The pass's fragments through the direct rasteriser: its keys are left for
-// the resolve, the shadow pass's targets are written.  n_draws and the
-// largest draw bound the launches' grids (direct_fits).
-static bool direct_fits(int n_draws, int max_faces, int max_pos, size_t px)
-{
-    const long long most = 0x7fffffffLL;
-    return (long long)n_draws * ((max_faces + 15) / 16) <= most &&
-           (long long)n_draws * ((max_pos + 255) / 256) + (long long)(px / 256) + 1 <= most;
-}
+// The direct rasteriser's launches of a pass: the draws' triangle groups and
+// vertex blocks (their bases in the draw records).
+struct DirectGrid {
+    int lanes;
+    long long groups, vblocks;
+};
 
-static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, int max_pos, int max_faces, long long nt,
-                       bool shadow, bool no_nan, int W, int H)
+// The pass's fragments through the direct rasteriser: its keys are left for
+// the resolve, the shadow pass's targets are written.
+static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const DirectGrid &g, long long nt, bool shadow,
+                       bool no_nan, int W, int H)
 {
     // large triangles' items: room for every 64 x 16 block of the screen many
     // times over; a pass that needs more rasterises the rest in place
@@ -1360,12 +1359,12 @@ static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, int max_
     c->direct_turn ^= 1;
     {
         KernelTimer t(c, "vertex");
-        launch_direct_vertex(shadow, a.draws, n_draws, max_pos, u, (int4 *)c->screen.p,
+        launch_direct_vertex(shadow, (int)g.vblocks, u, (int4 *)c->screen.p,
                              shadow ? (float *)c->ndc_z.p : nullptr, shadow ? nullptr : (float4 *)c->vary.p, a,
                              ctr + c->direct_turn, c->stream);
     }
     KernelTimer t(c, shadow ? "raster_shadow" : "raster");
-    launch_direct(a, max_faces, nt, c->stream);
+    launch_direct(a, g.lanes, (int)g.groups, nt, c->stream);
     if (shadow)
         launch_direct_shadow(a, (const float *)c->ndc_z.p, (float *)c->shadow_depth.p, (float *)c->shadow.p, c->stream);
     return FGL_OK;
@@ -1542,6 +1541,13 @@ static int flush_pass(fgl_ctx *c)
         max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
         max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
     }
+    DirectGrid grid = {direct_lanes(nt), 0, 0};
+    for (DevDraw &d : dd) {
+        d.group_base = (int)grid.groups;
+        d.vblock_base = (int)grid.vblocks;
+        grid.groups += direct_groups(d.n_faces, grid.lanes);
+        grid.vblocks += vertex_blocks(d.n_pos);
+    }
     const int n_draws = (int)c->draws.size();
     bool fits, no_nan;
     bound_pass(c, shadow, nt, W, H, shadow ? c->TS_shadow : c->TS, fits, no_nan);
@@ -1577,13 +1583,14 @@ static int flush_pass(fgl_ctx *c)
     // the tile lists.
     const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
     const size_t px = (size_t)W * H;
-    const bool direct = fresh && !stoch && fits && direct_fits(n_draws, max_faces, max_pos, px);
+    const bool direct = fresh && !stoch && fits && launch_fits(grid.groups) &&
+                        launch_fits(grid.vblocks + clear_blocks((long long)px));
     if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))) ||
         (!shadow && (rc = ensure(c, c->vary, (size_t)nv * 2 * sizeof(float4)))))
         return rc;
     uint32_t n_frag = 0;
     if (direct) {
-        if ((rc = direct_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, no_nan, W, H))) return rc;
+        if ((rc = direct_pass(c, u, n_draws, grid, nt, shadow, no_nan, W, H))) return rc;
     } else if ((rc = list_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, W, H, fresh, stoch, n_frag))) {
         return rc;
     }

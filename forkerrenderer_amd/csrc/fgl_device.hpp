@@ -57,6 +57,9 @@ struct DevDraw {
     int n_pos, n_faces, vert_base, tri_base;
     int has_tangents, support_pbr;
     int view;      // batched views: index of the draw's view (0 otherwise)
+    // the direct rasteriser's workgroups before the draw's: of the vertex pass,
+    // of the triangle groups (single passes)
+    int vblock_base, group_base;
     int pad0;
     float model[16];
     float normal[9];

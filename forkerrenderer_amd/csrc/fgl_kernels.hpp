@@ -3,6 +3,7 @@
 #pragma once
 
 #include "fgl_device.hpp"
+#include "pass_plan.hpp"
 
 namespace fgl {
 
@@ -160,13 +161,14 @@ void launch_tile_ranges(const uint32_t *keys, uint32_t n, const uint32_t *n_dev,
                         uint32_t *end, hipStream_t s);
 void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s);
 // The direct rasteriser.  launch_direct_vertex: launch_vertex, the key plane
-// cleared and the next pass's counters zeroed on the way; launch_direct: the
-// pass's fragments into the keys (max_faces: the largest draw's; n_tri: all
-// draws'); launch_direct_shadow: the shadow pass's depth and ShadowBuffer
+// cleared and the next pass's counters zeroed on the way (n_blocks: the draws'
+// vertex blocks in all); launch_direct: the pass's fragments into the keys
+// (n_groups: the draws' triangle groups in all at that many lanes, n_tri: their
+// triangles); launch_direct_shadow: the shadow pass's depth and ShadowBuffer
 // value of every texel from the keys.
-void launch_direct_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
-                          float *ndc_z, float4 *vary, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s);
-void launch_direct(const DirectArgs &a, int max_faces, long long n_tri, hipStream_t s);
+void launch_direct_vertex(bool shadow, int n_blocks, const FrameUniforms &u, int4 *out, float *ndc_z, float4 *vary,
+                          const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s);
+void launch_direct(const DirectArgs &a, int lanes, int n_groups, long long n_tri, hipStream_t s);
 void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth, float *shadow_out, hipStream_t s);
 void launch_gbuffer_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);
 void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);

@@ -194,9 +194,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TS == 32 
 // Direct rasteriser, first launch of a pass: the vertex records, the key
 // plane cleared (8 keys a thread) by the workgroups past the vertices', and
 // the counters of the next pass zeroed (this pass's were by the one before).
-constexpr int kClearKeys = 8;
 template <bool SHADOW>
-__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, int n_vert_blocks, int bx,
+__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, int n_draws, int n_vert_blocks,
                                                        FrameUniforms u, int4 *__restrict__ out,
                                                        float *__restrict__ ndc_z, float4 *__restrict__ vary,
                                                        unsigned long long *__restrict__ key,
@@ -216,8 +215,8 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
         }
         return;
     }
-    const DevDraw &dr = draws[b / bx];
-    const int vi = (b % bx) * 256 + threadIdx.x;
+    const DevDraw &dr = draws[draw_at<&DevDraw::vblock_base>(draws, n_draws, b)];
+    const int vi = (b - dr.vblock_base) * 256 + threadIdx.x;
     if (vi >= dr.n_pos) return;
     if (SHADOW) {
         const Vec4 n = depth_ndc(dr, vi);
@@ -229,16 +228,15 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
     }
 }
 
-// G lanes per triangle: as many as fill the chip (a triangle's pixels are
-// its lanes' serial work).  Workgroups are dealt to the XCDs in runs:
-// neighbouring triangles share vertices and pixels.
-constexpr long long kDirectTris16 = 32768, kDirectTris4 = 262144;
+// G lanes per triangle (direct_lanes, pass_plan.hpp).  Workgroups are dealt to
+// the XCDs in runs: neighbouring triangles share vertices and pixels.
 template <int G>
-__global__ __launch_bounds__(256) void k_direct(DirectArgs a, int bx)
+__global__ __launch_bounds__(256) void k_direct(DirectArgs a)
 {
     __shared__ DirectLds lds;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    direct_group<G>(a, a.draws[b / bx], (b % bx) * (256 / G), lds);
+    const DevDraw &dr = a.draws[draw_at<&DevDraw::group_base>(a.draws, a.n_draws, b)];
+    direct_group<G>(a, dr, (b - dr.group_base) * (256 / G), lds);
 }
 
 // The large triangles' items, a wavefront each.
@@ -252,15 +250,19 @@ __global__ __launch_bounds__(256) void k_direct_big(DirectArgs a)
     }
 }
 
-// The second walk of a pass with NaN marks.
-__global__ __launch_bounds__(256) void k_direct_nan(DirectArgs a, int bx, int blocks)
+// The second walk of a pass with NaN marks, over its n_tri triangles (each
+// draw's in its spatial order).
+__global__ __launch_bounds__(256) void k_direct_nan(DirectArgs a, uint32_t n_tri)
 {
     if (a.ctr->nan == 0u) return;
-    for (int b = blockIdx.x; b < blocks; b += gridDim.x) {
-        const DevDraw &dr = a.draws[b / bx];
-        const int n = (b % bx) * 256 + threadIdx.x;
+    for (uint32_t g0 = blockIdx.x * 256u; g0 < n_tri; g0 += gridDim.x * 256u) {
+        const uint32_t g = g0 + threadIdx.x;
         TriL t;
-        const bool keep = n < dr.n_faces && direct_stage(a, dr, n, t);
+        bool keep = g < n_tri;
+        if (keep) {
+            const DevDraw &dr = a.draws[draw_of(a.draws, a.n_draws, (int)g)];
+            keep = direct_stage(a, dr, (int)g - dr.tri_base, t);
+        }
         direct_walk<1>(t, keep, keep ? direct_area(t) : 0, FoldAfterNan{a});
     }
 }
@@ -606,37 +608,29 @@ void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s)
     else launch_raster_t<false>(TS, a, s);
 }
 
-void launch_direct_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
-                          float *ndc_z, float4 *vary, const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s)
+void launch_direct_vertex(bool shadow, int n_blocks, const FrameUniforms &u, int4 *out, float *ndc_z, float4 *vary,
+                          const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s)
 {
     const size_t P = (size_t)a.W * a.H;
-    const unsigned bx = blocks_for(max_pos, 256), nv = bx * (unsigned)n_draws;
-    const unsigned grid = nv + blocks_for(P, 256 * kClearKeys);
+    const unsigned grid = (unsigned)(n_blocks + clear_blocks((long long)P));
     if (shadow)
-        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z, vary,
-                           a.key, P, next_ctr);
+        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, a.draws, a.n_draws, n_blocks, u, out, ndc_z,
+                           vary, a.key, P, next_ctr);
     else
-        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, draws, (int)nv, (int)bx, u, out, ndc_z, vary,
-                           a.key, P, next_ctr);
+        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, a.draws, a.n_draws, n_blocks, u, out, ndc_z,
+                           vary, a.key, P, next_ctr);
 }
 
-void launch_direct(const DirectArgs &a, int max_faces, long long n_tri, hipStream_t s)
+void launch_direct(const DirectArgs &a, int lanes, int n_groups, long long n_tri, hipStream_t s)
 {
-    const unsigned nd = (unsigned)a.n_draws;
-    if (n_tri <= kDirectTris16) {
-        const unsigned bx = blocks_for(max_faces, 256 / 16);
-        hipLaunchKernelGGL(k_direct<16>, dim3(bx * nd), dim3(256), 0, s, a, (int)bx);
-    } else if (n_tri <= kDirectTris4) {
-        const unsigned bx = blocks_for(max_faces, 256 / 4);
-        hipLaunchKernelGGL(k_direct<4>, dim3(bx * nd), dim3(256), 0, s, a, (int)bx);
-    } else {
-        const unsigned bx = blocks_for(max_faces, 256);
-        hipLaunchKernelGGL(k_direct<1>, dim3(bx * nd), dim3(256), 0, s, a, (int)bx);
-    }
+    const dim3 grid((unsigned)n_groups);
+    if (lanes == 16) hipLaunchKernelGGL(k_direct<16>, grid, dim3(256), 0, s, a);
+    else if (lanes == 4) hipLaunchKernelGGL(k_direct<4>, grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_direct<1>, grid, dim3(256), 0, s, a);
     hipLaunchKernelGGL(k_direct_big, dim3(1024), dim3(256), 0, s, a);
     if (!a.fix) return;
-    const unsigned bx = blocks_for(max_faces, 256), nb = bx * nd;
-    hipLaunchKernelGGL(k_direct_nan, dim3(nb < 256u ? nb : 256u), dim3(256), 0, s, a, (int)bx, (int)nb);
+    const unsigned nb = blocks_for((size_t)n_tri, 256);
+    hipLaunchKernelGGL(k_direct_nan, dim3(nb < 256u ? nb : 256u), dim3(256), 0, s, a, (uint32_t)n_tri);
 }
 
 void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth, float *shadow_out, hipStream_t s)

@@ -441,6 +441,26 @@ constexpr int kDirectItemW = 64, kDirectItemH = 16;
 constexpr int kDirectBig = 4096;      // pixels of the bounding box
 constexpr int kDirectBox = 2048;      // pixels of a workgroup's LDS box: 16 KiB, nine workgroups a CU
 
+// The last draw whose base is at most g: the draw of pass-wide triangle (or
+// workgroup) g.  Bases ascend; of draws with none of their own the last one
+// of equal bases, which owns g, is found.
+template <int DevDraw::*BASE>
+__device__ __forceinline__ int draw_at(const DevDraw *draws, int n_draws, int g)
+{
+    int lo = 0, hi = n_draws - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (draws[mid].*BASE <= g) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+__device__ __forceinline__ int draw_of(const DevDraw *draws, int n_draws, int g)
+{
+    return draw_at<&DevDraw::tri_base>(draws, n_draws, g);
+}
+
 struct DirectLds {
     unsigned long long key[kDirectBox];
     uint32_t lo[4], hi[4];            // per wavefront: (min x | min y << 16), the complement of the maxima
@@ -670,18 +690,6 @@ __device__ __forceinline__ void direct_group(const DirectArgs &a, const DevDraw 
         const int y = p / w, x = p - y * w;
         if (k != ~0ull) direct_min(a.key + (size_t)(x0 + x) + (size_t)(y0 + y) * a.W, k);
     }
-}
-
-// The draw of pass-wide triangle g (their tri_base ascend).
-__device__ __forceinline__ int draw_of(const DevDraw *draws, int n_draws, int g)
-{
-    int lo = 0, hi = n_draws - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (draws[mid].tri_base <= g) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
 }
 
 // Triangle g staged from its face, and its vertex ids and draw.

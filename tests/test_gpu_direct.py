@@ -32,6 +32,13 @@ def _triangles(rng, n, size, spread=1.1):
     return c + rng.uniform(-size, size, (n, 3, 3)) * np.array([1, 1, 0.05])
 
 
+def _material(ctx):
+    m = F.Material()
+    for f in ("map_kd", "map_ks", "map_ke", "map_bump", "map_base", "map_rough", "map_metal", "map_ao", "map_pbr_ke"):
+        setattr(m, f, -1)
+    return ctx.upload_material(m)
+
+
 def _scene(name, rng):
     """(models, W, H): each model's triangles."""
     if name == "few_mixed":        # 16 lanes a triangle, boxes below and above the LDS box, items
@@ -66,11 +73,13 @@ def _scene(name, rng):
 def test_direct_equals_lists(ctx, name, shadow):
     rng = np.random.default_rng(len(name))
     tris, W, H = _scene(name, rng)
-    m = F.Material()
-    for f in ("map_kd", "map_ks", "map_ke", "map_bump", "map_base", "map_rough", "map_metal", "map_ao", "map_pbr_ke"):
-        setattr(m, f, -1)
-    mat = ctx.upload_material(m)
-    models = [_model(ctx, mat, t) for t in tris]
+    mat = _material(ctx)
+    models = [(_model(ctx, mat, t), EYE4) for t in tris]
+    _direct_against_lists(ctx, mat, models, W, H, shadow, name)
+
+
+def _direct_against_lists(ctx, mat, draws, W, H, shadow, name):
+    """draws: (model, matrix) in order."""
     off = _model(ctx, mat, np.full((1, 3, 3), 9.0) + np.eye(3)[None])
     ctx.set_tile_size(16)
     ctx.set_shadow(False)
@@ -91,8 +100,8 @@ def test_direct_equals_lists(ctx, name, shadow):
         if lists:
             ctx.draw_model(off, eye)
             ctx.set_eye((0.0, 0.0, 2.0))   # flushes the pass so far
-        for k in models:
-            ctx.draw_model(k, eye)
+        for k, at in draws:
+            ctx.draw_model(k, at)
         ctx.end_pass()
         which = (F.TARGET_SHADOW_DEPTH, F.TARGET_SHADOW) if shadow else (F.TARGET_DEPTH, F.TARGET_GBUFFER)
         out.append([ctx.read(t).view(np.uint32) for t in which])
@@ -104,3 +113,31 @@ def test_direct_equals_lists(ctx, name, shadow):
         assert np.array_equal(a, b), f"{what}: {(a != b).sum()} of {a.size} differ"
     depth = out[0][0].view(np.float32)
     assert (depth < 3e38).any()
+
+
+@pytest.mark.parametrize("shadow", [False, True])
+def test_many_small_draws_beside_a_large_one(ctx, shadow):
+    """8,200 draws of one triangle, draws of none among and after them, and
+    one of 131,072: the launches are sized by what each draw holds (their
+    number times the largest draw is more workgroups than a launch takes)."""
+    rng = np.random.default_rng(5)
+    mat = _material(ctx)
+    small = _model(ctx, mat, _triangles(rng, 1, 0.02, 0.0))
+    none = _model_without_faces(ctx)
+    draws = []
+    for k in range(8200):
+        at = EYE4.copy()
+        at[0, 3], at[1, 3], at[2, 3] = rng.uniform(-1, 1), rng.uniform(-1, 1), rng.uniform(-0.4, 0.4)
+        draws.append((small, np.ascontiguousarray(at)))
+        if k % 1000 == 3:
+            draws += [(none, EYE4)] * 2
+    draws.insert(4000, (_model(ctx, mat, _triangles(rng, 131072, 0.01)), EYE4))
+    draws += [(none, EYE4)] * 3
+    _direct_against_lists(ctx, mat, draws, 320, 200, shadow, "many draws")
+
+
+def _model_without_faces(ctx):
+    f = np.zeros((0, 3), np.int32)
+    return ctx.upload_model({"pos": np.ones((300, 3), np.float32), "uv": np.zeros((1, 2), np.float32),
+                             "nrm": np.ones((1, 3), np.float32), "tan": None, "vi": f, "ti": f, "ni": f,
+                             "face_material": np.zeros(0, np.int32), "support_pbr": False})
