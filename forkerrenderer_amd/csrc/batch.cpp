@@ -142,8 +142,7 @@ struct fgl_batch {
     Buf depth, vis, gbuf, ao, fb, img, shadow, shadow_depth;
     Buf screen, ndc_z, vary, rect, counts, offs, scan_tmp, tri_v, big_list, tile_start, tile_end;
     Buf keys[2], vals[2], keys_alt[2], vals_alt[2], sort_tmp[2];
-    Buf key, items, direct_ctr;   // pixel keys, large-triangle items, a counter record per pass
-    uint32_t n_direct_items = 0;
+    Buf key, big, direct_ctr;   // pixel keys, large triangles, a counter record per pass
     Buf d_dblocks[2], d_sblk_view;   // triangle groups of each pass; view of each 64 x 4 shadow-map block
     int n_dblocks[2] = {0, 0};
     uint32_t n_sblocks = 0;
@@ -295,7 +294,7 @@ static int plan(fgl_batch *b)
         const double per = area / (d.n_faces > 0 ? d.n_faces : 1);
         return per >= 48.0 ? 2u : per >= 6.0 ? 1u : 0u;
     };
-    b->direct_ok = b->direct_ok && launch_fits((long long)sblk_view.size());
+    b->direct_ok = b->direct_ok && launch_fits((long long)sblk_view.size()) && mt <= kDirectTrisMost;
     for (int p = 0; p < 2; ++p) {
         long long groups = 0, vblocks = 0;
         for (const DevDraw &d : dd[p]) {
@@ -306,10 +305,7 @@ static int plan(fgl_batch *b)
                        launch_fits(vblocks + clear_blocks((long long)(p == kBvShadow ? spx : px)));
     }
     if (b->direct_ok) {
-        // items: every view's 64 x 16 blocks several times over
-        const size_t kp = std::max(px, spx);
-        b->n_direct_items = (uint32_t)std::min<size_t>((size_t)1 << 28, std::max<size_t>((size_t)1 << 18, kp / 128 + 256 * b->n));
-        if (grow(b->key, kp * 8) || grow(b->items, (size_t)b->n_direct_items * sizeof(uint2)) ||
+        if (grow(b->key, std::max(px, spx) * 8) || grow(b->big, (size_t)mt * 12) ||
             grow(b->direct_ctr, 2 * sizeof(DirectCtr)) || grow(b->d_sblk_view, sblk_view.size() + 1))
             return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
         launch_fill_u32((uint32_t *)b->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, ctx_stream(c));
@@ -405,8 +401,8 @@ static BvDirectArgs direct_args(fgl_batch *b, int p)
     a.views = (const DevView *)b->d_views.p;
     a.screen = (const int4 *)b->screen.p;
     a.key = (unsigned long long *)b->key.p;
-    a.items = (uint2 *)b->items.p;
-    a.n_items = b->n_direct_items;
+    a.big_start = (unsigned long long *)b->big.p;
+    a.big_tri = (uint32_t *)(a.big_start + std::max(b->nt[0], b->nt[1]));
     a.ctr = (DirectCtr *)b->direct_ctr.p + p;
     return a;
 }
@@ -705,7 +701,7 @@ void fgl_batch_destroy(fgl_batch *b)
                    &b->d_lblk_view,
                    &b->d_pix_views, &b->depth, &b->vis, &b->gbuf, &b->ao, &b->fb, &b->img, &b->shadow,
                    &b->shadow_depth, &b->screen, &b->ndc_z, &b->vary, &b->rect, &b->counts, &b->offs, &b->scan_tmp, &b->tri_v,
-                   &b->big_list, &b->tile_start, &b->tile_end, &b->counters, &b->key, &b->items, &b->direct_ctr,
+                   &b->big_list, &b->tile_start, &b->tile_end, &b->counters, &b->key, &b->big, &b->direct_ctr,
                    &b->d_dblocks[0], &b->d_dblocks[1], &b->d_sblk_view};
     for (Buf *x : bufs) release(*x);
     for (int p = 0; p < 2; ++p) {

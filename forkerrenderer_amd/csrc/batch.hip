@@ -197,8 +197,8 @@ __device__ __forceinline__ DirectArgs bv_direct_args(const BvDirectArgs &b, cons
     a.screen = b.screen;
     a.key = b.key + (PASS == kBvShadow ? v.spx_off : v.px_off);
     a.fix = nullptr;
-    a.items = b.items;
-    a.n_items = b.n_items;
+    a.big_start = b.big_start;
+    a.big_tri = b.big_tri;
     a.ctr = b.ctr;
     a.W = PASS == kBvShadow ? v.S : v.W;
     a.H = PASS == kBvShadow ? v.S : v.H;
@@ -222,14 +222,7 @@ __global__ __launch_bounds__(256) void k_bv_direct(BvDirectArgs b, const uint2 *
 template <int PASS>
 __global__ __launch_bounds__(256) void k_bv_direct_big(BvDirectArgs b)
 {
-    const unsigned long long claimed = b.ctr->items;
-    const uint32_t n = claimed < b.n_items ? (uint32_t)claimed : b.n_items;
-    for (uint32_t k = blockIdx.x * 4 + (threadIdx.x >> 6); k < n; k += gridDim.x * 4) {
-        const uint2 it = b.items[k];
-        if (it.x == 0xffffffffu) continue;
-        const int d = draw_of(b.draws, b.n_draws, (int)it.x);
-        direct_item(bv_direct_args<PASS>(b, b.views[b.draws[d].view]), it, d);
-    }
+    direct_big<FoldPlane>(b, [&](int d) { return bv_direct_args<PASS>(b, b.views[b.draws[d].view]); });
 }
 
 // The shadow targets of every view, and the pass's counters zeroed.

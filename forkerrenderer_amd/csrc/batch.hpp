@@ -58,15 +58,15 @@ struct BvRasterArgs {
 };
 
 // A pass through the direct rasteriser: the key plane of every view's
-// targets (indexed as they are), the item list of all views' large triangles.
+// targets (indexed as they are), the list of all views' large triangles.
 struct BvDirectArgs {
     const DevDraw *draws;
     int n_draws;
     const DevView *views;
     const int4 *screen;
     unsigned long long *key;
-    uint2 *items;
-    uint32_t n_items;
+    unsigned long long *big_start;
+    uint32_t *big_tri;
     DirectCtr *ctr;
 };
 

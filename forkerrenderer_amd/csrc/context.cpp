@@ -104,8 +104,8 @@ struct fgl_ctx {
     DevBuf d_draws, screen, rect, counts, offs, scan_tmp, keys, vals, keys_alt, vals_alt, sort_tmp,
         tile_start, tile_end, tri_v, big_list, counters, ndc_z, vary;
     // the direct rasteriser: pixel keys, NaN plane (all ones between passes),
-    // large-triangle items and two passes' counters used in turn
-    DevBuf key, key_nan, items;
+    // large triangles, two passes' counters used in turn
+    DevBuf key, key_nan, big, direct_ctr;
     int direct_turn = 0;
     // forward pass with a stochastic shadow filter: per-pixel passing counts
     // (+ scan scratch), the passing fragments (triangle ids then pixels) and
@@ -416,7 +416,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
                       &c->screen, &c->rect, &c->counts, &c->offs, &c->scan_tmp, &c->keys,
                       &c->vals, &c->keys_alt, &c->vals_alt, &c->sort_tmp, &c->tile_start,
                       &c->tile_end, &c->tri_v, &c->big_list, &c->counters, &c->ndc_z, &c->vary,
-                      &c->key, &c->key_nan, &c->items,
+                      &c->key, &c->key_nan, &c->big, &c->direct_ctr,
                       &c->frag_cnt, &c->frag_tri, &c->frag_alt, &c->frag_tmp, &c->frag_planes,
                       &c->frag_offs_px};
     for (DevBuf *b : bufs) free_buf(*b);
@@ -1327,16 +1327,12 @@ struct DirectGrid {
 static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const DirectGrid &g, long long nt, bool shadow,
                        bool no_nan, int W, int H)
 {
-    // large triangles' items: room for every 64 x 16 block of the screen many
-    // times over; a pass that needs more rasterises the rest in place
-    constexpr uint32_t kItems = 1u << 18;
     const size_t px = (size_t)W * H;
     int rc;
-    if ((rc = ensure(c, c->key, px * 8))) return rc;
-    if (!c->items.p) {
-        // the items, then two passes' counters (one allocation)
-        if ((rc = ensure(c, c->items, (size_t)kItems * sizeof(uint2) + 2 * sizeof(DirectCtr)))) return rc;
-        launch_fill_u32((uint32_t *)((uint2 *)c->items.p + kItems), 0u, 2 * sizeof(DirectCtr) / 4, c->stream);
+    if ((rc = ensure(c, c->key, px * 8)) || (rc = ensure(c, c->big, (size_t)nt * 12))) return rc;
+    if (!c->direct_ctr.p) {
+        if ((rc = ensure(c, c->direct_ctr, 2 * sizeof(DirectCtr)))) return rc;
+        launch_fill_u32((uint32_t *)c->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, c->stream);
     }
     if (!no_nan) {
         const size_t cap = c->key_nan.cap;
@@ -1344,15 +1340,15 @@ static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const Di
         if (c->key_nan.cap != cap)
             launch_fill_u32((uint32_t *)c->key_nan.p, 0xffffffffu, c->key_nan.cap / 4, c->stream);
     }
-    DirectCtr *ctr = (DirectCtr *)((uint2 *)c->items.p + kItems);
+    DirectCtr *ctr = (DirectCtr *)c->direct_ctr.p;
     DirectArgs a;
     a.draws = (const DevDraw *)c->d_draws.p;
     a.n_draws = n_draws;
     a.screen = (const int4 *)c->screen.p;
     a.key = (unsigned long long *)c->key.p;
     a.fix = no_nan ? nullptr : (unsigned long long *)c->key_nan.p;
-    a.items = (uint2 *)c->items.p;
-    a.n_items = kItems;
+    a.big_start = (unsigned long long *)c->big.p;
+    a.big_tri = (uint32_t *)(a.big_start + nt);
     a.ctr = ctr + c->direct_turn;
     a.W = W;
     a.H = H;
@@ -1583,7 +1579,7 @@ static int flush_pass(fgl_ctx *c)
     // the tile lists.
     const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
     const size_t px = (size_t)W * H;
-    const bool direct = fresh && !stoch && fits && launch_fits(grid.groups) &&
+    const bool direct = fresh && !stoch && fits && nt <= kDirectTrisMost && launch_fits(grid.groups) &&
                         launch_fits(grid.vblocks + clear_blocks((long long)px));
     if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))) ||
         (!shadow && (rc = ensure(c, c->vary, (size_t)nv * 2 * sizeof(float4)))))

@@ -43,23 +43,28 @@ struct ShadowSamples {
     }
 };
 
-// Its counters: items claimed (64 bits: claims past the list's end still
-// count), and whether a NaN mark was made.
+// The direct rasteriser's counters: the large triangles claimed so far and, in
+// the low kBigShift bits, their items (one addition claims both, so the list is
+// in the order of its items); whether a NaN mark was made.  A pass has fewer
+// than 2^30 triangles (direct_pass, plan) and fewer than 2^33 items: an item is
+// at least half a (tile, triangle) pair, of which there are fewer than 2^32.
+constexpr int kBigShift = 34;
 struct DirectCtr {
-    unsigned long long items;
+    unsigned long long claims;
     uint32_t nan, pad;
 };
 
 // A pass of the direct rasteriser (raster_core.hpp): its key plane and the
-// second plane of pixels with NaN marks (null when none can be made), the item list of large triangles,
+// second plane of pixels with NaN marks (null when none can be made), the list
+// of large triangles (room for every triangle): each one's first item and id;
 // the counters.
 struct DirectArgs {
     const DevDraw *draws;
     int n_draws;
     const int4 *screen;
     unsigned long long *key, *fix;
-    uint2 *items;
-    uint32_t n_items;          // the list's capacity
+    unsigned long long *big_start;
+    uint32_t *big_tri;
     DirectCtr *ctr;
     int W, H;
 };

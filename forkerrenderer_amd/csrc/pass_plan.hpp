@@ -12,6 +12,9 @@ constexpr bool launch_fits(long long blocks) { return blocks <= kMaxBlocks; }
 constexpr long long kDirectTris16 = 32768, kDirectTris4 = 262144;
 constexpr int direct_lanes(long long n_tri) { return n_tri <= kDirectTris16 ? 16 : n_tri <= kDirectTris4 ? 4 : 1; }
 
+// Triangles of a pass that the direct rasteriser's claims count.
+constexpr long long kDirectTrisMost = (1LL << 30) - 1;
+
 // Workgroups of a draw: 256 / lanes triangles each; 256 vertices each.
 constexpr long long direct_groups(int n_faces, int lanes) { return ((long long)n_faces * lanes + 255) / 256; }
 constexpr long long vertex_blocks(int n_pos) { return ((long long)n_pos + 255) / 256; }

@@ -424,15 +424,15 @@ __device__ __forceinline__ void raster_tile(const RasterArgs &a, int tile, Raste
 // triangles are large, their own rows of pixels neighbours.
 //
 // kDirectBig bounds what one triangle costs the lanes that own it: a larger
-// one goes to the item list, 64 x 16 pixels an item, and any wavefront of
-// k_direct_big takes it (a list that is full leaves the triangle to its own
-// wavefront).
+// one goes to a list, and the wavefronts of k_direct_big share out its items of
+// 64 x 16 pixels.  The list has room for every triangle of the pass: what does
+// not go there is never more than kDirectBig pixels of one wavefront.
 //
 // NaN depths (a vertex on the camera plane) follow the rule above in two
 // more steps: the first walk marks the pixel with the NaN fragment's id --
 // high word 0, below every real depth's -- and the mark with the highest id
 // is the minimum; k_direct_nan, which returns at once unless a mark was made,
-// walks the triangles again and folds the fragments after the mark into a
+// walks the triangles and the items again and folds the fragments after the mark into a
 // second plane (all ones between passes: the resolve puts back what it
 // read).  A pass whose vertices the host has shown to have finite depths
 // (context.cpp, bound_pass) has neither that plane nor that walk.
@@ -481,9 +481,11 @@ __device__ __forceinline__ void direct_min(unsigned long long *key, unsigned lon
     (void)__hip_atomic_fetch_min(key, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Where a walk's fragments go: the key plane,
+// Where a walk's fragments go (wants: whether any fragment of an item's column
+// px, rows py to y1, can change it): the key plane,
 struct FoldPlane {
     const DirectArgs &a;
+    __device__ __forceinline__ bool wants(int, int, int) const { return true; }
     __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd) const
     {
         direct_min(a.key + (size_t)px + (size_t)py * a.W, direct_key(a, t, dd));
@@ -505,6 +507,17 @@ struct FoldBox {
 // fragments after the pixel's mark.
 struct FoldAfterNan {
     const DirectArgs &a;
+    // few pixels are marked, and the keys of a column load together
+    __device__ __forceinline__ bool wants(int px, int py, int y1) const
+    {
+        bool any = false;
+#pragma unroll
+        for (int e = 0; e < kDirectItemH; ++e) {
+            const int y = py + e < y1 ? py + e : y1 - 1;
+            any = any || (a.key[(size_t)px + (size_t)y * a.W] >> 32) == 0ull;
+        }
+        return any;
+    }
     __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd) const
     {
         const size_t i = (size_t)px + (size_t)py * a.W;
@@ -599,13 +612,12 @@ __device__ __forceinline__ void direct_walk(const TriL &t, bool keep, int area, 
     }
 }
 
-// Triangles of more than kDirectBig pixels to the item list, one claim a
-// wavefront, the items written by all its lanes; true when this lane's
-// triangle (n items of it, 0 if it is no such triangle) went there.
-__device__ __forceinline__ bool direct_items(const DirectArgs &a, int g, uint32_t n)
+// Triangles of more than kDirectBig pixels to the list, one claim a wavefront
+// (n: the items of this lane's triangle, 0 if it is no such triangle).
+__device__ __forceinline__ void direct_claim(const DirectArgs &a, int g, uint32_t n)
 {
-    unsigned long long m = __ballot(n != 0u);
-    if (!m) return false;
+    const unsigned long long m = __ballot(n != 0u);
+    if (!m) return;
     const int lane = threadIdx.x & 63;
     uint32_t inc = n;
 #pragma unroll
@@ -615,23 +627,13 @@ __device__ __forceinline__ bool direct_items(const DirectArgs &a, int g, uint32_
     }
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
     unsigned long long at = 0;
-    if (lane == 63) at = atomicAdd(&a.ctr->items, (unsigned long long)total);
+    if (lane == 63) at = atomicAdd(&a.ctr->claims, ((unsigned long long)__popcll(m) << kBigShift) | total);
     at = __shfl(at, 63, 64);
-    if (at + total > a.n_items) {
-        // no room: what was claimed inside the list holds no item
-        for (unsigned long long k = at + lane; k < a.n_items; k += 64) a.items[k] = make_uint2(0xffffffffu, 0u);
-        return false;
+    if (n) {
+        const size_t p = (size_t)(at >> kBigShift) + __popcll(m & ((1ull << lane) - 1ull));
+        a.big_start[p] = (at & ((1ull << kBigShift) - 1ull)) + (inc - n);
+        a.big_tri[p] = (uint32_t)g;
     }
-    const uint32_t off = (uint32_t)at + inc - n;
-    while (m) {
-        const int l = __builtin_ctzll(m);
-        m &= m - 1;
-        const uint32_t ln = (uint32_t)__builtin_amdgcn_readlane((int)n, l);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)off, l);
-        const uint32_t lg = (uint32_t)__builtin_amdgcn_readlane(g, l);
-        for (uint32_t k = lane; k < ln; k += 64) a.items[lo + k] = make_uint2(lg, k);
-    }
-    return n != 0u;
 }
 
 // A workgroup's 256 / G triangles of draw dr, from number first of its
@@ -649,9 +651,8 @@ __device__ __forceinline__ void direct_group(const DirectArgs &a, const DevDraw 
         const bool big = area > kDirectBig;
         const uint32_t k = big && lane % G == 0 ? (uint32_t)((w + kDirectItemW - 1) / kDirectItemW) *
                                                       (uint32_t)((h + kDirectItemH - 1) / kDirectItemH) : 0u;
-        // a group's first lane decides for the group
-        const int listed = __shfl((int)direct_items(a, keep ? t.g : 0, k), lane - lane % G, 64);
-        keep = keep && !listed;
+        direct_claim(a, keep ? t.g : 0, k);
+        keep = keep && !big;
     }
     // the box of what is left
     typedef unsigned short v2u __attribute__((ext_vector_type(2)));
@@ -703,21 +704,61 @@ __device__ __forceinline__ int4 direct_face(const DevDraw *draws, int d, const i
     return tv;
 }
 
-// Item it of the list, a triangle of draw d, by one wavefront.
-__device__ __forceinline__ void direct_item(const DirectArgs &a, uint2 it, int d)
+// Item k of triangle t by one wavefront.
+template <typename Fold>
+__device__ __forceinline__ void direct_item(const TriL &t, int k, const Fold &fold)
 {
-    TriL t;
-    direct_face(a.draws, d, a.screen, (int)it.x, a.W, a.H, t);
     const int bx = t.bb0 & 0xffff, by = t.bb0 >> 16, w = (t.bb1 & 0xffff) - bx + 1, h = (t.bb1 >> 16) - by + 1;
     const int nx = (w + kDirectItemW - 1) / kDirectItemW;
-    const int ox = ((int)it.y % nx) * kDirectItemW, oy = ((int)it.y / nx) * kDirectItemH;
+    const int ox = k % nx * kDirectItemW, oy = k / nx * kDirectItemH;
     const int x = ox + (int)(threadIdx.x & 63);
     if (x >= w) return;
     const int y1 = imin(oy + kDirectItemH, h);
-    const FoldPlane fold{a};
+    if (!fold.wants(bx + x, by + oy, by + y1)) return;
     for (int y = oy; y < y1; ++y) {
         float b0, b1, b2;
         if (cover(t, bx + x, by + y, b0, b1, b2)) fold(t, bx + x, by + y, tri_depth(t, b0, b1, b2));
+    }
+}
+
+// The large triangle that owns item i: the last whose first item is at most
+// i, of n (start[0] is 0); 64 probes a step.
+__device__ __forceinline__ uint32_t big_of(const unsigned long long *start, uint32_t n, unsigned long long i)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t lo = 0, len = n;
+    while (len > 1) {
+        const uint32_t step = (len + 63) / 64, at = lane * step;
+        const unsigned long long le = __ballot(at < len && start[lo + (at < len ? at : 0u)] <= i);
+        const uint32_t k = (uint32_t)__popcll(le) - 1u;
+        lo += k * step;
+        len = len - k * step < step ? len - k * step : step;
+    }
+    return lo;
+}
+
+// The items of a pass's large triangles shared out to the launch's wavefronts,
+// in runs of up to 16 (one search and one triangle's set-up a run or
+// triangle).  of(d): the arguments of draw d's target.
+template <typename Fold, typename Args, typename Of>
+__device__ __forceinline__ void direct_big(const Args &p, const Of &of)
+{
+    const unsigned long long claims = p.ctr->claims, n = claims & ((1ull << kBigShift) - 1ull);
+    const uint32_t n_big = (uint32_t)(claims >> kBigShift);
+    const unsigned long long waves = (unsigned long long)gridDim.x * (blockDim.x >> 6);
+    const unsigned long long share = n / (4 * waves), run = share < 1 ? 1 : share > 16 ? 16 : share;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
+    for (unsigned long long i = wave * run; i < n; i += waves * run) {
+        const unsigned long long end = i + run < n ? i + run : n;
+        uint32_t b = __builtin_amdgcn_readfirstlane(big_of(p.big_start, n_big, i));
+        for (unsigned long long k = i; k < end; ++b) {
+            const unsigned long long first = p.big_start[b], next = b + 1 < n_big ? p.big_start[b + 1] : n;
+            const int g = (int)p.big_tri[b], d = draw_of(p.draws, p.n_draws, g);
+            const DirectArgs a = of(d);
+            TriL t;
+            direct_face(a.draws, d, a.screen, g, a.W, a.H, t);
+            for (; k < end && k < next; ++k) direct_item(t, (int)(k - first), Fold{a});
+        }
     }
 }
 

@@ -1,7 +1,7 @@
 """The direct rasteriser (passes from cleared targets) against the tile lists
 (passes that go on from earlier depths), bit for bit, over what their rules
-divide: lanes per triangle, the workgroup's LDS box, the item list of large
-triangles and its overflow, NaN depths, screens of one pixel and wider than
+divide: lanes per triangle, the workgroup's LDS box, the list of large
+triangles and its runs of items, NaN depths, screens of one pixel and wider than
 the exact regime, several draws with equal depths.
 
 The second rendering starts with a draw that covers nothing and a change of
@@ -47,7 +47,7 @@ def _scene(name, rng):
         return [_triangles(rng, 40000, 0.02)], 640, 400
     if name == "one_lane":
         return [_triangles(rng, 270000, 0.004), _triangles(rng, 5, 1.5)], 512, 300
-    if name == "items_overflow":   # 1,200 full screens of 300 items each: more than the list holds
+    if name == "full_screens":     # 1,200 full screens of 300 items each: runs of 16, many searches
         full = np.array([[-3, -3, 0], [3, -3, 0], [0, 3, 0]]) + 0.0
         return [full[None] + rng.uniform(-0.4, 0.4, (1200, 3, 1)) * np.array([0, 0, 1]), _triangles(rng, 100, 0.1)], 640, 480
     if name == "ties":             # the same triangles drawn three times: the first draw's win
@@ -64,11 +64,15 @@ def _scene(name, rng):
         t[::7, 1, 2] = np.nan
         t[3::11, 2, 2] = np.inf
         return [t, _triangles(rng, 100, 0.4)], 120, 80
+    if name == "nan_large":        # the same with listed triangles before and after the marks
+        t = _triangles(rng, 300, 1.0)
+        t[::7, 1, 2] = np.nan
+        return [_triangles(rng, 60, 0.1), t, _triangles(rng, 60, 1.0)], 640, 480
     raise AssertionError(name)
 
 
-@pytest.mark.parametrize("name", ["few_mixed", "four_lanes", "one_lane", "items_overflow", "ties", "one_pixel", "thin",
-                                  "inexact", "nan"])
+@pytest.mark.parametrize("name", ["few_mixed", "four_lanes", "one_lane", "full_screens", "ties", "one_pixel", "thin",
+                                  "inexact", "nan", "nan_large"])
 @pytest.mark.parametrize("shadow", [False, True])
 def test_direct_equals_lists(ctx, name, shadow):
     rng = np.random.default_rng(len(name))
@@ -78,8 +82,9 @@ def test_direct_equals_lists(ctx, name, shadow):
     _direct_against_lists(ctx, mat, models, W, H, shadow, name)
 
 
-def _direct_against_lists(ctx, mat, draws, W, H, shadow, name):
-    """draws: (model, matrix) in order."""
+def _direct_against_lists(ctx, mat, draws, W, H, shadow, name, timed=False):
+    """draws: (model, matrix) in order.  timed: returns the ms of each
+    rendering's rasterisation (a second one, so that nothing is allocated)."""
     off = _model(ctx, mat, np.full((1, 3, 3), 9.0) + np.eye(3)[None])
     ctx.set_tile_size(16)
     ctx.set_shadow(False)
@@ -88,7 +93,7 @@ def _direct_against_lists(ctx, mat, draws, W, H, shadow, name):
     ctx.set_matrix(F.MAT_VIEW, eye)
     ctx.set_matrix(F.MAT_LIGHT_SPACE, eye)
     ctx.set_viewport(0, 0, W, H, shadow=shadow)
-    out = []
+    out, ms = [], []
     for lists in (False, True):
         print(f"direct test {name} {W}x{H} shadow {shadow} lists {lists}", flush=True)
         if shadow:
@@ -102,17 +107,33 @@ def _direct_against_lists(ctx, mat, draws, W, H, shadow, name):
             ctx.set_eye((0.0, 0.0, 2.0))   # flushes the pass so far
         for k, at in draws:
             ctx.draw_model(k, at)
+        if timed:
+            ctx.end_pass()
+            ctx.sync()
+            ctx.enable_timing(True)
+            ctx.init_targets(W, H)
+            ctx.begin_pass(F.PASS_GEOMETRY)
+            if lists:
+                ctx.draw_model(off, eye)
+                ctx.set_eye((0.0, 0.0, 1.0))
+            for k, at in draws:
+                ctx.draw_model(k, at)
         ctx.end_pass()
+        if timed:
+            ctx.sync()
+            ms.append(sum(t for k, t in ctx.read_timings() if k in ("vertex", "setup", "scan", "emit", "sort", "tile_ranges", "raster")))
+            ctx.enable_timing(False)
         which = (F.TARGET_SHADOW_DEPTH, F.TARGET_SHADOW) if shadow else (F.TARGET_DEPTH, F.TARGET_GBUFFER)
         out.append([ctx.read(t).view(np.uint32) for t in which])
     for a, b, what in zip(out[0], out[1], ("depth", "shadow value" if shadow else "G-buffer")):
-        if name == "nan":   # a NaN's payload is not the fold's
+        if name.startswith("nan"):   # a NaN's payload is not the fold's
             na, nb = np.isnan(a.view(np.float32)), np.isnan(b.view(np.float32))
             assert np.array_equal(na, nb), what
             a, b = np.where(na, 0, a), np.where(nb, 0, b)
         assert np.array_equal(a, b), f"{what}: {(a != b).sum()} of {a.size} differ"
     depth = out[0][0].view(np.float32)
     assert (depth < 3e38).any()
+    return ms
 
 
 @pytest.mark.parametrize("shadow", [False, True])
@@ -141,3 +162,21 @@ def _model_without_faces(ctx):
     return ctx.upload_model({"pos": np.ones((300, 3), np.float32), "uv": np.zeros((1, 2), np.float32),
                              "nrm": np.ones((1, 3), np.float32), "tan": None, "vi": f, "ti": f, "ni": f,
                              "face_material": np.zeros(0, np.int32), "support_pbr": False})
+
+
+@pytest.mark.parametrize("nan", [False, True])
+def test_large_triangles_are_shared_out(ctx, nan):
+    """Layers of full-screen triangles, more of them than 2^18 items of 64 x 16
+    pixels; with a NaN vertex among them the pass walks them twice.  No
+    wavefront is left with whole ones: the pass takes no more than a few times
+    what the tile lists take (an eighth of the layers on their own wavefronts
+    took 200 times as long)."""
+    rng = np.random.default_rng(3)
+    W, H, n = 1920, 1080, 256
+    full = np.array([[[-3, -3, 0.9], [3, -3, 0.9], [0, 3, 0.9]]]) + rng.uniform(0, 0.05, (n, 1, 1)) * np.array([0, 0, 1])
+    full[5, 1, 2] = np.nan if nan else 0.9
+    mat = _material(ctx)
+    m = _model(ctx, mat, full)
+    print("layers", nan, flush=True)
+    ms = _direct_against_lists(ctx, mat, [(m, EYE4)], W, H, False, "nan layers" if nan else "layers", timed=True)
+    assert ms[0] < 8 * ms[1] + 1.0, ms
