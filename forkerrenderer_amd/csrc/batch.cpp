@@ -401,6 +401,7 @@ static BvDirectArgs direct_args(fgl_batch *b, int p)
     a.views = (const DevView *)b->d_views.p;
     a.screen = (const int4 *)b->screen.p;
     a.key = (unsigned long long *)b->key.p;
+    a.deep_from = (unsigned long long)deep_items((long long)(p == kBvShadow ? b->total_spx : b->total_px));
     a.big_start = (unsigned long long *)b->big.p;
     a.big_tri = (uint32_t *)(a.big_start + std::max(b->nt[0], b->nt[1]));
     a.ctr = (DirectCtr *)b->direct_ctr.p + p;

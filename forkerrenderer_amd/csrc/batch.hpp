@@ -67,6 +67,7 @@ struct BvDirectArgs {
     unsigned long long *key;
     unsigned long long *big_start;
     uint32_t *big_tri;
+    unsigned long long deep_from;
     DirectCtr *ctr;
 };
 

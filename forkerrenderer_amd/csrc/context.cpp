@@ -1347,6 +1347,8 @@ static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const Di
     a.screen = (const int4 *)c->screen.p;
     a.key = (unsigned long long *)c->key.p;
     a.fix = no_nan ? nullptr : (unsigned long long *)c->key_nan.p;
+    a.bases = (const int *)(a.draws + n_draws);
+    a.deep_from = (unsigned long long)deep_items((long long)px);
     a.big_start = (unsigned long long *)c->big.p;
     a.big_tri = (uint32_t *)(a.big_start + nt);
     a.ctr = ctr + c->direct_turn;
@@ -1566,9 +1568,18 @@ static int flush_pass(fgl_ctx *c)
 
     if (dd.size() != c->last_draws.size() ||
         std::memcmp(dd.data(), c->last_draws.data(), dd.size() * sizeof(DevDraw)) != 0) {
-        if ((rc = ensure(c, c->d_draws, dd.size() * sizeof(DevDraw)))) return rc;
+        // the records, then their bases by themselves (DirectArgs::bases)
+        std::vector<int> bases(2 * dd.size());
+        for (size_t i = 0; i < dd.size(); ++i) {
+            bases[i] = dd[i].vblock_base;
+            bases[dd.size() + i] = dd[i].group_base;
+        }
+        const size_t records = dd.size() * sizeof(DevDraw), table = bases.size() * sizeof(int);
+        if ((rc = ensure(c, c->d_draws, records + table))) return rc;
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        HIPCHK(c, hipMemcpy(c->d_draws.p, dd.data(), dd.size() * sizeof(DevDraw), hipMemcpyHostToDevice));
+        c->last_draws.clear();
+        HIPCHK(c, hipMemcpy(c->d_draws.p, dd.data(), records, hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy((char *)c->d_draws.p + records, bases.data(), table, hipMemcpyHostToDevice));
         c->last_draws = dd;
     }
 

@@ -12,6 +12,10 @@ constexpr bool launch_fits(long long blocks) { return blocks <= kMaxBlocks; }
 constexpr long long kDirectTris16 = 32768, kDirectTris4 = 262144;
 constexpr int direct_lanes(long long n_tri) { return n_tri <= kDirectTris16 ? 16 : n_tri <= kDirectTris4 ? 4 : 1; }
 
+// Items (64 x 16 pixels) of large triangles that cover targets of so many pixels
+// three times over.
+constexpr long long deep_items(long long pixels) { return 3 * (pixels / 1024 + 1); }
+
 // Triangles of a pass that the direct rasteriser's claims count.
 constexpr long long kDirectTrisMost = (1LL << 30) - 1;
 

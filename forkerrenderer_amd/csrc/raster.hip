@@ -195,7 +195,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TS == 32 
 // plane cleared (8 keys a thread) by the workgroups past the vertices', and
 // the counters of the next pass zeroed (this pass's were by the one before).
 template <bool SHADOW>
-__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, int n_draws, int n_vert_blocks,
+__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, const int *__restrict__ bases,
+                                                       int n_draws, int n_vert_blocks,
                                                        FrameUniforms u, int4 *__restrict__ out,
                                                        float *__restrict__ ndc_z, float4 *__restrict__ vary,
                                                        unsigned long long *__restrict__ key,
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
         }
         return;
     }
-    const DevDraw &dr = draws[draw_at<&DevDraw::vblock_base>(draws, n_draws, b)];
+    const DevDraw &dr = draws[owner_of(bases, (uint32_t)n_draws, b)];
     const int vi = (b - dr.vblock_base) * 256 + threadIdx.x;
     if (vi >= dr.n_pos) return;
     if (SHADOW) {
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(256) void k_direct(DirectArgs a)
 {
     __shared__ DirectLds lds;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const DevDraw &dr = a.draws[draw_at<&DevDraw::group_base>(a.draws, a.n_draws, b)];
+    const DevDraw &dr = a.draws[owner_of(a.bases + a.n_draws, (uint32_t)a.n_draws, b)];
     direct_group<G>(a, dr, (b - dr.group_base) * (256 / G), lds);
 }
 
@@ -615,11 +616,11 @@ void launch_direct_vertex(bool shadow, int n_blocks, const FrameUniforms &u, int
     const size_t P = (size_t)a.W * a.H;
     const unsigned grid = (unsigned)(n_blocks + clear_blocks((long long)P));
     if (shadow)
-        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, a.draws, a.n_draws, n_blocks, u, out, ndc_z,
-                           vary, a.key, P, next_ctr);
+        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, a.draws, a.bases, a.n_draws, n_blocks, u, out,
+                           ndc_z, vary, a.key, P, next_ctr);
     else
-        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, a.draws, a.n_draws, n_blocks, u, out, ndc_z,
-                           vary, a.key, P, next_ctr);
+        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, a.draws, a.bases, a.n_draws, n_blocks, u, out,
+                           ndc_z, vary, a.key, P, next_ctr);
 }
 
 void launch_direct(const DirectArgs &a, int lanes, int n_groups, long long n_tri, hipStream_t s)

@@ -441,24 +441,34 @@ constexpr int kDirectItemW = 64, kDirectItemH = 16;
 constexpr int kDirectBig = 4096;      // pixels of the bounding box
 constexpr int kDirectBox = 2048;      // pixels of a workgroup's LDS box: 16 KiB, nine workgroups a CU
 
-// The last draw whose base is at most g: the draw of pass-wide triangle (or
-// workgroup) g.  Bases ascend; of draws with none of their own the last one
-// of equal bases, which owns g, is found.
-template <int DevDraw::*BASE>
-__device__ __forceinline__ int draw_at(const DevDraw *draws, int n_draws, int g)
+// The last of n ascending starts (start[0] is 0) that is at most i, by whole
+// wavefronts, 64 probes a step.  Of owners with nothing of their own the last
+// one of equal starts, which owns i, is found.
+template <typename T>
+__device__ __forceinline__ uint32_t owner_of(const T *start, uint32_t n, T i)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t lo = 0, len = n;
+    while (len > 1) {
+        const uint32_t step = (len + 63) / 64, at = lane * step;
+        const unsigned long long le = __ballot(at < len && start[lo + (at < len ? at : 0u)] <= i);
+        const uint32_t k = (uint32_t)__popcll(le) - 1u;
+        lo += k * step;
+        len = len - k * step < step ? len - k * step : step;
+    }
+    return __builtin_amdgcn_readfirstlane(lo);
+}
+
+// The draw of pass-wide triangle g (their tri_base ascend).
+__device__ __forceinline__ int draw_of(const DevDraw *draws, int n_draws, int g)
 {
     int lo = 0, hi = n_draws - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (draws[mid].*BASE <= g) lo = mid;
+        if (draws[mid].tri_base <= g) lo = mid;
         else hi = mid - 1;
     }
     return lo;
-}
-
-__device__ __forceinline__ int draw_of(const DevDraw *draws, int n_draws, int g)
-{
-    return draw_at<&DevDraw::tri_base>(draws, n_draws, g);
 }
 
 struct DirectLds {
@@ -489,6 +499,13 @@ struct FoldPlane {
     __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd) const
     {
         direct_min(a.key + (size_t)px + (size_t)py * a.W, direct_key(a, t, dd));
+    }
+    // of an item: not where the plane held a smaller key already (keys only fall)
+    __device__ __forceinline__ unsigned long long held(int px, int py) const { return a.key[(size_t)px + (size_t)py * a.W]; }
+    __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd, unsigned long long held) const
+    {
+        const unsigned long long k = direct_key(a, t, dd);
+        if (k < held) direct_min(a.key + (size_t)px + (size_t)py * a.W, k);
     }
 };
 
@@ -524,6 +541,11 @@ struct FoldAfterNan {
         const unsigned long long m = a.key[i];
         if ((m >> 32) != 0ull || dd != dd || t.g <= (int)~(uint32_t)m) return;
         direct_min(a.fix + i, ((unsigned long long)depth_order(dd) << 32) | (unsigned long long)(uint32_t)(t.g + 1));
+    }
+    __device__ __forceinline__ unsigned long long held(int, int) const { return 0ull; }
+    __device__ __forceinline__ void operator()(const TriL &t, int px, int py, float dd, unsigned long long) const
+    {
+        (*this)(t, px, py, dd);
     }
 };
 
@@ -610,6 +632,12 @@ __device__ __forceinline__ void direct_walk(const TriL &t, bool keep, int area, 
         m &= m - 1;
         direct_box(direct_lane(t, l), lane, 64, fold);
     }
+}
+
+__device__ __forceinline__ unsigned long long lane_u64(unsigned long long v, int l)
+{
+    return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
 }
 
 // Triangles of more than kDirectBig pixels to the list, one claim a wavefront
@@ -704,8 +732,9 @@ __device__ __forceinline__ int4 direct_face(const DevDraw *draws, int d, const i
     return tv;
 }
 
-// Item k of triangle t by one wavefront.
-template <typename Fold>
+// Item k of triangle t by one wavefront.  DEEP: where the plane already holds
+// a smaller key the atomic is left out.
+template <bool DEEP, typename Fold>
 __device__ __forceinline__ void direct_item(const TriL &t, int k, const Fold &fold)
 {
     const int bx = t.bb0 & 0xffff, by = t.bb0 >> 16, w = (t.bb1 & 0xffff) - bx + 1, h = (t.bb1 >> 16) - by + 1;
@@ -715,49 +744,57 @@ __device__ __forceinline__ void direct_item(const TriL &t, int k, const Fold &fo
     if (x >= w) return;
     const int y1 = imin(oy + kDirectItemH, h);
     if (!fold.wants(bx + x, by + oy, by + y1)) return;
-    for (int y = oy; y < y1; ++y) {
-        float b0, b1, b2;
-        if (cover(t, bx + x, by + y, b0, b1, b2)) fold(t, bx + x, by + y, tri_depth(t, b0, b1, b2));
+    constexpr int kRows = DEEP ? 4 : 1;   // their keys load together
+    for (int y = oy; y < y1; y += kRows) {
+        unsigned long long held[kRows];
+#pragma unroll
+        for (int e = 0; e < kRows; ++e) held[e] = DEEP ? fold.held(bx + x, by + imin(y + e, y1 - 1)) : ~0ull;
+#pragma unroll
+        for (int e = 0; e < kRows; ++e) {
+            float b0, b1, b2;
+            if (y + e < y1 && cover(t, bx + x, by + y + e, b0, b1, b2))
+                fold(t, bx + x, by + y + e, tri_depth(t, b0, b1, b2), held[e]);
+        }
     }
 }
 
-// The large triangle that owns item i: the last whose first item is at most
-// i, of n (start[0] is 0); 64 probes a step.
-__device__ __forceinline__ uint32_t big_of(const unsigned long long *start, uint32_t n, unsigned long long i)
-{
-    const uint32_t lane = threadIdx.x & 63;
-    uint32_t lo = 0, len = n;
-    while (len > 1) {
-        const uint32_t step = (len + 63) / 64, at = lane * step;
-        const unsigned long long le = __ballot(at < len && start[lo + (at < len ? at : 0u)] <= i);
-        const uint32_t k = (uint32_t)__popcll(le) - 1u;
-        lo += k * step;
-        len = len - k * step < step ? len - k * step : step;
-    }
-    return lo;
-}
-
-// The items of a pass's large triangles shared out to the launch's wavefronts,
-// in runs of up to 16 (one search and one triangle's set-up a run or
-// triangle).  of(d): the arguments of draw d's target.
+// The items of a pass's large triangles shared out to the launch's wavefronts.
+// of(d): the arguments of draw d's target.  Where the items cover the targets
+// several times over (deep_items, pass_plan.hpp) the fold is bound by the
+// atomics' traffic: a key is read before, and a wavefront takes runs of up to 16
+// items (one search and one triangle's set-up a run or triangle): 64 full screens
+// of 3840 x 2160 2.69 -> 1.02 ms.  With fewer an item's own time counts, to which
+// the read would add (640 x 400 frame 102 -> 111 us), and runs would put covered
+// items beside covered ones (24 views' shadow maps 81 -> 90).  Up to 64
+// triangles' starts are kept in the lanes.
 template <typename Fold, typename Args, typename Of>
 __device__ __forceinline__ void direct_big(const Args &p, const Of &of)
 {
     const unsigned long long claims = p.ctr->claims, n = claims & ((1ull << kBigShift) - 1ull);
     const uint32_t n_big = (uint32_t)(claims >> kBigShift);
     const unsigned long long waves = (unsigned long long)gridDim.x * (blockDim.x >> 6);
-    const unsigned long long share = n / (4 * waves), run = share < 1 ? 1 : share > 16 ? 16 : share;
+    const bool deep = n >= p.deep_from, few = n_big <= 64;
+    const unsigned long long rounds = (n + 16 * waves - 1) / (16 * waves);
+    const unsigned long long run = deep ? (n + rounds * waves - 1) / (rounds * waves) : 1;
+    const uint32_t lane = threadIdx.x & 63;
+    const unsigned long long start = few && lane < n_big ? p.big_start[lane] : ~0ull;
+    const uint32_t tri = few && lane < n_big ? p.big_tri[lane] : 0u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     for (unsigned long long i = wave * run; i < n; i += waves * run) {
         const unsigned long long end = i + run < n ? i + run : n;
-        uint32_t b = __builtin_amdgcn_readfirstlane(big_of(p.big_start, n_big, i));
+        uint32_t b = few ? (uint32_t)__popcll(__ballot(start <= i)) - 1u : owner_of(p.big_start, n_big, i);
         for (unsigned long long k = i; k < end; ++b) {
-            const unsigned long long first = p.big_start[b], next = b + 1 < n_big ? p.big_start[b + 1] : n;
-            const int g = (int)p.big_tri[b], d = draw_of(p.draws, p.n_draws, g);
+            const unsigned long long first = few ? lane_u64(start, b) : p.big_start[b];
+            const unsigned long long next = b + 1 >= n_big ? n : few ? lane_u64(start, b + 1) : p.big_start[b + 1];
+            const int g = few ? __builtin_amdgcn_readlane((int)tri, b) : (int)p.big_tri[b];
+            const int d = draw_of(p.draws, p.n_draws, g);
             const DirectArgs a = of(d);
             TriL t;
             direct_face(a.draws, d, a.screen, g, a.W, a.H, t);
-            for (; k < end && k < next; ++k) direct_item(t, (int)(k - first), Fold{a});
+            if (deep)
+                for (; k < end && k < next; ++k) direct_item<true>(t, (int)(k - first), Fold{a});
+            else
+                for (; k < end && k < next; ++k) direct_item<false>(t, (int)(k - first), Fold{a});
         }
     }
 }
