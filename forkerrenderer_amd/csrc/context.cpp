@@ -1202,9 +1202,11 @@ struct ClipBound {
     double m[16], a[16];
 };
 
-static void mat_mul_d(const double *x, const float *y, double *o, bool absolute)
+// Rows r0 .. 3 of x y (depths_finite needs the last, of absolute values the last
+// two).
+static void mat_mul_d(const double *x, const float *y, double *o, bool absolute, int r0 = 0)
 {
-    for (int r = 0; r < 4; ++r)
+    for (int r = r0; r < 4; ++r)
         for (int j = 0; j < 4; ++j) {
             double v = 0.0;
             for (int k = 0; k < 4; ++k) {
@@ -1232,9 +1234,11 @@ static ClipBound camera_bound(const fgl_ctx *c, bool shadow)
 // reach (they are about a millionth of it).
 constexpr double kClipMargin = 1e-4;
 
-// Whether every vertex of m has a finite window depth below 1e30: then no
-// fragment's depth is NaN.  Each vertex is tried for models of few vertices,
-// else the model's extent, which has to lie on one side of the camera plane.
+// Whether every vertex of m's faces has a finite window depth below 1e30: then
+// no fragment's depth is NaN.  The model's extent is tried, which has to lie on
+// one side of the camera plane; where it does not, each vertex of models of few
+// vertices (a ground plane the camera stands on).  The extent first: 4,096 draws
+// of 162 vertices, 640 x 400 view 6.4 -> 2.5 ms.
 static bool depths_finite(const ModelRes &m, const ClipBound &b)
 {
     if (!m.bounded) return false;
@@ -1251,7 +1255,8 @@ static bool depths_finite(const ModelRes &m, const ClipBound &b)
         const double least = std::fabs(w) - ext;
         return least > kClipMargin * mag && z < 1e30 * least && least > 1e-30 && mag < 1e30 && top < 1e30;
     };
-    if (m.few.empty()) return far_from_camera(m.lo, m.hi);
+    if (far_from_camera(m.lo, m.hi)) return true;
+    if (m.few.empty()) return false;
     for (size_t k = 0; k < m.few.size(); k += 3) {
         const double p[3] = {m.few[k], m.few[k + 1], m.few[k + 2]};
         if (!far_from_camera(p, p)) return false;
@@ -1307,8 +1312,9 @@ static void bound_pass(const fgl_ctx *c, bool shadow, long long nt, int W, int H
     for (const fgl_ctx::Rec &r : c->draws) {
         const ModelRes &m = c->models[r.model];
         ClipBound b;
-        mat_mul_d(cam.m, r.m, b.m, false);
-        mat_mul_d(cam.a, r.m, b.a, true);
+        if (!count && !no_nan) break;
+        mat_mul_d(cam.m, r.m, b.m, false, count ? 0 : 3);
+        mat_mul_d(cam.a, r.m, b.a, true, count ? 0 : 2);
         no_nan = no_nan && depths_finite(m, b);
         if (count) sum += pairs_bound(m, b, shadow ? c->shadow_viewport : c->viewport, W, H, TS);
     }
@@ -1525,8 +1531,10 @@ static int flush_pass(fgl_ctx *c)
 
     // draw table in submission order
     std::vector<DevDraw> dd(c->draws.size());
-    long long nt = 0, nv = 0;
+    long long nt = 0, nv = 0, tris = 0;
     int max_pos = 0, max_faces = 0;
+    for (const fgl_ctx::Rec &r : c->draws) tris += c->models[r.model].n_faces;
+    DirectGrid grid = {direct_lanes(tris), 0, 0};
     for (size_t i = 0; i < c->draws.size(); ++i) {
         const ModelRes &m = c->models[c->draws[i].model];
         DevDraw &d = dd[i];
@@ -1534,17 +1542,14 @@ static int flush_pass(fgl_ctx *c)
         if (c->draws[i].has_normal) std::memcpy(d.normal, c->draws[i].n, sizeof(d.normal));
         d.vert_base = (int)nv;
         d.tri_base = (int)nt;
-        nt += m.n_faces;
-        nv += m.n_pos;
-        max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
-        max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
-    }
-    DirectGrid grid = {direct_lanes(nt), 0, 0};
-    for (DevDraw &d : dd) {
         d.group_base = (int)grid.groups;
         d.vblock_base = (int)grid.vblocks;
         grid.groups += direct_groups(d.n_faces, grid.lanes);
         grid.vblocks += vertex_blocks(d.n_pos);
+        nt += m.n_faces;
+        nv += m.n_pos;
+        max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
+        max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
     }
     const int n_draws = (int)c->draws.size();
     bool fits, no_nan;
@@ -2115,8 +2120,8 @@ bool ctx_depths_finite(fgl_ctx *c, int model, const float M[16], bool shadow)
 {
     const ClipBound cam = camera_bound(c, shadow);
     ClipBound b;
-    mat_mul_d(cam.m, M, b.m, false);
-    mat_mul_d(cam.a, M, b.a, true);
+    mat_mul_d(cam.m, M, b.m, false, 3);
+    mat_mul_d(cam.a, M, b.a, true, 2);
     return depths_finite(c->models[model], b);
 }
 

@@ -7,6 +7,8 @@ the exact regime, several draws with equal depths.
 The second rendering starts with a draw that covers nothing and a change of
 state, which flushes it: the rest of the pass then continues from existing
 depths and takes the tile lists."""
+import time
+
 import numpy as np
 import pytest
 
@@ -180,3 +182,32 @@ def test_large_triangles_are_shared_out(ctx, nan):
     print("layers", nan, flush=True)
     ms = _direct_against_lists(ctx, mat, [(m, EYE4)], W, H, False, "nan layers" if nan else "layers", timed=True)
     assert ms[0] < 8 * ms[1] + 1.0, ms
+
+
+def test_draws_in_front_of_the_camera_are_bounded_by_their_box(ctx):
+    """Host time of a pass of many draws: models of few vertices, which are
+    tried one by one where the box of the model does not clear the camera
+    plane, cost no more than models of many (three times as much when they
+    were tried first)."""
+    rng = np.random.default_rng(9)
+    mat = _material(ctx)
+    ctx.set_shadow(False)
+    for which in (F.MAT_PROJ, F.MAT_VIEW):
+        ctx.set_matrix(which, np.ascontiguousarray(EYE4))
+    ctx.set_viewport(0, 0, 64, 64)
+    took = []
+    for faces in (85, 86):   # 255 and 258 vertices
+        m = _model(ctx, mat, _triangles(rng, faces, 0.05))
+        best = 1e9
+        for rep in range(6):
+            ctx.init_targets(64, 64)
+            ctx.begin_pass(F.PASS_GEOMETRY)
+            for k in range(2000):
+                ctx.draw_model(m, EYE4)
+            ctx.sync()
+            t0 = time.perf_counter()
+            ctx.end_pass()
+            best = min(best, time.perf_counter() - t0)
+        took.append(best)
+    print("2,000 draws, seconds:", took, flush=True)
+    assert took[0] < 1.5 * took[1], took
