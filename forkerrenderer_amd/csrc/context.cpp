@@ -517,7 +517,8 @@ int fgl_upload_material(fgl_ctx *c, const fgl_material *m, int *out_id)
 
 // The bundle (DevBundle) of material k's maps for the Blinn-Phong (0) or PBR
 // (1) shaders, made on first use from the maps that share the first one's
-// size, wrap and filter; a single map has none.
+// size, wrap and filter; a single map has none, and maps without room for it go
+// on by themselves.
 static int ensure_bundle(fgl_ctx *c, int k, int pbr)
 {
     DevMaterial &m = c->materials[k];
@@ -546,7 +547,10 @@ static int ensure_bundle(fgl_ctx *c, int k, int pbr)
         }
     const int w = first->w, h = first->h;
     void *mem = nullptr;
-    HIPCHK(c, hipMalloc(&mem, (size_t)((w + 3) / 4) * ((h + 3) / 4) * 16 * sizeof(uint2)));
+    if (hipMalloc(&mem, (size_t)((w + 3) / 4) * ((h + 3) / 4) * 16 * sizeof(uint2)) != hipSuccess) {
+        (void)hipGetLastError();
+        return FGL_OK;
+    }
     c->texture_mem.push_back(mem);
     launch_bundle(w, h, t[0] ? t[0]->texels : nullptr, t[1] ? t[1]->zb : nullptr, t[2] ? t[2]->texels : nullptr,
                   t[3] ? t[3]->zb : nullptr, (uint2 *)mem, c->stream);
