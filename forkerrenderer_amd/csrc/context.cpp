@@ -1332,24 +1332,36 @@ struct DirectGrid {
     long long groups, vblocks;
 };
 
-// The pass's fragments through the direct rasteriser: its keys are left for
-// the resolve, the shadow pass's targets are written.
-static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const DirectGrid &g, long long nt, bool shadow,
-                       bool no_nan, int W, int H)
+static void free_direct(fgl_ctx *c)
+{
+    (void)hipStreamSynchronize(c->stream);   // no kernel may still use it
+    (void)hipGetLastError();                 // of the allocation that failed
+    for (DevBuf *b : {&c->key, &c->big, &c->key_nan, &c->direct_ctr}) free_buf(*b);
+}
+
+// Memory for a direct pass; without it the tile lists, which need none of this,
+// take the pass.
+static bool direct_room(fgl_ctx *c, size_t px, long long nt, bool no_nan)
+{
+    const size_t nan_cap = c->key_nan.cap;
+    const bool first = !c->direct_ctr.p;
+    if (room(c, c->key, px * 8) && room(c, c->big, (size_t)nt * 12) && room(c, c->direct_ctr, 2 * sizeof(DirectCtr)) &&
+        (no_nan || room(c, c->key_nan, px * 8))) {
+        if (first) launch_fill_u32((uint32_t *)c->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, c->stream);
+        if (c->key_nan.cap != nan_cap)
+            launch_fill_u32((uint32_t *)c->key_nan.p, 0xffffffffu, c->key_nan.cap / 4, c->stream);
+        return true;
+    }
+    free_direct(c);
+    return false;
+}
+
+// The pass's fragments through the direct rasteriser (direct_room): its keys
+// are left for the resolve, the shadow pass's targets are written.
+static void direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const DirectGrid &g, long long nt, bool shadow,
+                        bool no_nan, int W, int H)
 {
     const size_t px = (size_t)W * H;
-    int rc;
-    if ((rc = ensure(c, c->key, px * 8)) || (rc = ensure(c, c->big, (size_t)nt * 12))) return rc;
-    if (!c->direct_ctr.p) {
-        if ((rc = ensure(c, c->direct_ctr, 2 * sizeof(DirectCtr)))) return rc;
-        launch_fill_u32((uint32_t *)c->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, c->stream);
-    }
-    if (!no_nan) {
-        const size_t cap = c->key_nan.cap;
-        if ((rc = ensure(c, c->key_nan, px * 8))) return rc;
-        if (c->key_nan.cap != cap)
-            launch_fill_u32((uint32_t *)c->key_nan.p, 0xffffffffu, c->key_nan.cap / 4, c->stream);
-    }
     DirectCtr *ctr = (DirectCtr *)c->direct_ctr.p;
     DirectArgs a;
     a.draws = (const DevDraw *)c->d_draws.p;
@@ -1375,7 +1387,6 @@ static int direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const Di
     launch_direct(a, g.lanes, (int)g.groups, nt, c->stream);
     if (shadow)
         launch_direct_shadow(a, (const float *)c->ndc_z.p, (float *)c->shadow_depth.p, (float *)c->shadow.p, c->stream);
-    return FGL_OK;
 }
 
 // The pass through the tile lists; with stoch also the sequence of passing
@@ -1584,9 +1595,9 @@ static int flush_pass(fgl_ctx *c)
             bases[dd.size() + i] = dd[i].group_base;
         }
         const size_t records = dd.size() * sizeof(DevDraw), table = bases.size() * sizeof(int);
+        c->last_draws.clear();   // nothing is known of the table until it is written
         if ((rc = ensure(c, c->d_draws, records + table))) return rc;
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        c->last_draws.clear();
         HIPCHK(c, hipMemcpy(c->d_draws.p, dd.data(), records, hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy((char *)c->d_draws.p + records, bases.data(), table, hipMemcpyHostToDevice));
         c->last_draws = dd;
@@ -1599,16 +1610,21 @@ static int flush_pass(fgl_ctx *c)
     // the tile lists.
     const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
     const size_t px = (size_t)W * H;
-    const bool direct = fresh && !stoch && fits && nt <= kDirectTrisMost && launch_fits(grid.groups) &&
-                        launch_fits(grid.vblocks + clear_blocks((long long)px));
     if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))) ||
         (!shadow && (rc = ensure(c, c->vary, (size_t)nv * 2 * sizeof(float4)))))
         return rc;
+    const bool direct = fresh && !stoch && fits && nt <= kDirectTrisMost && launch_fits(grid.groups) &&
+                        launch_fits(grid.vblocks + clear_blocks((long long)px)) && direct_room(c, px, nt, no_nan);
     uint32_t n_frag = 0;
     if (direct) {
-        if ((rc = direct_pass(c, u, n_draws, grid, nt, shadow, no_nan, W, H))) return rc;
-    } else if ((rc = list_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, W, H, fresh, stoch, n_frag))) {
-        return rc;
+        direct_pass(c, u, n_draws, grid, nt, shadow, no_nan, W, H);
+    } else {
+        rc = list_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, W, H, fresh, stoch, n_frag);
+        if (rc == FGL_ERR_NOMEM && c->key.p) {   // with the direct rasteriser's memory given back
+            free_direct(c);
+            rc = list_pass(c, u, n_draws, max_pos, max_faces, nt, shadow, W, H, fresh, stoch, n_frag);
+        }
+        if (rc) return rc;
     }
     if (shadow) {
         c->pend_shadow = false;

@@ -89,6 +89,24 @@ def _geometry(ctx, draws, W, H, started=lambda: None):
     return ctx.read(F.TARGET_DEPTH).view(np.uint32), ctx.read(F.TARGET_GBUFFER).view(np.uint32)
 
 
+def test_pass_without_room_for_keys():
+    """The key plane of 4096 x 4096 pixels is 128 MiB, the lists' winners 64."""
+    W = H = 4096
+    with_room, without = F.Context(0), F.Context(0)
+    try:
+        out = []
+        for c, left in ((with_room, None), (without, 112 * MB)):
+            _, ground, sphere = _world(c, 64)
+            _geometry(c, _draws(ground, sphere), 64, 64)   # kernels loaded, small buffers there
+            print("pass with", "all memory" if left is None else f"{left // MB} MiB left", flush=True)
+            out.append(_geometry(c, _draws(ground, sphere), W, H, (lambda: Held(left)) if left else (lambda: None)))
+        for a, b in zip(*out):
+            assert np.array_equal(a, b)
+    finally:
+        with_room.close()
+        without.close()
+
+
 def test_upload_without_room_for_bundles():
     """A 4096 x 4096 bundle is 128 MiB; the maps by themselves do as well."""
     c = F.Context(0)
