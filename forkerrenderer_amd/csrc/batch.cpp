@@ -305,14 +305,35 @@ static int plan(fgl_batch *b)
                        launch_fits(vblocks + clear_blocks((long long)(p == kBvShadow ? spx : px)));
     }
     if (b->direct_ok) {
+        std::vector<uint2> db[2];
+        for (int p = 0; p < 2; ++p)
+            for (size_t k = 0; k < dd[p].size(); ++k) {
+                const uint32_t code = lane_code(dd[p][k], p);
+                for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256 / bv_lanes(code))
+                    db[p].push_back(make_uint2((uint32_t)k, (uint32_t)f0 | code << 30));
+            }
+        Buf *bufs[] = {&b->key, &b->big, &b->direct_ctr, &b->d_sblk_view, &b->d_dblocks[0], &b->d_dblocks[1]};
         if (grow(b->key, std::max(px, spx) * 8) || grow(b->big, (size_t)mt * 12) ||
-            grow(b->direct_ctr, 2 * sizeof(DirectCtr)) || grow(b->d_sblk_view, sblk_view.size() + 1))
-            return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
-        launch_fill_u32((uint32_t *)b->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, ctx_stream(c));
-        if (!sblk_view.empty() &&
-            hipMemcpy(b->d_sblk_view.p, sblk_view.data(), sblk_view.size(), hipMemcpyHostToDevice))
-            return bfail(b, FGL_ERR_DEVICE, "upload failed");
-        b->n_sblocks = (uint32_t)sblk_view.size();
+            grow(b->direct_ctr, 2 * sizeof(DirectCtr)) || grow(b->d_sblk_view, sblk_view.size() + 1) ||
+            grow(b->d_dblocks[0], (db[0].size() + 1) * sizeof(uint2)) ||
+            grow(b->d_dblocks[1], (db[1].size() + 1) * sizeof(uint2))) {
+            // no room: the tile lists need none of these
+            (void)hipGetLastError();
+            for (Buf *x : bufs) release(*x);
+            b->direct_ok = false;
+        } else {
+            launch_fill_u32((uint32_t *)b->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, ctx_stream(c));
+            if (!sblk_view.empty() &&
+                hipMemcpy(b->d_sblk_view.p, sblk_view.data(), sblk_view.size(), hipMemcpyHostToDevice))
+                return bfail(b, FGL_ERR_DEVICE, "upload failed");
+            for (int p = 0; p < 2; ++p) {
+                b->n_dblocks[p] = (int)db[p].size();
+                if (!db[p].empty() &&
+                    hipMemcpy(b->d_dblocks[p].p, db[p].data(), db[p].size() * sizeof(uint2), hipMemcpyHostToDevice))
+                    return bfail(b, FGL_ERR_DEVICE, "upload failed");
+            }
+            b->n_sblocks = (uint32_t)sblk_view.size();
+        }
     }
     for (int p = 0; p < 2; ++p) {
         std::vector<uint2> vb, fb;
@@ -320,17 +341,6 @@ static int plan(fgl_batch *b)
             for (int v0 = 0; v0 < dd[p][k].n_pos; v0 += 256) vb.push_back(make_uint2((uint32_t)k, (uint32_t)v0));
             for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256) fb.push_back(make_uint2((uint32_t)k, (uint32_t)f0));
         }
-        std::vector<uint2> db;
-        for (size_t k = 0; b->direct_ok && k < dd[p].size(); ++k) {
-            const uint32_t code = lane_code(dd[p][k], p);
-            for (int f0 = 0; f0 < dd[p][k].n_faces; f0 += 256 / bv_lanes(code))
-                db.push_back(make_uint2((uint32_t)k, (uint32_t)f0 | code << 30));
-        }
-        b->n_dblocks[p] = (int)db.size();
-        if (grow(b->d_dblocks[p], (db.size() + 1) * sizeof(uint2)))
-            return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
-        if (!db.empty() && hipMemcpy(b->d_dblocks[p].p, db.data(), db.size() * sizeof(uint2), hipMemcpyHostToDevice))
-            return bfail(b, FGL_ERR_DEVICE, "upload failed");
         b->n_vblocks[p] = (int)vb.size();
         b->n_fblocks[p] = (int)fb.size();
         if (grow(b->d_vblocks[p], (vb.size() + 1) * sizeof(uint2)) || grow(b->d_fblocks[p], (fb.size() + 1) * sizeof(uint2)))

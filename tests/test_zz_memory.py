@@ -122,3 +122,38 @@ def test_upload_without_room_for_bundles():
         assert all(np.array_equal(x, y) for x, y in zip(a, b))
     finally:
         c.close()
+
+
+def test_batch_without_room_for_keys():
+    """A batch planned with room for all but its key plane renders through the
+    lists, in every replay."""
+    hip = _hip()
+    c = F.Context(0)
+    try:
+        _, ground, sphere = _world(c, 64)
+        view = VW.View(4096, 3072, (0.3, 1.5, 3.2), (0.0, -0.2, 0.0), _draws(ground, sphere),
+                       [(0, (2.0, 5.0, 5.0), (3.0, 3.0, 3.0))], VW.pcf_grid(3), 1024)
+
+        def render(b):
+            out = []
+            for _ in range(3):
+                b.render()
+                assert b.sync() == 0
+                out.append([b.read(0, t) for t in (F.TARGET_DEPTH, F.TARGET_IMAGE, F.TARGET_SHADOW)])
+            b.close()
+            for later in out[1:]:
+                assert all(np.array_equal(x, y) for x, y in zip(out[0], later))
+            return out[0]
+
+        c.sync()
+        before = _free(hip)
+        b = VW.Batch(c, [view])
+        took = before - _free(hip)
+        want = render(b)
+        print(f"batch of {took // MB} MiB with {(took - 48 * MB) // MB} MiB left", flush=True)
+        with Held(took - 48 * MB):
+            b = VW.Batch(c, [view])
+        got = render(b)
+        assert all(np.array_equal(x, y) for x, y in zip(want, got))
+    finally:
+        c.close()
