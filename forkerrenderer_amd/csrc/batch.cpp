@@ -634,6 +634,7 @@ int fgl_render_view(fgl_ctx *c, const fgl_view_desc *v, int ao_mode, fgl_nao *na
     if (ao_mode == FGL_AO_NEURAL && !nao) return ctx_fail(c, FGL_ERR_INVALID, "neural AO needs a network");
     int rc;
     if ((rc = check_view(c, *v))) return rc;
+    ctx_begin_frame(c, v->width, v->height);
     // DoShadowPass (render.cpp:60-97)
     if ((rc = apply_view_state(c, *v, true))) return rc;
     if (v->shadow_on) {

@@ -106,6 +106,7 @@ struct fgl_ctx {
     // the direct rasteriser: pixel keys, NaN plane (all ones between passes),
     // large triangles, two passes' counters used in turn
     DevBuf key, key_nan, big, direct_ctr;
+    size_t frame_px = 0;   // pixels of the frame begun, where its size is known before the shadow pass
     int direct_turn = 0;
     // forward pass with a stochastic shadow filter: per-pixel passing counts
     // (+ scan scratch), the passing fragments (triangle ids then pixels) and
@@ -1343,9 +1344,12 @@ static void free_direct(fgl_ctx *c)
 // take the pass.
 static bool direct_room(fgl_ctx *c, size_t px, long long nt, bool no_nan)
 {
+    // a shadow pass already takes what its frame's main pass will: growing the
+    // planes between them waits for the stream and frees
+    const size_t most = px > c->frame_px ? px : c->frame_px;
     const size_t nan_cap = c->key_nan.cap;
     const bool first = !c->direct_ctr.p;
-    if (room(c, c->key, px * 8) && room(c, c->big, (size_t)nt * 12) && room(c, c->direct_ctr, 2 * sizeof(DirectCtr)) &&
+    if ((room(c, c->key, most * 8) || room(c, c->key, px * 8)) && room(c, c->big, (size_t)nt * 12) && room(c, c->direct_ctr, 2 * sizeof(DirectCtr)) &&
         (no_nan || room(c, c->key_nan, px * 8))) {
         if (first) launch_fill_u32((uint32_t *)c->direct_ctr.p, 0u, 2 * sizeof(DirectCtr) / 4, c->stream);
         if (c->key_nan.cap != nan_cap)
@@ -2136,6 +2140,8 @@ int ctx_draw_record(fgl_ctx *c, int model, const float M[16], DevDraw *out)
     return FGL_OK;
 }
 
+void ctx_begin_frame(fgl_ctx *c, int w, int h) { c->frame_px = (size_t)w * h; }
+
 bool ctx_depths_finite(fgl_ctx *c, int model, const float M[16], bool shadow)
 {
     const ClipBound cam = camera_bound(c, shadow);
@@ -2310,6 +2316,7 @@ int fgl_render_scene(fgl_ctx *c, fgl_scene *sc)
     const float ratio = (float)I.width / I.height;
     // Preconfigure (render.cpp:33-38)
     fgl_set_viewport(c, 0, 0, 0, W, H);
+    c->frame_px = (size_t)W * H;
     const int S = I.shadow_map_size > 0 ? I.shadow_map_size : 0;
     fgl_set_viewport(c, 1, 0, 0, S ? S : W, S ? S : H);
     fgl_set_lights(c, I.n_lights, I.lights);

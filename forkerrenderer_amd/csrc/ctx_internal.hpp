@@ -37,6 +37,9 @@ void ctx_uniforms(fgl_ctx *c, FrameUniforms *u);
 // light-space matrix: geometry pointers, normal matrix, light * model.  The
 // pass-wide bases (vert_base, tri_base) and the view index are left zero.
 int ctx_draw_record(fgl_ctx *c, int model, const float M[16], DevDraw *out);
+// The size of the frame that the passes to come make: its shadow pass makes room
+// for its main pass.
+void ctx_begin_frame(fgl_ctx *c, int w, int h);
 // Whether every window depth of `model` under M is finite, in the shadow or
 // the main pass of the context's current matrices (then no fragment's depth
 // is NaN).
