@@ -44,8 +44,7 @@ __global__ __launch_bounds__(256) void k_bv_vertex(const DevDraw *__restrict__ d
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        const size_t v = (size_t)dr.vert_base + vi;
-        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_vertex_pass(dr, u, vi, vary));
     }
 }
 
@@ -183,8 +182,7 @@ __global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const 
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        const size_t v = (size_t)dr.vert_base + vi;
-        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_vertex_pass(dr, u, vi, vary));
     }
 }
 
@@ -259,7 +257,7 @@ __device__ __forceinline__ bool bv_pixel(const BvPixelArgs &a, int &vi, int &x, 
     return x < v.W && y < v.H;
 }
 
-template <bool DIRECT>
+template <bool DIRECT, bool CORNER>
 __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
 {
     int vi, x, y;
@@ -285,7 +283,7 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     a.textures = b.textures;
     a.shadow_map = nullptr;
     a.ss = ShadowSamples{};
-    gbuffer_px<DIRECT>(a, v.u, x, y);
+    gbuffer_px<DIRECT, CORNER>(a, v.u, x, y);
     // last: a store before them would keep the loads above from their scalar form
     if (DIRECT && blockIdx.x == 0 && threadIdx.x == 0) *b.ctr = DirectCtr{0ull, 0u, 0u};
 }
@@ -408,8 +406,10 @@ void launch_bv_direct_shadow(const BvDirectArgs &a, const uint8_t *sblk_view, ui
 void launch_bv_gbuffer(const BvPixelArgs &a, hipStream_t s)
 {
     if (!a.n_blocks) return;
-    if (a.key) hipLaunchKernelGGL(k_bv_gbuffer<true>, dim3(a.n_blocks), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(k_bv_gbuffer<false>, dim3(a.n_blocks), dim3(256), 0, s, a);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(a.n_blocks), dim3(256), 0, s, a); };
+    if (!a.key) go(k_bv_gbuffer<false, false>);
+    else if (a.vary) go(k_bv_gbuffer<true, false>);
+    else go(k_bv_gbuffer<true, true>);
 }
 
 void launch_bv_lighting(const BvPixelArgs &a, int mode, hipStream_t s)

@@ -78,7 +78,7 @@ struct BvPixelArgs {
     uint32_t n_blocks;
     const int4 *screen;
     const int4 *tri_v;
-    const float4 *vary;       // the main vertex pass's varyings
+    const float4 *vary;       // the main vertex pass's varyings; null: made from the corner records
     const int *vis;
     const unsigned long long *key;   // the direct rasteriser's keys instead of vis (null: vis)
     float *depth;                    // with key: written by the resolve

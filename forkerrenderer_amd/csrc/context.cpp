@@ -35,7 +35,7 @@ struct ModelRes {
     float *pos = nullptr, *uv = nullptr, *nrm = nullptr, *tan = nullptr;
     int *vi = nullptr, *ti = nullptr, *ni = nullptr, *fmat = nullptr;
     int4 *tri = nullptr;       // the faces in spatial order
-    float *corner = nullptr;   // per face corner: uv, normal, tangent (8 floats)
+    float *corner = nullptr;   // per face corner: uv, normal, tangent, position (12 floats)
     int n_pos = 0, n_faces = 0;
     bool has_tan = false, pbr = false;
     // extent of the faces' corners and the longest face edge; bounded: they
@@ -674,8 +674,8 @@ int fgl_upload_model(fgl_ctx *c, const fgl_model_desc *d, int *out_id)
     if ((rc = upload_array(c, &m.ti, (const int *)d->ti, 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.ni, (const int *)d->ni, 3 * nf))) return rc;
     if ((rc = upload_array(c, &m.fmat, (const int *)d->face_material, nf))) return rc;
-    HIPCHK(c, hipMalloc((void **)&m.corner, (nf ? 3 * nf * 8 : 1) * sizeof(float)));
-    launch_corners(m.uv, m.nrm, m.tan, m.vi, m.ti, m.ni, 3 * nf, (float4 *)m.corner, c->stream);
+    HIPCHK(c, hipMalloc((void **)&m.corner, (nf ? 3 * nf * 12 : 1) * sizeof(float)));
+    launch_corners(m.pos, m.uv, m.nrm, m.tan, m.vi, m.ti, m.ni, 3 * nf, (float4 *)m.corner, c->stream);
     HIPCHK(c, hipGetLastError());
     for (int k = 0; k < 3; ++k) {
         m.lo[k] = HUGE_VAL;
@@ -1331,6 +1331,7 @@ static void bound_pass(const fgl_ctx *c, bool shadow, long long nt, int W, int H
 struct DirectGrid {
     int lanes;
     long long groups, vblocks;
+    bool corner;   // varyings from the corner records (corner_form)
 };
 
 static void free_direct(fgl_ctx *c)
@@ -1384,7 +1385,7 @@ static void direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const D
     {
         KernelTimer t(c, "vertex");
         launch_direct_vertex(shadow, (int)g.vblocks, u, (int4 *)c->screen.p,
-                             shadow ? (float *)c->ndc_z.p : nullptr, shadow ? nullptr : (float4 *)c->vary.p, a,
+                             shadow ? (float *)c->ndc_z.p : nullptr, g.corner || shadow ? nullptr : (float4 *)c->vary.p, a,
                              ctr + c->direct_turn, c->stream);
     }
     KernelTimer t(c, shadow ? "raster_shadow" : "raster");
@@ -1553,7 +1554,7 @@ static int flush_pass(fgl_ctx *c)
     long long nt = 0, nv = 0, tris = 0;
     int max_pos = 0, max_faces = 0;
     for (const fgl_ctx::Rec &r : c->draws) tris += c->models[r.model].n_faces;
-    DirectGrid grid = {direct_lanes(tris), 0, 0};
+    DirectGrid grid = {direct_lanes(tris), 0, 0, corner_form((long long)W * H, tris)};
     for (size_t i = 0; i < c->draws.size(); ++i) {
         const ModelRes &m = c->models[c->draws[i].model];
         DevDraw &d = dd[i];
@@ -1639,7 +1640,7 @@ static int flush_pass(fgl_ctx *c)
         r.n_draws = n_draws;
         r.screen = (const int4 *)c->screen.p;
         r.tri_v = (const int4 *)c->tri_v.p;
-        r.vary = (const float4 *)c->vary.p;
+        r.vary = direct && grid.corner ? nullptr : (const float4 *)c->vary.p;
         r.vis = (const int *)c->vis.p;
         if (direct) {
             r.key = (unsigned long long *)c->key.p;

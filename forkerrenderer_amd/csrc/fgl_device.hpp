@@ -47,10 +47,10 @@ struct DevMaterial {
 struct DevDraw {
     const float *pos, *uv, *nrm, *tan;
     const int *vi, *ti, *ni, *face_mat;
-    // per face corner (3 per face), the attributes the main vertex programs
-    // read beside the position, interleaved as 2 float4: (uv, n.xy), (n.z,
-    // t.xyz), the normal and tangent normalised as ProcessVertex does -- one
-    // 32-byte record instead of three arrays behind three index streams
+    // per face, the attributes the main vertex programs read, 9 float4: for
+    // each corner (uv, n.xy), (n.z, t.xyz), the normal and tangent normalised as
+    // ProcessVertex does, then the three positions (corner_form alone reads
+    // them) -- one 144-byte record instead of four arrays behind three index streams
     const float4 *corner;
     // the faces in spatial order: position indices (as vi) and the face
     const int4 *tri;
@@ -253,16 +253,10 @@ struct Varying {
 };
 
 // BlinnPhong/PBR/G ProcessVertex (phongshader.h:35-85, pbrshader.h:35-85,
-// gshader.h:41-92), the part that depends on the position alone: made once a
-// vertex by the vertex pass (its NDC, and the varyings as two float4:
-// position / w and 1 / w, light NDC / w), where the resolves used to make it
-// for every corner of every pixel (some 120 operations each; 24-view batch
-// G-buffer 671 -> 628 us, 957 x 603 2x forward resolve 159 -> 154, 1920 x 1080
-// G-buffer 73 -> 65; where faces are a few pixels large the resolve is bound by
-// its gathers and stays as it was).
-__device__ __forceinline__ Vec4 main_position(const DevDraw &d, const FrameUniforms &u, int vi, float4 &v0, float4 &v1)
+// gshader.h:41-92), the part that depends on the position p alone: its NDC, and
+// the varyings as two float4 (position / w and 1 / w, light NDC / w).
+__device__ __forceinline__ Vec4 main_position(const DevDraw &d, const FrameUniforms &u, Vec4 p, float4 &v0, float4 &v1)
 {
-    Vec4 p = vec4(d.pos[3 * vi], d.pos[3 * vi + 1], d.pos[3 * vi + 2], 1.f);
     Vec4 ws = mv4(d.model, p);
     Vec4 cs = mv4(u.proj, mv4(u.view, ws));
     Vec4 l = vec4(0.f, 0.f, 0.f, 0.f);
@@ -278,13 +272,39 @@ __device__ __forceinline__ Vec4 main_position(const DevDraw &d, const FrameUnifo
     return divs4(cs, cs.w);
 }
 
+// main_position of vertex vi; vary (v0, v1 of each vertex; null where the
+// resolve makes them, corner_form) also takes its varyings.
+__device__ __forceinline__ Vec4 main_vertex_pass(const DevDraw &d, const FrameUniforms &u, int vi, float4 *vary)
+{
+    float4 v0, v1;
+    const Vec4 ndc = main_position(d, u, vec4(d.pos[3 * vi], d.pos[3 * vi + 1], d.pos[3 * vi + 2], 1.f), v0, v1);
+    if (vary) {
+        const size_t v = 2 * ((size_t)d.vert_base + vi);
+        vary[v] = v0;
+        vary[v + 1] = v1;
+    }
+    return ndc;
+}
+
 // Corner k of face f, a corner at vertex v of the pass's varyings, with its
 // attributes as Mesh::TexCoord / Normal / Tangent fetch them (mesh.cpp:34-56).
-__device__ __forceinline__ Varying main_vertex(const DevDraw &d, const float4 *vary, int v, int f, int k)
+// CORNER: the varyings made here from the position in the corner's record
+// (corner_form, pass_plan.hpp) instead of read from the vertex pass's.
+template <bool CORNER>
+__device__ __forceinline__ Varying main_vertex(const DevDraw &d, const FrameUniforms &u, const float4 *vary, int v, int f,
+                                               int k)
 {
     Varying o;
-    const float4 *r = d.corner + (size_t)(3 * f + k) * 2;
-    const float4 r0 = r[0], r1 = r[1], p0 = vary[2 * (size_t)v], p1 = vary[2 * (size_t)v + 1];
+    const float4 *face = d.corner + (size_t)f * 9;
+    const float4 r0 = face[2 * k], r1 = face[2 * k + 1];
+    float4 p0, p1;
+    if (CORNER) {
+        const float4 r2 = face[6 + k];
+        (void)main_position(d, u, vec4(r2.x, r2.y, r2.z, 1.f), p0, p1);
+    } else {
+        p0 = vary[2 * (size_t)v];
+        p1 = vary[2 * (size_t)v + 1];
+    }
     const float oow = p0.w;
     o.ws = vec3(p0.x, p0.y, p0.z);
     o.lndc = vec3(p1.x, p1.y, p1.z);

@@ -83,7 +83,7 @@ struct ResolveArgs {
     float clear[3];            // forward pass background colour
     float *gbuf;               // 19 planes (geometry pass)
     float *fb;                 // 3 planes (forward pass)
-    const float4 *vary;        // the vertex pass's varyings (main_position)
+    const float4 *vary;        // the vertex pass's varyings; null: made from the corner records
     const DevMaterial *materials;
     const DevTexture *textures;
     const float *shadow_map;
@@ -144,10 +144,10 @@ struct SsaoArgs {
 void launch_bundle(int w, int h, const uint32_t *a, const uint8_t *z, const uint32_t *n, const uint8_t *y, uint2 *out,
                    hipStream_t s);
 // The corner records of a model from its attribute arrays (tan may be null).
-void launch_corners(const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti, const int *ni,
+void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti, const int *ni,
                     size_t n, float4 *out, hipStream_t s);
 // Window records of every (draw, position); shadow pass: also the NDC z of
-// each vertex into ndc_z, main passes: its varyings into vary; zero (may be
+// each vertex into ndc_z, main passes: its varyings into vary (may be null); zero (may be
 // null): a word set to 0 on the way.
 void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, const FrameUniforms &u, int4 *out,
                    float *ndc_z, float4 *vary, uint32_t *zero, hipStream_t s);

@@ -12,6 +12,20 @@ constexpr bool launch_fits(long long blocks) { return blocks <= kMaxBlocks; }
 constexpr long long kDirectTris16 = 32768, kDirectTris4 = 262144;
 constexpr int direct_lanes(long long n_tri) { return n_tri <= kDirectTris16 ? 16 : n_tri <= kDirectTris4 ? 4 : 1; }
 
+// Whether a main pass's resolve makes the varyings that depend on a position
+// from the corner records, instead of reading what the vertex pass made of each
+// vertex.  Where faces are a pixel or two, a pixel's three corners are gathers of
+// their own: the corner records (one more line, some 120 operations a corner)
+// cost less than the vertices' (three more lines), and the vertex pass writes 32
+// bytes a vertex less.  Where more pixels share a vertex it is the other way.
+// G-buffer resolve and main vertex pass, from vertices / from corners, us:
+// 3840 x 2160, 64 objects of 81,920 faces (1.6 pixels a face) 297 / 250, 1920 x
+// 1080 (0.4) 108 / 76; 25 objects, 3840 x 2160 (4) 248 / 222.  With shadows, whose
+// light positions add to a corner's operations: 3840 x 2160 frame (1.6) 1,450 /
+// 1,413; 1280 x 800 (3.1) 329 / 330; 24 views (5.4) 3,099 / 3,136; 1914 x 1206
+// forward (13) 326 / 334.
+constexpr bool corner_form(long long pixels, long long n_tri) { return pixels < 2 * n_tri; }
+
 // Items (64 x 16 pixels) of large triangles that cover targets of so many pixels
 // three times over.
 constexpr long long deep_items(long long pixels) { return 3 * (pixels / 1024 + 1); }

@@ -25,9 +25,9 @@
 namespace fgl {
 
 // A model's corner records (DevDraw::corner), a thread per corner: gathered
-// here, not built on the host and copied (96 bytes a face).
-__global__ __launch_bounds__(256) void k_corners(const float *__restrict__ uv, const float *__restrict__ nrm,
-                                                 const float *__restrict__ tan, const int *__restrict__ vi,
+// here, not built on the host and copied (144 bytes a face).
+__global__ __launch_bounds__(256) void k_corners(const float *__restrict__ pos, const float *__restrict__ uv,
+                                                 const float *__restrict__ nrm, const float *__restrict__ tan, const int *__restrict__ vi,
                                                  const int *__restrict__ ti, const int *__restrict__ ni, size_t n,
                                                  float4 *__restrict__ out)
 {
@@ -40,8 +40,11 @@ __global__ __launch_bounds__(256) void k_corners(const float *__restrict__ uv, c
         const float *g = tan + 3 * (size_t)vi[k];
         tt = norm3(vec3(g[0], g[1], g[2]));
     }
-    out[2 * k] = make_float4(t[0], t[1], nn.x, nn.y);
-    out[2 * k + 1] = make_float4(nn.z, tt.x, tt.y, tt.z);
+    const float *p = pos + 3 * (size_t)vi[k];
+    const size_t f = k / 3, c = k - 3 * f;
+    out[9 * f + 2 * c] = make_float4(t[0], t[1], nn.x, nn.y);
+    out[9 * f + 2 * c + 1] = make_float4(nn.z, tt.x, tt.y, tt.z);
+    out[9 * f + 6 + c] = make_float4(p[0], p[1], p[2], 0.f);
 }
 
 // A bundle's texels (DevBundle) from its maps' own, a thread per texel in the
@@ -77,8 +80,7 @@ __global__ __launch_bounds__(256) void k_vertex(const DevDraw *__restrict__ draw
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        const size_t v = (size_t)dr.vert_base + vi;
-        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_vertex_pass(dr, u, vi, vary));
     }
 }
 
@@ -224,8 +226,7 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        const size_t v = (size_t)dr.vert_base + vi;
-        out[v] = to_screen(u.viewport, main_position(dr, u, vi, vary[2 * v], vary[2 * v + 1]));
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_vertex_pass(dr, u, vi, vary));
     }
 }
 
@@ -286,27 +287,27 @@ __global__ __launch_bounds__(256) void k_direct_shadow(DirectArgs a, const float
     if (w.mark) a.fix[i] = ~0ull;
 }
 
-template <bool DIRECT>
+template <bool DIRECT, bool CORNER>
 __global__ __launch_bounds__(256) void k_gbuffer_resolve(ResolveArgs a, FrameUniforms u)
 {
     int x, y;
     grid_px<32>(x, y);
     if (x >= a.W || y >= a.H) return;
-    gbuffer_px<DIRECT>(a, u, x, y);
+    gbuffer_px<DIRECT, CORNER>(a, u, x, y);
 }
 
 // Forward pass resolve: BlinnPhongShader / PBRShader::ProcessFragment
 // (phongshader.h:90-169, pbrshader.h:90-180) once for the visible fragment.
 // The forward fragment program for the winner (face f of draw dr, material
 // m, barycentrics b) at pixel i.
-template <bool STREAM, int MODE>
+template <bool STREAM, bool CORNER, int MODE>
 __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameUniforms &u, const DevDraw &dr,
                                               const DevMaterial &m, int f, const int4 &tv, const Vec3 &b, size_t i,
                                               size_t P)
 {
-    Varying v0 = main_vertex(dr, a.vary, tv.x, f, 0);
-    Varying v1 = main_vertex(dr, a.vary, tv.y, f, 1);
-    Varying v2 = main_vertex(dr, a.vary, tv.z, f, 2);
+    Varying v0 = main_vertex<CORNER>(dr, u, a.vary, tv.x, f, 0);
+    Varying v1 = main_vertex<CORNER>(dr, u, a.vary, tv.y, f, 1);
+    Varying v2 = main_vertex<CORNER>(dr, u, a.vary, tv.z, f, 2);
     const DevBundle &bn = m.bundle[dr.support_pbr ? 1 : 0];
     FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, bn);
     // the stochastic shadow filters: this fragment's samples in the stream
@@ -345,7 +346,7 @@ __device__ __forceinline__ void forward_shade(const ResolveArgs &a, const FrameU
 
 // Forward resolve, one thread per pixel; draw and material records through
 // readfirstlane when the wavefront shares them (as in gbuffer_px).
-template <bool STREAM, bool DIRECT, int MODE>
+template <bool STREAM, bool DIRECT, bool CORNER, int MODE>
 __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUniforms u)
 {
     int x, y;
@@ -370,14 +371,14 @@ __global__ __launch_bounds__(256) void k_forward_resolve(ResolveArgs a, FrameUni
         const int mi = dr.face_mat[f];
         const int m0 = __builtin_amdgcn_readfirstlane(mi);
         if (__ballot(mi != m0) == 0ull) {
-            forward_shade<STREAM, MODE>(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
+            forward_shade<STREAM, CORNER, MODE>(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
             resolve_end<DIRECT>(a, i, w);
             return;
         }
     }
     const DevDraw &dr = a.draws[w.tv.w];
     const int f = w.g - dr.tri_base;
-    forward_shade<STREAM, MODE>(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
+    forward_shade<STREAM, CORNER, MODE>(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
     resolve_end<DIRECT>(a, i, w);
 }
 
@@ -485,9 +486,9 @@ __global__ __launch_bounds__(256) void k_frag_shadow_inputs(ResolveArgs a, Frame
     const DevDraw &dr = a.draws[tv.w];
     const int f = g - dr.tri_base;
     const DevMaterial &m = a.materials[dr.face_mat[f]];
-    Varying v0 = main_vertex(dr, a.vary, tv.x, f, 0);
-    Varying v1 = main_vertex(dr, a.vary, tv.y, f, 1);
-    Varying v2 = main_vertex(dr, a.vary, tv.z, f, 2);
+    Varying v0 = main_vertex<false>(dr, u, a.vary, tv.x, f, 0);
+    Varying v1 = main_vertex<false>(dr, u, a.vary, tv.y, f, 1);
+    Varying v2 = main_vertex<false>(dr, u, a.vary, tv.z, f, 2);
     const FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, m.bundle[dr.support_pbr ? 1 : 0]);
     const size_t N = n;
     out[k] = fg.normal.x;
@@ -534,11 +535,11 @@ void launch_vertex(bool shadow, const DevDraw *draws, int n_draws, int max_pos, 
     else hipLaunchKernelGGL(k_vertex<false>, grid, dim3(256), 0, s, draws, u, out, ndc_z, vary, zero);
 }
 
-void launch_corners(const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti, const int *ni,
+void launch_corners(const float *pos, const float *uv, const float *nrm, const float *tan, const int *vi, const int *ti, const int *ni,
                     size_t n, float4 *out, hipStream_t s)
 {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_corners, dim3(blocks_for(n, 256)), dim3(256), 0, s, uv, nrm, tan, vi, ti, ni, n, out);
+    hipLaunchKernelGGL(k_corners, dim3(blocks_for(n, 256)), dim3(256), 0, s, pos, uv, nrm, tan, vi, ti, ni, n, out);
 }
 
 void launch_bundle(int w, int h, const uint32_t *a, const uint8_t *z, const uint32_t *n, const uint8_t *y, uint2 *out,
@@ -644,8 +645,10 @@ void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth,
 void launch_gbuffer_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s)
 {
     if (a.W <= 0 || a.H <= 0) return;
-    if (a.key) hipLaunchKernelGGL(k_gbuffer_resolve<true>, grid2(a.W, a.H), dim3(256), 0, s, a, u);
-    else hipLaunchKernelGGL(k_gbuffer_resolve<false>, grid2(a.W, a.H), dim3(256), 0, s, a, u);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid2(a.W, a.H), dim3(256), 0, s, a, u); };
+    if (!a.key) go(k_gbuffer_resolve<false, false>);
+    else if (a.vary) go(k_gbuffer_resolve<true, false>);
+    else go(k_gbuffer_resolve<true, true>);
 }
 
 void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s)
@@ -653,14 +656,24 @@ void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStr
     if (a.W <= 0 || a.H <= 0) return;
     const dim3 g = grid2(a.W, a.H);
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, g, dim3(256), 0, s, a, u); };
-    if (a.ss.sv.v) return go(k_forward_resolve<true, false, -1>);
-    if (!a.key) return go(k_forward_resolve<false, false, -1>);
-    switch (u.shadow_on ? u.shadow.mode : 0) {
-    case 0: return go(k_forward_resolve<false, true, 0>);
-    case 1: return go(k_forward_resolve<false, true, 1>);
-    case 2: return go(k_forward_resolve<false, true, 2>);
-    case 3: return go(k_forward_resolve<false, true, 3>);
-    default: return go(k_forward_resolve<false, true, -1>);
+    if (a.ss.sv.v) return go(k_forward_resolve<true, false, false, -1>);
+    if (!a.key) return go(k_forward_resolve<false, false, false, -1>);
+    const int mode = u.shadow_on ? u.shadow.mode : 0;
+    if (a.vary) {
+        switch (mode) {
+        case 0: return go(k_forward_resolve<false, true, false, 0>);
+        case 1: return go(k_forward_resolve<false, true, false, 1>);
+        case 2: return go(k_forward_resolve<false, true, false, 2>);
+        case 3: return go(k_forward_resolve<false, true, false, 3>);
+        default: return go(k_forward_resolve<false, true, false, -1>);
+        }
+    }
+    switch (mode) {
+    case 0: return go(k_forward_resolve<false, true, true, 0>);
+    case 1: return go(k_forward_resolve<false, true, true, 1>);
+    case 2: return go(k_forward_resolve<false, true, true, 2>);
+    case 3: return go(k_forward_resolve<false, true, true, 3>);
+    default: return go(k_forward_resolve<false, true, true, -1>);
     }
 }
 

@@ -880,14 +880,15 @@ __device__ __forceinline__ void resolve_end(const ResolveArgs &a, size_t i, cons
 // GShader::ProcessFragment + the seven buffer writes (gshader.h:95-202,
 // forkergl.cpp:211-223) for the winner (face f of draw dr, material m,
 // barycentrics b) at pixel i: the 19 G-buffer planes.
+template <bool CORNER>
 __device__ __forceinline__ void gbuffer_shade(const ResolveArgs &a, const FrameUniforms &u, const DevDraw &dr,
                                               const DevMaterial &m, int f, const int4 &tv, const Vec3 &b, size_t i,
                                               size_t P)
 {
     float *gb = a.gbuf;
-    Varying v0 = main_vertex(dr, a.vary, tv.x, f, 0);
-    Varying v1 = main_vertex(dr, a.vary, tv.y, f, 1);
-    Varying v2 = main_vertex(dr, a.vary, tv.z, f, 2);
+    Varying v0 = main_vertex<CORNER>(dr, u, a.vary, tv.x, f, 0);
+    Varying v1 = main_vertex<CORNER>(dr, u, a.vary, tv.y, f, 1);
+    Varying v2 = main_vertex<CORNER>(dr, u, a.vary, tv.z, f, 2);
     const DevBundle &bn = m.bundle[dr.support_pbr ? 1 : 0];
     FragGeom fg = frag_geometry(dr, u, a.textures, v0, v1, v2, b, m.map_bump, bn);
     Vec3 albedo, emissive, param;
@@ -937,7 +938,7 @@ __device__ __forceinline__ void gbuffer_shade(const ResolveArgs &a, const FrameU
 // descriptors) come in as scalar loads instead of one vector load per field.
 // DIRECT: winners come from the direct rasteriser's keys, and the depth
 // target is written here.
-template <bool DIRECT>
+template <bool DIRECT, bool CORNER>
 __device__ __forceinline__ void gbuffer_px(const ResolveArgs &a, const FrameUniforms &u, int x, int y)
 {
     const size_t i = (size_t)x + (size_t)y * a.W;
@@ -957,14 +958,14 @@ __device__ __forceinline__ void gbuffer_px(const ResolveArgs &a, const FrameUnif
         const int mi = dr.face_mat[f];
         const int m0 = __builtin_amdgcn_readfirstlane(mi);
         if (__ballot(mi != m0) == 0ull) {
-            gbuffer_shade(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
+            gbuffer_shade<CORNER>(a, u, dr, a.materials[m0], f, w.tv, w.b, i, P);
             resolve_end<DIRECT>(a, i, w);
             return;
         }
     }
     const DevDraw &dr = a.draws[w.tv.w];
     const int f = w.g - dr.tri_base;
-    gbuffer_shade(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
+    gbuffer_shade<CORNER>(a, u, dr, a.materials[dr.face_mat[f]], f, w.tv, w.b, i, P);
     resolve_end<DIRECT>(a, i, w);
 }
 

@@ -147,3 +147,20 @@ def test_batch_after_tables_and_ao_buffers_move(ctx, world, scene_dir):
         assert b.sync() == 0
         check(b, views, singles, f"after activation move, replay {rep}")
     b.close()
+
+
+def test_batch_of_dense_meshes(ctx):
+    """Fewer than two pixels a face over all views: replays make the varyings
+    from the corner records, the measuring render from the vertices'."""
+    views = VW.uneven_views(ctx, n_views=4, seed=17, subdivs=(4, 5), min_px=40 * 40, max_px=80 * 80, shadow_size=64, tex=32)
+    singles = []
+    for view in views:
+        VW.render_view(ctx, view)
+        singles.append({t: ctx.read(t).copy() for t in TARGETS})
+    b = VW.Batch(ctx, views)
+    assert b.stats()["pixels"] < 2 * b.stats()["tris_main"]
+    for rep in range(3):
+        b.render()
+        assert b.sync() == 0
+        check(b, views, singles, f"dense, render {rep}")
+    b.close()

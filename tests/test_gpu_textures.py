@@ -106,3 +106,21 @@ def test_grid_filter_sizes(ctx, scene_dir, mode, grid):
     assert_bitexact("shadow", got["shadow"], want["shadow"])
     mx, frac = lsb_stats(got["image"], want["image"])
     assert frac >= 0.999, (mx, frac)
+
+
+@pytest.mark.parametrize("shadow", ["hard", "pcf", "pcss", "grid"])
+@pytest.mark.parametrize("mode,pbr", [("deferred", True), ("deferred", False), ("forward", True), ("forward", False)])
+def test_dense_meshes(ctx, scene_dir, mode, pbr, shadow):
+    """Frames of fewer than two pixels a face, whose resolve makes the varyings
+    from the corner records, per mode, shading and shadow filter."""
+    p = G.tiny_scene(os.path.join(scene_dir, f"dense_{mode}_{pbr}_{shadow}"), seed=65, width=97, height=61, subdiv=5, tex=16,
+                     mode=mode, pbr=pbr, shadow=shadow)
+    sc = F.Scene(p)
+    print(f"dense: {mode} pbr {pbr} {shadow}", flush=True)
+    got = gpu_frame(ctx, sc, 16)
+    want = oracle_frame(sc)
+    assert_bitexact("depth", got["depth"], want["depth"])
+    if mode == "deferred":
+        assert_bitexact("gbuf", got["gbuf"], want["gbuf"])
+    mx, frac = lsb_stats(got["image"], want["image"])
+    assert frac >= 0.999, (mx, frac)
