@@ -288,13 +288,12 @@ static int plan(fgl_batch *b)
         grow(b->big_list, (size_t)mt * 4) || grow(b->tile_start, (size_t)mtiles * 4) ||
         grow(b->tile_end, (size_t)mtiles * 4) || grow(b->counters, 256))
         return bfail(b, FGL_ERR_NOMEM, "batch allocation failed");
-    // triangle groups of the direct rasteriser: lanes per triangle by the
-    // pixels the draw's view has for it
+    // triangle groups of the direct rasteriser: lanes by the draw and its view
     auto lane_code = [&](const DevDraw &d, int p) {
         const DevView &v = b->hv[d.view];
-        const double area = p == kBvShadow ? (double)v.S * v.S : (double)v.W * v.H;
-        const double per = area / (d.n_faces > 0 ? d.n_faces : 1);
-        return per >= 48.0 ? 2u : per >= 6.0 ? 1u : 0u;
+        const long long area = p == kBvShadow ? (long long)v.S * v.S : (long long)v.W * v.H;
+        const int lanes = direct_lanes(b->nt[p], d.n_faces, area, p == kBvShadow);
+        return lanes == 16 ? 2u : lanes == 4 ? 1u : 0u;
     };
     b->direct_ok = b->direct_ok && launch_fits((long long)sblk_view.size()) && mt <= kDirectTrisMost;
     for (int p = 0; p < 2; ++p) {

@@ -1554,7 +1554,7 @@ static int flush_pass(fgl_ctx *c)
     long long nt = 0, nv = 0, tris = 0;
     int max_pos = 0, max_faces = 0;
     for (const fgl_ctx::Rec &r : c->draws) tris += c->models[r.model].n_faces;
-    DirectGrid grid = {direct_lanes(tris), 0, 0, corner_form((long long)W * H, tris)};
+    DirectGrid grid = {direct_lanes(tris, tris, (long long)W * H, shadow), 0, 0, corner_form((long long)W * H, tris)};
     for (size_t i = 0; i < c->draws.size(); ++i) {
         const ModelRes &m = c->models[c->draws[i].model];
         DevDraw &d = dd[i];

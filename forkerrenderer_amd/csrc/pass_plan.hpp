@@ -7,10 +7,30 @@ namespace fgl {
 constexpr long long kMaxBlocks = 0xffffffffLL / 256;
 constexpr bool launch_fits(long long blocks) { return blocks <= kMaxBlocks; }
 
-// Lanes per triangle of the direct rasteriser in a pass of n_tri triangles: as
-// many as fill the chip (a triangle's pixels are its lanes' serial work).
-constexpr long long kDirectTris16 = 32768, kDirectTris4 = 262144;
-constexpr int direct_lanes(long long n_tri) { return n_tri <= kDirectTris16 ? 16 : n_tri <= kDirectTris4 ? 4 : 1; }
+// Lanes per triangle of the direct rasteriser: n_faces that share a target of
+// `pixels`, in a pass of n_tri triangles.  A triangle's pixels are its lanes'
+// serial work, its set-up every lane's; so by the pixels a face has (of a shadow
+// map, which holds the whole light volume, the scene covers a third of what it
+// covers of a view).  Passes of few triangles leave the chip idle with fewer lanes.
+// One sphere that fills the view, 16 / 4 / 1 lanes, us of the pass's raster
+// launches:
+//   faces      pixels a face    view                     pixels a face   shadow map
+//   20,480     12               11.4 / 11.9 / 41.0       20              19.2 / 15.3 / 37.2
+//   81,920     0.5              15.6 / 10.4 / 10.6       0.8             19.6 / 18.6 / 17.0
+//   81,920     3.1              17.0 / 11.9 / 22.5       5               20.8 / 18.2 / 22.2
+//   81,920     12               21.4 / 19.1 / 49.8       20              25.7 / 21.3 / 50.3
+//   81,920     25               23.8 / 39.8 / 60.7       45              32.1 / 29.2 / 62.6
+//   327,680    0.8              42.5 / 18.8 / 13.2       1.2             46.5 / 21.6 / 18.5
+//   327,680    6.3              49.1 / 26.6 / 83.7       11              58.6 / 35.7 / 39.6
+//   327,680    25               70.6 / 100 / 131         45              110 / 98 / 158
+//   1,310,720  1.6              145 / 55.5 / 38.0        2.8             162 / 69.8 / 46.4
+//   1,310,720  6.3              175 / 83 / 221           11              214 / 123 / 131
+constexpr long long kDirectFew = 32768;
+constexpr int direct_lanes(long long n_tri, long long n_faces, long long pixels, bool shadow)
+{
+    const long long px2 = 2 * pixels / (shadow ? 3 : 1);   // in halves
+    return n_tri <= kDirectFew || px2 >= 32 * n_faces ? 16 : px2 >= 5 * n_faces ? 4 : 1;
+}
 
 // Whether a main pass's resolve makes the varyings that depend on a position
 // from the corner records, instead of reading what the vertex pass made of each

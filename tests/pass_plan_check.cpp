@@ -32,9 +32,16 @@ int main()
     // many small draws beside a large one: what the draws hold, not the
     // number of draws times the largest
     const long long nt = 8192 + 131072;
-    const int lanes = direct_lanes(nt);
+    const int lanes = 4;
     CHECK(launch_fits(8192 * direct_groups(1, lanes) + direct_groups(131072, lanes)));
     CHECK(!launch_fits(8193 * direct_groups(131072, lanes)));
+    // lanes by pixels a face, all of them where triangles are few
+    CHECK(direct_lanes(32768, 32768, 1, false) == 16 && direct_lanes(32769, 32769, 1, false) == 1);
+    CHECK(direct_lanes(1 << 20, 1000, 16000, false) == 16 && direct_lanes(1 << 20, 1000, 15999, false) == 4);
+    CHECK(direct_lanes(1 << 20, 1000, 2500, false) == 4 && direct_lanes(1 << 20, 1000, 2499, false) == 1);
+    CHECK(direct_lanes(1 << 20, 1000, 48000, true) == 16 && direct_lanes(1 << 20, 1000, 47998, true) == 4);
+    CHECK(direct_lanes(1 << 20, 0, 1, false) == 16);   // a draw of none: no groups whatever its lanes
+    CHECK(direct_lanes(0x7fffffff, 0x7fffffff, 1LL << 34, false) == 4);
     // every face of the largest pass, 16 lanes each, does not fit
     CHECK(!launch_fits(direct_groups(0x7fffffff, 16)) && launch_fits(direct_groups(0x7fffffff, 1)));
     // 64 shadow maps of 8192 x 8192 in 64 x 4 blocks do not, 63 do

@@ -149,18 +149,26 @@ def test_batch_after_tables_and_ao_buffers_move(ctx, world, scene_dir):
     b.close()
 
 
-def test_batch_of_dense_meshes(ctx):
-    """Fewer than two pixels a face over all views: replays make the varyings
-    from the corner records, the measuring render from the vertices'."""
-    views = VW.uneven_views(ctx, n_views=4, seed=17, subdivs=(4, 5), min_px=40 * 40, max_px=80 * 80, shadow_size=64, tex=32)
+@pytest.mark.parametrize("dense", [True, False])
+def test_batch_of_larger_meshes(ctx, dense):
+    """More triangles than get 16 lanes whatever their size: one lane, four and
+    (the grounds) sixteen.  dense: fewer than two pixels a face over all views:
+    replays make the varyings from the corner records, the measuring render
+    from the vertices'."""
+    n, most, shadow = (4, 80, 64) if dense else (6, 560, 600)
+    views = VW.uneven_views(ctx, n_views=n, seed=17, subdivs=(5,), min_px=40 * 40, max_px=most * most, shadow_size=shadow, tex=32)
     singles = []
     for view in views:
         VW.render_view(ctx, view)
         singles.append({t: ctx.read(t).copy() for t in TARGETS})
     b = VW.Batch(ctx, views)
-    assert b.stats()["pixels"] < 2 * b.stats()["tris_main"]
+    st = b.stats()
+    assert st["tris_main"] > 32768 and (st["pixels"] < 2 * st["tris_main"]) == dense
+    if not dense:   # a sphere's pixels a face, in its view and in its map
+        faces = st["tris_main"] // n
+        assert min(v.pixels for v in views) < 2.5 * faces < max(v.pixels for v in views) and shadow ** 2 > 7.5 * faces
     for rep in range(3):
         b.render()
         assert b.sync() == 0
-        check(b, views, singles, f"dense, render {rep}")
+        check(b, views, singles, f"dense {dense}, render {rep}")
     b.close()

@@ -46,7 +46,7 @@ def _scene(name, rng):
     if name == "few_mixed":        # 16 lanes a triangle, boxes below and above the LDS box, items
         return [np.concatenate([_triangles(rng, 300, s) for s in (0.01, 0.05, 0.2, 0.9)])], 333, 201
     if name == "four_lanes":
-        return [_triangles(rng, 40000, 0.02)], 640, 400
+        return [_triangles(rng, 40000, 0.02)], 900, 500
     if name == "one_lane":
         return [_triangles(rng, 270000, 0.004), _triangles(rng, 5, 1.5)], 512, 300
     if name == "full_screens":     # 1,200 full screens of 300 items each: runs of 16, many searches
