@@ -295,6 +295,11 @@ class Context:
     def set_pass_tile_size(self, pass_, t):
         self._chk(lib().fgl_set_pass_tile_size(self._h, pass_, t), "fgl_set_pass_tile_size")
 
+    def pass_tile_size(self, pass_):
+        t = C.c_int()
+        self._chk(lib().fgl_get_pass_tile_size(self._h, pass_, C.byref(t)), "fgl_get_pass_tile_size")
+        return t.value
+
     def set_tile_size(self, t):
         self._chk(lib().fgl_set_tile_size(self._h, t), "fgl_set_tile_size")
 

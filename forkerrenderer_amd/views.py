@@ -99,6 +99,7 @@ class Batch:
     def __init__(self, ctx, views, ao_mode=AO_NONE, nao=None):
         L = _bind()
         self.ctx, self.views = ctx, list(views)
+        self.tiles, self.occupancy = (16, 16), 4   # as the library plans it
         arr = (ViewDesc * len(self.views))(*[v.desc for v in self.views])
         self._arr = arr
         self._h = C.c_void_p()
@@ -119,9 +120,11 @@ class Batch:
 
     def set_tiles(self, shadow_tile, main_tile):
         self.ctx._chk(_bind().fgl_batch_set_tiles(self._h, shadow_tile, main_tile), "fgl_batch_set_tiles")
+        self.tiles = (shadow_tile, main_tile)
 
     def set_occupancy(self, wg_per_cu):
         self.ctx._chk(_bind().fgl_batch_set_occupancy(self._h, wg_per_cu), "fgl_batch_set_occupancy")
+        self.occupancy = wg_per_cu
 
     def set_capacity(self, shadow_pairs, main_pairs):
         self.ctx._chk(_bind().fgl_batch_set_capacity(self._h, shadow_pairs, main_pairs), "fgl_batch_set_capacity")

@@ -143,7 +143,11 @@ const char *fgl_last_error(const fgl_ctx *ctx);
 int fgl_sync(fgl_ctx *ctx);
 /* Raster tuning: tile edge in pixels (8, 16 or 32).  Results do not depend
  * on it (each pixel's depth resolve is a minimum over (depth, submission id)
- * keys, whatever the tile). */
+ * keys, whatever the tile).  Only passes through the tile lists have tiles:
+ * forward passes with a stochastic shadow filter, passes that go on from
+ * earlier depths, and those that could reach 2^32 - 1 (tile, triangle) pairs
+ * or for whose per-pixel keys there is no memory; the others are rasterised
+ * without. */
 int fgl_set_tile_size(fgl_ctx *ctx, int tile);
 /* Per-pass tile edge (FGL_PASS_SHADOW, or FORWARD/GEOMETRY for the main pass);
  * the autotuner (forkerrenderer_amd/autotune.py) sets these. */
@@ -389,7 +393,11 @@ typedef struct fgl_batch fgl_batch;
 int fgl_batch_create(fgl_ctx *ctx, int n_views, const fgl_view_desc *views, int ao_mode, fgl_nao *nao,
                      fgl_batch **out);
 void fgl_batch_destroy(fgl_batch *b);
-/* raster tile edges (8, 16, 32) of the shadow and geometry passes */
+/* raster tile edges (8, 16, 32) of the shadow and geometry passes.  Tiles,
+ * workgroups and capacities apply to renders through the tile lists: the one
+ * that counts a plan's pairs, and all of a batch with explicit capacities for
+ * both passes (until one overflows), with a vertex on the camera plane, or
+ * without memory for its per-pixel keys.  Others rasterise without tiles. */
 int fgl_batch_set_tiles(fgl_batch *b, int shadow_tile, int main_tile);
 /* persistent rasteriser workgroups per compute unit (1..16) */
 int fgl_batch_set_occupancy(fgl_batch *b, int wg_per_cu);
