@@ -626,6 +626,17 @@ static int capture(fgl_batch *b)
     return FGL_OK;
 }
 
+namespace fgl {
+// The context goes first (its stream is idle): the batch keeps its memory
+// until it is destroyed, and takes no more calls.
+void batch_detach(void *p)
+{
+    fgl_batch *b = (fgl_batch *)p;
+    drop_graph(b);
+    b->ctx = nullptr;
+}
+}  // namespace fgl
+
 extern "C" {
 
 int fgl_render_view(fgl_ctx *c, const fgl_view_desc *v, int ao_mode, fgl_nao *nao)
@@ -671,6 +682,7 @@ int fgl_batch_create(fgl_ctx *c, int n, const fgl_view_desc *views, int ao_mode,
         if ((rc = check_view(c, views[i]))) return rc;
     fgl_batch *b = new fgl_batch();
     b->ctx = c;
+    ctx_register_batch(c, b);
     b->n = n;
     b->ao_mode = ao_mode;
     b->nao = nao;
@@ -703,7 +715,10 @@ int fgl_batch_create(fgl_ctx *c, int n, const fgl_view_desc *views, int ao_mode,
 void fgl_batch_destroy(fgl_batch *b)
 {
     if (!b) return;
-    (void)hipStreamSynchronize(ctx_stream(b->ctx));   // teardown: nothing to report to
+    if (b->ctx) {
+        (void)hipStreamSynchronize(ctx_stream(b->ctx));   // teardown: nothing to report to
+        ctx_unregister_batch(b->ctx, b);
+    }
     drop_graph(b);
     for (int l = 0; l < 2; ++l) release(b->d_conv_items[l]);
     for (int p = 0; p < 2; ++p) {
@@ -728,7 +743,7 @@ void fgl_batch_destroy(fgl_batch *b)
 
 int fgl_batch_set_tiles(fgl_batch *b, int shadow_tile, int main_tile)
 {
-    if (!b) return FGL_ERR_INVALID;
+    if (!b || !b->ctx) return FGL_ERR_INVALID;
     for (int t : {shadow_tile, main_tile})
         if (t != 8 && t != 16 && t != 32) return bfail(b, FGL_ERR_INVALID, "tile must be 8, 16 or 32");
     if (b->TS[0] == shadow_tile && b->TS[1] == main_tile) return FGL_OK;
@@ -740,7 +755,7 @@ int fgl_batch_set_tiles(fgl_batch *b, int shadow_tile, int main_tile)
 
 int fgl_batch_set_occupancy(fgl_batch *b, int wg_per_cu)
 {
-    if (!b) return FGL_ERR_INVALID;
+    if (!b || !b->ctx) return FGL_ERR_INVALID;
     if (wg_per_cu < 1 || wg_per_cu > 16) return bfail(b, FGL_ERR_INVALID, "occupancy must be 1..16");
     if (b->occupancy != wg_per_cu) drop_graph(b);
     b->occupancy = wg_per_cu;
@@ -749,7 +764,7 @@ int fgl_batch_set_occupancy(fgl_batch *b, int wg_per_cu)
 
 int fgl_batch_set_capacity(fgl_batch *b, uint32_t shadow_pairs, uint32_t main_pairs)
 {
-    if (!b) return FGL_ERR_INVALID;
+    if (!b || !b->ctx) return FGL_ERR_INVALID;
     if (hipStreamSynchronize(ctx_stream(b->ctx)) != hipSuccess) return bfail(b, FGL_ERR_DEVICE, "stream failed");
     b->cap_req[0] = shadow_pairs;
     b->cap_req[1] = main_pairs;
@@ -763,7 +778,7 @@ int fgl_batch_set_capacity(fgl_batch *b, uint32_t shadow_pairs, uint32_t main_pa
 
 int fgl_batch_use_graph(fgl_batch *b, int on)
 {
-    if (!b) return FGL_ERR_INVALID;
+    if (!b || !b->ctx) return FGL_ERR_INVALID;
     b->use_graph = on != 0;
     if (!on) drop_graph(b);
     return FGL_OK;
@@ -797,7 +812,7 @@ static int refresh_resources(fgl_batch *b)
 
 int fgl_batch_render(fgl_batch *b)
 {
-    if (!b) return FGL_ERR_INVALID;
+    if (!b || !b->ctx) return FGL_ERR_INVALID;
     const bool timed = ctx_timing(b->ctx);
     int rc;
     if ((rc = refresh_resources(b))) return rc;
@@ -815,7 +830,7 @@ int fgl_batch_render(fgl_batch *b)
 
 int fgl_batch_sync(fgl_batch *b, int *rerenders)
 {
-    if (!b) return FGL_ERR_INVALID;
+    if (!b || !b->ctx) return FGL_ERR_INVALID;
     if (rerenders) *rerenders = 0;
     hipStream_t s = ctx_stream(b->ctx);
     if (hipStreamSynchronize(s) != hipSuccess) return bfail(b, FGL_ERR_DEVICE, "batch failed");
@@ -836,7 +851,7 @@ int fgl_batch_sync(fgl_batch *b, int *rerenders)
 
 int fgl_batch_read(fgl_batch *b, int view, int which, void *dst, size_t bytes)
 {
-    if (!b || !dst || view < 0 || view >= b->n) return FGL_ERR_INVALID;
+    if (!b || !b->ctx || !dst || view < 0 || view >= b->n) return FGL_ERR_INVALID;
     const DevView &v = b->hv[view];
     const size_t P = (size_t)v.W * v.H, SP = (size_t)v.S * v.S;
     const char *src = nullptr;
@@ -863,7 +878,7 @@ int fgl_batch_read(fgl_batch *b, int view, int which, void *dst, size_t bytes)
 
 int fgl_batch_stats(fgl_batch *b, uint64_t stats[10])
 {
-    if (!b || !stats) return FGL_ERR_INVALID;
+    if (!b || !b->ctx || !stats) return FGL_ERR_INVALID;
     stats[0] = b->last_pairs[0];
     stats[1] = b->last_pairs[1];
     stats[2] = b->cap[0];

@@ -142,6 +142,7 @@ struct fgl_ctx {
     NetAo ao_net{};
     const void *ao_net_owner = nullptr;
     std::vector<void *> naos;   // networks created on this context
+    std::vector<void *> batches;
 
     // timing
     bool timing = false;
@@ -404,6 +405,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     for (void *n : c->naos) nao_detach(n);   // networks outliving their context stop using it
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    for (void *b : c->batches) batch_detach(b);
     for (void *p : c->texture_mem) (void)hipFree(p);
     for (auto &m : c->models) {
         (void)hipFree(m.pos); (void)hipFree(m.uv); (void)hipFree(m.nrm);
@@ -2121,14 +2123,20 @@ int ctx_settle_network_ao(fgl_ctx *c, const void *owner)
 
 void ctx_register_nao(fgl_ctx *c, void *n) { c->naos.push_back(n); }
 
-void ctx_unregister_nao(fgl_ctx *c, void *n)
+static void unregister(std::vector<void *> &list, void *p)
 {
-    for (size_t k = 0; k < c->naos.size(); ++k)
-        if (c->naos[k] == n) {
-            c->naos.erase(c->naos.begin() + (long)k);
+    for (size_t k = 0; k < list.size(); ++k)
+        if (list[k] == p) {
+            list.erase(list.begin() + (long)k);
             break;
         }
 }
+
+void ctx_unregister_nao(fgl_ctx *c, void *n) { unregister(c->naos, n); }
+
+void ctx_register_batch(fgl_ctx *c, void *b) { c->batches.push_back(b); }
+
+void ctx_unregister_batch(fgl_ctx *c, void *b) { unregister(c->batches, b); }
 
 int ctx_fail(fgl_ctx *c, int code, const char *msg) { return fail(c, code, msg); }
 

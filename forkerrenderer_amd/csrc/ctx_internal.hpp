@@ -93,6 +93,10 @@ void ctx_drop_network_ao(fgl_ctx *c, const void *owner);
 int ctx_settle_network_ao(fgl_ctx *c, const void *owner);
 void ctx_register_nao(fgl_ctx *c, void *n);
 void ctx_unregister_nao(fgl_ctx *c, void *n);
+// Batches, likewise: batch_detach from the context's end.
+void batch_detach(void *b);
+void ctx_register_batch(fgl_ctx *c, void *b);
+void ctx_unregister_batch(fgl_ctx *c, void *b);
 // Frame pixels per network pixel, each way (1, 2 or 4).
 int nao_scale(const fgl_nao *n);
 // Changes whenever nao_reserve moves the inference buffers (a graph that

@@ -388,7 +388,9 @@ int fgl_render_view(fgl_ctx *ctx, const fgl_view_desc *view, int ao_mode, fgl_na
 /* A batch renders many views of different sizes and meshes together: every
  * pass is one launch over all views (persistent rasteriser workgroups pull
  * (view, tile) items from a device queue), the pass sequence is captured in
- * a HIP graph and replayed.  Results equal fgl_render_view's bit for bit. */
+ * a HIP graph and replayed.  Results equal fgl_render_view's bit for bit.  A
+ * batch that outlives its context takes no more calls (FGL_ERR_INVALID) but
+ * its destruction. */
 typedef struct fgl_batch fgl_batch;
 int fgl_batch_create(fgl_ctx *ctx, int n_views, const fgl_view_desc *views, int ao_mode, fgl_nao *nao,
                      fgl_batch **out);

@@ -172,3 +172,17 @@ def test_batch_of_larger_meshes(ctx, dense):
         assert b.sync() == 0
         check(b, views, singles, f"dense {dense}, render {rep}")
     b.close()
+
+
+def test_batch_outlives_its_context():
+    c = F.Context(0)
+    b = VW.Batch(c, VW.uneven_views(c, n_views=2, seed=23, subdivs=(1,), min_px=256, max_px=512, shadow_size=32, tex=16))
+    for _ in range(2):   # the second captures a graph
+        b.render()
+        assert b.sync() == 0
+    c.close()
+    for call in (b.render, b.sync, b.stats, lambda: b.set_tiles(8, 8), lambda: b.set_occupancy(2), lambda: b.set_capacity(0, 0),
+                 lambda: b.use_graph(False), lambda: b.read(0, F.TARGET_IMAGE)):
+        with pytest.raises(F.FglError, match=r"\(-1\)"):
+            call()
+    b.close()
