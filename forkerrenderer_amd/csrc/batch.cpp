@@ -608,10 +608,12 @@ static int capture(fgl_batch *b)
 {
     hipStream_t s = ctx_stream(b->ctx);
     hipGraph_t g = nullptr;
+    std::unique_lock<std::mutex> lock(ctx_order_mutex());
     if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess)
         return bfail(b, FGL_ERR_DEVICE, "graph capture failed to start");
     int rc = enqueue(b, false, false);
     hipError_t e = hipStreamEndCapture(s, &g);
+    lock.unlock();
     if (rc) {
         if (g) (void)hipGraphDestroy(g);
         return rc;

@@ -136,6 +136,10 @@ struct fgl_ctx {
     // device address of the allocation-free entry point's scratch array
     float *noalloc_scratch = nullptr;
     int number = 0;   // of this context among its device's (0: none was free)
+    // what its calls have used of that array, and the event that other contexts'
+    // calls wait for where they use the same
+    size_t scratch_lo = 0, scratch_hi = 0;
+    hipEvent_t scratch_event = nullptr;
     // neural AO still on its network grid (lao != nullptr): the AO target's
     // content until something reads or replaces it; owner = the network
     // whose buffers hold it
@@ -180,7 +184,9 @@ static hipError_t scratch_address(int device, float **out)
 
 // Contexts on a device are numbered (the lowest free number), so that their
 // calls use different parts of `scratch` where it holds a part for each: parts
-// are the frame rounded up to a power of two, by the number.
+// are the frame rounded up to a power of two, by the number.  Where two
+// contexts' parts meet all the same (scratch_use), their calls are ordered.
+static std::vector<fgl_ctx *> g_scratch_users[kMaxDevices];
 static uint64_t g_ctx_numbers[kMaxDevices] = {};
 
 static int take_number(int device)
@@ -199,12 +205,42 @@ static void give_number(int device, int number)
     if (number > 0) g_ctx_numbers[device] &= ~(1ull << (number - 1));
 }
 
-static float *scratch_part(float *scratch_base, int number, size_t n)
+// The part of `scratch` for a call of c on n pixels; c's stream waits for the
+// calls of other contexts that used any of it.  The caller holds g_scratch_mu
+// until its own launches are enqueued, so an event recorded on a context's
+// stream comes after all of them.
+static hipError_t scratch_use(fgl_ctx *c, size_t n, float **out)
 {
     size_t part = 1 << 16;
     while (part < n) part *= 2;
     const size_t parts = FGL_SSAO_NOALLOC_MAX_PIXELS / part;   // n is at most that, a power of two
-    return scratch_base + (number > 0 ? (size_t)(number - 1) % parts : 0) * part;
+    const size_t lo = (c->number > 0 ? (size_t)(c->number - 1) % parts : 0) * part, hi = lo + n;
+    for (fgl_ctx *o : g_scratch_users[c->device]) {
+        if (o == c || o->scratch_hi <= lo || hi <= o->scratch_lo) continue;
+        hipError_t e = hipEventRecord(o->scratch_event, o->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(c->stream, o->scratch_event, 0);
+        if (e != hipSuccess) return e;
+    }
+    if (c->scratch_hi == 0) {
+        g_scratch_users[c->device].push_back(c);
+        c->scratch_lo = lo;
+    }
+    c->scratch_lo = lo < c->scratch_lo ? lo : c->scratch_lo;
+    c->scratch_hi = hi > c->scratch_hi ? hi : c->scratch_hi;
+    *out = c->noalloc_scratch + lo;
+    return hipSuccess;
+}
+
+// c's stream is idle and takes no more calls.
+static void scratch_leave(fgl_ctx *c)
+{
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    std::vector<fgl_ctx *> &users = g_scratch_users[c->device];
+    for (size_t k = 0; k < users.size(); ++k)
+        if (users[k] == c) {
+            users.erase(users.begin() + (long)k);
+            break;
+        }
 }
 
 static int fail(fgl_ctx *c, int code, const std::string &msg)
@@ -365,7 +401,8 @@ int fgl_ctx_create(int device, fgl_ctx **out)
         return FGL_ERR_NOMEM;
     }
     if (hipHostMalloc((void **)&c->h_pub, 64, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
-        hipHostGetDevicePointer((void **)&c->d_pub, c->h_pub, 0) != hipSuccess) {
+        hipHostGetDevicePointer((void **)&c->d_pub, c->h_pub, 0) != hipSuccess ||
+        hipEventCreateWithFlags(&c->scratch_event, hipEventDisableTiming) != hipSuccess) {
         if (c->h_pub) (void)hipHostFree(c->h_pub);
         (void)hipHostFree(c->h_total);
         (void)hipStreamDestroy(c->stream);
@@ -405,6 +442,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     for (void *n : c->naos) nao_detach(n);   // networks outliving their context stop using it
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    scratch_leave(c);
     for (void *b : c->batches) batch_detach(b);
     for (void *p : c->texture_mem) (void)hipFree(p);
     for (auto &m : c->models) {
@@ -426,6 +464,7 @@ void fgl_ctx_destroy(fgl_ctx *c)
     for (auto &t : c->timed) { (void)hipEventDestroy(t.a); (void)hipEventDestroy(t.b); }
     if (c->h_total) (void)hipHostFree(c->h_total);
     if (c->h_pub) (void)hipHostFree(c->h_pub);
+    (void)hipEventDestroy(c->scratch_event);
     (void)hipStreamDestroy(c->stream);
     give_number(c->device, c->number);
     delete c;
@@ -1820,7 +1859,12 @@ int fgl_ssao_noalloc(fgl_ctx *c, int w, int h, const float view[16], const float
     }
     // The separable blur reads the unblurred AO from the scratch array; the
     // SSAO kernel writes every pixel of it first, so nothing is cleared.
-    float *raw = cfg->blur == 2 ? scratch_part(c->noalloc_scratch, c->number, (size_t)w * h) : ao;
+    float *raw = ao;
+    std::unique_lock<std::mutex> lock(g_scratch_mu, std::defer_lock);
+    if (cfg->blur == 2) {
+        lock.lock();
+        HIPCHK(c, scratch_use(c, (size_t)w * h, &raw));
+    }
     launch_ssao(u, sa, depth, gbuf, raw, c->stream);
     if (cfg->blur == 1)
         launch_blur_recursive(ao, w, h, c->stream);
@@ -2150,6 +2194,8 @@ int ctx_draw_record(fgl_ctx *c, int model, const float M[16], DevDraw *out)
 }
 
 void ctx_begin_frame(fgl_ctx *c, int w, int h) { c->frame_px = (size_t)w * h; }
+
+std::mutex &ctx_order_mutex() { return g_scratch_mu; }
 
 bool ctx_depths_finite(fgl_ctx *c, int model, const float M[16], bool shadow)
 {

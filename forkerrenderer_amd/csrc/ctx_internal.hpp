@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <vector>
 
 #include "../../include/fgl.h"
@@ -40,6 +41,9 @@ int ctx_draw_record(fgl_ctx *c, int model, const float M[16], DevDraw *out);
 // The size of the frame that the passes to come make: its shadow pass makes room
 // for its main pass.
 void ctx_begin_frame(fgl_ctx *c, int w, int h);
+// Held while another context may record an event on a context's stream, and
+// while a context's stream is captured.
+std::mutex &ctx_order_mutex();
 // Whether every window depth of `model` under M is finite, in the shadow or
 // the main pass of the context's current matrices (then no fragment's depth
 // is NaN).

@@ -222,8 +222,10 @@ int fgl_ssao(fgl_ctx *ctx, const fgl_ssao_cfg *cfg);
  * library runs on, held until the process ends); larger frames fail with
  * FGL_ERR_CAPACITY.  Contexts whose frames round up to the same power of two
  * use parts of their own while the array holds one for each (64 contexts of
- * up to 2^17 pixels, one of more than 2^22); other calls that overlap on one
- * device (larger or mixed frames, two host threads on a context) race.  Work is
+ * up to 2^17 pixels, one of more than 2^22); where the parts of two contexts'
+ * calls meet (larger or mixed frames), the later call's work waits for the
+ * earlier one's on the device.  As for every call, a context is one host
+ * thread's at a time.  Work is
  * enqueued on the context's stream; nothing is allocated or freed, and the
  * context's targets and pending draws are left as they are.  Results equal
  * fgl_ssao's on the same frame bit for bit. */

@@ -127,16 +127,19 @@ def test_noalloc_ssao_rejects_what_it_cannot_run(ctx):
     assert fn(ctx._h, 64, 64, eye.ctypes.data, eye.ctypes.data, None, dummy, dummy, C.byref(cfg)) == F.ERR_INVALID
 
 
-def test_overlapping_calls_of_two_contexts_use_their_own_scratch(ctx, scene_dir):
-    """Two contexts (two streams), frames of one size, calls in turn with no
-    wait between: each result equals the one of a call by itself."""
+@pytest.mark.parametrize("sizes", [[(333, 201), (333, 201)], [(333, 201), (2000, 1100), (1100, 700)],
+                                   [(2400, 1800), (2300, 1900)]])
+def test_overlapping_calls_of_contexts(ctx, scene_dir, sizes):
+    """Contexts (a stream each), calls in turn with no wait between: each
+    result equals the one of a call by itself.  Frames of one size use their
+    own parts of the scratch; mixed ones and those of more than 2^22 pixels
+    share some of it and are ordered."""
     hip, fn = _hip(), _bind()
-    w, h = 333, 201
-    other = F.Context(0)
+    others = [F.Context(0) for _ in sizes[1:]]
     bufs, want, args = [], [], []
     try:
-        for k, c in enumerate((ctx, other)):
-            p = G.tiny_scene(os.path.join(scene_dir, f"noalloc_two_{k}"), seed=50 + k, width=w, height=h, subdiv=3, tex=16,
+        for k, (c, (w, h)) in enumerate(zip([ctx] + others, sizes)):
+            p = G.tiny_scene(os.path.join(scene_dir, f"noalloc_two_{k}_{w}"), seed=50 + k, width=w, height=h, subdiv=3, tex=16,
                              ssao=True, extra="aoblur gaussian 2")
             sc = F.Scene(p)
             c.render_scene(sc)
@@ -145,15 +148,16 @@ def test_overlapping_calls_of_two_contexts_use_their_own_scratch(ctx, scene_dir)
             b[0].put(c.read(F.TARGET_DEPTH))
             b[1].put(c.read(F.TARGET_GBUFFER))
             V, Pm = _camera(sc.info)
-            args.append((c, V, Pm, b, sc))
+            args.append((c, V, Pm, b, sc, w, h))
             want.append(c.read(F.TARGET_AO))
         for rep in range(40):
-            for c, V, Pm, b, sc in args:
+            for c, V, Pm, b, sc, w, h in args:
                 assert fn(c._h, w, h, V.ctypes.data, Pm.ctypes.data, b[0].p, b[1].p, b[2].p, C.byref(sc.info.ssao)) == 0
-        for (c, V, Pm, b, sc), ref in zip(args, want):
+        for (c, V, Pm, b, sc, w, h), ref in zip(args, want):
             c.sync()
             assert np.array_equal(b[2].get(w * h).view(np.uint32), ref.view(np.uint32))
     finally:
-        other.close()
+        for c in others:
+            c.close()
         for b in bufs:
             b.free()
