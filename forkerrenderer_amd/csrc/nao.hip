@@ -1258,11 +1258,10 @@ __global__ __launch_bounds__(256) void k_conv_wgrad(const uint16_t *__restrict__
     }
 }
 
-template <int DIL>
+template <int LAYER>
 static void launch_wgrad(hipStream_t s, const uint16_t *in, const uint16_t *dout, float *part, int S, int N)
 {
-    constexpr int CIN = DIL == layer_dil(0) ? C0 : CH;
-    hipLaunchKernelGGL((k_conv_wgrad<CIN, DIL>), dim3(S / 64, S / WG_ROWS, N), dim3(256), 0, s, in, dout, part, S, S);
+    hipLaunchKernelGGL((k_conv_wgrad<LAYER == 0 ? C0 : CH, layer_dil(LAYER)>), dim3(S / 64, S / WG_ROWS, N), dim3(256), 0, s, in, dout, part, S, S);
 }
 
 // Sum over b of part[b*len + i], in a fixed order (bitwise reproducible): 64
@@ -1739,10 +1738,10 @@ static int run_batch(fgl_nao *n, bool update, float lr, float *stats)
     for (int l = 3; l >= 0; --l) {
         const int len = CH * (l == 0 ? K1 : K2) + CH;
         switch (l) {
-        case 0: launch_wgrad<layer_dil(0)>(s, n->feat, n->d[0], n->part, S, N); break;
-        case 1: launch_wgrad<layer_dil(1)>(s, n->a[0], n->d[1], n->part, S, N); break;
-        case 2: launch_wgrad<layer_dil(2)>(s, n->a[1], n->d[2], n->part, S, N); break;
-        default: launch_wgrad<layer_dil(3)>(s, n->a[2], n->d[3], n->part, S, N); break;
+        case 0: launch_wgrad<0>(s, n->feat, n->d[0], n->part, S, N); break;
+        case 1: launch_wgrad<1>(s, n->a[0], n->d[1], n->part, S, N); break;
+        case 2: launch_wgrad<2>(s, n->a[1], n->d[2], n->part, S, N); break;
+        default: launch_wgrad<3>(s, n->a[2], n->d[3], n->part, S, N); break;
         }
         hipLaunchKernelGGL(k_reduce_cols, dim3((len + 63) / 64), dim3(64 * kReduceGroups), 0, s, n->part, nblk, len,
                            n->grads + woffs[l], len, (float *)nullptr);
