@@ -78,6 +78,124 @@ def test_batch_graph_replays_across_tiles(ctx, world, tiles, occ):
     b.close()
 
 
+def kernels(ctx, b):
+    """Names of the kernels of one render."""
+    ctx.read_timings()
+    ctx.enable_timing(True)
+    b.render()
+    assert b.sync() == 0
+    names = {n for n, _ in ctx.read_timings()}
+    ctx.enable_timing(False)
+    return names
+
+
+@pytest.mark.parametrize("tiles,occ", [((8, 8), 1), ((32, 16), 2), ((16, 32), 8)])
+def test_which_way_a_batch_rasterises(ctx, world, tiles, occ):
+    """The render that counts a plan's pairs goes through the lists, replays
+    through the direct rasteriser; explicit capacities keep every replay on
+    the lists (tiles, occupancy and graph replays of the list path)."""
+    views, net, singles = world
+    b = VW.Batch(ctx, views, VW.AO_NEURAL, net)
+    b.set_tiles(*tiles)
+    b.set_occupancy(occ)
+    assert "batch_main_sort" in kernels(ctx, b)
+    check(b, views, singles, "counting")
+    assert "batch_main_sort" not in kernels(ctx, b)
+    check(b, views, singles, "direct")
+    st = b.stats()
+    b.close()
+    b = VW.Batch(ctx, views, VW.AO_NEURAL, net)
+    b.set_tiles(*tiles)
+    b.set_occupancy(occ)
+    b.set_capacity(st["pairs_shadow"] + 1, st["pairs_main"] + 1)
+    for rep in range(3):
+        b.render()
+        assert b.sync() == 0
+        check(b, views, singles, f"lists, replay {rep}")
+        ctx.sync()
+    assert "batch_main_sort" in kernels(ctx, b)
+    b.close()
+
+
+def _filters(scene_dir):
+    """One configuration of each deterministic shadow filter."""
+    import os
+    from forkerrenderer_amd import scenegen as G
+    return [F.Scene(G.tiny_scene(os.path.join(scene_dir, f"batch_{k}"), shadow=k)).info.shadow
+            for k in ("hard", "pcf", "pcss", "grid")]
+
+
+@pytest.mark.parametrize("kinds", [(0, 1, 2, 3), (2, 2), (1, 3), (None, None), (None, 1)])
+def test_batch_of_shadow_filters(ctx, scene_dir, kinds):
+    """One filter over all shadowed views, several, none."""
+    cfgs = _filters(scene_dir)
+    base = VW.uneven_views(ctx, n_views=len(kinds), seed=29, subdivs=(3,), min_px=48 * 48, max_px=120 * 120, shadow_size=64,
+                           tex=16)
+    views = []
+    for v, k in zip(base, kinds):
+        d = v.desc
+        views.append(VW.View(d.width, d.height, tuple(d.eye), tuple(d.look_at),
+                             list(zip(v.models.tolist(), v.mats.reshape(-1, 4, 4))),
+                             [(0, (2.0, 5.0, 5.0), (3.0, 3.0, 3.0))], None if k is None else cfgs[k], 64))
+    singles = []
+    for view in views:
+        VW.render_view(ctx, view)
+        singles.append({t: ctx.read(t).copy() for t in TARGETS
+                        if view.desc.shadow_on or t not in (F.TARGET_SHADOW, F.TARGET_SHADOW_DEPTH)})
+    b = VW.Batch(ctx, views)
+    for rep in range(3):
+        b.render()
+        assert b.sync() == 0
+        check(b, views, singles, f"filters {kinds}, render {rep}")
+    b.close()
+
+
+@pytest.mark.parametrize("name", ["camera plane", "layers", "many large"])
+def test_batch_of_triangle_soups(ctx, name):
+    """A vertex on one view's camera plane (the whole batch stays on the
+    lists), full-screen layers enough for keys to be read first, and more
+    large triangles than a wavefront has lanes."""
+    rng = np.random.default_rng(11)
+    views = VW.uneven_views(ctx, n_views=3, seed=31, subdivs=(2,), min_px=150 * 150, max_px=320 * 240, shadow_size=128, tex=16)
+    v, d = views[1], views[1].desc
+    eye, at = np.array(d.eye, np.float64), np.array(d.look_at, np.float64)
+    fwd = (at - eye) / np.linalg.norm(at - eye)
+    right = np.cross(fwd, (0, 1, 0))
+    right /= np.linalg.norm(right)
+    up = np.cross(right, fwd)
+
+    def facing(n, dist, size, spread):   # triangles across the view, in world space
+        c = eye + fwd * dist.reshape(-1, 1) + (right * rng.uniform(-1, 1, (n, 1)) + up * rng.uniform(-1, 1, (n, 1))) * spread
+        return np.stack([c + right * size * a + up * size * b for a, b in ((-3, -1), (3, -1), (0, 3))], 1)
+    if name == "camera plane":
+        tris = facing(20, rng.uniform(1, 3, 20), 0.3, 0.6)
+        tris[0, 0] = eye - fwd          # the projection's w is 1 - z of the view space
+    elif name == "layers":
+        tris = facing(40, rng.uniform(0.5, 1.0, 40), 4.0, 0.0)
+    else:
+        tris = facing(80, rng.uniform(1.0, 2.5, 80), 0.6, 0.8)
+    n = len(tris)
+    f = np.arange(3 * n, dtype=np.int32).reshape(n, 3)
+    m = ctx.upload_model({"pos": tris.reshape(-1, 3).astype(np.float32), "uv": rng.uniform(0, 1, (3 * n, 2)).astype(np.float32),
+                          "nrm": np.tile(-fwd, (3 * n, 1)).astype(np.float32), "tan": None, "vi": f, "ti": f, "ni": f,
+                          "face_material": np.full(n, VW.pbr_material(ctx, 5, 16), np.int32), "support_pbr": True})
+    draws = list(zip(v.models.tolist(), v.mats.reshape(-1, 4, 4))) + [(m, np.eye(4, dtype=np.float32))]
+    views[1] = VW.View(d.width, d.height, tuple(d.eye), tuple(d.look_at), draws, [(0, (2.0, 5.0, 5.0), (3.0, 3.0, 3.0))],
+                       VW.pcf_grid(3), 128)
+    singles = []
+    for view in views:
+        VW.render_view(ctx, view)
+        singles.append({t: ctx.read(t).copy() for t in TARGETS})
+    b = VW.Batch(ctx, views)
+    print("batch of", name, flush=True)
+    for rep in range(3):
+        b.render()
+        assert b.sync() == 0
+        check(b, views, singles, f"{name}, render {rep}")
+    assert ("batch_main_sort" in kernels(ctx, b)) == (name == "camera plane")
+    b.close()
+
+
 def test_batch_overflow_rerenders(ctx, world):
     views, net, singles = world
     b = VW.Batch(ctx, views, VW.AO_NEURAL, net)

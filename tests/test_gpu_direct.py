@@ -4,9 +4,10 @@ divide: lanes per triangle, the workgroup's LDS box, the list of large
 triangles and its runs of items, NaN depths, screens of one pixel and wider than
 the exact regime, several draws with equal depths.
 
-The second rendering starts with a draw that covers nothing and a change of
-state, which flushes it: the rest of the pass then continues from existing
-depths and takes the tile lists."""
+The second rendering (one per tile size) starts with a draw that covers
+nothing and a change of state, which flushes it: the rest of the pass then
+continues from existing depths and takes the tile lists.  Which way each took
+is read from the kernels it ran."""
 import time
 
 import numpy as np
@@ -70,25 +71,26 @@ def _scene(name, rng):
         t = _triangles(rng, 300, 1.0)
         t[::7, 1, 2] = np.nan
         return [_triangles(rng, 60, 0.1), t, _triangles(rng, 60, 1.0)], 640, 480
+    if name == "off_screen":
+        return [_triangles(rng, 500, 0.3) + np.array([9.0, 0.0, 0.0])], 100, 70
     raise AssertionError(name)
 
 
 @pytest.mark.parametrize("name", ["few_mixed", "four_lanes", "one_lane", "full_screens", "ties", "one_pixel", "thin",
-                                  "inexact", "nan", "nan_large"])
+                                  "inexact", "nan", "nan_large", "off_screen"])
 @pytest.mark.parametrize("shadow", [False, True])
 def test_direct_equals_lists(ctx, name, shadow):
     rng = np.random.default_rng(len(name))
     tris, W, H = _scene(name, rng)
     mat = _material(ctx)
     models = [(_model(ctx, mat, t), EYE4) for t in tris]
-    _direct_against_lists(ctx, mat, models, W, H, shadow, name)
+    _direct_against_lists(ctx, mat, models, W, H, shadow, name, tiles=(16,) if name == "full_screens" else (8, 16, 32))
 
 
-def _direct_against_lists(ctx, mat, draws, W, H, shadow, name, timed=False):
+def _direct_against_lists(ctx, mat, draws, W, H, shadow, name, timed=False, tiles=(16,)):
     """draws: (model, matrix) in order.  timed: returns the ms of each
     rendering's rasterisation (a second one, so that nothing is allocated)."""
     off = _model(ctx, mat, np.full((1, 3, 3), 9.0) + np.eye(3)[None])
-    ctx.set_tile_size(16)
     ctx.set_shadow(False)
     eye = np.ascontiguousarray(EYE4)
     ctx.set_matrix(F.MAT_PROJ, eye)
@@ -96,8 +98,12 @@ def _direct_against_lists(ctx, mat, draws, W, H, shadow, name, timed=False):
     ctx.set_matrix(F.MAT_LIGHT_SPACE, eye)
     ctx.set_viewport(0, 0, W, H, shadow=shadow)
     out, ms = [], []
-    for lists in (False, True):
+    for lists in (0,) + tiles:   # 0: direct
         print(f"direct test {name} {W}x{H} shadow {shadow} lists {lists}", flush=True)
+        ctx.set_tile_size(lists or 16)
+        ctx.sync()
+        ctx.read_timings()
+        ctx.enable_timing(True)
         if shadow:
             ctx.init_shadow_buffer(W, H)
         else:
@@ -112,7 +118,7 @@ def _direct_against_lists(ctx, mat, draws, W, H, shadow, name, timed=False):
         if timed:
             ctx.end_pass()
             ctx.sync()
-            ctx.enable_timing(True)
+            ctx.read_timings()
             ctx.init_targets(W, H)
             ctx.begin_pass(F.PASS_GEOMETRY)
             if lists:
@@ -121,20 +127,23 @@ def _direct_against_lists(ctx, mat, draws, W, H, shadow, name, timed=False):
             for k, at in draws:
                 ctx.draw_model(k, at)
         ctx.end_pass()
-        if timed:
-            ctx.sync()
-            ms.append(sum(t for k, t in ctx.read_timings() if k in ("vertex", "setup", "scan", "emit", "sort", "tile_ranges", "raster")))
-            ctx.enable_timing(False)
+        ctx.sync()
+        kernels = ctx.read_timings()
+        ctx.enable_timing(False)
+        assert ("setup" in [k for k, _ in kernels]) == (lists > 0), (lists, kernels)
+        ms.append(sum(t for k, t in kernels if k in ("vertex", "setup", "scan", "emit", "sort", "tile_ranges", "raster")))
         which = (F.TARGET_SHADOW_DEPTH, F.TARGET_SHADOW) if shadow else (F.TARGET_DEPTH, F.TARGET_GBUFFER)
         out.append([ctx.read(t).view(np.uint32) for t in which])
-    for a, b, what in zip(out[0], out[1], ("depth", "shadow value" if shadow else "G-buffer")):
+    ctx.set_tile_size(16)
+    for tile, a, b, what in [(tile, a, b, what) for tile, got in zip(tiles, out[1:])
+                             for a, b, what in zip(out[0], got, ("depth", "shadow value" if shadow else "G-buffer"))]:
         if name.startswith("nan"):   # a NaN's payload is not the fold's
             na, nb = np.isnan(a.view(np.float32)), np.isnan(b.view(np.float32))
             assert np.array_equal(na, nb), what
             a, b = np.where(na, 0, a), np.where(nb, 0, b)
-        assert np.array_equal(a, b), f"{what}: {(a != b).sum()} of {a.size} differ"
+        assert np.array_equal(a, b), f"{what}, tile {tile}: {(a != b).sum()} of {a.size} differ"
     depth = out[0][0].view(np.float32)
-    assert (depth < 3e38).any()
+    assert (depth < 3e38).any() == (name != "off_screen")
     return ms
 
 

@@ -5,9 +5,11 @@ miss the screen (no (tile, triangle) pairs: the emit, sort and rasteriser
 run on nothing and every pixel keeps its clear value)."""
 import os
 
+import numpy as np
 import pytest
 
 import forkerrenderer_amd as F
+import oracle as O
 from forkerrenderer_amd import scenegen as G
 from tests.util import assert_bitexact, gpu_frame, lsb_stats, oracle_frame
 
@@ -46,3 +48,40 @@ def test_main_pass_with_every_triangle_off_screen(ctx, scene_dir):
     want = _compare(ctx, p, 16)
     assert (want["depth"] >= 3e38).all(), "the scene is not off screen"
     assert (want["shadow_depth"] < 3e38).any(), "the shadow pass should still see the models"
+
+
+@pytest.mark.parametrize("color", [(np.inf, 2.0, 2.0), (2.0, np.nan, -np.inf), (3e38, 3e38, 3e38)], ids=str)
+def test_empty_pixels_under_lights_that_are_not_finite(ctx, scene_dir, color):
+    """Pixels nothing was drawn to are left early only where every term of
+    theirs is a finite number times zero."""
+    p = G.tiny_scene(os.path.join(scene_dir, "nolight"), seed=66, width=97, height=61, subdiv=2, tex=16, shadow="grid")
+    sc = F.Scene(p)
+    sc.info.lights[0].color[:] = color
+    want = oracle_frame(sc)
+    gpu_frame(ctx, sc)
+    ctx.set_lights([(sc.info.lights[k].type, list(sc.info.lights[k].vec), list(sc.info.lights[k].color))
+                    for k in range(sc.info.n_lights)])
+    ctx.begin_pass(F.PASS_LIGHTING)
+    ctx.draw_screen_space_pixels()
+    ctx.end_pass()
+    got, ref = ctx.read(F.TARGET_FRAME).reshape(-1), np.asarray(want["fb"]).reshape(-1)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    ok = np.isfinite(ref)
+    assert np.allclose(got[ok], ref[ok], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("rng_bias", [(np.inf, 0.0005), (0.01, -np.inf), (1e38, 0.0005), (0.01, -1e38), (0.01, np.inf)], ids=str)
+def test_ssao_of_empty_pixels_with_extreme_thresholds(ctx, scene_dir, rng_bias):
+    """Ranges and biases that let an uncovered pixel's taps occlude."""
+    p = G.tiny_scene(os.path.join(scene_dir, "ssaoinf"), seed=67, width=97, height=61, subdiv=2, tex=16, ssao=True)
+    sc = F.Scene(p)
+    want = oracle_frame(sc)
+    gpu_frame(ctx, sc)
+    cfg = sc.info.ssao
+    cfg.range, cfg.bias, cfg.blur = rng_bias[0], rng_bias[1], 0
+    st = O.frame_setup(sc.info)
+    ref = O.ssao_kernel(st["fr"], st["W"], st["H"], want["depth"], want["gbuf"], cfg)
+    ctx.begin_pass(F.PASS_LIGHTING)
+    ctx.ssao(cfg)
+    ctx.end_pass()
+    assert_bitexact("ao", ctx.read(F.TARGET_AO), ref)

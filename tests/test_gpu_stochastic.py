@@ -273,6 +273,37 @@ def test_blocker_search_sample_counts_match_the_oracle(ctx, scene_dir, n_blocker
                                  n_blocker=n_blocker, n_pcf=n_pcf)
 
 
+@pytest.mark.parametrize("shadowmap,blocker_filter", [(96, 0.1), (128, 0.3), (64, 0.02)])
+def test_blocker_searches_over_texels_that_are_not_numbers(ctx, scene_dir, shadowmap, blocker_filter):
+    """Shadow maps holding NaNs, infinities, zeros and negative depths (a
+    window's extremes count a NaN as no blocker)."""
+    p = G.tiny_scene(os.path.join(scene_dir, f"rnan{shadowmap}_{blocker_filter}"), seed=36, width=64, height=48, subdiv=3, tex=16,
+                     shadowmap=shadowmap, extra="shadowfilter refpcss")
+    sc = F.Scene(p)
+    sc.info.shadow.blocker_filter = blocker_filter
+    want = oracle_frame(sc)
+    ctx.render_scene(sc)
+    rng = np.random.default_rng(shadowmap)
+    smap = want["shadow"].copy()
+    at = rng.permutation(smap.size)[:smap.size // 20]
+    smap[at] = rng.choice(np.array([np.nan, np.inf, -np.inf, 0.0, -0.3, 0.0005, 0.00105, 3.0], np.float32), at.size)
+    ctx.set_shadow(True, sc.info.shadow)
+    ctx.write(F.TARGET_SHADOW, smap)
+    ctx.rng_seed(5489)
+    O.rng_seed(5489)
+    ctx.begin_pass(F.PASS_LIGHTING)
+    ctx.draw_screen_space_pixels()
+    ctx.end_pass()
+    st = O.frame_setup(sc.info)
+    ref = O.lighting_pass(st["fr"], st["W"], st["H"], want["gbuf"], want["ao"], smap, st["SW"], st["SH"]).reshape(-1)
+    got = ctx.read(F.TARGET_FRAME).reshape(-1)
+    assert ctx.rng_draws() == O.rng_draws()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = np.isfinite(ref)
+    assert np.abs(got[ok] - ref[ok]).max() < 1e-4
+    ctx.rng_seed(5489)
+
+
 def _lighting_matches_the_oracle(ctx, path, shadowmap, **cfg):
     p = G.tiny_scene(path, seed=36, width=64, height=48, subdiv=3, tex=16, shadowmap=shadowmap,
                      extra="shadowfilter refpcss")
