@@ -119,7 +119,6 @@ struct fgl_batch {
     // the direct rasteriser: its passes' pairs are known (last_pairs) for this
     // plan; every draw's depths are finite
     bool pairs_known = false, direct_ok = false;
-    bool corner = false;   // varyings from the corner records (corner_form)
     bool use_graph = true;
     hipGraphExec_t exec = nullptr;
 
@@ -236,6 +235,7 @@ static int plan(fgl_batch *b)
             lpx += (size_t)pix[i].lW * pix[i].lH;
         }
         if (b->ao_mode == FGL_AO_NEURAL) nao_conv_items(i, pix[i].lW, pix[i].lH, conv_items);
+        const long long first_tri = b->nt[kBvMain];
         // draw records: light * model with this view's light space
         for (int k = 0; k < v.n_draws; ++k) {
             DevDraw d;
@@ -256,6 +256,7 @@ static int plan(fgl_batch *b)
                 dd[p].push_back(e);
             }
         }
+        dv.corner = corner_form((long long)v.width * v.height, b->nt[kBvMain] - first_tri);
         if (v.shadow_on) b->have_shadow = true;
     }
     for (int p = 0; p < 2; ++p) {
@@ -267,7 +268,6 @@ static int plan(fgl_batch *b)
         if (tiles[p] > (1u << 30)) return bfail(b, FGL_ERR_CAPACITY, "too many tiles");
     }
     b->total_px = px;
-    b->corner = corner_form((long long)px, b->nt[kBvMain]);
     b->total_spx = spx;
     b->n_blocks = blocks;
     b->total_lpx = lpx;
@@ -430,7 +430,7 @@ static void enqueue_direct(fgl_batch *b, bool timed, hipStream_t s)
         {
             CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_binning" : "batch_main_binning") : nullptr);
             launch_bv_direct_vertex(p, a, (const uint2 *)b->d_vblocks[p].p, b->n_vblocks[p], (int4 *)b->screen.p,
-                                    (float *)b->ndc_z.p, b->corner ? nullptr : (float4 *)b->vary.p,
+                                    (float *)b->ndc_z.p, (float4 *)b->vary.p,
                                     p == kBvShadow ? b->total_spx : b->total_px, flags, s);
         }
         CtxTimer t(b->ctx, timed ? (p == kBvShadow ? "batch_shadow_raster" : "batch_main_raster") : nullptr);
@@ -550,7 +550,7 @@ static int enqueue(fgl_batch *b, bool measure, bool timed)
     pa.n_blocks = b->n_blocks;
     pa.screen = (const int4 *)b->screen.p;
     pa.tri_v = (const int4 *)b->tri_v.p;
-    pa.vary = direct && b->corner ? nullptr : (const float4 *)b->vary.p;
+    pa.vary = (const float4 *)b->vary.p;
     pa.vis = (const int *)b->vis.p;
     pa.key = direct ? (const unsigned long long *)b->key.p : nullptr;
     pa.depth = (float *)b->depth.p;

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void k_bv_direct_vertex(BvDirectArgs a, const 
         out[dr.vert_base + vi] = to_screen(u.shadow_viewport, n);
         ndc_z[dr.vert_base + vi] = n.z;
     } else {
-        out[dr.vert_base + vi] = to_screen(u.viewport, main_vertex_pass(dr, u, vi, vary));
+        out[dr.vert_base + vi] = to_screen(u.viewport, main_vertex_pass(dr, u, vi, a.views[dr.view].corner ? nullptr : vary));
     }
 }
 
@@ -257,7 +257,7 @@ __device__ __forceinline__ bool bv_pixel(const BvPixelArgs &a, int &vi, int &x, 
     return x < v.W && y < v.H;
 }
 
-template <bool DIRECT, bool CORNER>
+template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
 {
     int vi, x, y;
@@ -283,7 +283,8 @@ __global__ __launch_bounds__(256) void k_bv_gbuffer(BvPixelArgs b)
     a.textures = b.textures;
     a.shadow_map = nullptr;
     a.ss = ShadowSamples{};
-    gbuffer_px<DIRECT, CORNER>(a, v.u, x, y);
+    if (DIRECT && v.corner) gbuffer_px<DIRECT, DIRECT>(a, v.u, x, y);
+    else gbuffer_px<DIRECT, false>(a, v.u, x, y);
     // last: a store before them would keep the loads above from their scalar form
     if (DIRECT && blockIdx.x == 0 && threadIdx.x == 0) *b.ctr = DirectCtr{0ull, 0u, 0u};
 }
@@ -407,9 +408,8 @@ void launch_bv_gbuffer(const BvPixelArgs &a, hipStream_t s)
 {
     if (!a.n_blocks) return;
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(a.n_blocks), dim3(256), 0, s, a); };
-    if (!a.key) go(k_bv_gbuffer<false, false>);
-    else if (a.vary) go(k_bv_gbuffer<true, false>);
-    else go(k_bv_gbuffer<true, true>);
+    if (a.key) go(k_bv_gbuffer<true>);
+    else go(k_bv_gbuffer<false>);
 }
 
 void launch_bv_lighting(const BvPixelArgs &a, int mode, hipStream_t s)

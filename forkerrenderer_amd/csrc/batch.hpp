@@ -25,7 +25,7 @@ struct DevView {
     uint32_t tile_base[2];
     uint32_t blk_base, sblk_base;
     int draw_base[2], n_draws;
-    int pad;
+    int corner;        // its resolve makes the varyings from the corner records (corner_form)
     size_t px_off, spx_off;
 };
 
@@ -78,7 +78,7 @@ struct BvPixelArgs {
     uint32_t n_blocks;
     const int4 *screen;
     const int4 *tri_v;
-    const float4 *vary;       // the main vertex pass's varyings; null: made from the corner records
+    const float4 *vary;       // the main vertex pass's varyings, of views without `corner`
     const int *vis;
     const unsigned long long *key;   // the direct rasteriser's keys instead of vis (null: vis)
     float *depth;                    // with key: written by the resolve
