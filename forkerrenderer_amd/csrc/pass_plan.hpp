@@ -25,11 +25,13 @@ constexpr bool launch_fits(long long blocks) { return blocks <= kMaxBlocks; }
 //   327,680    25               70.6 / 100 / 131         45              110 / 98 / 158
 //   1,310,720  1.6              145 / 55.5 / 38.0        2.8             162 / 69.8 / 46.4
 //   1,310,720  6.3              175 / 83 / 221           11              214 / 123 / 131
+// Between 12 and 25 pixels a batch places the upper line: 16 lanes from 16, 24, 48
+// pixels a face on, 64 views 9.13, 9.06, 9.07 ms, 24 views 2.102, 2.079, 2.099.
 constexpr long long kDirectFew = 32768;
 constexpr int direct_lanes(long long n_tri, long long n_faces, long long pixels, bool shadow)
 {
     const long long px2 = 2 * pixels / (shadow ? 3 : 1);   // in halves
-    return n_tri <= kDirectFew || px2 >= 32 * n_faces ? 16 : px2 >= 5 * n_faces ? 4 : 1;
+    return n_tri <= kDirectFew || px2 >= 48 * n_faces ? 16 : px2 >= 5 * n_faces ? 4 : 1;
 }
 
 // Whether a main pass's resolve makes the varyings that depend on a position

@@ -37,9 +37,9 @@ int main()
     CHECK(!launch_fits(8193 * direct_groups(131072, lanes)));
     // lanes by pixels a face, all of them where triangles are few
     CHECK(direct_lanes(32768, 32768, 1, false) == 16 && direct_lanes(32769, 32769, 1, false) == 1);
-    CHECK(direct_lanes(1 << 20, 1000, 16000, false) == 16 && direct_lanes(1 << 20, 1000, 15999, false) == 4);
+    CHECK(direct_lanes(1 << 20, 1000, 24000, false) == 16 && direct_lanes(1 << 20, 1000, 23999, false) == 4);
     CHECK(direct_lanes(1 << 20, 1000, 2500, false) == 4 && direct_lanes(1 << 20, 1000, 2499, false) == 1);
-    CHECK(direct_lanes(1 << 20, 1000, 48000, true) == 16 && direct_lanes(1 << 20, 1000, 47998, true) == 4);
+    CHECK(direct_lanes(1 << 20, 1000, 72000, true) == 16 && direct_lanes(1 << 20, 1000, 71998, true) == 4);
     CHECK(direct_lanes(1 << 20, 0, 1, false) == 16);   // a draw of none: no groups whatever its lanes
     CHECK(direct_lanes(0x7fffffff, 0x7fffffff, 1LL << 34, false) == 4);
     // every face of the largest pass, 16 lanes each, does not fit
