@@ -298,7 +298,7 @@ def run_batched_views(reps, n_views=64):
     the 1280x800 generator (2048^2 maps and shadow maps, 5x5 PCF, icosphere
     subdivision 4..8), 256^2 .. 1920x1080, deferred PBR + neural AO, as one
     batch: aggregate Mpix/s and Mtri/s of graph replays after the batch
-    autotuner (tiles, rasteriser workgroups per CU, pair capacity), and the
+    autotuner (which tunes only replays through the tile lists), and the
     per-view latency of the same views rendered one at a time (render_view,
     synchronised per view)."""
     import forkerrenderer_amd as F

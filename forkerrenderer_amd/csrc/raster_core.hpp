@@ -439,7 +439,7 @@ __device__ __forceinline__ void raster_tile(const RasterArgs &a, int tile, Raste
 constexpr unsigned long long kDirectClear = 0xff7fffffull << 32;   // depth_order(FLT_MAX), no fragment
 constexpr int kDirectItemW = 64, kDirectItemH = 16;
 constexpr int kDirectBig = 4096;      // pixels of the bounding box
-constexpr int kDirectBox = 2048;      // pixels of a workgroup's LDS box: 16 KiB, nine workgroups a CU
+constexpr int kDirectBox = 2048;      // pixels of a workgroup's LDS box: 16 KiB; a CU's 32 wavefronts are eight workgroups
 
 // The last of n ascending starts (start[0] is 0) that is at most i, by whole
 // wavefronts, 64 probes a step.  Of owners with nothing of their own the last
