@@ -1595,6 +1595,7 @@ static int flush_pass(fgl_ctx *c)
     long long nt = 0, nv = 0, tris = 0;
     int max_pos = 0, max_faces = 0;
     for (const fgl_ctx::Rec &r : c->draws) tris += c->models[r.model].n_faces;
+    long long groups[3] = {0, 0, 0};
     DirectGrid grid = {direct_lanes(tris, tris, (long long)W * H, shadow), 0, 0, corner_form((long long)W * H, tris)};
     for (size_t i = 0; i < c->draws.size(); ++i) {
         const ModelRes &m = c->models[c->draws[i].model];
@@ -1603,15 +1604,19 @@ static int flush_pass(fgl_ctx *c)
         if (c->draws[i].has_normal) std::memcpy(d.normal, c->draws[i].n, sizeof(d.normal));
         d.vert_base = (int)nv;
         d.tri_base = (int)nt;
-        d.group_base = (int)grid.groups;
         d.vblock_base = (int)grid.vblocks;
-        grid.groups += direct_groups(d.n_faces, grid.lanes);
         grid.vblocks += vertex_blocks(d.n_pos);
+        for (int lanes : {1, 4, 16}) {
+            long long &n = groups[lanes_slot(lanes)];
+            d.group_base[lanes_slot(lanes)] = (int)n;
+            n += direct_groups(d.n_faces, lanes);
+        }
         nt += m.n_faces;
         nv += m.n_pos;
         max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
         max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
     }
+    grid.groups = groups[lanes_slot(grid.lanes)];
     const int n_draws = (int)c->draws.size();
     bool fits, no_nan;
     bound_pass(c, shadow, nt, W, H, shadow ? c->TS_shadow : c->TS, fits, no_nan);
@@ -1635,17 +1640,19 @@ static int flush_pass(fgl_ctx *c)
     if (dd.size() != c->last_draws.size() ||
         std::memcmp(dd.data(), c->last_draws.data(), dd.size() * sizeof(DevDraw)) != 0) {
         // the records, then their bases by themselves (DirectArgs::bases)
-        std::vector<int> bases(2 * dd.size());
-        for (size_t i = 0; i < dd.size(); ++i) {
+        KernelTimer t(c, "draw_table");
+        const size_t n = dd.size(), records = n * sizeof(DevDraw);
+        std::vector<char> table(records + 4 * n * sizeof(int));
+        std::memcpy(table.data(), dd.data(), records);
+        int *bases = (int *)(table.data() + records);
+        for (size_t i = 0; i < n; ++i) {
             bases[i] = dd[i].vblock_base;
-            bases[dd.size() + i] = dd[i].group_base;
+            for (int k = 0; k < 3; ++k) bases[(1 + k) * n + i] = dd[i].group_base[k];
         }
-        const size_t records = dd.size() * sizeof(DevDraw), table = bases.size() * sizeof(int);
         c->last_draws.clear();   // nothing is known of the table until it is written
-        if ((rc = ensure(c, c->d_draws, records + table))) return rc;
+        if ((rc = ensure(c, c->d_draws, table.size()))) return rc;
         HIPCHK(c, hipStreamSynchronize(c->stream));
-        HIPCHK(c, hipMemcpy(c->d_draws.p, dd.data(), records, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy((char *)c->d_draws.p + records, bases.data(), table, hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_draws.p, table.data(), table.size(), hipMemcpyHostToDevice));
         c->last_draws = dd;
     }
 

@@ -63,7 +63,7 @@ struct DirectArgs {
     int n_draws;
     const int4 *screen;
     unsigned long long *key, *fix;
-    const int *bases;          // the draws' vertex blocks, then triangle groups, before each (single passes)
+    const int *bases;          // the draws' vertex blocks, then triangle groups by lanes_slot, before each (single passes)
     unsigned long long *big_start;
     uint32_t *big_tri;
     unsigned long long deep_from;   // items from which on keys are read first

@@ -56,6 +56,9 @@ constexpr long long deep_items(long long pixels) { return 3 * (pixels / 1024 + 1
 // Triangles of a pass that the direct rasteriser's claims count.
 constexpr long long kDirectTrisMost = (1LL << 30) - 1;
 
+// Their place among 1, 4 and 16.
+constexpr int lanes_slot(int lanes) { return lanes == 16 ? 2 : lanes == 4 ? 1 : 0; }
+
 // Workgroups of a draw: 256 / lanes triangles each; 256 vertices each.
 constexpr long long direct_groups(int n_faces, int lanes) { return ((long long)n_faces * lanes + 255) / 256; }
 constexpr long long vertex_blocks(int n_pos) { return ((long long)n_pos + 255) / 256; }

@@ -237,8 +237,9 @@ __global__ __launch_bounds__(256) void k_direct(DirectArgs a)
 {
     __shared__ DirectLds lds;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    const DevDraw &dr = a.draws[owner_of(a.bases + a.n_draws, (uint32_t)a.n_draws, b)];
-    direct_group<G>(a, dr, (b - dr.group_base) * (256 / G), lds);
+    constexpr int kSlot = lanes_slot(G);
+    const DevDraw &dr = a.draws[owner_of(a.bases + (size_t)(1 + kSlot) * a.n_draws, (uint32_t)a.n_draws, b)];
+    direct_group<G>(a, dr, (b - dr.group_base[kSlot]) * (256 / G), lds);
 }
 
 // The large triangles' items.

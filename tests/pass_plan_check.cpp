@@ -42,6 +42,7 @@ int main()
     CHECK(direct_lanes(1 << 20, 1000, 72000, true) == 16 && direct_lanes(1 << 20, 1000, 71998, true) == 4);
     CHECK(direct_lanes(1 << 20, 0, 1, false) == 16);   // a draw of none: no groups whatever its lanes
     CHECK(direct_lanes(0x7fffffff, 0x7fffffff, 1LL << 34, false) == 4);
+    CHECK(lanes_slot(1) == 0 && lanes_slot(4) == 1 && lanes_slot(16) == 2);
     // every face of the largest pass, 16 lanes each, does not fit
     CHECK(!launch_fits(direct_groups(0x7fffffff, 16)) && launch_fits(direct_groups(0x7fffffff, 1)));
     // 64 shadow maps of 8192 x 8192 in 64 x 4 blocks do not, 63 do

@@ -220,3 +220,36 @@ def test_draws_in_front_of_the_camera_are_bounded_by_their_box(ctx):
         took.append(best)
     print("2,000 draws, seconds:", took, flush=True)
     assert took[0] < 1.5 * took[1], took
+
+
+def test_passes_of_a_frame_share_their_draw_table(ctx):
+    """The draw table is written when the draws change, not when a pass takes
+    another number of lanes per triangle than the one before (each write waits
+    for the stream): 40,000 triangles, a shadow map of 64 x 64 (one lane) and a
+    view of 640 x 400 (four)."""
+    rng = np.random.default_rng(11)
+    mat = _material(ctx)
+    a, b = (_model(ctx, mat, _triangles(rng, 20000, 0.02)) for _ in range(2))
+    ctx.set_shadow(False)
+    for which in (F.MAT_PROJ, F.MAT_VIEW, F.MAT_LIGHT_SPACE):
+        ctx.set_matrix(which, np.ascontiguousarray(EYE4))
+    ctx.set_viewport(0, 0, 640, 400)
+    ctx.set_viewport(0, 0, 64, 64, shadow=True)
+    writes = []
+    for order in ((a, b), (a, b), (b, a), (b, a)):
+        ctx.sync()
+        ctx.read_timings()
+        ctx.enable_timing(True)
+        ctx.init_shadow_buffer(64, 64)
+        ctx.init_targets(640, 400)
+        for which in (F.PASS_SHADOW, F.PASS_GEOMETRY):
+            ctx.begin_pass(which)
+            for m in order:
+                ctx.draw_model(m, EYE4)
+            ctx.end_pass()
+        ctx.sync()
+        names = [n for n, _ in ctx.read_timings()]
+        ctx.enable_timing(False)
+        assert "raster_shadow" in names and "raster" in names and "setup" not in names, names
+        writes.append(names.count("draw_table"))
+    assert writes == [1, 0, 1, 0], writes
