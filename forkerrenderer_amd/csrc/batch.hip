@@ -195,7 +195,6 @@ __device__ __forceinline__ DirectArgs bv_direct_args(const BvDirectArgs &b, cons
     a.screen = b.screen;
     a.key = b.key + (PASS == kBvShadow ? v.spx_off : v.px_off);
     a.fix = nullptr;
-    a.bases = nullptr;
     a.deep_from = b.deep_from;
     a.big_start = b.big_start;
     a.big_tri = b.big_tri;

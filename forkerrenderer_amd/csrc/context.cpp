@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <climits>
 #include <cstddef>
 #include <cmath>
 #include <cstdio>
@@ -1368,11 +1369,12 @@ static void bound_pass(const fgl_ctx *c, bool shadow, long long nt, int W, int H
 }
 
 // The direct rasteriser's launches of a pass: the draws' triangle groups and
-// vertex blocks (their bases in the draw records).
+// vertex blocks, and where each draw's begin.
 struct DirectGrid {
     int lanes;
     long long groups, vblocks;
     bool corner;   // varyings from the corner records (corner_form)
+    DrawStarts group_starts, vblock_starts;
 };
 
 static void free_direct(fgl_ctx *c)
@@ -1415,7 +1417,6 @@ static void direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const D
     a.screen = (const int4 *)c->screen.p;
     a.key = (unsigned long long *)c->key.p;
     a.fix = no_nan ? nullptr : (unsigned long long *)c->key_nan.p;
-    a.bases = (const int *)(a.draws + n_draws);
     a.deep_from = (unsigned long long)deep_items((long long)px);
     a.big_start = (unsigned long long *)c->big.p;
     a.big_tri = (uint32_t *)(a.big_start + nt);
@@ -1427,10 +1428,10 @@ static void direct_pass(fgl_ctx *c, const FrameUniforms &u, int n_draws, const D
         KernelTimer t(c, "vertex");
         launch_direct_vertex(shadow, (int)g.vblocks, u, (int4 *)c->screen.p,
                              shadow ? (float *)c->ndc_z.p : nullptr, g.corner || shadow ? nullptr : (float4 *)c->vary.p, a,
-                             ctr + c->direct_turn, c->stream);
+                             g.vblock_starts, ctr + c->direct_turn, c->stream);
     }
     KernelTimer t(c, shadow ? "raster_shadow" : "raster");
-    launch_direct(a, g.lanes, (int)g.groups, nt, c->stream);
+    launch_direct(a, g.group_starts, g.lanes, (int)g.groups, nt, c->stream);
     if (shadow)
         launch_direct_shadow(a, (const float *)c->ndc_z.p, (float *)c->shadow_depth.p, (float *)c->shadow.p, c->stream);
 }
@@ -1595,8 +1596,9 @@ static int flush_pass(fgl_ctx *c)
     long long nt = 0, nv = 0, tris = 0;
     int max_pos = 0, max_faces = 0;
     for (const fgl_ctx::Rec &r : c->draws) tris += c->models[r.model].n_faces;
-    long long groups[3] = {0, 0, 0};
-    DirectGrid grid = {direct_lanes(tris, tris, (long long)W * H, shadow), 0, 0, corner_form((long long)W * H, tris)};
+    DirectGrid grid = {direct_lanes(tris, tris, (long long)W * H, shadow), 0, 0, corner_form((long long)W * H, tris),
+                       {}, {}};
+    for (int k = 1; k < kFewDraws; ++k) grid.group_starts.few[k] = grid.vblock_starts.few[k] = INT_MAX;
     for (size_t i = 0; i < c->draws.size(); ++i) {
         const ModelRes &m = c->models[c->draws[i].model];
         DevDraw &d = dd[i];
@@ -1604,19 +1606,17 @@ static int flush_pass(fgl_ctx *c)
         if (c->draws[i].has_normal) std::memcpy(d.normal, c->draws[i].n, sizeof(d.normal));
         d.vert_base = (int)nv;
         d.tri_base = (int)nt;
-        d.vblock_base = (int)grid.vblocks;
-        grid.vblocks += vertex_blocks(d.n_pos);
-        for (int lanes : {1, 4, 16}) {
-            long long &n = groups[lanes_slot(lanes)];
-            d.group_base[lanes_slot(lanes)] = (int)n;
-            n += direct_groups(d.n_faces, lanes);
+        if (i < kFewDraws) {
+            grid.vblock_starts.few[i] = (int)grid.vblocks;
+            grid.group_starts.few[i] = (int)grid.groups;
         }
+        grid.vblocks += vertex_blocks(d.n_pos);
+        grid.groups += direct_groups(d.n_faces, grid.lanes);
         nt += m.n_faces;
         nv += m.n_pos;
         max_pos = m.n_pos > max_pos ? m.n_pos : max_pos;
         max_faces = m.n_faces > max_faces ? m.n_faces : max_faces;
     }
-    grid.groups = groups[lanes_slot(grid.lanes)];
     const int n_draws = (int)c->draws.size();
     bool fits, no_nan;
     bound_pass(c, shadow, nt, W, H, shadow ? c->TS_shadow : c->TS, fits, no_nan);
@@ -1639,15 +1639,19 @@ static int flush_pass(fgl_ctx *c)
 
     if (dd.size() != c->last_draws.size() ||
         std::memcmp(dd.data(), c->last_draws.data(), dd.size() * sizeof(DevDraw)) != 0) {
-        // the records, then their bases by themselves (DirectArgs::bases)
+        // The records, then where each draw's workgroups begin (DrawStarts): the
+        // vertex pass's, the triangle groups' at 1, 4 and 16 lanes.  Nothing of it
+        // is one pass's own: the shadow pass's table serves the main pass.
         KernelTimer t(c, "draw_table");
         const size_t n = dd.size(), records = n * sizeof(DevDraw);
         std::vector<char> table(records + 4 * n * sizeof(int));
         std::memcpy(table.data(), dd.data(), records);
-        int *bases = (int *)(table.data() + records);
+        int *starts = (int *)(table.data() + records);
+        long long at[4] = {0, 0, 0, 0};
         for (size_t i = 0; i < n; ++i) {
-            bases[i] = dd[i].vblock_base;
-            for (int k = 0; k < 3; ++k) bases[(1 + k) * n + i] = dd[i].group_base[k];
+            for (int k = 0; k < 4; ++k) starts[k * n + i] = (int)at[k];
+            at[0] += vertex_blocks(dd[i].n_pos);
+            for (int lanes : {1, 4, 16}) at[1 + lanes_slot(lanes)] += direct_groups(dd[i].n_faces, lanes);
         }
         c->last_draws.clear();   // nothing is known of the table until it is written
         if ((rc = ensure(c, c->d_draws, table.size()))) return rc;
@@ -1662,6 +1666,8 @@ static int flush_pass(fgl_ctx *c)
     // that goes on from earlier depths, or replays the fragment sequence, takes
     // the tile lists.
     const DevDraw *ddraws = (const DevDraw *)c->d_draws.p;
+    grid.vblock_starts.table = (const int *)(ddraws + n_draws);
+    grid.group_starts.table = grid.vblock_starts.table + (size_t)(1 + lanes_slot(grid.lanes)) * n_draws;
     const size_t px = (size_t)W * H;
     if ((rc = ensure(c, c->screen, (size_t)nv * sizeof(int4))) || (shadow && (rc = ensure(c, c->ndc_z, (size_t)nv * 4))) ||
         (!shadow && (rc = ensure(c, c->vary, (size_t)nv * 2 * sizeof(float4)))))

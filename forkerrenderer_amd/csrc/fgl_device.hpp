@@ -57,10 +57,7 @@ struct DevDraw {
     int n_pos, n_faces, vert_base, tri_base;
     int has_tangents, support_pbr;
     int view;      // batched views: index of the draw's view (0 otherwise)
-    // the direct rasteriser's workgroups before the draw's: of the vertex pass,
-    // of the triangle groups at 1, 4 and 16 lanes (lanes_slot; single passes).
-    // Nothing here is one pass's own: the shadow pass's records serve the main pass
-    int vblock_base, group_base[3];
+    int pad0;
     float model[16];
     float normal[9];
     float lm[16];  // light_space * model (DepthShader, src/shaders/depthshader.h:23-25)

@@ -63,12 +63,21 @@ struct DirectArgs {
     int n_draws;
     const int4 *screen;
     unsigned long long *key, *fix;
-    const int *bases;          // the draws' vertex blocks, then triangle groups by lanes_slot, before each (single passes)
     unsigned long long *big_start;
     uint32_t *big_tri;
     unsigned long long deep_from;   // items from which on keys are read first
     DirectCtr *ctr;
     int W, H;
+};
+
+// Where the draws' workgroups of one launch begin: the table's (ascending, the
+// first 0) and the first of them as kernel arguments, so that a workgroup of a
+// pass of few draws finds its own without a load (485 x 303 view, two objects:
+// 0.3 us of each of its four launches); INT_MAX past the last draw.
+constexpr int kFewDraws = 8;
+struct DrawStarts {
+    const int *table;
+    int few[kFewDraws];
 };
 
 struct ResolveArgs {
@@ -174,8 +183,8 @@ void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s);
 // triangles); launch_direct_shadow: the shadow pass's depth and ShadowBuffer
 // value of every texel from the keys.
 void launch_direct_vertex(bool shadow, int n_blocks, const FrameUniforms &u, int4 *out, float *ndc_z, float4 *vary,
-                          const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s);
-void launch_direct(const DirectArgs &a, int lanes, int n_groups, long long n_tri, hipStream_t s);
+                          const DirectArgs &a, const DrawStarts &starts, DirectCtr *next_ctr, hipStream_t s);
+void launch_direct(const DirectArgs &a, const DrawStarts &starts, int lanes, int n_groups, long long n_tri, hipStream_t s);
 void launch_direct_shadow(const DirectArgs &a, const float *ndc_z, float *depth, float *shadow_out, hipStream_t s);
 void launch_gbuffer_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);
 void launch_forward_resolve(const ResolveArgs &a, const FrameUniforms &u, hipStream_t s);

@@ -197,7 +197,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TS == 32 
 // plane cleared (8 keys a thread) by the workgroups past the vertices', and
 // the counters of the next pass zeroed (this pass's were by the one before).
 template <bool SHADOW>
-__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, const int *__restrict__ bases,
+__global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict__ draws, DrawStarts starts,
                                                        int n_draws, int n_vert_blocks,
                                                        FrameUniforms u, int4 *__restrict__ out,
                                                        float *__restrict__ ndc_z, float4 *__restrict__ vary,
@@ -218,8 +218,9 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
         }
         return;
     }
-    const DevDraw &dr = draws[owner_of(bases, (uint32_t)n_draws, b)];
-    const int vi = (b - dr.vblock_base) * 256 + threadIdx.x;
+    int before;
+    const DevDraw &dr = draws[draw_of_group(starts, n_draws, b, before)];
+    const int vi = (b - before) * 256 + threadIdx.x;
     if (vi >= dr.n_pos) return;
     if (SHADOW) {
         const Vec4 n = depth_ndc(dr, vi);
@@ -233,13 +234,13 @@ __global__ __launch_bounds__(256) void k_direct_vertex(const DevDraw *__restrict
 // G lanes per triangle (direct_lanes, pass_plan.hpp).  Workgroups are dealt to
 // the XCDs in runs: neighbouring triangles share vertices and pixels.
 template <int G>
-__global__ __launch_bounds__(256) void k_direct(DirectArgs a)
+__global__ __launch_bounds__(256) void k_direct(DirectArgs a, DrawStarts starts)
 {
     __shared__ DirectLds lds;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
-    constexpr int kSlot = lanes_slot(G);
-    const DevDraw &dr = a.draws[owner_of(a.bases + (size_t)(1 + kSlot) * a.n_draws, (uint32_t)a.n_draws, b)];
-    direct_group<G>(a, dr, (b - dr.group_base[kSlot]) * (256 / G), lds);
+    int before;
+    const DevDraw &dr = a.draws[draw_of_group(starts, a.n_draws, b, before)];
+    direct_group<G>(a, dr, (b - before) * (256 / G), lds);
 }
 
 // The large triangles' items.
@@ -613,23 +614,23 @@ void launch_raster(bool shadow, int TS, const RasterArgs &a, hipStream_t s)
 }
 
 void launch_direct_vertex(bool shadow, int n_blocks, const FrameUniforms &u, int4 *out, float *ndc_z, float4 *vary,
-                          const DirectArgs &a, DirectCtr *next_ctr, hipStream_t s)
+                          const DirectArgs &a, const DrawStarts &starts, DirectCtr *next_ctr, hipStream_t s)
 {
     const size_t P = (size_t)a.W * a.H;
     const unsigned grid = (unsigned)(n_blocks + clear_blocks((long long)P));
     if (shadow)
-        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, a.draws, a.bases, a.n_draws, n_blocks, u, out,
+        hipLaunchKernelGGL(k_direct_vertex<true>, dim3(grid), dim3(256), 0, s, a.draws, starts, a.n_draws, n_blocks, u, out,
                            ndc_z, vary, a.key, P, next_ctr);
     else
-        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, a.draws, a.bases, a.n_draws, n_blocks, u, out,
+        hipLaunchKernelGGL(k_direct_vertex<false>, dim3(grid), dim3(256), 0, s, a.draws, starts, a.n_draws, n_blocks, u, out,
                            ndc_z, vary, a.key, P, next_ctr);
 }
 
-void launch_direct(const DirectArgs &a, int lanes, int n_groups, long long n_tri, hipStream_t s)
+void launch_direct(const DirectArgs &a, const DrawStarts &starts, int lanes, int n_groups, long long n_tri, hipStream_t s)
 {
     const dim3 grid((unsigned)n_groups);
     auto go = [&](auto groups, auto nan) {
-        hipLaunchKernelGGL(groups, grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL(groups, grid, dim3(256), 0, s, a, starts);
         hipLaunchKernelGGL(k_direct_big, dim3(1024), dim3(256), 0, s, a);
         if (a.fix) hipLaunchKernelGGL(nan, dim3(1024), dim3(256), 0, s, a, (uint32_t)n_tri);
     };

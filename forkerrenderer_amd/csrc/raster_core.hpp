@@ -459,6 +459,25 @@ __device__ __forceinline__ uint32_t owner_of(const T *start, uint32_t n, T i)
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
+// The draw of workgroup b and the workgroups before the draw's.
+__device__ __forceinline__ int draw_of_group(const DrawStarts &s, int n_draws, int b, int &before)
+{
+    if (n_draws > kFewDraws) {
+        const int d = (int)owner_of(s.table, (uint32_t)n_draws, b);
+        before = s.table[d];
+        return d;
+    }
+    int d = 0;
+    before = 0;
+#pragma unroll
+    for (int k = 1; k < kFewDraws; ++k)
+        if (s.few[k] <= b) {
+            d = k;
+            before = s.few[k];
+        }
+    return d;
+}
+
 // The draw of pass-wide triangle g (their tri_base ascend).
 __device__ __forceinline__ int draw_of(const DevDraw *draws, int n_draws, int g)
 {

@@ -168,6 +168,19 @@ def test_many_small_draws_beside_a_large_one(ctx, shadow):
     _direct_against_lists(ctx, mat, draws, 320, 200, shadow, "many draws")
 
 
+@pytest.mark.parametrize("n", [2, 7, 8, 9, 10])
+@pytest.mark.parametrize("shadow", [False, True])
+def test_few_draws(ctx, n, shadow):
+    """Around eight draws, up to which a workgroup finds its draw in the kernel's
+    arguments: draws of none first, in the middle and last."""
+    rng = np.random.default_rng(n)
+    mat = _material(ctx)
+    none = _model_without_faces(ctx)
+    models = [none if k in (0, n // 2, n - 1) and n > 2 else _model(ctx, mat, _triangles(rng, 40 + 700 * (k % 3), 0.1))
+              for k in range(n)]
+    _direct_against_lists(ctx, mat, [(m, EYE4) for m in models], 250, 130, shadow, f"{n} draws")
+
+
 def _model_without_faces(ctx):
     f = np.zeros((0, 3), np.int32)
     return ctx.upload_model({"pos": np.ones((300, 3), np.float32), "uv": np.zeros((1, 2), np.float32),
